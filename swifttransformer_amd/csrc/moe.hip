@@ -4,7 +4,7 @@
 // Everything stays on the device and has a fixed launch shape, so a step can be recorded:
 //   route    per token the `top` best experts and their weights (five rules, see st_moe_route);
 //   align    the (token, choice) pairs sorted by expert into tiles of 16, 64 or 128 places, a tile
-//            holding pairs of one expert only (places left over are marked -1);
+//            holding pairs of one expert only, an expert's tiles neighbours (places left over are marked -1);
 //   up       per tile and 64 inner features: both input products on the matrix cores, rows
 //            gathered through the sorted list, then clamp, gate and product of the two halves (experts
 //            without a gate: one product and the exact GELU);
@@ -480,106 +480,151 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
         }
 }
 
-// ---- prompts in bfloat16: tiles of 128 places, operands staged through LDS ----------------------
-// With a hundred rows and more an expert the products are bound by arithmetic, not by the weights'
-// stream, and operands read straight from memory leave the matrix cores waiting.  Here a workgroup
-// computes 128 places x 128 weight rows in steps of 64 in depth: all threads bring the two operand
-// tiles into registers with 16-byte loads (the next step's while this one is multiplied), store
-// them into LDS with the rows' chunks rotated so that the matrix instruction's reads spread over
-// the banks, and every wave multiplies a 64 x 64 part (v_mfma_f32_32x32x16_bf16).
-// UP: the 128 weight rows are 64 inner features of the gate matrix and the same 64 of the other
-// one, dealt so that a lane holds both halves of a result; rows of x are gathered through the
-// sorted list.  Otherwise: 128 output features of the expert's output matrix over the rows of y.
+// ---- prompts in bfloat16: tiles of 64 or 128 places, operands by direct loads into LDS -----------
+// With some dozens of rows and more an expert a tile of 64 NJ places meets 128 rows of its expert's matrix, steps of 64 in depth.
+// Both operand tiles go from memory into LDS without passing through registers (16 bytes a lane; a row's chunks are rotated by
+// the lane's choice of address, so that the matrix instruction's reads spread over the banks), the next step's into the other of
+// two buffers while this one is multiplied: one barrier a step.  Each of four waves multiplies a 64 x 32 NJ part
+// (v_mfma_f32_32x32x16_bf16), the operands of a product of depth 16 read ahead of the one before.
+// UP: of every 64 weight rows 32 are inner features of the gate matrix and 32 the same features of the other one, so that a
+// lane holds both halves of a result; rows of x are gathered through the sorted list.  GELU: the one input matrix of experts
+// without a gate.  Otherwise: output features of the expert's output matrix over the rows of y.
+//
+// What bounds it: the path from L2 into LDS (about 19 bytes a cycle and unit; the weights' own stream from memory is the floor
+// below it, all experts' matrices whatever the rows).  Workgroups go round the eight dies by their number; here each die takes
+// an eighth of the work in the order (expert, weight rows, tile of that expert), so that an expert's matrix passes through one
+// die's L2 once, its tiles next to each other, and a die gets the same number of tiles as any other, however the tokens chose.
+// Measured beside the kernels before it (operands through registers into LDS for 128 places, straight from memory for 64), 16
+// experts of 2,048 x 2,048, two a token, up + down: 2,011 tokens 299 -> 201 us, 1,024 tokens 257 -> 135, 512 tokens (tiles of 64)
+// 319 -> 122, 256 tokens 223 -> 100 us; 14 experts of 4,096 x 4,096 at 2,048 tokens 1,034 -> 660 us.  Tried and no better: 256
+// weight rows a workgroup (four waves of 128 x 64, or eight waves), steps of 32 in depth in three to five buffers.
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-__device__ inline int rot(int row, int chunk) { return row * 8 + (chunk ^ ((row >> 1) & 7)); }
+#define ST_LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
+#define ST_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void*)(p))
+// a row's chunk of 8 in depth lies at chunk ^ swizzle(row): 16 neighbouring rows' like chunks lie in different banks
+__device__ inline int swizzle(int row) { return (row >> 1) & 7; }
 
-// GELU: as UP, but the 128 weight rows are 128 inner features of the one input matrix of experts without a gate.
-enum TiledKind : int { kTiledDown = 0, kTiledUp = 1, kTiledGelu = 2 };
-template <int KIND>
-__global__ __launch_bounds__(256) void moe_tiled_kernel(
-    bf16_t* __restrict__ y_out, float* __restrict__ out, const float* __restrict__ residual,
-    float* __restrict__ pair_out, const bf16_t* __restrict__ a_rows, const bf16_t* __restrict__ w0,
-    const bf16_t* __restrict__ w1, const int* __restrict__ sorted, const int* __restrict__ tile_expert,
-    const float* __restrict__ weights, int top, int N, int K, float limit, float out_scale, int style) {
-    constexpr bool UP = KIND == kTiledUp, GATHER = KIND != kTiledDown;
-    __shared__ uint4 sw[128 * 8];      // weight rows: [row][chunk of 8 in depth]
-    __shared__ uint4 sx[128 * 8];      // places
-    const int tile = blockIdx.x;
-    const int e = tile_expert[tile];
-    if (e < 0) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wn = wave & 1, wm = wave >> 1, l32 = lane & 31, lh = lane >> 5;
-    const int base = tile * 128;
-    const int n0 = blockIdx.y * (UP ? 64 : 128);
-    // the four rows of each tile that this thread brings in, fixed over the steps
-    const bf16_t* wrow[4];
-    const bf16_t* xrow[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = (tid + i * 256) >> 3;
-        int n;
-        const bf16_t* m;
-        if (UP) { n = n0 + (row >> 6) * 32 + (row & 31); m = ((row >> 5) & 1) ? w1 : w0; }
-        else { n = n0 + row; m = w0; }
-        wrow[i] = n < N ? m + ((int64_t)e * N + n) * K : nullptr;
-        const int p = sorted[base + row];
-        xrow[i] = GATHER ? (p >= 0 ? a_rows + (int64_t)(p / top) * K : nullptr) : a_rows + (int64_t)(base + row) * K;
+// the tile and the block of weight rows of a workgroup; false where there is none left
+__device__ inline bool moe_work_item(int& tile, int& block, int& expert, const int* __restrict__ tile_expert, int max_tiles, int blocks) {
+    const int lane = threadIdx.x & 63;
+    int tiles = 0;
+    for (int b = 0; b < max_tiles; b += 64)
+        tiles += __popcll(__ballot(b + lane < max_tiles && tile_expert[min(b + lane, max_tiles - 1)] >= 0));
+    const int items = tiles * blocks, share = (items + 7) / 8;       // (the host checks that the numbers fit)
+    const int j = blockIdx.x >> 3, i = (blockIdx.x & 7) * share + j;
+    if (j >= share || i >= items) return false;
+    expert = tile_expert[i / blocks];                                // (an expert's tiles are neighbours)
+    int before = 0, own = 0;
+    for (int b = 0; b < max_tiles; b += 64) {
+        const int v = tile_expert[min(b + lane, max_tiles - 1)];
+        const bool in = b + lane < max_tiles && v >= 0;
+        before += __popcll(__ballot(in && v < expert));
+        own += __popcll(__ballot(in && v == expert));
     }
-    floatx16 acc[2][2];
+    const int r = i - before * blocks;
+    block = r / own;
+    tile = before + (r - block * own);
+    return true;
+}
+
+enum TiledKind : int { kTiledDown = 0, kTiledUp = 1, kTiledGelu = 2 };
+template <int KIND, int NJ>
+__global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
+    bf16_t* __restrict__ y_out, float* out, const float* residual, float* __restrict__ pair_out, const bf16_t* __restrict__ a_rows,
+    const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, const int* __restrict__ sorted, const int* __restrict__ tile_expert,
+    const float* __restrict__ weights, int max_tiles, int blocks, int top, int N, int K, float limit, float out_scale, int style) {
+    constexpr bool UP = KIND == kTiledUp, GATHER = KIND != kTiledDown;
+    constexpr int PLACES = 64 * NJ;
+    constexpr int BUF = (128 + PLACES) * 8;        // 16-byte pieces a buffer: weight rows, then places
+    constexpr int NL = (128 + PLACES) / 32;        // direct loads a wave and step, eight rows each
+    __shared__ uint4 lds[2 * BUF];
+    int tile, block, e;
+    if (!moe_work_item(tile, block, e, tile_expert, max_tiles, blocks)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave & 1, wm = wave >> 1, l32 = lane & 31, lh = lane >> 5;
+    const int base = tile * PLACES, n0 = block * (UP ? 64 : 128);
+    // Load t of a wave brings rows 8 (wave + 4 t) on, a lane 16 bytes of row + lane / 8: piece lane % 8 of the row's place in
+    // LDS, which is the chunk that the row's swizzle puts there, the same for all t.  Rows past the matrix and places without a
+    // pair stand for row 0: their results are not stored, or stored as zeros.
+    const int chunk = (lane & 7) ^ swizzle(8 * wave + (lane >> 3));
+    const bf16_t* src[NL];
+#pragma unroll
+    for (int t = 0; t < NL; ++t) {
+        const int row = 8 * (wave + 4 * t) + (lane >> 3);
+        if (t < 4) {
+            const int n = UP ? n0 + (row >> 6) * 32 + (row & 31) : n0 + row;
+            const bf16_t* m = UP && ((row >> 5) & 1) ? w1 : w0;
+            src[t] = m + ((int64_t)e * N + (n < N ? n : 0)) * K;
+        } else {
+            const int place = base + row - 128, p = sorted[place];
+            src[t] = GATHER ? a_rows + (int64_t)(p >= 0 ? p / top : 0) * K : a_rows + (int64_t)place * K;
+        }
+        src[t] += chunk * 8;
+    }
+    const int whole = K >> 6, steps = (K + 63) >> 6;
+    auto stage = [&](int s) {
+        uint4* dst = lds + (s & 1) * BUF + wave * 64;
+        if (s < whole) {
+#pragma unroll
+            for (int t = 0; t < NL; ++t)
+                __builtin_amdgcn_global_load_lds(ST_GLOBAL_PTR(src[t] + s * 64), ST_LDS_PTR(void, dst + t * 256), 16, 0, 0);
+        } else {                                   // the last, shorter step: zeros past the depth
+            const bool in = s * 64 + chunk * 8 < K;
+#pragma unroll
+            for (int t = 0; t < NL; ++t) {
+                const uint4 v = *reinterpret_cast<const uint4*>(src[t] + (in ? s * 64 : -chunk * 8));
+                dst[t * 256 + lane] = in ? v : make_uint4(0, 0, 0, 0);
+            }
+        }
+    };
+    floatx16 acc[2][NJ];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-    uint4 rw[4], rx[4];
-    auto load_global = [&](int k0) {
-        const int k = k0 + (tid & 7) * 8;
-        const bool in = k < K;
+    // (the swizzle of a lane's rows is that of l32: the rows before it are a multiple of 32)
+    const uint4* own = lds + l32 * 8;
+    const int swz = swizzle(l32);
+    bf16x8 a[2][2], b[2][NJ];
+    auto fetch = [&](int buf, int kk) {            // the operands of a product of depth 16
+        const uint4* at = own + buf * BUF + ((kk * 2 + lh) ^ swz);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            // (addresses clamped and values cleared rather than loads behind a branch)
-            const bf16_t* pw = wrow[i] ? wrow[i] : w0;
-            const bf16_t* px = xrow[i] ? xrow[i] : a_rows;
-            const uint4 vw = *reinterpret_cast<const uint4*>(pw + (in ? k : 0));
-            const uint4 vx = *reinterpret_cast<const uint4*>(px + (in ? k : 0));
-            rw[i] = (in && wrow[i]) ? vw : make_uint4(0, 0, 0, 0);
-            rx[i] = (in && xrow[i]) ? vx : make_uint4(0, 0, 0, 0);
-        }
+        for (int i = 0; i < 2; ++i) a[kk & 1][i] = __builtin_bit_cast(bf16x8, at[(wn * 64 + i * 32) * 8]);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) b[kk & 1][j] = __builtin_bit_cast(bf16x8, at[(128 + (wm * NJ + j) * 32) * 8]);
     };
-    load_global(0);
-    for (int k0 = 0; k0 < K; k0 += 64) {
-        __syncthreads();               // the step before has been read
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + i * 256;
-            sw[rot(c >> 3, c & 7)] = rw[i];
-            sx[rot(c >> 3, c & 7)] = rx[i];
-        }
-        __syncthreads();
-        if (k0 + 64 < K) load_global(k0 + 64);
+    stage(0);
+    for (int s = 0; s < steps; ++s) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's loads of this step have landed
+        __syncthreads();                                             // everyone's have, and the other buffer has been read
+        fetch(s & 1, 0);
+        if (s + 1 < steps) stage(s + 1);
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
-            const int chunk = kk * 2 + lh;
-            bf16x8 a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = __builtin_bit_cast(bf16x8, sw[rot(wn * 64 + i * 32 + l32, chunk)]);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = __builtin_bit_cast(bf16x8, sx[rot(wm * 64 + j * 32 + l32, chunk)]);
+            if (kk < 3) fetch(s & 1, kk + 1);
+            __builtin_amdgcn_sched_barrier(0);     // (the next operands are on their way before these are multiplied)
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kk & 1][i], b[kk & 1][j], acc[i][j], 0, 0, 0);
         }
     }
-    // acc[i][j][q]: weight row wn*64 + i*32 + 8*(q/4) + 4*lh + q%4, place base + wm*64 + j*32 + l32
+    // acc[i][j][q]: weight row wn * 64 + i * 32 + 8 * (q / 4) + 4 * lh + q % 4, place base + (wm * NJ + j) * 32 + l32
+    auto store_row = [&](int place, int f, const float* r) {
+        bf16_t* dst = y_out + (int64_t)place * N + f;
+        if (f + 3 < N && (N & 3) == 0) Elem<bf16_t>::store4(dst, r);
+        else
+            for (int u = 0; u < 4 && f + u < N; ++u) Elem<bf16_t>::store(dst + u, r[u]);
+    };
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int place = base + wm * 64 + j * 32 + l32;
+    for (int j = 0; j < NJ; ++j) {
+        const int place = base + (wm * NJ + j) * 32 + l32;
         const int p = sorted[place];
         if (UP) {
-            const float s = p >= 0 && style == 0 ? weights[p] : 1.f;
+            const float scale = p >= 0 && style == 0 ? weights[p] : 1.f;
 #pragma unroll
             for (int q4 = 0; q4 < 4; ++q4) {
                 const int f = n0 + wn * 32 + 8 * q4 + 4 * lh;
@@ -592,14 +637,11 @@ __global__ __launch_bounds__(256) void moe_tiled_kernel(
                         r[u] = p >= 0 ? gv / (1.f + expf(-gv)) * acc[1][j][4 * q4 + u] : 0.f;
                         continue;
                     }
-                    const float gv = fminf(s * acc[0][j][4 * q4 + u], limit);
-                    const float uv = fminf(fmaxf(s * acc[1][j][4 * q4 + u], -limit), limit);
+                    const float gv = fminf(scale * acc[0][j][4 * q4 + u], limit);
+                    const float uv = fminf(fmaxf(scale * acc[1][j][4 * q4 + u], -limit), limit);
                     r[u] = p >= 0 ? gv / (1.f + expf(-1.702f * gv)) * (uv + 1.f) : 0.f;
                 }
-                bf16_t* dst = y_out + (int64_t)place * N + f;
-                if (f + 3 < N && (N & 3) == 0) Elem<bf16_t>::store4(dst, r);
-                else
-                    for (int u = 0; u < 4 && f + u < N; ++u) Elem<bf16_t>::store(dst + u, r[u]);
+                store_row(place, f, r);
             }
         } else if (KIND == kTiledGelu) {
 #pragma unroll
@@ -611,10 +653,7 @@ __global__ __launch_bounds__(256) void moe_tiled_kernel(
                     float r[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) r[u] = p >= 0 ? apply_activation(kActGeluErf, acc[i][j][4 * q4 + u]) : 0.f;
-                    bf16_t* dst = y_out + (int64_t)place * N + f;
-                    if (f + 3 < N && (N & 3) == 0) Elem<bf16_t>::store4(dst, r);
-                    else
-                        for (int u = 0; u < 4 && f + u < N; ++u) Elem<bf16_t>::store(dst + u, r[u]);
+                    store_row(place, f, r);
                 }
         } else {
             if (p < 0) continue;
@@ -623,6 +662,11 @@ __global__ __launch_bounds__(256) void moe_tiled_kernel(
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) {
                     const int n = n0 + wn * 64 + i * 32 + 8 * q4 + 4 * lh;
+                    if (pair_out && (N & 3) == 0 && n + 3 < N) {
+                        *reinterpret_cast<float4*>(pair_out + (int64_t)place * N + n) = make_float4(
+                            acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
+                        continue;
+                    }
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
                         if (n + u >= N) continue;
@@ -636,6 +680,23 @@ __global__ __launch_bounds__(256) void moe_tiled_kernel(
                 }
         }
     }
+}
+
+template <int KIND>
+static int launch_tiled(bf16_t* y, float* out, const float* residual, float* pair_out, const void* a_rows, const void* w0,
+                        const void* w1, const int* sorted, const int* tile_expert, const float* weights, int capacity, int tile, int top,
+                        int N, int K, float limit, float out_scale, int style, hipStream_t stream) {
+    const int features = KIND == kTiledUp ? 64 : 128, tiles = capacity / tile, blocks = (N + features - 1) / features;
+    ST_CHECK((int64_t)tiles * blocks < (1ll << 30), "moe: too many tiles");
+    const unsigned grid = (unsigned)((tiles * blocks + 7) / 8 * 8);
+    if (tile == 64)
+        moe_tiled_kernel<KIND, 1><<<grid, 256, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
+            (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
+    else
+        moe_tiled_kernel<KIND, 2><<<grid, 256, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
+            (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
+    ST_LAUNCH_CHECK("moe (tiled)");
+    return 0;
 }
 
 // V columns a thread and turn (4: 16-byte accesses).  x (or null): the tokens' own vectors, the results of the identity
@@ -755,18 +816,12 @@ extern "C" int st_moe_up(void* y, const void* x, const void* w_gate, const void*
     const dim3 grid(capacity / kTile, (inner + 63) / 64);
     ST_CHECK(grid.y <= 65535, "moe_up: too many inner features");
     const int vec = rows_vectorised(x, w_gate, w_up, width, dtype);
-    if (dtype == kBF16 && tile == 128 && vec) {
-        if (style == 2) {
-            moe_tiled_kernel<kTiledGelu><<<dim3(capacity / 128, (inner + 127) / 128), 256, 0, stream>>>((bf16_t*)y, nullptr, nullptr,
-                nullptr, (const bf16_t*)x, (const bf16_t*)w_up, nullptr, sorted, tile_expert, weights, top, inner, width, limit, 1.f, style);
-            ST_LAUNCH_CHECK("moe_up (tiled, no gate)");
-            return 0;
-        }
-        const dim3 g2(capacity / 128, (inner + 63) / 64);
-        moe_tiled_kernel<kTiledUp><<<g2, 256, 0, stream>>>((bf16_t*)y, nullptr, nullptr, nullptr, (const bf16_t*)x,
-            (const bf16_t*)w_gate, (const bf16_t*)w_up, sorted, tile_expert, weights, top, inner, width, limit, 1.f, style);
-        ST_LAUNCH_CHECK("moe_up (tiled)");
-        return 0;
+    if (dtype == kBF16 && tile >= 64 && vec) {
+        if (style == 2)
+            return launch_tiled<kTiledGelu>((bf16_t*)y, nullptr, nullptr, nullptr, x, w_up, nullptr, sorted, tile_expert, weights,
+                                            capacity, tile, top, inner, width, limit, 1.f, style, stream);
+        return launch_tiled<kTiledUp>((bf16_t*)y, nullptr, nullptr, nullptr, x, w_gate, w_up, sorted, tile_expert, weights,
+                                      capacity, tile, top, inner, width, limit, 1.f, style, stream);
     }
 #define ST_UP_G(T, RT, G)                                                                                    \
     moe_up_kernel<T, RT, G><<<grid, 256, 0, stream>>>((T*)y, (const T*)x, (const T*)w_gate, (const T*)w_up, sorted, \
@@ -806,13 +861,9 @@ extern "C" int st_moe_down(float* out, const float* residual, float* pair_out, c
     const dim3 grid(capacity / kTile, (width + 63) / 64);
     ST_CHECK(grid.y <= 65535, "moe_down: too wide");
     const int vec = rows_vectorised(y, w_down, w_down, inner, dtype);
-    if (dtype == kBF16 && tile == 128 && vec) {
-        const dim3 g2(capacity / 128, (width + 127) / 128);
-        moe_tiled_kernel<kTiledDown><<<g2, 256, 0, stream>>>(nullptr, out, residual, pair_out, (const bf16_t*)y,
-            (const bf16_t*)w_down, nullptr, sorted, tile_expert, nullptr, top, width, inner, 0.f, out_scale, 0);
-        ST_LAUNCH_CHECK("moe_down (tiled)");
-        return 0;
-    }
+    if (dtype == kBF16 && tile >= 64 && vec)
+        return launch_tiled<kTiledDown>(nullptr, out, residual, pair_out, y, w_down, nullptr, sorted, tile_expert, nullptr, capacity,
+                                        tile, top, width, inner, 0.f, out_scale, 0, stream);
     if (tile == 16) {
         const dim3 few(capacity / 16, (width + 15) / 16);
         ST_CHECK(few.y <= 65535, "moe_down: too wide");

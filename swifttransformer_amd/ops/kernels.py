@@ -1274,11 +1274,16 @@ def latent_write(cache: torch.Tensor, x: torch.Tensor, gain: torch.Tensor, eps: 
 
 
 # ---------------------------------------------------------------- routed experts
-def moe_tile(num_tokens: int, top: int, experts: int) -> int:
-    """Places a tile: 16 for few rows an expert (only the weights' stream counts), 64 or 128 where an
-    expert gets some dozens or a hundred rows on average (a tile's weight operands then meet four or
-    eight blocks of 16 rows, and the expert's weights are read once a tile)."""
+def moe_tile(num_tokens: int, top: int, experts: int, staged: bool = False) -> int:
+    """Places a tile: 16 for few rows an expert (only the weights' stream counts), 64 or 128 for more.
+    ``staged``: bfloat16 rows in whole 16-byte pieces, whose larger tiles go through LDS.  Up + down of 16
+    experts of 2,048 x 2,048, two a token, us with tiles of 16 / 64 / 128 places: 79 / 89 / 93 at 6 pairs an
+    expert, 79 / 72 at 7, 112 / 93 / 98 at 12, 361 / 122 / 135 at 64, 137 / 137 at 112 (64 / 128),
+    144 / 135 at 128.  Otherwise a tile's weight operands come from memory for four or eight blocks of 16
+    rows, which takes some dozens of pairs an expert to pay."""
     pairs = num_tokens * top
+    if staged:
+        return 128 if pairs >= 112 * experts else 64 if pairs >= 7 * experts else 16
     return 128 if pairs >= 96 * experts else 64 if pairs >= 32 * experts else 16
 
 
@@ -1359,7 +1364,7 @@ def routed_experts(x: torch.Tensor, logits: torch.Tensor, w_gate: Optional[torch
     if token_item is not None:
         _need(token_item, "token_item", torch.int32, (T,))
     lib, dev, code, st = _lib(), x.device, dtype_code(x.dtype), _stream()
-    tile = moe_tile(T, top, E)
+    tile = moe_tile(T, top, E, x.dtype == torch.bfloat16 and W % 8 == 0 and F % 8 == 0)
     cap = moe_capacity(T, top, E, tile)
     ids = empty((T * top,), torch.int32, dev)
     wts = empty((T * top,), torch.float32, dev)

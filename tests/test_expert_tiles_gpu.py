@@ -1,0 +1,80 @@
+"""Routed experts in tiles of 64 and 128 places (bfloat16): row counts around a tile, feature counts and depths that leave part of a
+block or of a step, experts without a pair, one expert with all of them, padding rows, every unit and the single-choice sum."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+
+
+def _experts(x, ids, weights, wg, wu, wd, unit, on_input, limit):
+    """float64 sums of a token's experts, and of their absolute values (what the rounding is relative to)."""
+    out, size = torch.zeros(x.shape[0], wd.shape[1], dtype=F64), torch.zeros(x.shape[0], wd.shape[1], dtype=F64)
+    for j in range(ids.shape[1]):
+        for e in ids[:, j].unique().tolist():
+            rows = (ids[:, j] == e).nonzero()[:, 0]
+            s = weights[rows, j][:, None]
+            h = x[rows] * s if on_input else x[rows]
+            u = h @ wu[e].T
+            if unit == "gelu":
+                y = 0.5 * u * (1 + torch.erf(u / 2 ** 0.5))
+            else:
+                g = h @ wg[e].T
+                if unit == "silu":
+                    y = g * torch.sigmoid(g) * u
+                else:
+                    g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+                    y = g * torch.sigmoid(1.702 * g) * (u + 1)
+            y = y if on_input else y * s
+            out[rows] += y @ wd[e].T
+            size[rows] += y.abs() @ wd[e].abs().T
+    return out, size
+
+
+@pytest.mark.parametrize("T,W,F,E,top,style,clamped,same", [
+    (64, 64, 64, 3, 2, "softmax_output", False, False),
+    (65, 136, 72, 5, 2, "scaled_input", False, False),        # depths of 136 and 72: two whole steps and one, and 8 more
+    (127, 8, 200, 4, 1, "scaled_input", False, True),         # a depth below one step; one choice a token: straight into the stream
+    (128, 200, 8, 2, 2, "softmax_output", False, False),
+    (129, 72, 130 * 8, 3, 1, "sigmoid_output", False, True),  # one expert has 129 rows, the others none
+    (500, 264, 328, 4, 3, "softmax_corrected", True, False),
+    (333, 96, 160, 9, 2, "sigmoid_output", False, False),
+    (1100, 128, 96, 300, 8, "softmax_output", False, False),  # more tiles than a wave has lanes
+])
+def test_tiles_of_64_and_128_places(T, W, F, E, top, style, clamped, same):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(T + W + F)
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).bfloat16().to(F64)
+    x, wu, wd = rnd(T, W), rnd(E, F, W, std=W ** -0.5), rnd(E, W, F, std=F ** -0.5)
+    gated = style != "sigmoid_output"
+    wg = rnd(E, F, W, std=W ** -0.5) if gated else None
+    z = torch.randn(T, E, generator=g) * 2
+    if same:
+        z = torch.arange(E, dtype=torch.float32).flip(0).repeat(T, 1)
+    limit = 0.9
+    corrected = style in ("sigmoid_output", "softmax_corrected")
+    correction = torch.randn(E, generator=g) if corrected else None
+    zd = z.to(F64)
+    score = {"scaled_input": torch.sigmoid(zd), "softmax_output": zd, "sigmoid_output": torch.sigmoid(zd),
+             "softmax_corrected": torch.softmax(zd, 1)}[style]
+    ids = torch.topk(score + (correction.to(F64) if corrected else 0), top, dim=1).indices
+    wts = score.gather(1, ids)
+    if style == "softmax_output":
+        wts = torch.softmax(wts, 1)
+    elif style == "sigmoid_output":
+        wts = wts / wts.sum(1, keepdim=True) * 1.5
+    unit = "gelu" if not gated else "clamped" if clamped or style == "scaled_input" else "silu"
+    want, size = _experts(x, ids, wts, wg, wu, wd, unit, style == "scaled_input", limit)
+    dev = lambda t, d=torch.bfloat16: None if t is None else t.to("cuda").to(d)
+    res = torch.randn(T, W, generator=g)
+    item = torch.zeros(T, dtype=torch.int32, device="cuda")
+    item[T - 3:] = -1                                          # padding rows keep what they held
+    r = dev(res, torch.float32)
+    got = K.routed_experts(dev(x), dev(z, torch.float32), dev(wg), dev(wu), dev(wd), r, top=top, limit=limit, out_scale=0.5,
+                           token_item=item, style=style, clamped=clamped, correction=dev(correction, torch.float32), scale=1.5)
+    assert K.moe_tile(T, top, E, True) in (64, 128)
+    # an expert's inner values are rounded to bfloat16 once (8 significant bits: by 2^-8 of each at most); every sum is float
+    bound = 0.5 * (2.0 ** -8 + 1e-4) * size + 1e-5
+    err = (got.double().cpu() - (res.to(F64) + 0.5 * want)).abs()
+    assert bool((err[:T - 3] <= bound[:T - 3]).all()), float((err / bound)[:T - 3].max())
+    assert torch.equal(got[T - 3:].cpu(), res[T - 3:])
