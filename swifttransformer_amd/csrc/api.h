@@ -207,6 +207,15 @@ int st_gla_scan(float* o_part, int64_t part_stride, int part_dim, const void* q,
                 float* state, const int* item_len, const int* item_tok_off, const int* item_slot,
                 int num_items, int heads, int key_dim, int value_dim, float scale, int dtype, hipStream_t stream);
 int st_gla_scan_parts(int key_dim, int part_dim);
+// The same recurrence, the head norm and the gate (as st_gated_head_norm) over prompts and portions, in chunks of 64 rows
+// (csrc/gla_chunks.hip): out [T, heads * value_dim] of `dtype`, rows of no item left as they are.  Up to 128 key and value channels
+// a head.  z [T, heads * key_dim]: the decays' logits, a = sigmoid(z)^inv_tau.  scratch: scratch_chunks >= num_rows / 64 + num_items times heads * key_dim * (value_dim + 1) floats; none where every
+// item has at most one row (`single`).
+int st_gla_chunks(void* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
+                  const float* z, float inv_tau, const void* gate, int64_t gate_stride, const float* gain, float* state, const int* item_len,
+                  const int* item_tok_off, const int* item_slot, int num_items, int num_rows, int heads, int key_dim,
+                  int value_dim, float scale, float eps, float* scratch, int64_t scratch_chunks, int single, int dtype,
+                  hipStream_t stream);
 // With o the sum of `parts` planes (part_stride floats apart):
 // out[t, h, j] = o[t, h, j] * rsqrt(mean_j o[t, h, :]^2 + eps) * gain[j] * silu(g[t, h, j]); g: rows
 // of `dtype` with stride g_stride; out: rows of `dtype`, dense.  Up to 256 value channels a head.

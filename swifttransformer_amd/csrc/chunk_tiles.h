@@ -7,21 +7,44 @@ namespace st {
 
 constexpr int kChunkRows = 64;       // counted from an item's first row of the step
 
-// the chunk of an item that a global chunk index means; false past the last one
-__device__ inline bool find_chunk(int idx, const int* __restrict__ item_len, const int* __restrict__ item_slot,
-                                         int num_items, int& item, int& chunk) {
+__device__ inline int chunks_of(int len, int slot, int rows) { return slot >= 0 && len > 0 ? (len + rows - 1) / rows : 0; }
+
+// The chunk of an item that a global chunk index means; false past the last one (`chunk` is then how far).  Whole waves: a lane an item, so that the items'
+// lengths are one trip to memory and not one after the other (48 rows beside 24 single tokens through gla_chunks: 109 -> 91 us).
+__device__ inline bool find_chunk(int idx, const int* __restrict__ item_len, const int* __restrict__ item_slot, int num_items, int& item,
+                                  int& chunk, int rows = kChunkRows) {
+    const int lane = threadIdx.x & 63;
     int base = 0;
-    for (int b = 0; b < num_items; ++b) {
-        const int len = item_len[b];
-        const int n = (item_slot[b] >= 0 && len > 0) ? (len + kChunkRows - 1) / kChunkRows : 0;
-        if (idx < base + n) {
-            item = b;
-            chunk = idx - base;
+    for (int b0 = 0; b0 < num_items; b0 += 64) {
+        const int b = min(b0 + lane, num_items - 1), len = item_len[b], slot = item_slot[b];
+        const int own = b0 + lane < num_items ? chunks_of(len, slot, rows) : 0;
+        int upto = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += up;
+        }
+        const uint64_t past = __ballot(base + upto > idx);
+        if (past) {
+            const int at = __ffsll((unsigned long long)past) - 1;
+            item = __builtin_amdgcn_readfirstlane(b0 + at);
+            chunk = __builtin_amdgcn_readfirstlane(idx - base - __shfl(upto - own, at, 64));
             return true;
         }
-        base += n;
+        base += __shfl(upto, 63, 64);
     }
+    chunk = __builtin_amdgcn_readfirstlane(idx - base);
     return false;
+}
+
+// the chunks of all items before `item`; whole waves
+__device__ inline int chunks_before(int item, const int* __restrict__ item_len, const int* __restrict__ item_slot, int rows = kChunkRows) {
+    const int lane = threadIdx.x & 63;
+    int sum = 0;
+    for (int b = lane; b < item; b += 64) sum += chunks_of(item_len[b], item_slot[b], rows);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    return __builtin_amdgcn_readfirstlane(sum);
 }
 
 // Four neighbouring floats of a row, zeros past its `limit` numbers or where the row does not exist.  VEC: the row starts

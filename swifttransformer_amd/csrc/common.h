@@ -139,6 +139,14 @@ __device__ inline float tanh_fast(float x) {
     return fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(2.88539008177792681f * x)), 1.f);
 }
 
+// e^x for finite x <= 0 to a few 2^-24 of itself by the hardware's 2^x: the product with log2(e) and what its rounding lost
+__device__ inline float exp_le0(float x) {
+    const float t = x * 1.44269504f;
+    const float lost = fmaf(x, 1.44269504f, -t) + x * 1.92596299e-8f;
+    const float p = __builtin_amdgcn_exp2f(t);
+    return fmaf(p, lost * 0.693147181f, p);
+}
+
 __device__ inline float wave_sum(float v) {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);

@@ -86,6 +86,8 @@ def _lib():
         lib.st_gated_group_norm.argtypes = [_c_p, _c_p, _c_p, _c_i64, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                             _c_int, _c_f, _c_int, _c_p]
         lib.st_decay_gate.argtypes = [_c_p, _c_p, _c_i64, _c_f, _c_p]
+        lib.st_gla_chunks.argtypes = [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_f, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_p,
+                                      _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _c_p, _c_i64, _c_int, _c_int, _c_p]
         lib.st_gla_scan.argtypes = [_c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p,
                                     _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_p]
         lib.st_gated_head_norm.argtypes = [_c_p, _c_p, _c_int, _c_i64, _c_p, _c_i64, _c_p, _c_int, _c_int, _c_int,
@@ -1214,6 +1216,43 @@ def gla_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Ten
                               _ptr(v), v.stride(0), _ptr(decay), _ptr(state), _ptr(item_len), _ptr(item_tok_off),
                               _ptr(item_slot), B, heads, kd, vd, float(scale), dtype_code(q.dtype), _stream()))
     return PartialSums(planes)
+
+
+GLA_CHUNK_DIM = 128              # key and value channels a head that the chunk kernels take
+
+
+@_timed("gla_chunks", lambda q, k, v, logits, tau, state, *a, **kw: {
+    "rows": q.shape[0], "width": v.shape[1], "flops": 4 * q.shape[0] * v.shape[1] * (q.shape[1] // state.shape[1]),
+    "bytes": (2 * q.shape[1] + 3 * v.shape[1]) * q.shape[0] * q.element_size() + logits.numel() * 4})
+def gla_chunks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, logits: torch.Tensor, tau: float, state: torch.Tensor, ctx_arrays, heads: int,
+               scale: float, gate: torch.Tensor, gain: torch.Tensor, eps: float, single: bool = False) -> torch.Tensor:
+    """``gated_head_norm(gla_scan(.., decay_gate(logits, 1 / tau), ..), gate, gain, ...)``: the recurrence as products within chunks of 64 rows and a carry between
+    chunks, norm and gate in the last kernel; items of up to 16 rows row by row.  ``single``: no item has more than one row.  Up to ``GLA_CHUNK_DIM`` key and value channels
+    a head; gate: rows like v's.  Rows of no item are left as they are."""
+    _token_item, item_len, item_tok_off, item_slot = ctx_arrays
+    T = q.shape[0]
+    kd, vd = q.shape[1] // heads, v.shape[1] // heads
+    if kd > GLA_CHUNK_DIM or vd > GLA_CHUNK_DIM:
+        raise KernelError(f"gla_chunks: up to {GLA_CHUNK_DIM} key and value channels a head, not {kd} and {vd}")
+    for name, t, w in (("q", q, heads * kd), ("k", k, heads * kd), ("v", v, heads * vd), ("gate", gate, heads * vd)):
+        _need(t, name, q.dtype, (T, w), contiguous=False)
+        if t.stride(1) != 1:
+            raise KernelError(f"{name}: rows must be dense")
+    _need(logits, "logits", torch.float32, (T, heads * kd))
+    _need(state, "state", torch.float32, (state.shape[0], heads, kd, vd))
+    if tau <= 0:
+        raise KernelError(f"gla_chunks: tau must be positive, not {tau}")
+    _need(gain, "gain", torch.float32, (vd,))
+    B = item_slot.shape[0]
+    for name, t in (("item_len", item_len), ("item_tok_off", item_tok_off), ("item_slot", item_slot)):
+        _need(t, name, torch.int32, (B,))
+    out = empty((T, heads * vd), q.dtype, q.device)
+    chunks = 0 if single else T // 64 + B
+    scratch = empty((chunks * heads * kd * (vd + 1),), torch.float32, q.device) if chunks else None
+    _check(_lib().st_gla_chunks(_ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(logits), 1.0 / float(tau), _ptr(gate),
+                                gate.stride(0), _ptr(gain), _ptr(state), _ptr(item_len), _ptr(item_tok_off), _ptr(item_slot), B, T,
+                                heads, kd, vd, float(scale), float(eps), _ptr(scratch), chunks, int(single), dtype_code(q.dtype), _stream()))
+    return out
 
 
 @_timed("gated_head_norm", lambda o, gate, *a, **k: {

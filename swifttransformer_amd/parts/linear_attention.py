@@ -6,7 +6,8 @@
     y = Wo (rmsnorm_head(o) * gain * silu(Wg x))
 
 The state lives in the request's state slot (``CacheNeed("state")``) and is carried from step to
-step, so prompts, portions and decoded tokens run through the same kernel.  Products take the
+step: prompts and portions by chunks of rows, single tokens row by row, heads of more than 128 channels
+by the scan.  Products take the
 engine's storage type; the decay, the state and the head norm are float.  The result is added to
 the residual stream with ``residual_scale`` in the output product's epilogue.  The reference has
 no such mixer."""
@@ -74,10 +75,15 @@ class GatedLinearAttention(Mixer):
         qk, vs = self.qk_size, self.v_size
         proj = K.gemm(x_t, self.w_in)
         low = K.gemm(x_t, self.w_decay_in)
-        decay = K.decay_gate(K.gemm(low, self.w_decay_out, bias=self.b_decay, out_f32=True), 1.0 / self.tau)
+        logits = K.gemm(low, self.w_decay_out, bias=self.b_decay, out_f32=True)
         items = (ctx.token_item, ctx.item_len, ctx.item_tok_off, ctx.item_slot)
-        o = K.gla_scan(proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + vs], decay, cache.state, items,
-                       self.num_heads, self.scale,
-                       tuning.gla_part_dim_decode if ctx.all_single else tuning.gla_part_dim_prompt)
-        y = K.gated_head_norm(o, proj[:, 2 * qk + vs:], self.gain, self.num_heads, self.eps, self.dtype)
+        q, k, v, gate = proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + vs], proj[:, 2 * qk + vs:]
+        if max(self.key_dim, self.value_dim) <= K.GLA_CHUNK_DIM:
+            y = K.gla_chunks(q, k, v, logits, self.tau, cache.state, items, self.num_heads, self.scale, gate, self.gain, self.eps,
+                             single=ctx.all_single)
+        else:
+            decay = K.decay_gate(logits, 1.0 / self.tau)
+            o = K.gla_scan(q, k, v, decay, cache.state, items, self.num_heads, self.scale,
+                           tuning.gla_part_dim_decode if ctx.all_single else tuning.gla_part_dim_prompt)
+            y = K.gated_head_norm(o, gate, self.gain, self.num_heads, self.eps, self.dtype)
         return K.gemm(y, self.w_out, residual=residual32, out_f32=True, out_scale=self.residual_scale)

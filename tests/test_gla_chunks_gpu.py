@@ -1,0 +1,90 @@
+"""Gated linear attention by chunks against the recurrence in float64: items of 1 row to several chunks around the limits of a block (16),
+of a walk (16) and of a chunk (64), sizes with and without whole 16-byte pieces, decays of exactly 0 and 1, padding items, and a
+portion that goes on from the state another one left."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, F64 = "cuda", torch.float64
+
+
+def _walk(q, k, v, a, S):
+    out = torch.empty(q.shape[0], q.shape[1], v.shape[2], dtype=F64)
+    for t in range(q.shape[0]):
+        S = a[t][:, :, None] * S + k[t][:, :, None] * v[t][:, None, :]
+        out[t] = (S * q[t][:, :, None]).sum(1)
+    return out, S
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("lens,heads,kd,vd", [((1, 15, 16, 17, 63), 3, 64, 64), ((64, 65, 1, 129), 2, 128, 128), ((200, 2), 2, 5, 7),
+                                              ((33, 80, 3), 3, 80, 48), ((130,), 2, 20, 100), ((1,) * 70, 2, 64, 32),
+                                              ((70,) + (1,) * 66, 1, 16, 16)])
+def test_chunks_are_the_recurrence(dtype, lens, heads, kd, vd):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(sum(lens) + kd)
+    T, B = sum(lens) + 2, len(lens) + 1                        # two rows of no item; one padding item
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype)
+    proj = rnd(T, heads * (2 * kd + 2 * vd) + (3 if kd == 5 else 0))
+    logits = torch.randn(T, heads * kd, generator=g) * 3
+    logits[::7, ::3] = -1e5                                    # decays of exactly 0 and 1
+    logits[::5, 1::3] = 1e5
+    logits[9, :] = -1e5
+    a = torch.sigmoid(logits.to(F64)) ** 0.25
+    state = torch.randn(B + 2, heads, kd, vd, generator=g)
+    gain = torch.rand(vd, generator=g) + 0.5
+    eps, scale = 1e-5, kd ** -0.5
+    off = [sum(lens[:i]) for i in range(len(lens))]
+    slots = list(range(len(lens), 0, -1))                      # slot 0 and the last stay untouched
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    items = (None, i32(list(lens) + [0]), i32(off + [0]), i32(slots + [-1]))
+    d = proj.to(DEV)
+    cut = [heads * kd, 2 * heads * kd, 2 * heads * kd + heads * vd, 2 * heads * (kd + vd)]
+    q, k, v, gate = (d[:, lo:hi] for lo, hi in zip([0] + cut, cut))
+    st = state.to(DEV)
+    y = K.gla_chunks(q, k, v, logits.to(DEV), 4.0, st, items, heads, scale, gate, gain.to(DEV), eps, single=max(lens) == 1)
+    # the roundings on a number's way: up to 16 + 4 + 32 decays of a few each, 64 + 128 products and sums in chains of fours; in units
+    # of 2^-24 of the sum of magnitudes
+    unit = 512 * 2.0 ** -24
+    f = lambda x, w: x.cpu().to(F64).reshape(T, heads, w)
+    q6, k6, v6, a6, g6 = f(q, kd) * scale, f(k, kd), f(v, vd), a.to(F64).reshape(T, heads, kd), f(gate, vd)
+    for n, lo, slot in zip(lens, off, slots):
+        r = slice(lo, lo + n)
+        o, S = _walk(q6[r], k6[r], v6[r], a6[r], state[slot].to(F64))
+        oa, Sa = _walk(q6[r].abs(), k6[r].abs(), v6[r].abs(), a6[r], state[slot].to(F64).abs())
+        rms = torch.sqrt(o.square().mean(-1, keepdim=True) + eps)
+        b = unit * oa
+        by = gain.to(F64) * (g6[r] * torch.sigmoid(g6[r]))
+        want = o / rms * by
+        err_rms = b.square().mean(-1, keepdim=True).sqrt() / rms
+        bound = by.abs() * (b / rms + o.abs() / rms * err_rms) + (2.0 ** -8 if dtype == torch.bfloat16 else 1e-6) * want.abs() + 1e-12
+        got = y[r].cpu().to(F64).reshape(n, heads, vd)
+        assert bool(((got - want).abs() <= bound).all()), (n, float(((got - want).abs() / bound).max()))
+        assert bool(((st[slot].cpu().to(F64) - S).abs() <= unit * Sa + 1e-12).all()), n
+    assert torch.equal(st[0].cpu(), state[0]) and torch.equal(st[-1].cpu(), state[-1])
+
+
+def test_a_portion_goes_on_from_the_one_before():
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(4)
+    heads, kd, vd, T = 2, 64, 64, 150
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    x = torch.randn(T, 2 * heads * (kd + vd), generator=g).to(DEV)
+    q, k, v, gate = x.split([heads * kd, heads * kd, heads * vd, heads * vd], 1)
+    z = torch.randn(T, heads * kd, generator=g).to(DEV)
+    gain = torch.ones(vd, device=DEV)
+
+    def run(cuts):
+        state = torch.zeros(1, heads, kd, vd, device=DEV)
+        out = []
+        for lo, hi in zip(cuts, cuts[1:]):
+            items = (None, i32([hi - lo]), i32([0]), i32([0]))
+            out.append(K.gla_chunks(q[lo:hi], k[lo:hi], v[lo:hi], z[lo:hi].contiguous(), 8.0, state, items, heads, 0.125, gate[lo:hi], gain, 1e-5,
+                                    single=hi - lo == 1))
+        return torch.cat(out), state
+
+    y0, s0 = run([0, T])
+    for cuts in ([0, 1, 17, 64, 65, T], [0, 100, 101, T]):
+        y, s = run(cuts)
+        # float sums in another order (see above: 256 roundings), of numbers up to 5 after the norm
+        assert float((y - y0).abs().max()) < 256 * 2.0 ** -24 * 5 * 8 and float((s - s0).norm() / s0.norm()) < 1e-6
