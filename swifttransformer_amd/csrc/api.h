@@ -150,6 +150,17 @@ int st_concat_cast(void* out, const float* a, int wa, const float* b, int wb, in
                    hipStream_t stream);
 
 // ---- attention with heads coupled before the softmax, a sink and a window (csrc/sink_attention.hip)
+// The same for prompts and portions in bfloat16 (csrc/sink_tiles.hip): key sizes in whole 8, value sizes in whole 16, both up to 128;
+// mixed heads up to 32.  st_sink_tiles_fit: whether these sizes are taken.
+int st_sink_tiles_fit(int heads, int kv_heads, int key_dim, int value_dim, int mixed, int window, int keep_first, int max_pages, int page_size);
+int st_sink_tiles(void* out, float* part_o, float* part_ml, const void* q, int64_t q_stride, const void* k_cache,
+                  int64_t k_page_stride, const void* v_cache, int64_t v_page_stride, const float* mix, const int* token_item,
+                  const int* positions, const int* block_table, int max_pages, int page_size, const int* item_len,
+                  const int* item_tok_off, const int* item_slot, int num_items, int num_tokens, int heads, int kv_heads,
+                  int key_dim, int value_dim, float scale, int window, int keep_first, int sink, int splits, hipStream_t stream);
+// out[t, h, :] = the splits' partial results of a row added up by their maxima and sums
+int st_sink_attention_merge(void* out, const float* part_o, const float* part_ml, int num_tokens, int heads, int value_dim, int splits,
+                            int dtype, hipStream_t stream);
 int64_t st_sink_attention_lds(int heads, int key_dim, int mixed);
 int st_sink_attention(void* out, float* part_o, float* part_ml, const void* q, int64_t q_stride,
                       const void* k_cache, int64_t k_page_stride, const void* v_cache, int64_t v_page_stride,

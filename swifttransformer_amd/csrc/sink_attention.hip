@@ -332,17 +332,24 @@ static int launch_sink_attention(const SinkAttnArgs& a, int num_tokens, size_t l
         else sink_attention_kernel<T, 32, 1><<<grid, 256, lds_bytes, stream>>>(a);
     }
     ST_LAUNCH_CHECK("sink_attention");
-    if (a.splits > 1) {
-        sink_attention_merge_kernel<T><<<num_tokens, 256, 0, stream>>>((T*)a.out, a.part_o, a.part_ml, a.splits,
-                                                                      a.heads, a.value_dim);
-        ST_LAUNCH_CHECK("sink_attention_merge");
-    }
-    return 0;
+    return a.splits > 1 ? st_sink_attention_merge(a.out, a.part_o, a.part_ml, num_tokens, a.heads, a.value_dim, a.splits,
+                                                  sizeof(T) == 4 ? kF32 : kBF16, stream) : 0;
 }
 
 }  // namespace st
 
 using namespace st;
+
+extern "C" int st_sink_attention_merge(void* out, const float* part_o, const float* part_ml, int num_tokens, int heads, int value_dim,
+                                       int splits, int dtype, hipStream_t stream) {
+    ST_CHECK(heads > 0 && heads <= 256 && splits >= 1 && splits <= 16, "sink_attention_merge: bad sizes");
+    if (dtype == kF32)
+        sink_attention_merge_kernel<float><<<num_tokens, 256, 0, stream>>>((float*)out, part_o, part_ml, splits, heads, value_dim);
+    else
+        sink_attention_merge_kernel<bf16_t><<<num_tokens, 256, 0, stream>>>((bf16_t*)out, part_o, part_ml, splits, heads, value_dim);
+    ST_LAUNCH_CHECK("sink_attention_merge");
+    return 0;
+}
 
 // LDS bytes a workgroup of st_sink_attention needs (the host checks it against the device's limit)
 extern "C" int64_t st_sink_attention_lds(int heads, int key_dim, int mixed) {

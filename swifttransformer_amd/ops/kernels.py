@@ -86,6 +86,10 @@ def _lib():
         lib.st_gated_group_norm.argtypes = [_c_p, _c_p, _c_p, _c_i64, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                             _c_int, _c_f, _c_int, _c_p]
         lib.st_decay_gate.argtypes = [_c_p, _c_p, _c_i64, _c_f, _c_p]
+        lib.st_sink_tiles_fit.argtypes = [_c_int] * 9
+        lib.st_sink_tiles.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int,
+                                      _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_int, _c_int,
+                                      _c_int, _c_p]
         lib.st_gla_chunks.argtypes = [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_f, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_p,
                                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _c_p, _c_i64, _c_int, _c_int, _c_p]
         lib.st_gla_scan.argtypes = [_c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p,
@@ -956,11 +960,12 @@ def _d_sink_attention(q, k_cache, v_cache, token_item, positions, block_table, h
 def sink_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, token_item: torch.Tensor,
                    positions: torch.Tensor, block_table: torch.Tensor, heads: int, scale: float, *,
                    window: int = 0, sink: bool = True, head_mix: Optional[torch.Tensor] = None,
-                   num_splits: int = 1, out: Optional[torch.Tensor] = None, keep_first: int = 0) -> torch.Tensor:
+                   num_splits: int = 1, out: Optional[torch.Tensor] = None, keep_first: int = 0, items=None) -> torch.Tensor:
     """Each query row attends over its request's cached keys [max(0, p - window + 1), p] (window 0: from
     0) and, with ``keep_first`` > 0, over the keys at positions below ``keep_first`` as well.  Every head's scaled products with a key are mixed over the heads by ``head_mix`` (float
     [heads, heads], row = receiving head; None: no mix) before the softmax; ``sink``: one is added to the
-    softmax's denominator.
+    softmax's denominator.  ``items`` (the step's token_item, item_len, item_tok_off, item_slot; for steps with prompts
+    or portions): tiles of 16 rows on the matrix cores where ``sink_tiles_fit`` has the sizes and rows are bfloat16.
 
     q: [T, heads * key_dim] (dense rows, any stride); k_cache [pages, kv_heads, page, key_dim];
     v_cache [pages, kv_heads, page, value_dim].  Returns [T, heads * value_dim]."""
@@ -982,10 +987,31 @@ def sink_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     if out is None:
         out = empty((T, heads * dv), q.dtype, q.device)
     _need(out, "out", q.dtype, (T, heads * dv))
+    # (from 128 rows: 32 heads of 64 with a mix and a window of 1,024 take 21 us by rows and 32 by tiles at 40 rows, 31 and 25 at 130)
+    tiled = (items is not None and T >= 128 and q.dtype == torch.bfloat16 and (q.stride(0) | k_cache.stride(0) | v_cache.stride(0)) % 8 == 0 and
+             (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr() | out.data_ptr()) % 16 == 0 and
+             bool(_lib().st_sink_tiles_fit(heads, nkv, dk, dv, int(head_mix is not None), int(window), int(keep_first),
+                                           block_table.shape[1], ps)))
+    if tiled:
+        # keys are split where a tile's workgroups (mixed: one, else one for sixteen heads) leave most of the chip idle
+        groups = 1 if head_mix is not None else max(1, heads // 16)
+        span = window + keep_first if window > 0 else block_table.shape[1] * ps
+        num_splits = max(1, min(256 // max(1, -(-T // 16) * groups), span // 128, 8))
     part_o = part_ml = None
     if num_splits > 1:
         part_o = empty((T, num_splits, heads * dv), torch.float32, q.device)
         part_ml = empty((T, num_splits, heads, 2), torch.float32, q.device)
+    if tiled:
+        _t, item_len, item_tok_off, item_slot = items
+        B = item_slot.shape[0]
+        for name, t in (("item_len", item_len), ("item_tok_off", item_tok_off), ("item_slot", item_slot)):
+            _need(t, name, torch.int32, (B,))
+        _check(_lib().st_sink_tiles(_ptr(out), _ptr(part_o), _ptr(part_ml), _ptr(q), q.stride(0), _ptr(k_cache), k_cache.stride(0),
+                                    _ptr(v_cache), v_cache.stride(0), _ptr(head_mix), _ptr(token_item), _ptr(positions),
+                                    _ptr(block_table), block_table.shape[1], ps, _ptr(item_len), _ptr(item_tok_off), _ptr(item_slot),
+                                    B, T, heads, nkv, dk, dv, float(scale), int(window), int(keep_first), int(bool(sink)),
+                                    int(num_splits), _stream()))
+        return out
     _check(_lib().st_sink_attention(_ptr(out), _ptr(part_o), _ptr(part_ml), _ptr(q), q.stride(0), _ptr(k_cache),
                                     k_cache.stride(0), _ptr(v_cache), v_cache.stride(0), _ptr(head_mix),
                                     _ptr(token_item), _ptr(positions), _ptr(block_table), block_table.shape[1], ps, T,

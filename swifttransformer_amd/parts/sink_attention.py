@@ -118,7 +118,8 @@ class SinkAttention(Mixer):
             K.paged_write(cache.v, v, ctx.token_item, ctx.positions, bt, unit_eps=self.value_norm_eps)
         o = K.sink_attention(q, cache.k, cache.v, ctx.token_item, ctx.positions, bt, self.num_heads, self.scale,
                              window=self.window, sink=self.sink, head_mix=self.mix,
-                             num_splits=self._splits(ctx, qkv.shape[0]))
+                             num_splits=self._splits(ctx, qkv.shape[0]),
+                             items=None if ctx.all_single else (ctx.token_item, ctx.item_len, ctx.item_tok_off, ctx.item_slot))
         return K.gemm(o, self.w_out, bias=self.b_out, residual=residual32, out_f32=True)
 
 

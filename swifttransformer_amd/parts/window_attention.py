@@ -122,7 +122,8 @@ class GatedWindowAttention(Mixer):
         K.paged_write(kv.v, v, ctx.token_item, ctx.positions, bt)
         o = K.sink_attention(q, kv.k, kv.v, ctx.token_item, ctx.positions, bt, self.num_heads, self.scale,
                              window=self.window, keep_first=self.keep_first, sink=False, head_mix=None,
-                             num_splits=self._splits(ctx, proj.shape[0]))
+                             num_splits=self._splits(ctx, proj.shape[0]),
+                             items=None if ctx.all_single else (ctx.token_item, ctx.item_len, ctx.item_tok_off, ctx.item_slot))
         if self.gate is not None:
             o = K.activation_multiply(proj[:, self.qkv_size:], o, self.gate)
         return K.gemm(o, self.w_out, residual=residual32, out_f32=True, out_scale=self.out_scale)

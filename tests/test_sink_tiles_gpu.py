@@ -1,0 +1,70 @@
+"""Window attention of prompts in tiles on the matrix cores, against float64: tiles with a last short one, single rows beside a
+portion, portions that start behind the window, windows that are no multiple of a block and keep the first tokens, every key in one
+block, heads alone, in fours and mixed (up to 16 and up to 32 of them), sizes up to the largest, rows of no item."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, F64 = "cuda", torch.float64
+
+
+@pytest.mark.parametrize("lens,starts,H,G,dk,dv,window,keep,sink,mixed", [
+    ((128,), (0,), 4, 1, 64, 64, 0, 0, False, False),                         # whole tiles, everything visible
+    ((129, 1, 1), (0, 40, 200), 8, 2, 64, 64, 33, 0, True, True),             # eight heads: one tile of the mix, partly empty
+    ((17, 15, 100), (300, 0, 70), 5, 5, 24, 48, 40, 5, True, True),           # heads alone, key size below a step
+    ((140,), (1000,), 32, 8, 64, 64, 100, 20, False, False),                  # a portion far behind the kept tokens
+    ((150,), (90,), 32, 8, 64, 64, 128, 16, True, True),                      # kept tokens and a mix of 32 heads
+    ((131,), (500,), 6, 2, 128, 32, 0, 0, False, False),                      # heads alone in waves of one workgroup and a half
+    ((70, 66), (33, 2), 24, 6, 80, 112, 64, 3, True, True),                   # sizes between the instances
+    ((160,), (0,), 8, 2, 128, 128, 1, 0, False, False),                       # a row sees itself alone
+    ((130,), (0,), 32, 8, 128, 128, 50, 7, True, True),                       # the largest
+])
+def test_tiles_are_the_attention(lens, starts, H, G, dk, dv, window, keep, sink, mixed):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(sum(lens) + H + dk)
+    T, B, ps = sum(lens), len(lens), 8
+    total = [s + n for s, n in zip(starts, lens)]
+    pages = [-(-t // ps) for t in total]
+    order = torch.randperm(sum(pages), generator=g)
+    table = torch.full((B, max(pages) + 1), -1, dtype=torch.int32)
+    for b in range(B):
+        table[b, :pages[b]] = order[sum(pages[:b]):sum(pages[:b + 1])].int()
+    kc = torch.randn(sum(pages), G, ps, dk, generator=g).bfloat16()
+    vc = torch.randn(sum(pages), G, ps, dv, generator=g).bfloat16()
+    q = (torch.randn(T + 2, H * dk + 8, generator=g) * 2).bfloat16()[:, :H * dk]
+    mix = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g) if mixed else None
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    off = [sum(lens[:i]) for i in range(B)]
+    item = i32([b for b, n in enumerate(lens) for _ in range(n)] + [-1, -1])
+    pos = i32([s + i for s, n in zip(starts, lens) for i in range(n)] + [-1, 0])
+    items = (item, i32(list(lens) + [0]), i32(off + [0]), i32(list(range(B)) + [-1]))
+    scale = dk ** -0.5
+    assert T >= 128 and K._lib().st_sink_tiles_fit(H, G, dk, dv, int(mixed), window, keep, table.shape[1], ps)
+    args = (q.to(DEV), kc.to(DEV), vc.to(DEV), item, pos, table.to(DEV), H, scale)
+    kw = dict(window=window, sink=sink, head_mix=mix.to(DEV) if mixed else None, keep_first=keep)
+    got = K.sink_attention(*args, items=items, **kw).cpu().to(F64)
+    rows = K.sink_attention(*args, **kw).cpu().to(F64)                        # the row kernel
+    assert float(got[T:].abs().max()) == 0.0
+    for b in range(B):
+        idx = table[b, :pages[b]].long()
+        flat = lambda c, w: c[idx].transpose(0, 1).reshape(G, -1, w)[:, :total[b]].to(F64).repeat_interleave(H // G, 0)
+        k, v = flat(kc, dk), flat(vc, dv)
+        r = slice(off[b], off[b] + lens[b])
+        s = torch.einsum("ihd,hjd->hij", q[r].to(F64).reshape(-1, H, dk), k) * scale
+        if mixed:
+            s = torch.einsum("hg,gij->hij", mix.to(F64), s)
+        i, j = torch.arange(starts[b], total[b])[:, None], torch.arange(total[b])[None]
+        seen = (j <= i) & ((i - j < window) | (j < keep)) if window else j <= i
+        s = s.masked_fill(~seen[None], float("-inf"))
+        top = s.amax(-1, keepdim=True).clamp(min=0.0) if sink else s.amax(-1, keepdim=True)
+        p = torch.exp(s - top)
+        p = p / (p.sum(-1, keepdim=True) + (torch.exp(-top) if sink else 0))
+        want = torch.einsum("hij,hjv->ihv", p, v).reshape(lens[b], -1)
+        size = torch.einsum("hij,hjv->ihv", p, v.abs()).reshape(lens[b], -1)
+        # the result is rounded to bfloat16 (2^-8 of it); a weight is off by its score's rounding (sums of up to 128 + 32 products
+        # of numbers up to 40: 40 * 160 * 2^-24 = 4e-4 at most) and by 2^-17
+        bound = 2.0 ** -8 * want.abs() + (4e-4 + 2.0 ** -17) * size + 1e-6
+        assert bool(((got[r] - want).abs() <= bound).all()), float(((got[r] - want).abs() / bound).max())
+        # and on the whole no further from it than the row kernel, whose weights are floats throughout
+        err = lambda x: float((x[r] - want).norm() / want.norm())
+        assert err(got) <= 1.05 * err(rows) + 1e-5, (err(got), err(rows))
