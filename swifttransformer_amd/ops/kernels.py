@@ -98,6 +98,7 @@ def _lib():
                                            _c_f, _c_int, _c_p]
         lib.st_latent_write.argtypes = [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int,
                                         _c_int, _c_int, _c_f, _c_int, _c_p, _c_f, _c_int, _c_p]
+        lib.st_moe_route_align.argtypes = [_c_p] * 6 + [_c_int, _c_p, _c_p, _c_f] + [_c_int] * 9 + [_c_p]
         lib.st_moe_route.argtypes = [_c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_f, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_p]
         lib.st_moe_align.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_p]
         lib.st_moe_up.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int,
@@ -1352,6 +1353,11 @@ def moe_tile(num_tokens: int, top: int, experts: int, staged: bool = False) -> i
     return 128 if pairs >= 96 * experts else 64 if pairs >= 32 * experts else 16
 
 
+def moe_routes_at_once(num_tokens: int, outputs: int) -> bool:
+    """Whether routing and sorting are one workgroup's: a lane an output, 16, 32 or 64 lanes a token, 1,024 in all."""
+    return outputs <= 64 and num_tokens * (16 if outputs <= 16 else 32 if outputs <= 32 else 64) <= 1024
+
+
 def moe_capacity(num_tokens: int, top: int, experts: int, tile: int) -> int:
     """Places of the sorted pair list: every expert's pairs start a tile of their own."""
     return -(-num_tokens * top // tile) * tile + tile * experts
@@ -1437,9 +1443,16 @@ def routed_experts(x: torch.Tensor, logits: torch.Tensor, w_gate: Optional[torch
     place = empty((T * top,), torch.int32, dev)
     tile_expert = empty((cap // tile,), torch.int32, dev)
     y = empty((cap, F), x.dtype, dev)
-    _check(lib.st_moe_route(_ptr(ids), _ptr(wts), _ptr(logits), logits.stride(0) if T > 1 else logits.shape[1], _ptr(token_item),
-                            _ptr(correction) if mode >= 3 else None, float(scale), T, outputs, int(top), mode, int(groups), int(keep), st))
-    _check(lib.st_moe_align(_ptr(sorted_pairs), _ptr(place), _ptr(tile_expert), _ptr(ids), T * top, E, cap, tile, st))
+    stride = logits.stride(0) if T > 1 else logits.shape[1]
+    corr = _ptr(correction) if mode >= 3 else None
+    if moe_routes_at_once(T, outputs):
+        _check(lib.st_moe_route_align(_ptr(ids), _ptr(wts), _ptr(sorted_pairs), _ptr(place), _ptr(tile_expert), _ptr(logits), stride,
+                                      _ptr(token_item), corr, float(scale), T, outputs, E, int(top), mode, int(groups), int(keep), cap,
+                                      tile, st))
+    else:
+        _check(lib.st_moe_route(_ptr(ids), _ptr(wts), _ptr(logits), stride, _ptr(token_item), corr, float(scale), T, outputs, int(top),
+                                mode, int(groups), int(keep), st))
+        _check(lib.st_moe_align(_ptr(sorted_pairs), _ptr(place), _ptr(tile_expert), _ptr(ids), T * top, E, cap, tile, st))
     _check(lib.st_moe_up(_ptr(y), _ptr(x), _ptr(w_gate), _ptr(w_up), _ptr(sorted_pairs), _ptr(tile_expert),
                          _ptr(wts), cap, tile, int(top), W, F, float(limit), 2 if w_gate is None else 3 if clamped else int(on_output), code, st))
     if on_output:
