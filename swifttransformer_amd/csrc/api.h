@@ -149,6 +149,15 @@ int st_paged_write(void* cache, int64_t page_stride, const void* src, int64_t sr
 int st_concat_cast(void* out, const float* a, int wa, const float* b, int wb, int num_rows, int dtype,
                    hipStream_t stream);
 
+// The additive form of st_state_scan over prompts and portions in chunks of 64 rows, for decays gate_b between 0 and 1
+// (csrc/state_chunks.hip); `single` (no item has more than 16 rows): row by row, any decay, no scratch.  Up to 128 key and value channels a
+// head.  scratch: scratch_chunks >= num_rows / 64 + num_items times heads * (key_dim * value_dim + 1) floats.
+int st_state_chunks(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v,
+                    int64_t v_stride, const float* gate_a, const float* gate_b, int64_t gate_stride, const float* skip,
+                    float* state, int64_t slot_stride, const int* item_len, const int* item_tok_off, const int* item_slot,
+                    int num_items, int num_rows, int heads, int qk_heads, int key_dim, int value_dim, float* scratch,
+                    int64_t scratch_chunks, int single, hipStream_t stream);
+
 // ---- attention with heads coupled before the softmax, a sink and a window (csrc/sink_attention.hip)
 // The same for prompts and portions in bfloat16 (csrc/sink_tiles.hip): key sizes in whole 8, value sizes in whole 16, both up to 128;
 // mixed heads up to 32.  st_sink_tiles_fit: whether these sizes are taken.

@@ -1,0 +1,424 @@
+// The additive recurrence with one decay a head and token, over prompts and portions in chunks of 64 rows:
+//
+//   S_t = b_t S_(t-1) + (a_t k_t) v_t^T,   o_t = S_t^T q_t + skip v_t          (S [key channels x value channels] a head)
+//
+// With F_i the sum of log b over a chunk's rows up to i (double; a decay of zero counts as e^-10000), a chunk of n rows that starts
+// from the state S is
+//
+//   o_i = e^(F_i) S^T q_i + sum_(j<=i) e^(F_i - F_j) a_j (q_i . k_j) v_j + skip v_i
+//   S'  = e^(F_n) S + sum_j e^(F_n - F_j) a_j k_j v_j^T
+//
+// with every exponent a difference that is never positive.  Three kernels as in gla_chunks.hip: the chunks' sums (all chunks side by
+// side), the carry (a thread an element of the state), the outputs; all products float on the matrix cores.  Heads share queries
+// and keys in groups.  Items of up to 16 rows are walked row by row in the third kernel, which is all that steps of single tokens
+// launch.  The scan (state_scan.hip) keeps the delta rule and heads of more than 128 channels.
+//
+// Per chunk and head the products are 2 * 64 * (64 + 2 dv) * dk flops at 154 Tflop/s, the chunks' sums are written, walked and read
+// once (4 dk dv bytes each): both take less than the launches' own time up to some 500 rows; from there the sums' passes bound it.  Sums
+// go in four chains a product and the exponents keep their double's rest, which holds the error at the scan's (2048 rows: y 6.3e-8
+// against 6.2e-8 of its norm, 7.4e-8 with one chain).  32 heads of 64 x 64, one prompt of 2048 rows: scan 530 us, here 59; three that
+// make 2048: 222 and 61; 512 rows and 24 single ones: 141 and 33; 130 rows: 45 and 24; 33 rows: 23 and 24; 48 single rows: 23 and 16, 8:
+// 17 and 16.  32 heads of 128 x 128, 2048 rows: 893 and 155; with 128 key channels 24 single rows take 27 and 31, (17, 16, 3) rows 24
+// and 40, 64 rows 37 and 25: such heads come here from 64 rows on, and never in steps of single tokens.
+#include "api.h"
+#include "common.h"
+#include "chunk_tiles.h"
+#include "fragment.h"
+
+#include <type_traits>
+
+namespace st {
+
+constexpr int kStateShort = 16;      // rows up to which an item is walked row by row
+
+struct StateArgs {
+    float* out;
+    const float *q, *k, *v;
+    int64_t q_stride, k_stride, v_stride;
+    const float *gate_a, *gate_b;    // rows gate_stride apart (0: one row for all tokens)
+    int64_t gate_stride;
+    const float* skip;               // [heads] or null
+    float* state;
+    int64_t slot_stride;
+    float *U, *fall;                 // [chunks][heads][dk * dv], [chunks][heads]
+    const int *item_len, *item_tok_off, *item_slot;
+    int num_items, heads, qk_heads, dk, dv;
+};
+
+// the first wave: F_i of a chunk's n rows; past them the last one's
+__device__ inline double state_log_decays(const float* __restrict__ b, int64_t stride, int n) {
+    const int lane = threadIdx.x & 63;
+    const double x = log((double)b[(int64_t)min(lane, n - 1) * stride]);
+    double F = lane < n ? (x < -10000.0 ? -10000.0 : x) : 0.0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const double up = __shfl_up(F, o, 64);
+        if (lane >= o) F += up;
+    }
+    return F;
+}
+
+// e^x of a double, x <= 0, to a float's last place: what x loses as a float goes on as a factor
+__device__ __forceinline__ float state_exp(double x) {
+    const float hi = (float)x, e = expf(hi);
+    return fmaf(e, (float)(x - (double)hi), e);
+}
+
+// U[idx, head] and fall[idx, head].  Grid (heads, chunks, blocks of 64 value channels).  LDS: k [64][4 KQ + 4] | v [64][68] | w [64].
+template <int KQ, bool VEC>
+__global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float state_lds[];
+    const int head = blockIdx.x, idx = blockIdx.y, vb = blockIdx.z * 64, tid = threadIdx.x;
+    int item, chunk;
+    if (!find_chunk(idx, a.item_len, a.item_slot, a.num_items, item, chunk)) return;
+    if (a.item_len[item] <= kStateShort) return;
+    const int n = min(kChunkRows, a.item_len[item] - chunk * kChunkRows), dk = a.dk, dv = a.dv;
+    const int64_t row0 = (int64_t)a.item_tok_off[item] + (int64_t)chunk * kChunkRows;
+    const int group = head / (a.heads / a.qk_heads);
+    constexpr int KS = 4 * KQ + 4, VS = 68;
+    float* ks = state_lds;
+    float* vs = ks + 64 * KS;
+    float* w = vs + 64 * VS;
+    Tile<KQ> tk;
+    Tile<16> tv;
+    tk.template load<VEC>(a.k + row0 * a.k_stride + (int64_t)group * dk, a.k_stride, n, 0, dk);
+    tv.template load<VEC>(a.v + row0 * a.v_stride + (int64_t)head * dv, a.v_stride, n, vb, dv);
+    if (tid < 64) {
+        const double F = state_log_decays(a.gate_b + row0 * a.gate_stride + head, a.gate_stride, n), last = __shfl(F, n - 1, 64);
+        const float f = a.gate_a[(row0 + min(tid, n - 1)) * a.gate_stride + head];
+        w[tid] = tid < n ? f * state_exp(last - F) : 0.f;
+        if (blockIdx.z == 0 && tid == 0) a.fall[(int64_t)idx * a.heads + head] = state_exp(last);
+    }
+    tv.store(vs, VS);
+    __syncthreads();                                // the weights
+    tk.store_weighted(ks, KS, w);
+    __syncthreads();
+    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    const int steps = (n + 15) >> 4, ktiles = (dk + 15) >> 4;
+    float* u = a.U + ((int64_t)idx * a.heads + head) * dk * dv;
+    for (int kt = wave; kt < ktiles; kt += 4) {
+        floatx4 acc[4][4];                          // (sums in four short chains: their error is the scan's)
+#pragma unroll
+        for (int vt = 0; vt < 4; ++vt) acc[0][vt] = acc[1][vt] = acc[2][vt] = acc[3][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < steps; ++s) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int j = 16 * s + 4 * g + r;
+                const float x = ks[j * KS + 16 * kt + r16];
+#pragma unroll
+                for (int vt = 0; vt < 4; ++vt)
+                    acc[r][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, vs[j * VS + 16 * vt + r16], acc[r][vt], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int vt = 0; vt < 4; ++vt) acc[0][vt] = (acc[0][vt] + acc[1][vt]) + (acc[2][vt] + acc[3][vt]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int kk = 16 * kt + 4 * g + r;
+            if (kk >= dk) continue;
+#pragma unroll
+            for (int vt = 0; vt < 4; ++vt) {
+                const int col = vb + 16 * vt + r16;
+                if (col < dv) u[(int64_t)kk * dv + col] = acc[0][vt][r];
+            }
+        }
+    }
+}
+
+// A thread an element of a request's state: S walks the item's chunks, leaving at U's place the state each chunk starts from.
+__global__ __launch_bounds__(256) void state_carry_kernel(StateArgs a) {
+    const int head = blockIdx.x, item = blockIdx.y;
+    const int e = blockIdx.z * 256 + threadIdx.x;
+    const int slot = a.item_slot[item], len = a.item_len[item];
+    if (slot < 0 || len <= kStateShort) return;
+    const int base = chunks_before(item, a.item_len, a.item_slot), chunks = (len + kChunkRows - 1) / kChunkRows;
+    if (e >= a.dk * a.dv) return;
+    const int64_t plane = (int64_t)a.dk * a.dv, first = (int64_t)base * a.heads + head;
+    float* home = a.state + (int64_t)slot * a.slot_stride + (int64_t)head * plane + e;
+    float* u = a.U + first * plane + e;
+    const float* f = a.fall + first;
+    float S = *home;
+    int c0 = 0;
+    auto batch = [&](auto count) {                             // so many chunks' operands on their way at once
+        constexpr int B = decltype(count)::value;
+        for (; c0 + B <= chunks; c0 += B) {
+            float add[B], keep[B];
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                add[b] = u[(int64_t)(c0 + b) * a.heads * plane];
+                keep[b] = f[(int64_t)(c0 + b) * a.heads];
+            }
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                u[(int64_t)(c0 + b) * a.heads * plane] = S;
+                S = fmaf(keep[b], S, add[b]);
+            }
+        }
+    };
+    batch(std::integral_constant<int, 16>());
+    batch(std::integral_constant<int, 4>());
+    batch(std::integral_constant<int, 1>());
+    *home = S;
+}
+
+// 64 value channels (from vb) of an item of up to kStateShort rows from its slot's state, row by row.  Thread (wave, lane): KQ key
+// channels from KQ * wave, value channel vb + lane; the waves' partial read-outs meet in LDS once a row.  (Value channels never meet:
+// a wave with 128 of them holds twice the state and leaves a unit half as many workgroups: 49 against 31 us for 24 items of 32 heads of
+// 128 x 128.)
+template <int KQ>
+__device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int item, int head, int vb) {
+    constexpr int C = 4 * KQ, V = 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = a.dk, dv = a.dv, n = a.item_len[item];
+    const int64_t row0 = a.item_tok_off[item];
+    const int group = head / (a.heads / a.qk_heads), col = vb + lane, colc = min(col, dv - 1);
+    float* sq = lds;                       // [n][C], keys (times their factor) likewise, zeros past dk
+    float* sk = sq + kStateShort * C;
+    float* sv = sk + kStateShort * C;      // [n][V]
+    float* sb = sv + kStateShort * V;      // [n]
+    float* part = sb + kStateShort;        // [2][4][V]
+    float* home = a.state + (int64_t)a.item_slot[item] * a.slot_stride + (int64_t)head * dk * dv;
+    float S[KQ];
+#pragma unroll
+    for (int c = 0; c < KQ; ++c) {
+        const int kk = wave * KQ + c;
+        const float x = home[(int64_t)min(kk, dk - 1) * dv + colc];
+        S[c] = kk < dk && col < dv ? x : 0.f;
+    }
+    for (int e = tid; e < n * C; e += 256) {
+        const int j = e / C, c = e - j * C;
+        const int64_t at = (int64_t)group * dk + min(c, dk - 1), row = row0 + j;
+        const float x = a.q[row * a.q_stride + at], y = a.k[row * a.k_stride + at], f = a.gate_a[row * a.gate_stride + head];
+        sq[e] = c < dk ? x : 0.f;
+        sk[e] = c < dk ? f * y : 0.f;
+    }
+    for (int j = wave; j < n; j += 4) {
+        const float x = a.v[(row0 + j) * a.v_stride + (int64_t)head * dv + colc];
+        sv[j * V + lane] = col < dv ? x : 0.f;
+    }
+    if (tid < n) sb[tid] = a.gate_b[(row0 + tid) * a.gate_stride + head];
+    const float skip = a.skip ? a.skip[head] : 0.f;
+    __syncthreads();
+    for (int j = 0; j < n; ++j) {
+        float* p = part + (j & 1) * 4 * V;
+        const float b = sb[j], vv = sv[j * V + lane];
+        float acc = 0.f;
+#pragma unroll
+        for (int c = 0; c < KQ; c += 4) {
+            const float4 q4 = *reinterpret_cast<const float4*>(sq + j * C + wave * KQ + c);
+            const float4 k4 = *reinterpret_cast<const float4*>(sk + j * C + wave * KQ + c);
+            S[c] = fmaf(b, S[c], k4.x * vv);         acc = fmaf(S[c], q4.x, acc);
+            S[c + 1] = fmaf(b, S[c + 1], k4.y * vv); acc = fmaf(S[c + 1], q4.y, acc);
+            S[c + 2] = fmaf(b, S[c + 2], k4.z * vv); acc = fmaf(S[c + 2], q4.z, acc);
+            S[c + 3] = fmaf(b, S[c + 3], k4.w * vv); acc = fmaf(S[c + 3], q4.w, acc);
+        }
+        p[wave * V + lane] = acc;
+        __syncthreads();                   // (the other half of `part` was read before this row's sums were written)
+        if (wave == 0 && col < dv)
+            a.out[((row0 + j) * a.heads + head) * dv + col] = fmaf(skip, vv, (p[lane] + p[V + lane]) + (p[2 * V + lane] + p[3 * V + lane]));
+    }
+#pragma unroll
+    for (int c = 0; c < KQ; ++c) {
+        const int kk = wave * KQ + c;
+        if (kk < dk && col < dv) home[(int64_t)kk * dv + col] = S[c];
+    }
+}
+
+// Steps of single tokens: grid (heads, items, blocks of 64 value channels), a kernel of its own with few registers.
+template <int KQ>
+__global__ __launch_bounds__(256) void state_walk_kernel(StateArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float state_lds[];
+    const int item = blockIdx.y;
+    if (a.item_slot[item] < 0 || a.item_len[item] <= 0 || a.item_len[item] > kStateShort) return;
+    state_walk<KQ>(state_lds, a, item, blockIdx.x, blockIdx.z * 64);
+}
+
+// Rows of a chunk, transposed as in gla_chunks.hip and the matrix memory's outputs.  LDS: F doubles [64] | a [64] | k [64][4 KQ + 4],
+// later 64 key channels of the start state [64][16 NV + 4] | v [64][16 NV + 4].
+template <int KQ, int NV>
+struct StateOutLds {
+    static constexpr int KS = 4 * KQ + 4, VS = 16 * NV + 4;
+    static constexpr int first = KS > VS ? 64 * KS : 64 * VS;
+    static constexpr size_t bytes = sizeof(double) * 64 + sizeof(float) * (size_t)(64 + first + 64 * VS);
+    static constexpr size_t walk = sizeof(float) * (size_t)(kStateShort * (8 * KQ + 65) + 512);
+    static constexpr size_t both = bytes > walk ? bytes : walk;
+};
+
+template <int KQ, int NV, bool VEC>
+__global__ __launch_bounds__(256) void state_out_kernel(StateArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float state_lds[];
+    using L = StateOutLds<KQ, NV>;
+    const int head = blockIdx.x, idx = blockIdx.y, tid = threadIdx.x;
+    int item, chunk;
+    if (!find_chunk(idx, a.item_len, a.item_slot, a.num_items, item, chunk)) return;
+    if (a.item_len[item] <= kStateShort) {
+        for (int vb = 0; vb < a.dv; vb += 64) {
+            if (vb > 0) __syncthreads();                       // the rows before have been read
+            state_walk<KQ>(state_lds, a, item, head, vb);
+        }
+        return;
+    }
+    const int n = min(kChunkRows, a.item_len[item] - chunk * kChunkRows), dk = a.dk, dv = a.dv;
+    const int64_t row0 = (int64_t)a.item_tok_off[item] + (int64_t)chunk * kChunkRows;
+    const int group = head / (a.heads / a.qk_heads);
+    double* sF = reinterpret_cast<double*>(state_lds);
+    float* sa = reinterpret_cast<float*>(sF + 64);
+    float* ks = sa + 64;
+    float* vs = ks + L::first;
+    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    const int i = wave * 16 + r16;                             // this lane's row of the chunk
+    const bool row_ok = i < n;
+    {
+        Tile<KQ> tk;
+        Tile<4 * NV> tv;
+        tk.template load<VEC>(a.k + row0 * a.k_stride + (int64_t)group * dk, a.k_stride, n, 0, dk);
+        tv.template load<VEC>(a.v + row0 * a.v_stride + (int64_t)head * dv, a.v_stride, n, 0, dv);
+        if (tid < 64) {
+            sF[tid] = state_log_decays(a.gate_b + row0 * a.gate_stride + head, a.gate_stride, n);
+            sa[tid] = tid < n ? a.gate_a[(row0 + tid) * a.gate_stride + head] : 0.f;
+        }
+        tk.store(ks, L::KS);
+        tv.store(vs, L::VS);
+    }
+    float qf[KQ];                                              // key channels 16 s + 4 g .. + 3
+    {
+        const float* qr = a.q + (row0 + min(i, n - 1)) * a.q_stride + (int64_t)group * dk;
+#pragma unroll
+        for (int s = 0; s < KQ / 4; ++s) {
+            const float4 x = load_piece<VEC>(qr, 16 * s + 4 * g, dk, row_ok);
+            qf[4 * s] = x.x; qf[4 * s + 1] = x.y; qf[4 * s + 2] = x.z; qf[4 * s + 3] = x.w;
+        }
+    }
+    // the start state's first 64 key channels, on their way during the scores
+    const float* s0 = a.U + ((int64_t)idx * a.heads + head) * dk * dv;
+    Tile<4 * NV> ts;
+    ts.template load<VEC>(s0, dv, min(dk, 64), 0, dv);
+    __syncthreads();
+    const double Fi = sF[i];
+    const float carried = state_exp(Fi);
+    floatx4 st[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        st[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        if (t > wave || 16 * t >= n) continue;                 // uniform over the wave
+        floatx4 second = floatx4{0.f, 0.f, 0.f, 0.f}, third = second, fourth = second;     // (sums in short chains)
+#pragma unroll
+        for (int s = 0; s < KQ / 4; ++s) {
+            const float4 x = *reinterpret_cast<const float4*>(ks + (16 * t + r16) * L::KS + 16 * s + 4 * g);
+            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, qf[4 * s], st[t], 0, 0, 0);
+            second = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, qf[4 * s + 1], second, 0, 0, 0);
+            third = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, qf[4 * s + 2], third, 0, 0, 0);
+            fourth = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, qf[4 * s + 3], fourth, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 16 * t + 4 * g + r;
+            st[t][r] = j <= i ? ((st[t][r] + second[r]) + (third[r] + fourth[r])) * (sa[j] * state_exp(Fi - sF[j])) : 0.f;
+        }
+    }
+    floatx4 o[4][NV];
+#pragma unroll
+    for (int vt = 0; vt < NV; ++vt) o[0][vt] = o[1][vt] = o[2][vt] = o[3][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < (KQ + 15) / 16; ++b) {                 // S_0^T q, then times the row's factor
+        if (64 * b >= dk) continue;
+        __syncthreads();                                       // the keys (or the channels before) have been read
+        ts.store(ks, L::VS);
+        __syncthreads();
+        if (64 * (b + 1) < dk) ts.template load<VEC>(s0 + (int64_t)64 * (b + 1) * dv, dv, min(dk - 64 * (b + 1), 64), 0, dv);
+#pragma unroll
+        for (int s = 0; s < (KQ < 16 ? KQ : 16); ++s) {
+            const float* sr = ks + (16 * (s >> 2) + 4 * g + (s & 3)) * L::VS + r16;
+#pragma unroll
+            for (int vt = 0; vt < NV; ++vt)
+                o[s & 3][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sr[16 * vt], qf[(16 * b + s) % KQ], o[s & 3][vt], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int vt = 0; vt < NV; ++vt) {
+        o[0][vt] = ((o[0][vt] + o[1][vt]) + (o[2][vt] + o[3][vt])) * carried;
+        o[1][vt] = o[2][vt] = o[3][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        if (t > wave || 16 * t >= n) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float* vr = vs + (16 * t + 4 * g + r) * L::VS + r16;
+#pragma unroll
+            for (int vt = 0; vt < NV; ++vt) o[r][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[16 * vt], st[t][r], o[r][vt], 0, 0, 0);
+        }
+    }
+    if (!row_ok) return;
+    // o[.][vt][r]: value channel 16 vt + 4 g + r of row i
+    const float skip = a.skip ? a.skip[head] : 0.f;
+    float* dst = a.out + ((row0 + i) * a.heads + head) * dv;
+#pragma unroll
+    for (int vt = 0; vt < NV; ++vt) {
+        const int v0 = 16 * vt + 4 * g;
+        if (v0 >= dv) continue;
+        const float* own = vs + i * L::VS + v0;
+        const floatx4 sum = (o[0][vt] + o[1][vt]) + (o[2][vt] + o[3][vt]);
+        const float4 y = make_float4(fmaf(skip, own[0], sum[0]), fmaf(skip, own[1], sum[1]), fmaf(skip, own[2], sum[2]), fmaf(skip, own[3], sum[3]));
+        if (VEC) *reinterpret_cast<float4*>(dst + v0) = y;
+        else {
+            const float z[4] = {y.x, y.y, y.z, y.w};
+            for (int r = 0; r < 4 && v0 + r < dv; ++r) dst[v0 + r] = z[r];
+        }
+    }
+}
+
+template <int KQ, int NV, bool VEC>
+static int launch_state_chunks(const StateArgs& a, unsigned chunks, bool single, hipStream_t stream) {
+    using L = StateOutLds<KQ, NV>;
+    if constexpr (KQ == 16) if (single) {
+        state_walk_kernel<KQ><<<dim3(a.heads, a.num_items, (a.dv + 63) / 64), 256, L::walk, stream>>>(a);
+        ST_LAUNCH_CHECK("state_chunks (single rows)");
+        return 0;
+    }
+    constexpr int kSums = (int)sizeof(float) * (64 * (4 * KQ + 4) + 64 * 68 + 64), kOut = (int)L::both;
+    ST_CHECK(hipFuncSetAttribute((const void*)state_sums_kernel<KQ, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kSums) == hipSuccess &&
+             hipFuncSetAttribute((const void*)state_out_kernel<KQ, NV, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kOut) == hipSuccess,
+             "state_chunks: cannot raise the LDS limit");
+    state_sums_kernel<KQ, VEC><<<dim3(a.heads, chunks, (a.dv + 63) / 64), 256, kSums, stream>>>(a);
+    ST_LAUNCH_CHECK("state_chunks (sums)");
+    state_carry_kernel<<<dim3(a.heads, a.num_items, (unsigned)((a.dk * a.dv + 255) / 256)), 256, 0, stream>>>(a);
+    ST_LAUNCH_CHECK("state_chunks (carry)");
+    state_out_kernel<KQ, NV, VEC><<<dim3(a.heads, chunks), 256, kOut, stream>>>(a);
+    ST_LAUNCH_CHECK("state_chunks (outputs)");
+    return 0;
+}
+
+}  // namespace st
+
+using namespace st;
+
+extern "C" int st_state_chunks(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v,
+                               int64_t v_stride, const float* gate_a, const float* gate_b, int64_t gate_stride, const float* skip,
+                               float* state, int64_t slot_stride, const int* item_len, const int* item_tok_off, const int* item_slot,
+                               int num_items, int num_rows, int heads, int qk_heads, int key_dim, int value_dim, float* scratch,
+                               int64_t scratch_chunks, int single, hipStream_t stream) {
+    ST_CHECK(num_items >= 0 && num_rows >= 0 && heads > 0 && qk_heads > 0 && heads % qk_heads == 0 && key_dim > 0 && value_dim > 0,
+             "state_chunks: bad sizes");
+    ST_CHECK(key_dim <= 128 && value_dim <= 128, "state_chunks: up to 128 key and 128 value channels a head, not %d and %d", key_dim, value_dim);
+    ST_CHECK(!single || key_dim <= 64, "state_chunks: steps of single tokens take up to 64 key channels a head, not %d", key_dim);
+    if (num_items == 0 || num_rows == 0) return 0;
+    ST_CHECK(out && q && k && v && gate_a && gate_b && state && item_len && item_tok_off && item_slot && (scratch || single),
+             "state_chunks: null operand");
+    const int64_t chunks = single ? num_items : num_rows / kChunkRows + num_items;   // (every item's last chunk may be a short one)
+    ST_CHECK(single || scratch_chunks >= chunks, "state_chunks: scratch for %lld chunks, %lld needed", (long long)scratch_chunks, (long long)chunks);
+    ST_CHECK(chunks <= 65535 && num_items <= 65535, "state_chunks: too many chunks or items");
+    StateArgs a;
+    a.out = out; a.q = q; a.k = k; a.v = v; a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride;
+    a.gate_a = gate_a; a.gate_b = gate_b; a.gate_stride = gate_stride; a.skip = skip; a.state = state; a.slot_stride = slot_stride;
+    a.U = scratch; a.fall = scratch + scratch_chunks * heads * key_dim * value_dim;
+    a.item_len = item_len; a.item_tok_off = item_tok_off; a.item_slot = item_slot; a.num_items = num_items;
+    a.heads = heads; a.qk_heads = qk_heads; a.dk = key_dim; a.dv = value_dim;
+    // four numbers at a time: rows and heads start on their size
+    const bool vec = ((key_dim | value_dim) & 3) == 0 && ((q_stride | k_stride | v_stride) & 3) == 0 &&
+                     (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)scratch) & 15) == 0;
+#define ST_STATE(KQ, NV) \
+    (vec ? launch_state_chunks<KQ, NV, true>(a, (unsigned)chunks, single != 0, stream) : launch_state_chunks<KQ, NV, false>(a, (unsigned)chunks, single != 0, stream))
+    if (key_dim <= 64) return value_dim <= 64 ? ST_STATE(16, 4) : ST_STATE(16, 8);
+    return value_dim <= 64 ? ST_STATE(32, 4) : ST_STATE(32, 8);
+#undef ST_STATE
+}

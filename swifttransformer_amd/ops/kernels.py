@@ -90,6 +90,8 @@ def _lib():
         lib.st_sink_tiles.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int,
                                       _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_int, _c_int,
                                       _c_int, _c_p]
+        lib.st_state_chunks.argtypes = [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p,
+                                        _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_p, _c_i64, _c_int, _c_p]
         lib.st_gla_chunks.argtypes = [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_f, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_p,
                                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _c_p, _c_i64, _c_int, _c_int, _c_p]
         lib.st_gla_scan.argtypes = [_c_p, _c_i64, _c_int, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p,
@@ -1056,7 +1058,7 @@ def unit_norm(x: torch.Tensor, heads: int, eps: float, scale: float = 1.0) -> to
     return x
 
 
-def _d_state_scan(q, k, v, gate_a, gate_b, state, ctx_arrays, heads, mode, skip=None, max_item_rows=0):
+def _d_state_scan(q, k, v, gate_a, gate_b, state, ctx_arrays, heads, mode, skip=None, max_item_rows=0, chunks=False):
     T = q.shape[0]
     vd = v.shape[1] // heads
     kd = state.shape[2]
@@ -1066,10 +1068,13 @@ def _d_state_scan(q, k, v, gate_a, gate_b, state, ctx_arrays, heads, mode, skip=
                      8 * ctx_arrays[2].shape[0] * heads * kd * vd}
 
 
+STATE_CHUNK_DIM = 128            # key and value channels a head that the chunk kernels of the additive recurrence take
+
+
 @_timed("state_scan", _d_state_scan)
 def state_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_a: torch.Tensor, gate_b: torch.Tensor,
                state: torch.Tensor, ctx_arrays, heads: int, mode: str, skip: Optional[torch.Tensor] = None,
-               max_item_rows: int = 0) -> torch.Tensor:
+               max_item_rows: int = 0, chunks: bool = False) -> torch.Tensor:
     """Per item and head, from the slot's state S [key_dim, value_dim] and over the item's rows in order
     (a = gate_a[t, head], b = gate_b[t, head]):
     ``"additive"``: S <- b S + (a k_t) v_t^T, o_t = S^T q_t + skip[head] v_t;
@@ -1078,7 +1083,8 @@ def state_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_a: torch.
     rows, any stride; head h reads q/k head h // (heads / qk_heads)); state: float
     [slots, heads, key_dim, value_dim] (slots may be parts of a larger per-slot state).  ``max_item_rows``: a
     bound on the rows of any item where the caller knows one (1 in steps of single tokens; 0: the launch's
-    rows); it sizes the kernel's staging, nothing else.  Returns float [T, heads * value_dim]."""
+    rows); it sizes the kernel's staging, nothing else.  ``chunks`` (additive; the caller's decays lie between 0 and 1): prompts
+    and portions go by chunks of 64 rows, up to ``STATE_CHUNK_DIM`` key and value channels a head.  Returns float [T, heads * value_dim]."""
     _token_item, item_len, item_tok_off, item_slot = ctx_arrays
     T = q.shape[0]
     _, sh, kd, vd = state.shape
@@ -1105,6 +1111,16 @@ def state_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_a: torch.
     for name, t in (("item_len", item_len), ("item_tok_off", item_tok_off), ("item_slot", item_slot)):
         _need(t, name, torch.int32, (B,))
     out = empty((T, heads * vd), torch.float32, q.device)
+    single = max_item_rows == 1
+    # more than 64 key channels: the scan is the faster one for few rows (figures in state_chunks.hip)
+    n = 0 if single else T // 64 + B
+    if (mode == "additive" and (single or chunks) and max(kd, vd) <= STATE_CHUNK_DIM and (kd <= 64 or not single and T >= 64) and
+            n <= 65535):
+        scratch = empty((n * heads * (kd * vd + 1),), torch.float32, q.device) if n else None
+        _check(_lib().st_state_chunks(_ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_a),
+                                      _ptr(gate_b), gate_stride, _ptr(skip), _ptr(state), slot_stride, _ptr(item_len), _ptr(item_tok_off),
+                                      _ptr(item_slot), B, T, heads, qk_heads, kd, vd, _ptr(scratch), n, int(single), _stream()))
+        return out
     _check(_lib().st_state_scan(_ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0),
                                 _ptr(gate_a), _ptr(gate_b), gate_stride, _ptr(skip), _ptr(state), slot_stride, _ptr(item_len),
                                 _ptr(item_tok_off), _ptr(item_slot), B, int(max_item_rows) or T, heads, qk_heads, kd, vd,

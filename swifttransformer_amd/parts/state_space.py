@@ -117,7 +117,7 @@ class Mamba2Mixer(_RecurrentMixer):
         xbc = K.token_conv(proj[:, inner:], self.w_conv, conv_state, items, torch.float32, add_input=False,
                            bias=self.b_conv, activation="silu")
         y = K.state_scan(xbc[:, inner + bc:], xbc[:, inner:inner + bc], xbc[:, :inner], steps, decay, state, items,
-                         self.num_heads, "additive", skip=self.skip, max_item_rows=1 if ctx.all_single else 0)
+                         self.num_heads, "additive", skip=self.skip, max_item_rows=1 if ctx.all_single else 0, chunks=True)
         g = K.gated_group_norm(y, proj[:, :inner], self.gain, self.norm_groups, self.eps, self.dtype, gate_first=True)
         return K.gemm(g, self.w_out, residual=residual32, out_f32=True)
 
