@@ -25,6 +25,7 @@
 #include "chunk_tiles.h"
 #include "common.h"
 
+#include <algorithm>
 #include <mutex>
 #include <set>
 
@@ -372,43 +373,80 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(
     }
 }
 
-// Grid (heads, blocks of 16 value channels, items): walks a request's chunks.  wv becomes U, start [chunk, head, dk, dv]
+// The nth item with rows and a slot: its slot and length and the chunks of the items before it; len 0 where there is none.  `live`: how many
+// such items there are.  Whole waves, one trip to memory for 64 items.
+struct LiveItem { int slot, len, first, live; };
+__device__ inline LiveItem live_item(int nth, const int* __restrict__ item_len, const int* __restrict__ item_slot, int num_items) {
+    const int lane = threadIdx.x & 63;
+    LiveItem it{-1, 0, 0, 0};
+    int base = 0;
+    for (int b0 = 0; b0 < num_items; b0 += 64) {
+        const int b = min(b0 + lane, num_items - 1), len = item_len[b], slot = item_slot[b];
+        const int own = b0 + lane < num_items ? chunks_of(len, slot, kChunkRows) : 0;
+        const uint64_t mask = __ballot(own > 0), mine = __ballot(own > 0 && it.live + __popcll(mask & ((1ull << lane) - 1)) == nth);
+        int upto = own;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += up;
+        }
+        if (mine) {
+            const int at = __ffsll((unsigned long long)mine) - 1;
+            it.slot = __builtin_amdgcn_readfirstlane(__shfl(slot, at, 64));
+            it.len = __builtin_amdgcn_readfirstlane(__shfl(len, at, 64));
+            it.first = __builtin_amdgcn_readfirstlane(base + __shfl(upto - own, at, 64));
+        }
+        base += __shfl(upto, 63, 64);
+        it.live += __popcll(mask);
+    }
+    return it;
+}
+
+// Grid (heads, blocks of 16 W value channels, items): walks a request's chunks.  wv becomes U, start [chunk, head, dk, dv]
 // receives the chunks' start states.  A wave owns 16 rows of U and every fourth tile of 16 key channels of S; both meet in
-// LDS: S [16 KT][20] | U [64][20].  The matrix instruction's four depth slots are key channels (rows) 4 g + r, so that the
+// LDS: S [16 KT][16 W + 4] | U [64][16 W + 4].  The matrix instruction's four depth slots are key channels (rows) 4 g + r, so that the
 // results of one product are the operands of the next as they lie.  KT: dk <= 16 KT; AHEAD: chunks whose operands are on
 // their way at a time (a trip to memory takes longer than a chunk).
-template <int KT, int AHEAD>
-__global__ __launch_bounds__(256) void delta_carry_kernel(
+// W: with few requests the chip is filled by value channels, 16 a workgroup, and each request's chunks are a chain that wants its
+// operands early (AHEAD, at the price of one workgroup a unit).  Every workgroup reads all of wk and kt, so where the requests fill the chip
+// (`many` of them with rows) a workgroup takes 32 channels and two share a unit; 64 channels want more registers than two have.  Which
+// of the two launches does the work is seen here, not on the host: a recorded step's list has room for more requests than it holds (one
+// prompt of 2048 rows in a list for 32: 353 us and 354 with the launch that finds nothing to do).  All kernels of a call, 32 heads of
+// 128 x 128, narrow and wide: 16 requests of 2048 rows in a list for 24 521 and 395 us, 512 rows beside 23 single ones 433 and 271, three
+// requests of 2048 382 and 343; 64 x 64, 40 requests of 2048 rows 252 and 187.  Same sums in the same order.
+template <int KT, int AHEAD, int W>
+__global__ __launch_bounds__(256, W > 1 ? 2 : 1) void delta_carry_kernel(
     float* __restrict__ wv, const float* __restrict__ wk, const float* __restrict__ kt, const float* __restrict__ fall,
     float* __restrict__ start, float* __restrict__ state, int64_t slot_stride, const int* __restrict__ item_len,
-    const int* __restrict__ item_slot, DeltaShape sh) {
-    __shared__ float ss[16 * KT][20];
-    __shared__ float su[kChunkRows][20];
-    const int head = blockIdx.x, vb = blockIdx.y * 16, item = blockIdx.z, tid = threadIdx.x;
-    const int slot = item_slot[item], len = item_len[item];
-    if (slot < 0 || len <= 0) return;
-    int first = 0;
-    for (int b = 0; b < item; ++b) {
-        const int l = item_len[b];
-        first += (item_slot[b] >= 0 && l > 0) ? (l + kChunkRows - 1) / kChunkRows : 0;
-    }
+    const int* __restrict__ item_slot, int num_items, int many, DeltaShape sh) {
+    constexpr int WS = 16 * W + 4;
+    __shared__ float ss[16 * KT][WS];
+    __shared__ float su[kChunkRows][WS];
+    const int head = blockIdx.x, vb = blockIdx.y * 16 * W, tid = threadIdx.x;
+    const LiveItem it = live_item(blockIdx.z, item_len, item_slot, num_items);
+    if (it.len <= 0 || (it.live >= many) != (W > 1)) return;
+    const int slot = it.slot, len = it.len, first = it.first;
     const int chunks = (len + kChunkRows - 1) / kChunkRows, dk = sh.dk, dv = sh.dv;
-    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4, col = vb + r16, colc = min(col, dv - 1);
+    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4, col0 = vb + r16;
     constexpr int MT = (KT + 3) / 4;                 // a wave's tiles of S
     float* home = state + (int64_t)slot * slot_stride + sh.s_base() + (int64_t)head * dk * dv;
-    floatx4 S[MT];
+    floatx4 S[MT][W];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int kk = 16 * (wave + 4 * m) + 4 * g + r;
-            const float v = home[(int64_t)min(kk, dk - 1) * dv + colc];
-            S[m][r] = kk < dk && col < dv ? v : 0.f;
-            if (wave + 4 * m < KT) ss[kk][r16] = S[m][r];
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const int col = col0 + 16 * w;
+                const float v = home[(int64_t)min(kk, dk - 1) * dv + min(col, dv - 1)];
+                S[m][w][r] = kk < dk && col < dv ? v : 0.f;
+                if (wave + 4 * m < KT) ss[kk][16 * w + r16] = S[m][w][r];
+            }
         }
     const bool quads = dk % 4 == 0;
     struct Operands {
-        floatx4 fk[KT], ft[MT][4], fv;
+        floatx4 fk[KT], ft[MT][4], fv[W];
     };
     auto load = [&](Operands& p, int c) {
         const int64_t at = (int64_t)(first + c) * sh.heads + head;
@@ -435,7 +473,9 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
             }
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p.fv[r] = wv[(at * kChunkRows + 16 * wave + 4 * g + r) * dv + colc];
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int w = 0; w < W; ++w) p.fv[w][r] = wv[(at * kChunkRows + 16 * wave + 4 * g + r) * dv + min(col0 + 16 * w, dv - 1)];
     };
     // (a lane holds the factor of chunk lane of the present 64: a load that is the same for all lanes would be a scalar one,
     // and every barrier waits for those)
@@ -444,38 +484,56 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
         if ((c & 63) == 0) falls = fall[(int64_t)(first + min(c + lane, chunks - 1)) * sh.heads + head];
         const float keep = __shfl(falls, c & 63, 64);
         const int64_t at = (int64_t)(first + c) * sh.heads + head;
-        floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+        floatx4 acc[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) acc[w] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int t = 0; t < KT; ++t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(p.fk[t][r], ss[16 * t + 4 * g + r][r16], acc, 0, 0, 0);
-        const floatx4 u = p.fv - acc;
+            for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            su[16 * wave + 4 * g + r][r16] = u[r];
-            if (col < dv) wv[(at * kChunkRows + 16 * wave + 4 * g + r) * dv + col] = u[r];
-        }
+                for (int w = 0; w < W; ++w)
+                    acc[w] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.fk[t][r], ss[16 * t + 4 * g + r][16 * w + r16], acc[w], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const int col = col0 + 16 * w;
+                const float u = p.fv[w][r] - acc[w][r];
+                su[16 * wave + 4 * g + r][16 * w + r16] = u;
+                if (col < dv) wv[(at * kChunkRows + 16 * wave + 4 * g + r) * dv + col] = u;
+            }
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int kk = 16 * (wave + 4 * m) + 4 * g + r;
-                if (kk < dk && col < dv) start[(at * dk + kk) * dv + col] = S[m][r];
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    if (kk < dk && col0 + 16 * w < dv) start[(at * dk + kk) * dv + col0 + 16 * w] = S[m][w][r];
             }
         __syncthreads();                             // U is there, S has been read
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             if (wave + 4 * m >= KT) continue;
-            floatx4 d = S[m] * keep;
+            floatx4 d[W];
+#pragma unroll
+            for (int w = 0; w < W; ++w) d[w] = S[m][w] * keep;
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) d = __builtin_amdgcn_mfma_f32_16x16x4f32(p.ft[m][s][r], su[16 * s + 4 * g + r][r16], d, 0, 0, 0);
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int w = 0; w < W; ++w)
+                        d[w] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.ft[m][s][r], su[16 * s + 4 * g + r][16 * w + r16], d[w], 0, 0, 0);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int kk = 16 * (wave + 4 * m) + 4 * g + r;
-                S[m][r] = kk < dk ? d[r] : 0.f;
-                ss[kk][r16] = S[m][r];
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    S[m][w][r] = kk < dk ? d[w][r] : 0.f;
+                    ss[kk][16 * w + r16] = S[m][w][r];
+                }
             }
         }
         if (c + AHEAD < chunks) load(p, c + AHEAD);
@@ -495,7 +553,9 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int kk = 16 * (wave + 4 * m) + 4 * g + r;
-            if (kk < dk && col < dv) home[(int64_t)kk * dv + col] = S[m][r];
+#pragma unroll
+            for (int w = 0; w < W; ++w)
+                if (kk < dk && col0 + 16 * w < dv) home[(int64_t)kk * dv + col0 + 16 * w] = S[m][w][r];
         }
 }
 
@@ -754,13 +814,23 @@ extern "C" int st_delta_chunks(void* out, const float* proj, int64_t stride, flo
 #undef ST_DP
 #undef ST_DP2
     ST_LAUNCH_CHECK("delta_chunks (prep)");
-    const dim3 grid_c(heads, (value_dim + 15) / 16, num_items);
-#define ST_DC(KT, AHEAD) delta_carry_kernel<KT, AHEAD><<<grid_c, 256, 0, stream>>>(wv, wk, kt, fall, start, state, slot_stride, item_len, item_slot, sh)
-    if (key_dim <= 16) ST_DC(1, 4);
-    else if (key_dim <= 32) ST_DC(2, 4);
-    else if (key_dim <= 64) ST_DC(4, 4);
-    else if (key_dim <= 128) ST_DC(8, 2);
-    else ST_DC(16, 1);
+    // `many`: requests whose wide workgroups give every unit one, or one and a half where those are short (four requests of 32 heads of
+    // 64: 168 us narrow, 177 wide, eight: 158 and 153); below, only many - 1 can have work for the narrow ones
+    const int wide_blocks = heads * ((value_dim + 31) / 32), fill = key_dim <= 64 ? 384 : 256;
+    const int many = key_dim <= 128 ? std::max(2, (fill + wide_blocks - 1) / wide_blocks) : num_items + 1;
+    const dim3 grid_c(heads, (value_dim + 15) / 16, std::min(num_items, many - 1)), grid_w(heads, (value_dim + 31) / 32, num_items);
+#define ST_DC(KT, AHEAD, W, GRID) \
+    delta_carry_kernel<KT, AHEAD, W><<<GRID, 256, 0, stream>>>(wv, wk, kt, fall, start, state, slot_stride, item_len, item_slot, num_items, many, sh)
+    if (key_dim <= 16) ST_DC(1, 4, 1, grid_c);
+    else if (key_dim <= 32) ST_DC(2, 4, 1, grid_c);
+    else if (key_dim <= 64) ST_DC(4, 4, 1, grid_c);
+    else if (key_dim <= 128) ST_DC(8, 2, 1, grid_c);
+    else ST_DC(16, 1, 1, grid_c);
+    ST_LAUNCH_CHECK("delta_chunks (carry)");
+    if (num_items >= many) {
+        if (key_dim <= 64) ST_DC(4, 2, 2, grid_w);
+        else ST_DC(8, 1, 2, grid_w);
+    }
 #undef ST_DC
     ST_LAUNCH_CHECK("delta_chunks (carry)");
 #define ST_DO_E(T, KQ, NV, VEC)                                                                                        \

@@ -273,12 +273,9 @@ __global__ __launch_bounds__(256) void memory_carry_kernel(
     const int slot = item_slot[item], len = item_len[item];
     const int plane = sh.dk * sh.dv;
     const int e = blockIdx.z * 256 + threadIdx.x;
-    if (slot < 0 || len <= 0 || e >= plane + sh.dk) return;
-    int base = 0;
-    for (int b = 0; b < item; ++b) {
-        const int l = item_len[b];
-        base += (item_slot[b] >= 0 && l > 0) ? (l + kMemChunk - 1) / kMemChunk : 0;
-    }
+    if (slot < 0 || len <= 0) return;
+    const int base = chunks_before(item, item_len, item_slot, kMemChunk);
+    if (e >= plane + sh.dk) return;
     const int chunks = (len + kMemChunk - 1) / kMemChunk;
     float* sl = state + (int64_t)slot * slot_stride;
     const bool in_n = e >= plane;

@@ -15,6 +15,7 @@
 // Everything is float: the scan's recurrence in another order of sums.  Steps of single tokens keep the
 // scan (csrc/state_scan.hip), whose walk is then one token long.
 #include "api.h"
+#include "chunk_tiles.h"
 #include "common.h"
 
 namespace st {
@@ -101,12 +102,9 @@ __global__ __launch_bounds__(256) void retention_carry_kernel(
     const int head = blockIdx.x, item = blockIdx.y;
     const int e = blockIdx.z * 256 + threadIdx.x;
     const int slot = item_slot[item], len = item_len[item];
-    if (slot < 0 || len <= 0 || e >= dk * dv) return;
-    int base = 0;
-    for (int b = 0; b < item; ++b) {
-        const int l = item_len[b];
-        base += (item_slot[b] >= 0 && l > 0) ? (l + C - 1) / C : 0;
-    }
+    if (slot < 0 || len <= 0) return;
+    const int base = chunks_before(item, item_len, item_slot, C);
+    if (e >= dk * dv) return;
     const int chunks = (len + C - 1) / C;
     const float g = decay[head];
     const float gC = decay_pow(g, C), gLast = decay_pow(g, len - (chunks - 1) * C);
