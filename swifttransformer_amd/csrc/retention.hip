@@ -12,8 +12,8 @@
 // channels), the carry (a thread an element of the state; U's place then holds the chunk's start state),
 // the outputs (a workgroup a head, chunk and value block).  Chunks are counted from an item's first row of
 // the step, so a portion may start anywhere; the state comes from and goes back to the request's slot.
-// Everything is float: the scan's recurrence in another order of sums.  Steps of single tokens keep the
-// scan (csrc/state_scan.hip), whose walk is then one token long.
+// Everything is float: the scan's recurrence in another order of sums.  Steps of single tokens take the
+// walk of csrc/state_chunks.hip (wide heads the scan, csrc/state_scan.hip).
 #include "api.h"
 #include "chunk_tiles.h"
 #include "common.h"

@@ -26,3 +26,15 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture(autouse=True)
+def _memory_of_tests_before(request):
+    """A test that measures the card's free memory starts from what is really free: engines of the tests before that wait for the
+    collector, and the allocator's cache, would otherwise go back during the test or not by when the collector happens to run."""
+    if "free_memory" in request.node.name and _gpu_available():
+        import gc
+        import torch
+        gc.collect()
+        torch.cuda.empty_cache()
+    yield
