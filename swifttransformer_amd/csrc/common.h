@@ -139,8 +139,10 @@ __device__ inline float tanh_fast(float x) {
     return fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(2.88539008177792681f * x)), 1.f);
 }
 
-// e^x for finite x <= 0 to a few 2^-24 of itself by the hardware's 2^x: the product with log2(e) and what its rounding lost
+// e^x for x <= 0 by the hardware's 2^x: the product with log2(e) and what its rounding lost.  To a few 2^-24 of itself down to
+// x = -87, zero below (the hardware gives no denormal numbers; the limit at -200 keeps the product finite), NaN for NaN.
 __device__ inline float exp_le0(float x) {
+    x = x < -200.f ? -200.f : x;
     const float t = x * 1.44269504f;
     const float lost = fmaf(x, 1.44269504f, -t) + x * 1.92596299e-8f;
     const float p = __builtin_amdgcn_exp2f(t);

@@ -41,7 +41,7 @@ constexpr int kGlaShort = 16;        // rows up to which an item is walked row b
 // largest float, which stands for rows that do not exist.  (The exponent is right to 2^-24 of itself or of one, as it is by the
 // library's functions, which take five times as long: 85 against 62 us for 2,011 rows of 32 heads.)
 __device__ inline float gla_decay(float z, float inv_tau) {
-    const float u = exp_le0(fabsf(z) > 200.f ? -200.f : -fabsf(z));
+    const float u = exp_le0(-fabsf(z));
     const float m = z < -1e30f ? -1e30f : z < 0.f ? z : 0.f, t = m * 1.44269504f;
     const float l = (t - __builtin_amdgcn_logf(1.f + u)) + (fmaf(m, 1.44269504f, -t) + m * 1.92596299e-8f);
     const float e = l * inv_tau, p = __builtin_amdgcn_exp2f(e);

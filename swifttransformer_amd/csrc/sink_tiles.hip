@@ -266,13 +266,13 @@ __global__ __launch_bounds__(MT ? 512 : 256, MT || HW * NV >= 32 ? 1 : 2) void s
             // (rows of which nothing was seen yet: any finite maximum makes their weights zeros)
             const float base = top == -INFINITY ? 0.f : top;
             const bool moved = __any(top != m[h]);
-            const float alpha = moved ? (m[h] == -INFINITY ? 0.f : exp_le0(m[h] - base)) : 1.f;
+            const float alpha = moved ? exp_le0(m[h] - base) : 1.f;
             m[h] = top;
             uint32_t hb[4], lb[4];
             float sum = 0.f;
 #pragma unroll
             for (int u = 0; u < 8; u += 2) {
-                const float x = p[u] == -INFINITY ? 0.f : exp_le0(p[u] - base), y = p[u + 1] == -INFINITY ? 0.f : exp_le0(p[u + 1] - base);
+                const float x = exp_le0(p[u] - base), y = exp_le0(p[u + 1] - base);        // (unseen: e^-inf)
                 sum += x + y;
                 const uint32_t both = pack_bf16x2(x, y);
                 hb[u >> 1] = both;

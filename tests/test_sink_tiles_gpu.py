@@ -68,3 +68,34 @@ def test_tiles_are_the_attention(lens, starts, H, G, dk, dv, window, keep, sink,
         # and on the whole no further from it than the row kernel, whose weights are floats throughout
         err = lambda x: float((x[r] - want).norm() / want.norm())
         assert err(got) <= 1.05 * err(rows) + 1e-5, (err(got), err(rows))
+
+
+def _attend(q, kc, vc, start, H, window, keep, sink, mix, tiles=True, scale=1.0):
+    """One request whose T rows start at position ``start``; caches by whole pages in order."""
+    from swifttransformer_amd.ops import kernels as K
+    T = q.shape[0]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    item, pos = i32([0] * T), i32(list(range(start, start + T)))
+    table = torch.arange(kc.shape[0], dtype=torch.int32, device=DEV)[None].contiguous()
+    return K.sink_attention(q.to(DEV), kc.to(DEV), vc.to(DEV), item, pos, table, H, scale, window=window, sink=sink, keep_first=keep,
+                            head_mix=mix.to(DEV) if mix is not None else None,
+                            items=(item, i32([T]), i32([0]), i32([0])) if tiles else None)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_scores_as_far_apart_as_floats_go(mixed):
+    """Products of +-1.3e38: the weight of the smaller ones is e^-2.6e38, zero, whichever of the two a row (or a block of 32 keys)
+    meets first."""
+    H, d, ps, T = 4, 16, 16, 144
+    g = torch.Generator().manual_seed(1)
+    q, kc, vc = torch.zeros(T, H * d), torch.zeros(T // ps, H, ps, d), torch.randn(T // ps, H, ps, d, generator=g).bfloat16()
+    q[:, ::d] = 1e19
+    high = torch.rand(T, generator=g) < 0.3
+    high[:40], high[40:72] = False, True                       # whole blocks of either kind
+    kc[..., 0] = torch.where(high, 1.3e19, -1.3e19).view(T // ps, 1, ps)
+    got = _attend(q.bfloat16(), kc.bfloat16(), vc, 0, H, 0, 0, False, torch.eye(H) if mixed else None).cpu().to(F64).view(T, H, d)
+    v = vc.transpose(1, 2).reshape(T, H, d).to(F64)
+    for i in range(T):
+        best = high[:i + 1] if bool(high[:i + 1].any()) else ~high[:i + 1]
+        want = v[:i + 1][best].mean(0)
+        assert bool(((got[i] - want).abs() <= 2.0 ** -8 * want.abs() + 144 * 2.0 ** -22).all()), i
