@@ -8,6 +8,10 @@
 // the row kernel: scores, mix, maxima, sums; a weight meets the values as the sum of two bfloat16 numbers, its nearest and the
 // nearest to what is left (together off by 2^-18 of it, where one alone would be off by 2^-9), in two products.
 //
+// A product of whole blocks meets the values of keys that a row does not see with a weight of zero, which an infinity or NaN among
+// them would turn into NaN.  A tile whose results are not finite is therefore walked once more, the keys that a row sees one by one
+// on the vector units: the row kernel's answer, for such inputs alone.
+//
 // MIX: the workgroup holds all heads.  Their products with a block lie in LDS as [head][key][row]; a wave takes some of the
 // block's keys and mixes them over the heads in place (M is one operand, in registers for the whole walk, a key's products of all
 // heads and rows the other: v_mfma_f32_16x16x4_f32), then every wave takes its own heads back.  Two barriers a block.
@@ -22,6 +26,8 @@
 #include "common.h"
 #include "chunk_tiles.h"
 #include "fragment.h"
+
+#include <type_traits>
 
 namespace st {
 
@@ -54,7 +60,7 @@ __global__ __launch_bounds__(MT ? 512 : 256, MT || HW * NV >= 32 ? 1 : 2) void s
     constexpr bool MIX = MT > 0;                                     // heads in tiles of 16, up to 16 MT of them
     constexpr int ROWB = 32 * NV + 16;                               // bytes between a block's values in LDS
     // eight waves have 256 registers a lane: the largest heads' queries and next values are not kept there
-    constexpr bool KEEP_Q = !(MIX && HW * DS >= 16), AHEAD_V = !(MIX && HW * NV >= 32);
+    constexpr bool KEEP_Q = !(MIX && HW * DS >= 16), AHEAD_V = !(HW * NV >= 32 && (MIX || DS >= 4));
     const int W = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r16 = lane & 15, g = lane >> 4;
     const int H = a.heads, dk = a.key_dim, dv = a.value_dim, width = H * dv, per = H / a.kv_heads;
@@ -124,13 +130,6 @@ __global__ __launch_bounds__(MT ? 512 : 256, MT || HW * NV >= 32 ? 1 : 2) void s
     }
     floatx4 o[HW][NV];
     float m[HW], l[HW];
-#pragma unroll
-    for (int h = 0; h < HW; ++h) {
-        m[h] = a.sink && split == 0 ? 0.f : -INFINITY;
-        l[h] = a.sink && split == 0 && g == 0 ? 1.f : 0.f;           // (a lane's own keys; summed over the groups at the end)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) o[h][v] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
     const int pos = p0 + r16;
     __syncthreads();                                                 // the pages
 
@@ -173,131 +172,174 @@ __global__ __launch_bounds__(MT ? 512 : 256, MT || HW * NV >= 32 ? 1 : 2) void s
             *reinterpret_cast<u32x4*>(vs + key * ROWB + 16 * c) = vr[i];
         }
     };
-    if (b0 < b1) {
-        load_k(b0);
-        if (AHEAD_V) load_v(b0);
-    }
-    for (int b = b0; b < b1; ++b) {
-        int j0, nk;
-        block_of(b, j0, nk);
-        if (AHEAD_V) store_v();
-        // a head's products with the block; kept (or, mixed, put into LDS) one head after the other, so that few are in registers
-        floatx4 sc[MIX ? 1 : HW][2];
+    auto walk = [&](auto one_by_one) __attribute__((always_inline)) {
 #pragma unroll
         for (int h = 0; h < HW; ++h) {
-            if (!KEEP_Q) load_q(h, qf[0]);
-            floatx4* x = sc[MIX ? 0 : h];
+            m[h] = a.sink && split == 0 ? 0.f : -INFINITY;
+            l[h] = a.sink && split == 0 && g == 0 ? 1.f : 0.f;           // (a lane's own keys; summed over the groups at the end)
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                x[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int v = 0; v < NV; ++v) o[h][v] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (b0 < b1) {
+            load_k(b0);
+            if (AHEAD_V) load_v(b0);
+        }
+        for (int b = b0; b < b1; ++b) {
+            int j0, nk;
+            block_of(b, j0, nk);
+            if (AHEAD_V) store_v();
+            // a head's products with the block; kept (or, mixed, put into LDS) one head after the other, so that few are in registers
+            floatx4 sc[MIX ? 1 : HW][2];
 #pragma unroll
-                for (int s = 0; s < DS; ++s) {
-                    const u32x4 k = 32 * s + 8 * g < dk ? kr[t][s] : u32x4{0, 0, 0, 0};
-                    x[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k), qf[KEEP_Q ? h : 0][s], x[t], 0, 0, 0);
+            for (int h = 0; h < HW; ++h) {
+                if (!KEEP_Q) load_q(h, qf[0]);
+                floatx4* x = sc[MIX ? 0 : h];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    x[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int s = 0; s < DS; ++s) {
+                        const u32x4 k = 32 * s + 8 * g < dk ? kr[t][s] : u32x4{0, 0, 0, 0};
+                        x[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k), qf[KEEP_Q ? h : 0][s], x[t], 0, 0, 0);
+                    }
+                    x[t] *= a.scale;
+                    if (MIX && own)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) rs[(h0 + h) * kSinkHeadStride + (16 * t + 4 * g + e) * kSinkKeyStride + r16] = x[t][e];
                 }
-                x[t] *= a.scale;
-                if (MIX && own)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) rs[(h0 + h) * kSinkHeadStride + (16 * t + 4 * g + e) * kSinkKeyStride + r16] = x[t][e];
             }
-        }
-        if (!AHEAD_V) load_v(b);
-        if (b + 1 < b1) {
-            load_k(b + 1);
-            if (AHEAD_V) load_v(b + 1);
-        }
-        if constexpr (MIX) {
-            __syncthreads();
-            for (int key = wave; key < kSinkKeys; key += 2 * W) {    // two keys at a time: chains of products side by side
-                const bool second = key + W < kSinkKeys;
-                float* col = rs + key * kSinkKeyStride + r16;
-                float* col2 = rs + (second ? key + W : key) * kSinkKeyStride + r16;
-                float x[4 * MT], y[4 * MT];
+            if (!AHEAD_V) load_v(b);
+            if (b + 1 < b1) {
+                load_k(b + 1);
+                if (AHEAD_V) load_v(b + 1);
+            }
+            if constexpr (MIX) {
+                __syncthreads();
+                for (int key = wave; key < kSinkKeys; key += 2 * W) {    // two keys at a time: chains of products side by side
+                    const bool second = key + W < kSinkKeys;
+                    float* col = rs + key * kSinkKeyStride + r16;
+                    float* col2 = rs + (second ? key + W : key) * kSinkKeyStride + r16;
+                    float x[4 * MT], y[4 * MT];
 #pragma unroll
-                for (int s = 0; s < 4 * MT; ++s) { x[s] = col[(4 * s + g) * kSinkHeadStride]; y[s] = col2[(4 * s + g) * kSinkHeadStride]; }
-                floatx4 acc[MT][2];
+                    for (int s = 0; s < 4 * MT; ++s) { x[s] = col[(4 * s + g) * kSinkHeadStride]; y[s] = col2[(4 * s + g) * kSinkHeadStride]; }
+                    floatx4 acc[MT][2];
 #pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t][0] = acc[t][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    for (int t = 0; t < MT; ++t) acc[t][0] = acc[t][1] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int s = 0; s < 4 * MT; ++s)
+                    for (int s = 0; s < 4 * MT; ++s)
 #pragma unroll
-                    for (int t = 0; t < MT; ++t) {
-                        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(mf[t][s], x[s], acc[t][0], 0, 0, 0);
-                        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(mf[t][s], y[s], acc[t][1], 0, 0, 0);
+                        for (int t = 0; t < MT; ++t) {
+                            acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(mf[t][s], x[s], acc[t][0], 0, 0, 0);
+                            acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(mf[t][s], y[s], acc[t][1], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            if (H < 16 * MT && 16 * t + g + 4 * r >= H) continue;        // (these stay zeros)
+                            col[(16 * t + g + 4 * r) * kSinkHeadStride] = acc[t][0][r];
+                            if (second) col2[(16 * t + g + 4 * r) * kSinkHeadStride] = acc[t][1][r];
+                        }
+                }
+                __syncthreads();
+            }
+            if (!AHEAD_V) store_v();
+            // bit 4 t + e: key 16 t + 4 g + e is visible to this row (most blocks: every key to every row)
+            uint32_t seen = 0xff;
+            const bool whole = nk == kSinkKeys && j0 + nk - 1 <= p0 && (a.window <= 0 || last - j0 < a.window);
+            if (!whole) seen = 0;
+#pragma unroll
+            for (int t = 0; t < 2 && !whole; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int kk = 16 * t + 4 * g + e, j = j0 + kk;
+                    if (kk < nk && j <= pos && (a.window <= 0 || pos - j < a.window || j < a.keep_first)) seen |= 1u << (4 * t + e);
+                }
+            // (the wave's own values: stored above, read here by other lanes of the same wave, whose LDS accesses keep their order)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int h = 0; h < HW; ++h) {
+                float p[8];
+                float top = -INFINITY;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    p[u] = MIX ? rs[(own ? h0 + h : 0) * kSinkHeadStride + (16 * (u >> 2) + 4 * g + (u & 3)) * kSinkKeyStride + r16]
+                               : sc[MIX ? 0 : h][u >> 2][u & 3];
+                    if (!whole) p[u] = seen >> u & 1 ? p[u] : -INFINITY;
+                    top = fmaxf(top, p[u]);
+                }
+                top = fmaxf(m[h], rows4_max(top));
+                // (rows of which nothing was seen yet: any finite maximum makes their weights zeros)
+                const float base = top == -INFINITY ? 0.f : top;
+                const bool moved = __any(top != m[h]);
+                const float alpha = moved ? exp_le0(m[h] - base) : 1.f;
+                m[h] = top;
+                uint32_t hb[4], lb[4];
+                float sum = 0.f;
+#pragma unroll
+                for (int u = 0; u < 8; u += 2) {
+                    const float x = exp_le0(p[u] - base), y = exp_le0(p[u + 1] - base);        // (unseen: e^-inf)
+                    sum += x + y;
+                    if (one_by_one) { p[u] = x; p[u + 1] = y; }
+                    const uint32_t both = pack_bf16x2(x, y);
+                    hb[u >> 1] = both;
+                    lb[u >> 1] = pack_bf16x2(x - __uint_as_float(both << 16), y - __uint_as_float(both & 0xffff0000u));
+                }
+                l[h] = fmaf(l[h], alpha, sum);
+                const bf16x8 hi = __builtin_bit_cast(bf16x8, u32x4{hb[0], hb[1], hb[2], hb[3]});
+                const bf16x8 rest = __builtin_bit_cast(bf16x8, u32x4{lb[0], lb[1], lb[2], lb[3]});
+                if (moved)
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) o[h][v] *= alpha;
+                if constexpr (one_by_one) {
+#pragma unroll 1
+                    for (int gg = 0; gg < 4; ++gg) {
+                        const uint32_t visible = __shfl(seen, r16 + 16 * gg, 64);
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            const float w = __shfl(p[u], r16 + 16 * gg, 64);
+                            const char* at = vs + (16 * (u >> 2) + 4 * gg + (u & 3)) * ROWB + 8 * g;
+                            if (visible >> u & 1)
+#pragma unroll
+                                for (int v = 0; v < NV; ++v) {
+                                    const uint2 x = *reinterpret_cast<const uint2*>(at + 32 * v);
+                                    o[h][v][0] = fmaf(w, __uint_as_float(x.x << 16), o[h][v][0]);
+                                    o[h][v][1] = fmaf(w, __uint_as_float(x.x & 0xffff0000u), o[h][v][1]);
+                                    o[h][v][2] = fmaf(w, __uint_as_float(x.y << 16), o[h][v][2]);
+                                    o[h][v][3] = fmaf(w, __uint_as_float(x.y & 0xffff0000u), o[h][v][3]);
+                                }
+                            __builtin_amdgcn_sched_barrier(0);           // (one key's values in registers at a time)
+                        }
                     }
+                    continue;
+                }
 #pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        col[(16 * t + g + 4 * r) * kSinkHeadStride] = acc[t][0][r];
-                        if (second) col2[(16 * t + g + 4 * r) * kSinkHeadStride] = acc[t][1][r];
-                    }
+                for (int v = 0; v < NV; ++v) {
+                    if (16 * v >= dv) continue;                          // uniform
+                    const char* at = vs + (4 * g + (r16 >> 2)) * ROWB + 32 * v + 8 * (r16 & 3);
+                    const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ST_LDS_PTR(short4v, at)));
+                    const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ST_LDS_PTR(short4v, at + 16 * ROWB)));
+                    const bf16x8 v8 = __builtin_bit_cast(bf16x8, u32x4{x.x, x.y, y.x, y.y});
+                    o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, rest, o[h][v], 0, 0, 0);
+                    o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, hi, o[h][v], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0x100);                   // (one head's weights in registers at a time; LDS reads may go ahead)
             }
-            __syncthreads();
+            __builtin_amdgcn_wave_barrier();
         }
-        if (!AHEAD_V) store_v();
-        // bit 4 t + e: key 16 t + 4 g + e is visible to this row (most blocks: every key to every row)
-        uint32_t seen = 0xff;
-        const bool whole = nk == kSinkKeys && j0 + nk - 1 <= p0 && (a.window <= 0 || last - j0 < a.window);
-        if (!whole) seen = 0;
+    };
+    walk(std::false_type());
+    float finite = 0.f;
 #pragma unroll
-        for (int t = 0; t < 2 && !whole; ++t)
+    for (int h = 0; h < HW; ++h)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int kk = 16 * t + 4 * g + e, j = j0 + kk;
-                if (kk < nk && j <= pos && (a.window <= 0 || pos - j < a.window || j < a.keep_first)) seen |= 1u << (4 * t + e);
-            }
-        // (the wave's own values: stored above, read here by other lanes of the same wave, whose LDS accesses keep their order)
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int v = 0; v < NV; ++v)
 #pragma unroll
-        for (int h = 0; h < HW; ++h) {
-            float p[8];
-            float top = -INFINITY;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                p[u] = MIX ? rs[(own ? h0 + h : 0) * kSinkHeadStride + (16 * (u >> 2) + 4 * g + (u & 3)) * kSinkKeyStride + r16]
-                           : sc[MIX ? 0 : h][u >> 2][u & 3];
-                if (!whole) p[u] = seen >> u & 1 ? p[u] : -INFINITY;
-                top = fmaxf(top, p[u]);
-            }
-            top = fmaxf(m[h], rows4_max(top));
-            // (rows of which nothing was seen yet: any finite maximum makes their weights zeros)
-            const float base = top == -INFINITY ? 0.f : top;
-            const bool moved = __any(top != m[h]);
-            const float alpha = moved ? exp_le0(m[h] - base) : 1.f;
-            m[h] = top;
-            uint32_t hb[4], lb[4];
-            float sum = 0.f;
-#pragma unroll
-            for (int u = 0; u < 8; u += 2) {
-                const float x = exp_le0(p[u] - base), y = exp_le0(p[u + 1] - base);        // (unseen: e^-inf)
-                sum += x + y;
-                const uint32_t both = pack_bf16x2(x, y);
-                hb[u >> 1] = both;
-                lb[u >> 1] = pack_bf16x2(x - __uint_as_float(both << 16), y - __uint_as_float(both & 0xffff0000u));
-            }
-            l[h] = fmaf(l[h], alpha, sum);
-            const bf16x8 hi = __builtin_bit_cast(bf16x8, u32x4{hb[0], hb[1], hb[2], hb[3]});
-            const bf16x8 rest = __builtin_bit_cast(bf16x8, u32x4{lb[0], lb[1], lb[2], lb[3]});
-            if (moved)
-#pragma unroll
-                for (int v = 0; v < NV; ++v) o[h][v] *= alpha;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                if (16 * v >= dv) continue;                          // uniform
-                const char* at = vs + (4 * g + (r16 >> 2)) * ROWB + 32 * v + 8 * (r16 & 3);
-                const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ST_LDS_PTR(short4v, at)));
-                const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ST_LDS_PTR(short4v, at + 16 * ROWB)));
-                const bf16x8 v8 = __builtin_bit_cast(bf16x8, u32x4{x.x, x.y, y.x, y.y});
-                o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, rest, o[h][v], 0, 0, 0);
-                o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, hi, o[h][v], 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0x100);                   // (one head's weights in registers at a time; LDS reads may go ahead)
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
+            for (int r = 0; r < 4; ++r) finite = fmaf(o[h][v][r], 0.f, finite);
+    // (mixed: every wave walks, or none)
+    if (MIX ? __syncthreads_or(!(finite == 0.f)) : __any(!(finite == 0.f))) walk(std::true_type());
     // o[h][v][r]: value channel 16 v + 4 g + r of row r16
     const bool row_ok = r16 < n && own;
     const int64_t row = row0 + r16;

@@ -99,3 +99,31 @@ def test_scores_as_far_apart_as_floats_go(mixed):
         best = high[:i + 1] if bool(high[:i + 1].any()) else ~high[:i + 1]
         want = v[:i + 1][best].mean(0)
         assert bool(((got[i] - want).abs() <= 2.0 ** -8 * want.abs() + 144 * 2.0 ** -22).all()), i
+
+
+@pytest.mark.parametrize("H,G,dv,mixed,keep", [(32, 8, 64, False, 0), (5, 5, 48, False, 3), (8, 2, 128, True, 0), (32, 8, 64, True, 7)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_value_that_is_not_finite_reaches_the_rows_that_see_it_and_no_others(H, G, dv, mixed, keep, bad):
+    """An infinity or NaN in one channel of one key head's value at position 75, in a key at position 90: rows before, rows behind the
+    window and other channels are what they are without it; the rows and channels that see it are not finite."""
+    dk, ps, T, window = 32, 16, 160, 50
+    g = torch.Generator().manual_seed(H + dv)
+    q = torch.randn(T, H * dk, generator=g).bfloat16()
+    kc, vc = (torch.randn(T // ps, G, ps, w, generator=g).bfloat16() for w in (dk, dv))
+    mix = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g) if mixed else None
+    clean = _attend(q, kc, vc, 0, H, window, keep, True, mix, scale=dk ** -0.5).float().cpu().view(T, H, dv)
+    v2 = vc.clone()
+    v2[75 // ps, G - 1, 75 % ps, 7] = bad
+    got = _attend(q, kc, v2, 0, H, window, keep, True, mix, scale=dk ** -0.5).float().cpu().view(T, H, dv)
+    hit = torch.zeros(T, H, dv, dtype=torch.bool)
+    hit[75:75 + window, H - H // G:, 7] = True
+    assert not bool(got[hit].isfinite().any())
+    # the same weights and values, summed in another order where a tile was made again (see the bound above)
+    assert bool(((got - clean).abs() <= 2.0 ** -7 * clean.abs() + 4e-3)[~hit].all())
+    k2 = kc.clone()
+    k2[90 // ps, 0, 90 % ps, 3] = float("nan")
+    got = _attend(q, k2, vc, 0, H, window, keep, True, mix, scale=dk ** -0.5).float().cpu().view(T, H, dv)
+    hit = torch.zeros(T, H, dv, dtype=torch.bool)
+    hit[90:90 + window, :H if mixed else H // G] = True
+    assert not bool(got[hit].isfinite().any())
+    assert bool(((got - clean).abs() <= 2.0 ** -7 * clean.abs() + 4e-3)[~hit].all())
