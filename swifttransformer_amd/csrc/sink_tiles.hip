@@ -5,8 +5,8 @@
 // A wave has the tile's rows with HW heads that share a key head.  S^T = K Q^T (v_mfma_f32_16x16x32_bf16) leaves a lane with keys
 // 16 t + 4 g + e of one row; keys come straight from the pages in the instruction's layout, values through the wave's own LDS, read
 // back transposed (ds_read_b64_tr_b16) as the operand of O^T += V^T P^T.  Everything between the two products stays float, as in
-// the row kernel: scores, mix, maxima, sums; a weight meets the values as the sum of two bfloat16 numbers, its nearest and the
-// nearest to what is left (together off by 2^-18 of it, where one alone would be off by 2^-9), in two products.
+// the row kernel: scores, mix, maxima, sums; a weight meets the values as the sum of three bfloat16 numbers, which hold its 24 bits,
+// in three products.
 //
 // A product of whole blocks meets the values of keys that a row does not see with a weight of zero, which an infinity or NaN among
 // them would turn into NaN.  A tile whose results are not finite is therefore walked once more, the keys that a row sees one by one
@@ -19,9 +19,10 @@
 // What bounds it: vector instructions around the products (exponentials, roundings, masks) and, with the mix, its float products
 // (heads^2 multiply-adds a row and key) with two barriers a block and one workgroup a unit.  Rows whose tiles leave units idle have their keys split over workgroups;
 // the row kernel's merge adds them up.
-// Measured beside the row kernel, 32 heads of 64 on 8 key heads, window 1,024: mixed, one prompt of 2,048 rows 755 -> 224 us, three
-// of them together 450 -> 166; not mixed 671 -> 104; 512 rows beside 16 single tokens 222 -> 71; 32 heads of 128 x 128, 1,024 rows,
-// 510 -> 240 (mixed), 451 -> 151.  The results' distance from float64 is the row kernel's (1.66e-3: their rounding to bfloat16).
+// Measured beside the row kernel, 32 heads of 64 on 8 key heads, window 1,024: mixed, one prompt of 2,048 rows 755 -> 247 us, three
+// that make 2,048 437 -> 181; not mixed 671 -> 107; 512 rows beside 16 single tokens 225 -> 77; 32 heads of 128 x 128, 1,024 rows,
+// 510 -> 241 (mixed), 454 -> 190.  The sums' distance from float64 before they are rounded to bfloat16: 512 rows behind 600 keys, mixed
+// 3.8e-7 -> 3.3e-7, not mixed 3.0e-7 -> 1.8e-7; with weights of two bfloat16 numbers (230 and 99 us for 2,048 rows) 1.7e-6 and 2.0e-6.
 #include "api.h"
 #include "common.h"
 #include "chunk_tiles.h"
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(MT ? 512 : 256, MT || HW * NV >= 32 ? 1 : 2) void s
                 const bool moved = __any(top != m[h]);
                 const float alpha = moved ? exp_le0(m[h] - base) : 1.f;
                 m[h] = top;
-                uint32_t hb[4], lb[4];
+                uint32_t hb[4], mb[4], lb[4];
                 float sum = 0.f;
 #pragma unroll
                 for (int u = 0; u < 8; u += 2) {
@@ -285,11 +286,15 @@ __global__ __launch_bounds__(MT ? 512 : 256, MT || HW * NV >= 32 ? 1 : 2) void s
                     if (one_by_one) { p[u] = x; p[u + 1] = y; }
                     const uint32_t both = pack_bf16x2(x, y);
                     hb[u >> 1] = both;
-                    lb[u >> 1] = pack_bf16x2(x - __uint_as_float(both << 16), y - __uint_as_float(both & 0xffff0000u));
+                    const float dx = x - __uint_as_float(both << 16), dy = y - __uint_as_float(both & 0xffff0000u);
+                    const uint32_t rest = pack_bf16x2(dx, dy);
+                    mb[u >> 1] = rest;
+                    lb[u >> 1] = pack_bf16x2(dx - __uint_as_float(rest << 16), dy - __uint_as_float(rest & 0xffff0000u));
                 }
                 l[h] = fmaf(l[h], alpha, sum);
                 const bf16x8 hi = __builtin_bit_cast(bf16x8, u32x4{hb[0], hb[1], hb[2], hb[3]});
-                const bf16x8 rest = __builtin_bit_cast(bf16x8, u32x4{lb[0], lb[1], lb[2], lb[3]});
+                const bf16x8 mid = __builtin_bit_cast(bf16x8, u32x4{mb[0], mb[1], mb[2], mb[3]});
+                const bf16x8 low = __builtin_bit_cast(bf16x8, u32x4{lb[0], lb[1], lb[2], lb[3]});
                 if (moved)
 #pragma unroll
                     for (int v = 0; v < NV; ++v) o[h][v] *= alpha;
@@ -322,7 +327,8 @@ __global__ __launch_bounds__(MT ? 512 : 256, MT || HW * NV >= 32 ? 1 : 2) void s
                     const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ST_LDS_PTR(short4v, at)));
                     const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ST_LDS_PTR(short4v, at + 16 * ROWB)));
                     const bf16x8 v8 = __builtin_bit_cast(bf16x8, u32x4{x.x, x.y, y.x, y.y});
-                    o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, rest, o[h][v], 0, 0, 0);
+                    o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, low, o[h][v], 0, 0, 0);
+                    o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, mid, o[h][v], 0, 0, 0);
                     o[h][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v8, hi, o[h][v], 0, 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0x100);                   // (one head's weights in registers at a time; LDS reads may go ahead)

@@ -127,3 +127,50 @@ def test_a_value_that_is_not_finite_reaches_the_rows_that_see_it_and_no_others(H
     hit[90:90 + window, :H if mixed else H // G] = True
     assert not bool(got[hit].isfinite().any())
     assert bool(((got - clean).abs() <= 2.0 ** -7 * clean.abs() + 4e-3)[~hit].all())
+
+
+@pytest.mark.parametrize("T,start,H,G,dk,dv,window,keep,sink,mixed,spread", [
+    (512, 600, 32, 8, 64, 64, 1024, 0, True, True, 1), (512, 600, 32, 8, 64, 64, 1024, 16, False, False, 1),
+    (700, 10, 32, 8, 128, 128, 300, 16, True, True, 1), (200, 900, 12, 3, 64, 64, 256, 0, True, True, 2),
+    (300, 0, 8, 8, 80, 48, 0, 0, False, False, 3)])
+def test_sums_before_the_rounding_are_no_further_from_float64_than_the_row_kernels(monkeypatch, T, start, H, G, dk, dv, window, keep, sink,
+                                                                                   mixed, spread):
+    """The float partial results of split keys, added up in float64: weights that met the values in fewer than 24 bits would show."""
+    from swifttransformer_amd.ops import kernels as K
+    made, make = [], K.empty
+    monkeypatch.setattr(K, "empty", lambda *a: made.append(make(*a)) or made[-1])
+    g = torch.Generator().manual_seed(T + H)
+    ps, total = 16, start + T
+    kc, vc = (torch.randn(-(-total // ps), G, ps, w, generator=g).bfloat16() for w in (dk, dv))
+    q = (spread * torch.randn(T, H * dk, generator=g)).bfloat16()
+    mix = torch.eye(H) + 0.1 * torch.randn(H, H, generator=g) if mixed else None
+
+    def sums():
+        o, ml = (t.to(F64) for t in made if t.dtype == torch.float32)
+        o, m, l = o.view(T, -1, H, dv), ml[..., 0, None], ml[..., 1, None]
+        w = torch.exp(m - m.amax(1, keepdim=True))
+        return (w * torch.where(w > 0, o, 0.0)).sum(1) / (w * l).sum(1), o.shape[1]
+
+    _attend(q, kc, vc, start, H, window, keep, sink, mix, scale=dk ** -0.5)
+    tiles, splits = sums()
+    assert splits > 1
+    made.clear()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    item, pos = i32([0] * T), i32(list(range(start, total)))
+    table = torch.arange(kc.shape[0], dtype=torch.int32, device=DEV)[None].contiguous()
+    K.sink_attention(q.to(DEV), kc.to(DEV), vc.to(DEV), item, pos, table, H, dk ** -0.5, window=window, sink=sink, keep_first=keep,
+                     head_mix=mix.to(DEV) if mixed else None, num_splits=splits)
+    rows, _ = sums()
+    flat = lambda c, w: c.to(DEV).transpose(0, 1).reshape(G, -1, w)[:, :total].to(F64).repeat_interleave(H // G, 0)
+    k, v = flat(kc, dk), flat(vc, dv)
+    s = torch.matmul(q.to(DEV).to(F64).view(T, H, dk).transpose(0, 1).contiguous(), k.transpose(1, 2).contiguous()) * dk ** -0.5
+    if mixed:
+        s = torch.matmul(mix.to(DEV).to(F64), s.reshape(H, -1)).view(s.shape)
+    i, j = torch.arange(start, total, device=DEV)[:, None], torch.arange(total, device=DEV)[None]
+    s = s.masked_fill(~((j <= i) & ((i - j < window) | (j < keep)) if window else j <= i), float("-inf"))
+    top = s.amax(-1, keepdim=True).clamp(min=0.0) if sink else s.amax(-1, keepdim=True)
+    p = torch.exp(s - top)
+    want = torch.matmul(p / (p.sum(-1, keepdim=True) + (torch.exp(-top) if sink else 0)), v).transpose(0, 1)
+    err = lambda x: float((x - want).norm() / want.norm())
+    # (by a tenth to a half nearer; two bfloat16 numbers a weight: 1.4 to 7 times as far)
+    assert err(tiles) <= err(rows), (err(tiles), err(rows))
