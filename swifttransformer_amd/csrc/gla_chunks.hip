@@ -475,6 +475,30 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
     for (int t = 0; t < 4; ++t) {
         if (t > wave || 16 * wave >= n) continue;
         const floatx4 p = t == wave ? diag : st[t];
+        if (t == wave) {
+            // A row meets the later rows of its block with a weight of zero, which an infinity or NaN among their values would turn
+            // into NaN: such a block's rows are summed one by one.
+            float finite = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int vt = 0; vt < NV; ++vt) finite = fmaf(vs[(16 * t + 4 * g + r) * L::VS + 16 * vt + r16], 0.f, finite);
+            if (__any(!(finite == 0.f))) {
+#pragma unroll 1
+                for (int j4 = 0; j4 < 4; ++j4)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float w = __shfl(p[e], r16 + 16 * j4, 64);
+                        if (4 * j4 + e <= r16)
+#pragma unroll
+                            for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+                                for (int r = 0; r < 4; ++r) ok[vt][r] = fmaf(w, vs[(16 * t + 4 * j4 + e) * L::VS + 16 * vt + 4 * g + r], ok[vt][r]);
+                        __builtin_amdgcn_sched_barrier(0);   // (one row's values in registers at a time)
+                    }
+                continue;
+            }
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float* vr = vs + (16 * t + 4 * g + r) * L::VS + r16;

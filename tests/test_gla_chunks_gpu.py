@@ -88,3 +88,34 @@ def test_a_portion_goes_on_from_the_one_before():
         y, s = run(cuts)
         # float sums in another order (see above: 256 roundings), of numbers up to 5 after the norm
         assert float((y - y0).abs().max()) < 256 * 2.0 ** -24 * 5 * 8 and float((s - s0).norm() / s0.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("what", ["q", "k", "v", "z"])
+def test_a_number_that_is_not_finite_reaches_no_row_before_it(what, bad):
+    from swifttransformer_amd.ops import kernels as K
+    heads, kd, vd, lens, at = 2, 64, 48, (130, 70), 130 + 25
+    g = torch.Generator().manual_seed(8)
+    T = sum(lens)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    items = (None, i32(list(lens)), i32([0, lens[0]]), i32([0, 1]))
+    x = {n: torch.randn(T, heads * w, generator=g) for n, w in (("q", kd), ("k", kd), ("v", vd), ("z", kd), ("g", vd))}
+
+    def run(y):
+        state = torch.ones(2, heads, kd, vd, device=DEV)
+        d = {n: t.to(DEV) for n, t in y.items()}
+        out = K.gla_chunks(d["q"], d["k"], d["v"], d["z"], 8.0, state, items, heads, 0.125, d["g"], torch.ones(vd, device=DEV), 1e-5)
+        return out.view(T, heads, vd).cpu(), state.cpu()
+
+    y0, s0 = run(x)
+    spoilt = {n: t.clone() for n, t in x.items()}
+    spoilt[what][at, 5] = float("nan") if what == "z" else bad            # the first head of the second item's row 25
+    y, s = run(spoilt)
+    assert not bool(y[at, 0].isfinite().all())                             # (an infinite root mean square makes the other channels zero)
+    ok = torch.ones(T, heads, dtype=torch.bool)
+    ok[at:, 0] = False
+    # (a block that holds such a value is summed in another order: 16 products, of numbers up to 50 after the norm)
+    assert bool(((y - y0)[ok].abs() <= 16 * 2.0 ** -24 * 50).all())
+    assert torch.equal(s[0], s0[0]) and torch.equal(s[1, 1], s0[1, 1])
+    hit = s[1, 0] if what == "q" else s[1, 0, :, 5] if what == "v" else s[1, 0, 5]
+    assert torch.equal(s[1, 0], s0[1, 0]) if what == "q" else not bool(hit.isfinite().any())
