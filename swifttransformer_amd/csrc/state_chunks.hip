@@ -244,7 +244,7 @@ struct StateOutLds {
 };
 
 template <int KQ, int NV, bool VEC>
-__global__ __launch_bounds__(256) void state_out_kernel(StateArgs a) {
+__global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_kernel(StateArgs a) {
     extern __shared__ __attribute__((aligned(16))) float state_lds[];
     using L = StateOutLds<KQ, NV>;
     const int head = blockIdx.x, idx = blockIdx.y, tid = threadIdx.x;
@@ -338,9 +338,17 @@ __global__ __launch_bounds__(256) void state_out_kernel(StateArgs a) {
         o[0][vt] = ((o[0][vt] + o[1][vt]) + (o[2][vt] + o[3][vt])) * carried;
         o[1][vt] = o[2][vt] = o[3][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
+    // A row meets the later rows of its own block with a weight of zero, which an infinity or NaN among their values would turn into
+    // NaN: such a block's rows are summed one by one instead, below.
+    float zero = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int vt = 0; vt < NV; ++vt) zero = fmaf(vs[(16 * wave + 4 * g + r) * L::VS + 16 * vt + r16], 0.f, zero);
+    const bool finite = !__any(!(zero == 0.f));
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        if (t > wave || 16 * t >= n) continue;
+        if (t > wave || 16 * t >= n || (t == wave && !finite)) continue;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float* vr = vs + (16 * t + 4 * g + r) * L::VS + r16;
@@ -348,8 +356,25 @@ __global__ __launch_bounds__(256) void state_out_kernel(StateArgs a) {
             for (int vt = 0; vt < NV; ++vt) o[r][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[16 * vt], st[t][r], o[r][vt], 0, 0, 0);
         }
     }
+    floatx4 sum[NV];
+#pragma unroll
+    for (int vt = 0; vt < NV; ++vt) sum[vt] = (o[0][vt] + o[1][vt]) + (o[2][vt] + o[3][vt]);
+    if (!finite) {
+        const floatx4 p = wave == 0 ? st[0] : wave == 1 ? st[1] : wave == 2 ? st[2] : st[3];
+#pragma unroll 1
+        for (int j4 = 0; j4 < 4; ++j4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float w = __shfl(p[e], r16 + 16 * j4, 64);
+                if (4 * j4 + e > r16) continue;
+#pragma unroll
+                for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sum[vt][r] = fmaf(w, vs[(16 * wave + 4 * j4 + e) * L::VS + 16 * vt + 4 * g + r], sum[vt][r]);
+            }
+    }
     if (!row_ok) return;
-    // o[.][vt][r]: value channel 16 vt + 4 g + r of row i
+    // sum[vt][r]: value channel 16 vt + 4 g + r of row i
     const float skip = a.skip ? a.skip[head] : 0.f;
     float* dst = a.out + ((row0 + i) * a.heads + head) * dv;
 #pragma unroll
@@ -357,8 +382,7 @@ __global__ __launch_bounds__(256) void state_out_kernel(StateArgs a) {
         const int v0 = 16 * vt + 4 * g;
         if (v0 >= dv) continue;
         const float* own = vs + i * L::VS + v0;
-        const floatx4 sum = (o[0][vt] + o[1][vt]) + (o[2][vt] + o[3][vt]);
-        const float4 y = make_float4(fmaf(skip, own[0], sum[0]), fmaf(skip, own[1], sum[1]), fmaf(skip, own[2], sum[2]), fmaf(skip, own[3], sum[3]));
+        const float4 y = make_float4(fmaf(skip, own[0], sum[vt][0]), fmaf(skip, own[1], sum[vt][1]), fmaf(skip, own[2], sum[vt][2]), fmaf(skip, own[3], sum[vt][3]));
         if (VEC) *reinterpret_cast<float4*>(dst + v0) = y;
         else {
             const float z[4] = {y.x, y.y, y.z, y.w};

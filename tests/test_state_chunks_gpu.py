@@ -89,3 +89,35 @@ def test_a_portion_goes_on_from_the_one_before():
     for cuts in ([0, 1, 17, 64, 65, T], [0, 100, 101, T]):
         y, s = run(cuts)
         assert bool(((y - y0).abs() <= 2 * UNIT * ya + 1e-30).all()) and float((s - s0).norm() / s0.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("what", ["q", "k", "v", "a", "b"])
+def test_a_number_that_is_not_finite_reaches_no_row_before_it(what, bad):
+    from swifttransformer_amd.ops import kernels as K
+    heads, kd, vd, lens, at = 2, 64, 80, (130, 70), 130 + 25
+    g = torch.Generator().manual_seed(8)
+    T = sum(lens)
+    items = (None, i32(list(lens)), i32([0, lens[0]]), i32([0, 1]))
+    x = {n: torch.randn(T, heads * w, generator=g) for n, w in (("q", kd), ("k", kd), ("v", vd))}
+    x["a"] = torch.rand(T, heads, generator=g) * 0.1
+    x["b"] = torch.exp(-4 * x["a"])
+
+    def run(y):
+        state = torch.ones(2, heads, kd, vd, device=DEV)
+        d = {n: t.to(DEV) for n, t in y.items()}
+        out = K.state_scan(d["q"], d["k"], d["v"], d["a"], d["b"], state, items, heads, "additive", chunks=True)
+        return out.view(T, heads, vd).cpu(), state.cpu()
+
+    y0, s0 = run(x)
+    spoilt = {n: t.clone() for n, t in x.items()}
+    spoilt[what][at, 0 if what in "ab" else 5] = float("nan") if what == "b" else bad      # the first head of the second item's row 25
+    y, s = run(spoilt)
+    assert not bool((y[at, 0, 5] if what == "v" else y[at, 0]).isfinite().any())
+    ok = torch.ones(T, heads, dtype=torch.bool)
+    ok[at:, 0] = False
+    # (a block that holds such a value is summed in another order: 16 products of weights and values up to 10 each)
+    assert bool(((y - y0)[ok].abs() <= 16 * 2.0 ** -24 * 100).all())
+    assert torch.equal(s[0], s0[0]) and torch.equal(s[1, 1], s0[1, 1])
+    hit = s[1, 0, :, 5] if what == "v" else s[1, 0, 5] if what == "k" else s[1, 0]
+    assert torch.equal(s, s0) if what == "q" else not bool(hit.isfinite().any())
