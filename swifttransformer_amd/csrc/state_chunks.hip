@@ -9,17 +9,22 @@
 //   S'  = e^(F_n) S + sum_j e^(F_n - F_j) a_j k_j v_j^T
 //
 // with every exponent a difference that is never positive.  Three kernels as in gla_chunks.hip: the chunks' sums (all chunks side by
-// side), the carry (a thread an element of the state), the outputs; all products float on the matrix cores.  Heads share queries
+// side), the carry (a thread an element of the state), the outputs.  Operands are float, weights and sums double, on the matrix cores
+// (v_mfma_f64_16x16x4_f64, half as fast as float): chains of 64 rows and channels in float were up to a tenth further from float64
+// than the scan, which does as many roundings but of smaller sums.  Heads share queries
 // and keys in groups.  Items of up to 16 rows are walked row by row in the third kernel, which is all that steps of single tokens
 // launch.  The scan (state_scan.hip) keeps the delta rule and heads of more than 128 channels.
 //
-// Per chunk and head the products are 2 * 64 * (64 + 2 dv) * dk flops at 154 Tflop/s, the chunks' sums are written, walked and read
-// once (4 dk dv bytes each): both take less than the launches' own time up to some 500 rows; from there the sums' passes bound it.  Sums
-// go in four chains a product and the exponents keep their double's rest, which holds the error at the scan's (2048 rows: y 6.3e-8
-// against 6.2e-8 of its norm, 7.4e-8 with one chain).  32 heads of 64 x 64, one prompt of 2048 rows: scan 530 us, here 59; three that
-// make 2048: 222 and 61; 512 rows and 24 single ones: 141 and 33; 130 rows: 45 and 24; 33 rows: 23 and 24; 48 single rows: 23 and 16, 8:
-// 17 and 16.  32 heads of 128 x 128, 2048 rows: 893 and 155; with 128 key channels 24 single rows take 27 and 31, (17, 16, 3) rows 24
-// and 40, 64 rows 37 and 25: such heads come here from 64 rows on, and never in steps of single tokens.
+// Per chunk and head the products are 2 * 64 * (64 + 2 dv) * dk flops at 77 Tflop/s (double), the chunks' sums are written, walked and
+// read once (4 dk dv bytes each): both take less than the launches' own time up to some 250 rows; from there the products bound it.
+// Distance from float64, 32 heads of 64 x 64: outputs 6.2e-8 (scan) and 2.6e-8, states 5.5e-8 and 3.0e-8 of their norm at 2,048 rows,
+// 8.6e-8 and 2.6e-8, 6.3e-8 and 3.5e-8 at 33; single rows 9.1e-8 and 7.6e-8 (sums in four chains).  With float products it was
+// 6.3e-8, 6.2e-8, 9.0e-8, 6.6e-8.
+// Times, 32 heads of 64 x 64, one prompt of 2,048 rows: scan 530 us, here 73 (with float products 57); three that make 2,048: 222 and 79;
+// 512 rows and 24 single ones: 141 and 37; 130 rows: 44 and 25; 33 rows: 20 and 24; 48 single rows: 23 and 16, 8: 17 and 15.  32 heads of
+// 128 x 128, 2,048 rows: 895 and 182, 256: 122 and 53, 96: 52 and 44, 64: 38 and 43; beside 24 single rows 200: 100 and 86, 104: 78 and
+// 83; 24 single rows alone 27 and 31: heads of more than 64 key channels come here from a number of rows on that grows with the items,
+// and never in steps of single tokens.
 #include "api.h"
 #include "common.h"
 #include "chunk_tiles.h"
@@ -28,6 +33,12 @@
 #include <type_traits>
 
 namespace st {
+
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// The matrix instruction for doubles (v_mfma_f64_16x16x4_f64) leaves rows g + 4 r of its result with a lane's group g, the one for floats
+// rows 4 g + r; with the first operand's rows dealt like this a lane gets what it gets from the one for floats.
+__device__ inline int double_row(int r16) { return 4 * (r16 & 3) + (r16 >> 2); }
 
 constexpr int kStateShort = 16;      // rows up to which an item is walked row by row
 
@@ -58,13 +69,25 @@ __device__ inline double state_log_decays(const float* __restrict__ b, int64_t s
     return F;
 }
 
-// e^x of a double, x <= 0, to a float's last place: what x loses as a float goes on as a factor
-__device__ __forceinline__ float state_exp(double x) {
-    const float hi = (float)x, e = expf(hi);
-    return fmaf(e, (float)(x - (double)hi), e);
+// e^x for x <= 0 to 2^-31 of itself (the Taylor sum up to r^8 on |r| <= ln(2) / 2), so that a weight is rounded to float once, with
+// all its factors; 0 below e^-200, which is none in float.  Doubles take as long as floats here, and a dozen of them no longer than
+// the library's expf.
+__device__ __forceinline__ double state_exp(double x) {
+    x = x < -200.0 ? -200.0 : x;
+    const double n = rint(x * 1.4426950408889634), r = fma(n, -0.69314718055994531, x);
+    double y = 1.0 / 40320.0;
+    y = fma(y, r, 1.0 / 5040.0);
+    y = fma(y, r, 1.0 / 720.0);
+    y = fma(y, r, 1.0 / 120.0);
+    y = fma(y, r, 1.0 / 24.0);
+    y = fma(y, r, 1.0 / 6.0);
+    y = fma(y, r, 0.5);
+    y = fma(y, r, 1.0);
+    y = fma(y, r, 1.0);
+    return ldexp(y, (int)n);
 }
 
-// U[idx, head] and fall[idx, head].  Grid (heads, chunks, blocks of 64 value channels).  LDS: k [64][4 KQ + 4] | v [64][68] | w [64].
+// U[idx, head] and fall[idx, head].  Grid (heads, chunks, blocks of 64 value channels).  LDS: w doubles [64] | k [64][4 KQ + 4] | v [64][68].
 template <int KQ, bool VEC>
 __global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
     extern __shared__ __attribute__((aligned(16))) float state_lds[];
@@ -76,9 +99,9 @@ __global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
     const int64_t row0 = (int64_t)a.item_tok_off[item] + (int64_t)chunk * kChunkRows;
     const int group = head / (a.heads / a.qk_heads);
     constexpr int KS = 4 * KQ + 4, VS = 68;
-    float* ks = state_lds;
+    double* w = reinterpret_cast<double*>(state_lds);
+    float* ks = state_lds + 128;
     float* vs = ks + 64 * KS;
-    float* w = vs + 64 * VS;
     Tile<KQ> tk;
     Tile<16> tv;
     tk.template load<VEC>(a.k + row0 * a.k_stride + (int64_t)group * dk, a.k_stride, n, 0, dk);
@@ -86,32 +109,29 @@ __global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
     if (tid < 64) {
         const double F = state_log_decays(a.gate_b + row0 * a.gate_stride + head, a.gate_stride, n), last = __shfl(F, n - 1, 64);
         const float f = a.gate_a[(row0 + min(tid, n - 1)) * a.gate_stride + head];
-        w[tid] = tid < n ? f * state_exp(last - F) : 0.f;
-        if (blockIdx.z == 0 && tid == 0) a.fall[(int64_t)idx * a.heads + head] = state_exp(last);
+        w[tid] = tid < n ? f * state_exp(last - F) : 0.0;
+        if (blockIdx.z == 0 && tid == 0) a.fall[(int64_t)idx * a.heads + head] = (float)state_exp(last);
     }
     tv.store(vs, VS);
-    __syncthreads();                                // the weights
-    tk.store_weighted(ks, KS, w);
+    tk.store(ks, KS);
     __syncthreads();
-    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4, p16 = double_row(r16);
     const int steps = (n + 15) >> 4, ktiles = (dk + 15) >> 4;
     float* u = a.U + ((int64_t)idx * a.heads + head) * dk * dv;
     for (int kt = wave; kt < ktiles; kt += 4) {
-        floatx4 acc[4][4];                          // (sums in four short chains: their error is the scan's)
+        doublex4 acc[4];
 #pragma unroll
-        for (int vt = 0; vt < 4; ++vt) acc[0][vt] = acc[1][vt] = acc[2][vt] = acc[3][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int vt = 0; vt < 4; ++vt) acc[vt] = doublex4{0.0, 0.0, 0.0, 0.0};
         for (int s = 0; s < steps; ++s) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int j = 16 * s + 4 * g + r;
-                const float x = ks[j * KS + 16 * kt + r16];
+                const double x = ks[j * KS + 16 * kt + p16] * w[j];
 #pragma unroll
                 for (int vt = 0; vt < 4; ++vt)
-                    acc[r][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, vs[j * VS + 16 * vt + r16], acc[r][vt], 0, 0, 0);
+                    acc[vt] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, (double)vs[j * VS + 16 * vt + r16], acc[vt], 0, 0, 0);
             }
         }
-#pragma unroll
-        for (int vt = 0; vt < 4; ++vt) acc[0][vt] = (acc[0][vt] + acc[1][vt]) + (acc[2][vt] + acc[3][vt]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int kk = 16 * kt + 4 * g + r;
@@ -119,7 +139,7 @@ __global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
 #pragma unroll
             for (int vt = 0; vt < 4; ++vt) {
                 const int col = vb + 16 * vt + r16;
-                if (col < dv) u[(int64_t)kk * dv + col] = acc[0][vt][r];
+                if (col < dv) u[(int64_t)kk * dv + col] = (float)acc[vt][r];
             }
         }
     }
@@ -171,11 +191,11 @@ __device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int i
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = a.dk, dv = a.dv, n = a.item_len[item];
     const int64_t row0 = a.item_tok_off[item];
     const int group = head / (a.heads / a.qk_heads), col = vb + lane, colc = min(col, dv - 1);
-    float* sq = lds;                       // [n][C], keys (times their factor) likewise, zeros past dk
+    float* sq = lds;                       // [n][C], keys likewise, zeros past dk
     float* sk = sq + kStateShort * C;
     float* sv = sk + kStateShort * C;      // [n][V]
-    float* sb = sv + kStateShort * V;      // [n]
-    float* part = sb + kStateShort;        // [2][4][V]
+    float* sb = sv + kStateShort * V;      // [n], and the keys' factors [n]
+    float* part = sb + 2 * kStateShort;    // [2][4][V]
     float* home = a.state + (int64_t)a.item_slot[item] * a.slot_stride + (int64_t)head * dk * dv;
     float S[KQ];
 #pragma unroll
@@ -187,31 +207,34 @@ __device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int i
     for (int e = tid; e < n * C; e += 256) {
         const int j = e / C, c = e - j * C;
         const int64_t at = (int64_t)group * dk + min(c, dk - 1), row = row0 + j;
-        const float x = a.q[row * a.q_stride + at], y = a.k[row * a.k_stride + at], f = a.gate_a[row * a.gate_stride + head];
+        const float x = a.q[row * a.q_stride + at], y = a.k[row * a.k_stride + at];
         sq[e] = c < dk ? x : 0.f;
-        sk[e] = c < dk ? f * y : 0.f;
+        sk[e] = c < dk ? y : 0.f;
     }
     for (int j = wave; j < n; j += 4) {
         const float x = a.v[(row0 + j) * a.v_stride + (int64_t)head * dv + colc];
         sv[j * V + lane] = col < dv ? x : 0.f;
     }
-    if (tid < n) sb[tid] = a.gate_b[(row0 + tid) * a.gate_stride + head];
+    if (tid < n) {
+        sb[tid] = a.gate_b[(row0 + tid) * a.gate_stride + head];
+        sb[kStateShort + tid] = a.gate_a[(row0 + tid) * a.gate_stride + head];
+    }
     const float skip = a.skip ? a.skip[head] : 0.f;
     __syncthreads();
     for (int j = 0; j < n; ++j) {
         float* p = part + (j & 1) * 4 * V;
-        const float b = sb[j], vv = sv[j * V + lane];
-        float acc = 0.f;
+        const float b = sb[j], vv = sv[j * V + lane], av = sb[kStateShort + j] * vv;
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};                   // (sums in short chains)
 #pragma unroll
         for (int c = 0; c < KQ; c += 4) {
             const float4 q4 = *reinterpret_cast<const float4*>(sq + j * C + wave * KQ + c);
             const float4 k4 = *reinterpret_cast<const float4*>(sk + j * C + wave * KQ + c);
-            S[c] = fmaf(b, S[c], k4.x * vv);         acc = fmaf(S[c], q4.x, acc);
-            S[c + 1] = fmaf(b, S[c + 1], k4.y * vv); acc = fmaf(S[c + 1], q4.y, acc);
-            S[c + 2] = fmaf(b, S[c + 2], k4.z * vv); acc = fmaf(S[c + 2], q4.z, acc);
-            S[c + 3] = fmaf(b, S[c + 3], k4.w * vv); acc = fmaf(S[c + 3], q4.w, acc);
+            S[c] = fmaf(b, S[c], k4.x * av);         acc[0] = fmaf(S[c], q4.x, acc[0]);
+            S[c + 1] = fmaf(b, S[c + 1], k4.y * av); acc[1] = fmaf(S[c + 1], q4.y, acc[1]);
+            S[c + 2] = fmaf(b, S[c + 2], k4.z * av); acc[2] = fmaf(S[c + 2], q4.z, acc[2]);
+            S[c + 3] = fmaf(b, S[c + 3], k4.w * av); acc[3] = fmaf(S[c + 3], q4.w, acc[3]);
         }
-        p[wave * V + lane] = acc;
+        p[wave * V + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
         __syncthreads();                   // (the other half of `part` was read before this row's sums were written)
         if (wave == 0 && col < dv)
             a.out[((row0 + j) * a.heads + head) * dv + col] = fmaf(skip, vv, (p[lane] + p[V + lane]) + (p[2 * V + lane] + p[3 * V + lane]));
@@ -239,7 +262,7 @@ struct StateOutLds {
     static constexpr int KS = 4 * KQ + 4, VS = 16 * NV + 4;
     static constexpr int first = KS > VS ? 64 * KS : 64 * VS;
     static constexpr size_t bytes = sizeof(double) * 64 + sizeof(float) * (size_t)(64 + first + 64 * VS);
-    static constexpr size_t walk = sizeof(float) * (size_t)(kStateShort * (8 * KQ + 65) + 512);
+    static constexpr size_t walk = sizeof(float) * (size_t)(kStateShort * (8 * KQ + 66) + 512);
     static constexpr size_t both = bytes > walk ? bytes : walk;
 };
 
@@ -264,7 +287,7 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
     float* sa = reinterpret_cast<float*>(sF + 64);
     float* ks = sa + 64;
     float* vs = ks + L::first;
-    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4, p16 = double_row(r16);
     const int i = wave * 16 + r16;                             // this lane's row of the chunk
     const bool row_ok = i < n;
     {
@@ -294,30 +317,29 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
     ts.template load<VEC>(s0, dv, min(dk, 64), 0, dv);
     __syncthreads();
     const double Fi = sF[i];
-    const float carried = state_exp(Fi);
-    floatx4 st[4];
+    const double carried = state_exp(Fi);
+    doublex4 st[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        st[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        st[t] = doublex4{0.0, 0.0, 0.0, 0.0};
         if (t > wave || 16 * t >= n) continue;                 // uniform over the wave
-        floatx4 second = floatx4{0.f, 0.f, 0.f, 0.f}, third = second, fourth = second;     // (sums in short chains)
 #pragma unroll
         for (int s = 0; s < KQ / 4; ++s) {
-            const float4 x = *reinterpret_cast<const float4*>(ks + (16 * t + r16) * L::KS + 16 * s + 4 * g);
-            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, qf[4 * s], st[t], 0, 0, 0);
-            second = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, qf[4 * s + 1], second, 0, 0, 0);
-            third = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, qf[4 * s + 2], third, 0, 0, 0);
-            fourth = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, qf[4 * s + 3], fourth, 0, 0, 0);
+            const float4 x = *reinterpret_cast<const float4*>(ks + (16 * t + p16) * L::KS + 16 * s + 4 * g);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.x, (double)qf[4 * s], st[t], 0, 0, 0);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.y, (double)qf[4 * s + 1], st[t], 0, 0, 0);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.z, (double)qf[4 * s + 2], st[t], 0, 0, 0);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.w, (double)qf[4 * s + 3], st[t], 0, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int j = 16 * t + 4 * g + r;
-            st[t][r] = j <= i ? ((st[t][r] + second[r]) + (third[r] + fourth[r])) * (sa[j] * state_exp(Fi - sF[j])) : 0.f;
+            st[t][r] = j <= i ? st[t][r] * (sa[j] * state_exp(Fi - sF[j])) : 0.0;
         }
     }
-    floatx4 o[4][NV];
+    doublex4 o[NV];
 #pragma unroll
-    for (int vt = 0; vt < NV; ++vt) o[0][vt] = o[1][vt] = o[2][vt] = o[3][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int vt = 0; vt < NV; ++vt) o[vt] = doublex4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int b = 0; b < (KQ + 15) / 16; ++b) {                 // S_0^T q, then times the row's factor
         if (64 * b >= dk) continue;
@@ -327,17 +349,14 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
         if (64 * (b + 1) < dk) ts.template load<VEC>(s0 + (int64_t)64 * (b + 1) * dv, dv, min(dk - 64 * (b + 1), 64), 0, dv);
 #pragma unroll
         for (int s = 0; s < (KQ < 16 ? KQ : 16); ++s) {
-            const float* sr = ks + (16 * (s >> 2) + 4 * g + (s & 3)) * L::VS + r16;
+            const float* sr = ks + (16 * (s >> 2) + 4 * g + (s & 3)) * L::VS + p16;
 #pragma unroll
             for (int vt = 0; vt < NV; ++vt)
-                o[s & 3][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sr[16 * vt], qf[(16 * b + s) % KQ], o[s & 3][vt], 0, 0, 0);
+                o[vt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)sr[16 * vt], (double)qf[(16 * b + s) % KQ], o[vt], 0, 0, 0);
         }
     }
 #pragma unroll
-    for (int vt = 0; vt < NV; ++vt) {
-        o[0][vt] = ((o[0][vt] + o[1][vt]) + (o[2][vt] + o[3][vt])) * carried;
-        o[1][vt] = o[2][vt] = o[3][vt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int vt = 0; vt < NV; ++vt) o[vt] *= carried;
     // A row meets the later rows of its own block with a weight of zero, which an infinity or NaN among their values would turn into
     // NaN: such a block's rows are summed one by one instead, below.
     float zero = 0.f;
@@ -351,38 +370,36 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
         if (t > wave || 16 * t >= n || (t == wave && !finite)) continue;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float* vr = vs + (16 * t + 4 * g + r) * L::VS + r16;
+            const float* vr = vs + (16 * t + 4 * g + r) * L::VS + p16;
 #pragma unroll
-            for (int vt = 0; vt < NV; ++vt) o[r][vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[16 * vt], st[t][r], o[r][vt], 0, 0, 0);
+            for (int vt = 0; vt < NV; ++vt) o[vt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)vr[16 * vt], st[t][r], o[vt], 0, 0, 0);
         }
     }
-    floatx4 sum[NV];
-#pragma unroll
-    for (int vt = 0; vt < NV; ++vt) sum[vt] = (o[0][vt] + o[1][vt]) + (o[2][vt] + o[3][vt]);
     if (!finite) {
-        const floatx4 p = wave == 0 ? st[0] : wave == 1 ? st[1] : wave == 2 ? st[2] : st[3];
+        const doublex4 p = wave == 0 ? st[0] : wave == 1 ? st[1] : wave == 2 ? st[2] : st[3];
 #pragma unroll 1
         for (int j4 = 0; j4 < 4; ++j4)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float w = __shfl(p[e], r16 + 16 * j4, 64);
+                const double w = __shfl(p[e], r16 + 16 * j4, 64);
                 if (4 * j4 + e > r16) continue;
 #pragma unroll
                 for (int vt = 0; vt < NV; ++vt)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) sum[vt][r] = fmaf(w, vs[(16 * wave + 4 * j4 + e) * L::VS + 16 * vt + 4 * g + r], sum[vt][r]);
+                    for (int r = 0; r < 4; ++r) o[vt][r] = fma(w, (double)vs[(16 * wave + 4 * j4 + e) * L::VS + 16 * vt + 4 * g + r], o[vt][r]);
             }
     }
     if (!row_ok) return;
-    // sum[vt][r]: value channel 16 vt + 4 g + r of row i
-    const float skip = a.skip ? a.skip[head] : 0.f;
+    // o[vt][r]: value channel 16 vt + 4 g + r of row i
+    const double skip = a.skip ? a.skip[head] : 0.f;
     float* dst = a.out + ((row0 + i) * a.heads + head) * dv;
 #pragma unroll
     for (int vt = 0; vt < NV; ++vt) {
         const int v0 = 16 * vt + 4 * g;
         if (v0 >= dv) continue;
         const float* own = vs + i * L::VS + v0;
-        const float4 y = make_float4(fmaf(skip, own[0], sum[vt][0]), fmaf(skip, own[1], sum[vt][1]), fmaf(skip, own[2], sum[vt][2]), fmaf(skip, own[3], sum[vt][3]));
+        const float4 y = make_float4((float)fma(skip, (double)own[0], o[vt][0]), (float)fma(skip, (double)own[1], o[vt][1]),
+                                     (float)fma(skip, (double)own[2], o[vt][2]), (float)fma(skip, (double)own[3], o[vt][3]));
         if (VEC) *reinterpret_cast<float4*>(dst + v0) = y;
         else {
             const float z[4] = {y.x, y.y, y.z, y.w};
@@ -399,7 +416,7 @@ static int launch_state_chunks(const StateArgs& a, unsigned chunks, bool single,
         ST_LAUNCH_CHECK("state_chunks (single rows)");
         return 0;
     }
-    constexpr int kSums = (int)sizeof(float) * (64 * (4 * KQ + 4) + 64 * 68 + 64), kOut = (int)L::both;
+    constexpr int kSums = (int)sizeof(float) * (128 + 64 * (4 * KQ + 4) + 64 * 68), kOut = (int)L::both;
     ST_CHECK(hipFuncSetAttribute((const void*)state_sums_kernel<KQ, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kSums) == hipSuccess &&
              hipFuncSetAttribute((const void*)state_out_kernel<KQ, NV, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kOut) == hipSuccess,
              "state_chunks: cannot raise the LDS limit");

@@ -11,6 +11,7 @@ import torch
 
 from . import arena, library
 from .arena import empty
+from .tuning import tuning
 
 F32, BF16 = 0, 1
 _CODE = {torch.float32: F32, torch.bfloat16: BF16}
@@ -1112,10 +1113,9 @@ def state_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_a: torch.
         _need(t, name, torch.int32, (B,))
     out = empty((T, heads * vd), torch.float32, q.device)
     single = max_item_rows == 1
-    # more than 64 key channels: the scan is the faster one for few rows (figures in state_chunks.hip)
     n = 0 if single else T // 64 + B
-    if (mode == "additive" and (single or chunks) and max(kd, vd) <= STATE_CHUNK_DIM and (kd <= 64 or not single and T >= 64) and
-            n <= 65535):
+    if (mode == "additive" and (single or chunks) and max(kd, vd) <= STATE_CHUNK_DIM and (kd <= 64 or not single and
+            T >= tuning.state_chunks_wide_rows + tuning.state_chunks_wide_rows_per_item * B) and n <= 65535):
         scratch = empty((n * heads * (kd * vd + 1),), torch.float32, q.device) if n else None
         _check(_lib().st_state_chunks(_ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_a),
                                       _ptr(gate_b), gate_stride, _ptr(skip), _ptr(state), slot_stride, _ptr(item_len), _ptr(item_tok_off),

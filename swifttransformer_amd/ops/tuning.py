@@ -45,6 +45,11 @@ class Tuning:
     # norm sums).
     gla_part_dim_decode: int = 16
     gla_part_dim_prompt: int = 8
+    # The additive recurrence of heads with more than 64 key channels goes by chunks from so many rows on, and so many more for
+    # each item of the step (figures beside csrc/state_chunks.hip: 32 heads of 128 x 128, one prompt of 64 rows 38 us row by row
+    # and 43 by chunks, 96 rows 52 and 44; 104 rows beside 24 single ones 78 and 83, 200 rows 100 and 86).
+    state_chunks_wide_rows: int = 80
+    state_chunks_wide_rows_per_item: int = 4
 
 
 tuning = Tuning()

@@ -121,3 +121,40 @@ def test_a_number_that_is_not_finite_reaches_no_row_before_it(what, bad):
     assert torch.equal(s[0], s0[0]) and torch.equal(s[1, 1], s0[1, 1])
     hit = s[1, 0, :, 5] if what == "v" else s[1, 0, 5] if what == "k" else s[1, 0]
     assert torch.equal(s, s0) if what == "q" else not bool(hit.isfinite().any())
+
+
+@pytest.mark.parametrize("lens,heads,groups,kd,vd", [((2048,), 8, 1, 64, 64), ((700, 600, 33), 8, 2, 64, 128), ((33,), 16, 4, 64, 64),
+                                                     ((130,), 16, 4, 64, 64), ((257, 77), 6, 6, 20, 36), ((300,), 4, 1, 128, 128), ((1,) * 48, 16, 4, 64, 64)])
+def test_sums_are_no_further_from_float64_than_the_scans(monkeypatch, lens, heads, groups, kd, vd):
+    """Against the kernel that goes row by row, on the same numbers."""
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + kd)
+    T, B = sum(lens), len(lens)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    q, k, v = rnd(T, groups * kd), rnd(T, groups * kd), rnd(T, heads * vd)
+    step = torch.rand(T, heads, generator=g, device=DEV) * 0.1 + 0.001
+    decay = torch.exp(-(torch.rand(heads, generator=g, device=DEV) * 15 + 1) * step)
+    skip, state = rnd(heads), rnd(B, heads, kd, vd)
+    off = [sum(lens[:i]) for i in range(B)]
+    items = (None, i32(list(lens)), i32(off), i32(list(range(B))))
+
+    def run():
+        s = state.clone()
+        return K.state_scan(q, k, v, step, decay, s, items, heads, "additive", skip=skip, max_item_rows=1 if max(lens) == 1 else 0, chunks=True), s
+
+    y, s = run()
+    monkeypatch.setattr(K, "STATE_CHUNK_DIM", 0)
+    y0, s0 = run()
+    f = lambda t, n, w: t.to(F64).view(T, n, w).repeat_interleave(heads // n, 1)
+    q6, k6, v6, a6, b6 = f(q, groups, kd), f(k, groups, kd), f(v, heads, vd), step.to(F64), decay.to(F64)
+    want, last = torch.empty(T, heads, vd, dtype=F64, device=DEV), state.to(F64)
+    for b in range(B):
+        S = last[b]
+        for t in range(off[b], off[b] + lens[b]):
+            S = b6[t][:, None, None] * S + (a6[t][:, None] * k6[t])[:, :, None] * v6[t][:, None, :]
+            want[t] = (S * q6[t][:, :, None]).sum(1) + skip.to(F64)[:, None] * v6[t]
+        last[b] = S
+    err = lambda x, z: float((x.to(F64).view(z.shape) - z).norm() / z.norm())
+    # (prompts: 0.3 to 0.6 of the scan's; single rows 0.8, with the same state, whose one multiplication and addition are the scan's)
+    assert err(y, want) <= err(y0, want), (err(y, want), err(y0, want))
+    assert err(s, last) <= err(s0, last), (err(s, last), err(s0, last))
