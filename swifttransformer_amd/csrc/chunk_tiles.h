@@ -47,6 +47,30 @@ __device__ inline int chunks_before(int item, const int* __restrict__ item_len, 
     return __builtin_amdgcn_readfirstlane(sum);
 }
 
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// The matrix instruction for doubles (v_mfma_f64_16x16x4_f64) leaves rows g + 4 r of its result with a lane's group g, the one for floats
+// rows 4 g + r; with the first operand's rows dealt like this a lane gets what it gets from the one for floats.
+__device__ inline int double_row(int r16) { return 4 * (r16 & 3) + (r16 >> 2); }
+
+// e^x for x <= 0 to 2^-31 of itself (the Taylor sum up to r^8 on |r| <= ln(2) / 2), so that a weight is rounded to float once, with
+// all its factors; 0 below e^-200, which is none in float.  Doubles take as long as floats here, and a dozen of them no longer than
+// the library's expf.
+__device__ __forceinline__ double exp_le0_double(double x) {
+    x = x < -200.0 ? -200.0 : x;
+    const double n = rint(x * 1.4426950408889634), r = fma(n, -0.69314718055994531, x);
+    double y = 1.0 / 40320.0;
+    y = fma(y, r, 1.0 / 5040.0);
+    y = fma(y, r, 1.0 / 720.0);
+    y = fma(y, r, 1.0 / 120.0);
+    y = fma(y, r, 1.0 / 24.0);
+    y = fma(y, r, 1.0 / 6.0);
+    y = fma(y, r, 0.5);
+    y = fma(y, r, 1.0);
+    y = fma(y, r, 1.0);
+    return ldexp(y, (int)n);
+}
+
 // Four neighbouring floats of a row, zeros past its `limit` numbers or where the row does not exist.  VEC: the row starts
 // on 16 bytes and the limit is a multiple of 4.  (Addresses are clamped and values cleared rather than loads behind a
 // branch: the loads of a tile are then all on their way at once.)

@@ -2,8 +2,9 @@
 //
 //   S_t = diag(a_t) S_(t-1) + k_t v_t^T,   o_t = scale * S_t^T q_t,   y_t = o_t / rms(o_t) * gain * silu(gate_t)
 //
-// a_t = sigmoid(z_t)^(1 / tau) is a decay a key channel and token, between 0 and 1.  A chunk's outputs are products on the matrix cores (float,
-// v_mfma_f32_16x16x4_f32) once decays are folded into queries and keys.  Nothing is divided by a product of decays (it may be
+// a_t = sigmoid(z_t)^(1 / tau) is a decay a key channel and token, between 0 and 1.  A chunk's outputs are products on the matrix cores
+// once decays are folded into queries and keys.  Operands in memory and LDS are float; products of decays, sums and what meets them are
+// double (v_mfma_f64_16x16x4_f64): chains of 64 rows and channels in float were up to a fifth further from float64 than the scan.  Nothing is divided by a product of decays (it may be
 // zero): a chunk is four blocks of 16 rows, and only products over rows that lie between two points are formed, never above one:
 //
 //   q^_i = q_i * prod of a from its block's first row to i
@@ -21,10 +22,11 @@
 // LDS.
 //
 // Measured beside decay gates, scan and norm kernel (which sums the scan's planes): one item of 2,011 rows, 32 heads of 64 x 64,
-// 427 -> 64 us (the scan's 2,011 dependent steps; now the carry's 32, and the products at a few workgroups a unit); three items of
-// 2,048 rows together 219 -> 69; 32 heads of 128 x 128 637 -> 232; 33 rows 35 -> 24; 512 rows beside 24 single tokens 123 -> 32; 8
-// single tokens 34 -> 15, 24 of 32 heads of 128 x 128 58 -> 30 us.  Relative error against float64, all in float: state 9.7e-8 ->
-// 1.0e-7, read-outs 1.5e-7 -> 1.7e-7 (the scan sums 8 channels a plane), a tenth of what the float products around them lose.
+// 427 -> 99 us (the scan's 2,011 dependent steps; now the carry's 32, and the products at a few workgroups a unit; with everything in
+// float 65); three items of 2,048 rows together 219 -> 107; 32 heads of 128 x 128 637 -> 304; 33 rows 35 -> 31; 512 rows beside 24 single
+// tokens 123 -> 49; 8 single tokens 34 -> 15, 24 of 32 heads of 128 x 128 58 -> 29 us.  Relative distance from float64 behind norm and
+// gate, in float: 2,011 rows outputs 1.5e-7 -> 9.3e-8, state 9.6e-8 -> 6.5e-8; 33 rows 1.4e-7 -> 7.7e-8 and 4.4e-8 -> 3.2e-8; 48 single
+// tokens 1.4e-7 -> 1.2e-7 and 3.6e-8 -> 3.5e-8 (with everything in float 1.7e-7 and 9.9e-8, 1.3e-7 and 5.0e-8, 1.4e-7 and 3.9e-8).
 #include "api.h"
 #include "common.h"
 #include "chunk_tiles.h"
@@ -37,15 +39,22 @@ namespace st {
 
 constexpr int kGlaShort = 16;        // rows up to which an item is walked row by row
 
-// sigmoid(z)^inv_tau = 2^(inv_tau (log2(e) min(z, 0) - log2(1 + e^-|z|))) with what the products' roundings lost; 1 for the
-// largest float, which stands for rows that do not exist.  (The exponent is right to 2^-24 of itself or of one, as it is by the
-// library's functions, which take five times as long: 85 against 62 us for 2,011 rows of 32 heads.)
+// sigmoid(z)^inv_tau = e^(inv_tau (min(z, 0) - log(1 + e^-|z|))), rounded to float once; 1 for the largest float, which stands for
+// rows that do not exist.  log(1 + u) = 2 artanh(u / (2 + u)), nine terms of its series for u up to 1 (the tenth is below 2^-32).  (The
+// library's float functions, off by up to 2^-24 each, take 23 us more for 2,011 rows of 32 heads of 64.)
 __device__ inline float gla_decay(float z, float inv_tau) {
-    const float u = exp_le0(-fabsf(z));
-    const float m = z < -1e30f ? -1e30f : z < 0.f ? z : 0.f, t = m * 1.44269504f;
-    const float l = (t - __builtin_amdgcn_logf(1.f + u)) + (fmaf(m, 1.44269504f, -t) + m * 1.92596299e-8f);
-    const float e = l * inv_tau, p = __builtin_amdgcn_exp2f(e);
-    return fmaf(p, fmaf(l, inv_tau, -e) * 0.693147181f, p);
+    const double u = exp_le0_double(-fabs((double)z));
+    const double r0 = __builtin_amdgcn_rcpf((float)(2.0 + u)), s = u * (r0 * fma(-(2.0 + u), r0, 2.0)), s2 = s * s;
+    double y = 1.0 / 17.0;
+    y = fma(y, s2, 1.0 / 15.0);
+    y = fma(y, s2, 1.0 / 13.0);
+    y = fma(y, s2, 1.0 / 11.0);
+    y = fma(y, s2, 1.0 / 9.0);
+    y = fma(y, s2, 1.0 / 7.0);
+    y = fma(y, s2, 1.0 / 5.0);
+    y = fma(y, s2, 1.0 / 3.0);
+    y = fma(y, s2, 1.0);
+    return (float)exp_le0_double(((z < 0.f ? (double)z : 0.0) - 2.0 * s * y) * inv_tau);
 }
 
 // four neighbouring numbers of a row as floats, `fill` past its end or where the row does not exist (see load_piece)
@@ -102,7 +111,7 @@ struct GlaTile {
 };
 
 // U[idx, head] [dk, dv] and A[idx, head] [dk].  Grid (heads, chunks, blocks of 64 value channels); a wave takes rows of 16 x 16
-// tiles.  KQ: dk <= 4 KQ.  LDS: k [64][4 KQ + 4] | a [64][4 KQ + 4] | v [64][68] | B [4][4 KQ].
+// tiles.  KQ: dk <= 4 KQ.  LDS: k [64][4 KQ + 4] | a [64][4 KQ + 4] | v [64][68] | B doubles [4][4 KQ].
 template <typename T, int KQ, bool VEC>
 __global__ __launch_bounds__(256) void gla_sums_kernel(
     float* __restrict__ U, float* __restrict__ A, const T* __restrict__ k, int64_t k_stride, const T* __restrict__ v, int64_t v_stride,
@@ -119,7 +128,7 @@ __global__ __launch_bounds__(256) void gla_sums_kernel(
     float* ks = gla_lds;
     float* as = ks + 64 * KS;
     float* vs = as + 64 * KS;
-    float* bp = vs + 64 * VS;
+    double* bp = reinterpret_cast<double*>(vs + 64 * VS);
     const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
     {
         GlaTile<KQ> tk, ta;
@@ -132,7 +141,7 @@ __global__ __launch_bounds__(256) void gla_sums_kernel(
         tv.store(vs, VS);
     }
     __syncthreads();
-    // a wave's block of 16 rows: each key times the decays behind it in the block, then those of the blocks behind
+    // a wave's block of 16 rows: each key times the decays behind it in the block (those of the blocks behind meet it in the product)
     float* kw = ks + wave * 16 * KS;
     const float* aw = as + wave * 16 * KS;
     for (int c = lane; c < 4 * KQ; c += 64) {
@@ -142,31 +151,32 @@ __global__ __launch_bounds__(256) void gla_sums_kernel(
             kw[j * KS + c] = (float)(kw[j * KS + c] * run);
             run *= aw[j * KS + c];
         }
-        bp[wave * 4 * KQ + c] = (float)run;
+        bp[wave * 4 * KQ + c] = run;
     }
     __syncthreads();
-    for (int c = lane; c < 4 * KQ; c += 64) {
-        float run = 1.f;
-        for (int w = wave + 1; w < 4; ++w) run *= bp[w * 4 * KQ + c];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) kw[j * KS + c] *= run;
-        if (wave == 0 && blockIdx.z == 0 && c < dk) A[((int64_t)idx * heads + head) * dk + c] = run * bp[c];
-    }
-    __syncthreads();
+    const int p16 = double_row(r16);
     const int steps = (n + 15) >> 4, ktiles = (dk + 15) >> 4;    // steps of 16 keys
     float* u = U + ((int64_t)idx * heads + head) * dk * dv;
     for (int kt = wave; kt < ktiles; kt += 4) {
-        floatx4 acc[4];
+        double behind[4];
+        behind[3] = 1.0;
 #pragma unroll
-        for (int vt = 0; vt < 4; ++vt) acc[vt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        for (int s = 0; s < steps; ++s) {
+        for (int s = 2; s >= 0; --s) behind[s] = behind[s + 1] * bp[(s + 1) * 4 * KQ + 16 * kt + p16];
+        if (blockIdx.z == 0 && g == 0 && 16 * kt + p16 < dk)
+            A[((int64_t)idx * heads + head) * dk + 16 * kt + p16] = (float)(behind[0] * bp[16 * kt + p16]);
+        doublex4 acc[4];
+#pragma unroll
+        for (int vt = 0; vt < 4; ++vt) acc[vt] = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (s >= steps) continue;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int j = 16 * s + 4 * g + r;
-                const float x = ks[j * KS + 16 * kt + r16];
+                const double x = ks[j * KS + 16 * kt + p16] * behind[s];
 #pragma unroll
                 for (int vt = 0; vt < 4; ++vt)
-                    acc[vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, vs[j * VS + 16 * vt + r16], acc[vt], 0, 0, 0);
+                    acc[vt] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, (double)vs[j * VS + 16 * vt + r16], acc[vt], 0, 0, 0);
             }
         }
         // acc[vt][r]: key channel 16 kt + 4 g + r, value channel 16 vt + r16
@@ -177,7 +187,7 @@ __global__ __launch_bounds__(256) void gla_sums_kernel(
 #pragma unroll
             for (int vt = 0; vt < 4; ++vt) {
                 const int col = vb + 16 * vt + r16;
-                if (col < dv) u[(int64_t)kk * dv + col] = acc[vt][r];
+                if (col < dv) u[(int64_t)kk * dv + col] = (float)acc[vt][r];
             }
         }
     }
@@ -226,7 +236,7 @@ __global__ __launch_bounds__(256) void gla_carry_kernel(
 // Rows of a chunk, transposed as in the matrix memory's outputs: a wave has a block of 16 rows, lane (r16, g) row r16 of it with
 // the key channels 16 s + 4 g .. + 3; S^T = K Q^T leaves a lane with keys 4 g + r of its row, which is the next product's operand
 // as it lies (O^T += V^T P^T).  LDS: k [64][4 KQ + 4] | a [64][4 KQ + 4], later 64 key channels of the start state
-// [64][16 NV + 4] | v [64][16 NV + 4] | B [4][4 KQ].
+// [64][16 NV + 4] | v [64][16 NV + 4] | B doubles [4][4 KQ].
 //
 // An item of up to kGlaShort rows is walked here from its slot's state instead, row by row, and leaves its state there: 16 x less
 // traffic than a chunk for a single token.  Thread (wave, lane): KQ key channels from KQ * wave, value channels lane (and lane + 64);
@@ -269,9 +279,10 @@ __device__ __forceinline__ void gla_walk(float* lds, T* __restrict__ out, const 
     __syncthreads();
     for (int j = 0; j < n; ++j) {
         float* p = part + (j & 1) * 4 * V;
-        float vv[VL], acc[VL];
+        float vv[VL];
+        float4 acc[VL];                    // (sums in short chains)
 #pragma unroll
-        for (int u = 0; u < VL; ++u) { vv[u] = sv[j * V + lane + 64 * u]; acc[u] = 0.f; }
+        for (int u = 0; u < VL; ++u) { vv[u] = sv[j * V + lane + 64 * u]; acc[u] = make_float4(0.f, 0.f, 0.f, 0.f); }
 #pragma unroll
         for (int c = 0; c < KQ; c += 4) {
             const float4 q4 = *reinterpret_cast<const float4*>(sq + j * C + wave * KQ + c);
@@ -279,14 +290,14 @@ __device__ __forceinline__ void gla_walk(float* lds, T* __restrict__ out, const 
             const float4 a4 = *reinterpret_cast<const float4*>(sa + j * C + wave * KQ + c);
 #pragma unroll
             for (int u = 0; u < VL; ++u) {
-                S[c][u] = fmaf(a4.x, S[c][u], k4.x * vv[u]);         acc[u] = fmaf(S[c][u], q4.x, acc[u]);
-                S[c + 1][u] = fmaf(a4.y, S[c + 1][u], k4.y * vv[u]); acc[u] = fmaf(S[c + 1][u], q4.y, acc[u]);
-                S[c + 2][u] = fmaf(a4.z, S[c + 2][u], k4.z * vv[u]); acc[u] = fmaf(S[c + 2][u], q4.z, acc[u]);
-                S[c + 3][u] = fmaf(a4.w, S[c + 3][u], k4.w * vv[u]); acc[u] = fmaf(S[c + 3][u], q4.w, acc[u]);
+                S[c][u] = fmaf(a4.x, S[c][u], k4.x * vv[u]);         acc[u].x = fmaf(S[c][u], q4.x, acc[u].x);
+                S[c + 1][u] = fmaf(a4.y, S[c + 1][u], k4.y * vv[u]); acc[u].y = fmaf(S[c + 1][u], q4.y, acc[u].y);
+                S[c + 2][u] = fmaf(a4.z, S[c + 2][u], k4.z * vv[u]); acc[u].z = fmaf(S[c + 2][u], q4.z, acc[u].z);
+                S[c + 3][u] = fmaf(a4.w, S[c + 3][u], k4.w * vv[u]); acc[u].w = fmaf(S[c + 3][u], q4.w, acc[u].w);
             }
         }
 #pragma unroll
-        for (int u = 0; u < VL; ++u) p[wave * V + lane + 64 * u] = acc[u];
+        for (int u = 0; u < VL; ++u) p[wave * V + lane + 64 * u] = (acc[u].x + acc[u].y) + (acc[u].z + acc[u].w);
         __syncthreads();                   // (the other half of `part` was read before this row's sums were written)
         if (tid < V) so[j * V + tid] = (p[tid] + p[V + tid]) + (p[2 * V + tid] + p[3 * V + tid]);
     }
@@ -315,7 +326,7 @@ __device__ __forceinline__ void gla_walk(float* lds, T* __restrict__ out, const 
 
 // Steps of single tokens: grid (heads, items), a kernel of its own, whose few registers leave room for three workgroups a unit.
 template <typename T, int KQ, int NV>
-__global__ __launch_bounds__(256) void gla_walk_kernel(
+__global__ __launch_bounds__(256, 3) void gla_walk_kernel(
     T* __restrict__ out, const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k, int64_t k_stride, const T* __restrict__ v,
     int64_t v_stride, const float* __restrict__ z, float inv_tau, float* __restrict__ state, const T* __restrict__ gate, int64_t gate_stride,
     const float* __restrict__ gain, const int* __restrict__ item_len, const int* __restrict__ item_tok_off,
@@ -331,13 +342,13 @@ template <int KQ, int NV>
 struct GlaOutLds {
     static constexpr int KS = 4 * KQ + 4, VS = 16 * NV + 4;
     static constexpr int second = KS > VS ? 64 * KS : 64 * VS;
-    static constexpr size_t bytes = sizeof(float) * (size_t)(64 * KS + second + 64 * VS + 16 * KQ);
+    static constexpr size_t bytes = sizeof(float) * (size_t)(64 * KS + second + 64 * VS + 32 * KQ);
     static constexpr size_t walk = sizeof(float) * (size_t)(kGlaShort * (12 * KQ + 32 * NV) + 128 * NV);
     static_assert(walk <= bytes, "the short items' rows fit the chunks' LDS");
 };
 
 template <typename T, int KQ, int NV, bool VEC>
-__global__ __launch_bounds__(256) void gla_out_kernel(
+__global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void gla_out_kernel(
     T* __restrict__ out, const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k, int64_t k_stride, const T* __restrict__ v,
     int64_t v_stride, const float* __restrict__ z, float inv_tau, const float* __restrict__ S0, float* __restrict__ state, const T* __restrict__ gate, int64_t gate_stride,
     const float* __restrict__ gain, const int* __restrict__ item_len, const int* __restrict__ item_tok_off,
@@ -358,8 +369,8 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
     float* ks = gla_lds;
     float* as = ks + 64 * L::KS;
     float* vs = as + L::second;
-    float* bp = vs + 64 * L::VS;
-    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    double* bp = reinterpret_cast<double*>(vs + 64 * L::VS);
+    const int lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4, p16 = double_row(r16);
     const int i = wave * 16 + r16;                             // this lane's row of the chunk
     const bool row_ok = i < n;
     {
@@ -372,13 +383,13 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
         ta.store_decays(as, L::KS, inv_tau);
         tv.store(vs, L::VS);
     }
-    float qd[KQ];
+    double qd[KQ];
     {
         const T* qr = q + (row0 + min(i, n - 1)) * q_stride + (int64_t)head * dk;
 #pragma unroll
         for (int s = 0; s < KQ / 4; ++s) {
             const float4 x = gla_piece<T, VEC>(qr, 16 * s + 4 * g, dk, row_ok, 0.f);
-            qd[4 * s] = x.x * scale; qd[4 * s + 1] = x.y * scale; qd[4 * s + 2] = x.z * scale; qd[4 * s + 3] = x.w * scale;
+            qd[4 * s] = x.x * (double)scale; qd[4 * s + 1] = x.y * (double)scale; qd[4 * s + 2] = x.z * (double)scale; qd[4 * s + 3] = x.w * (double)scale;
         }
     }
     // the start state's first 64 key channels, on their way during the scores
@@ -386,10 +397,10 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
     GlaTile<4 * NV> ts;
     ts.template load<float, VEC>(s0, dv, min(dk, 64), 0, dv, 0.f);
     __syncthreads();
-    floatx4 st[4];
+    doublex4 st[4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) st[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    floatx4 diag = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 4; ++t) st[t] = doublex4{0.0, 0.0, 0.0, 0.0};
+    doublex4 diag = doublex4{0.0, 0.0, 0.0, 0.0};
     float* kw = ks + wave * 16 * L::KS + 4 * g;
     const float* aw = as + wave * 16 * L::KS + 4 * g;
     if (wave * 16 < n) {                                       // (uniform over the wave)
@@ -402,15 +413,17 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
                     qd[4 * s] *= f.x; qd[4 * s + 1] *= f.y; qd[4 * s + 2] *= f.z; qd[4 * s + 3] *= f.w;
                 }
             }
-            float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
+            double d[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int s = 0; s < KQ / 4; ++s) {
                 const float4 x = *reinterpret_cast<const float4*>(kw + j * L::KS + 16 * s);
-                d.x = fmaf(qd[4 * s], x.x, d.x); d.y = fmaf(qd[4 * s + 1], x.y, d.y);
-                d.z = fmaf(qd[4 * s + 2], x.z, d.z); d.w = fmaf(qd[4 * s + 3], x.w, d.w);
+                d[0] = fma(qd[4 * s], (double)x.x, d[0]); d[1] = fma(qd[4 * s + 1], (double)x.y, d[1]);
+                d[2] = fma(qd[4 * s + 2], (double)x.z, d[2]); d[3] = fma(qd[4 * s + 3], (double)x.w, d[3]);
             }
-            const float dot = rows4_sum((d.x + d.y) + (d.z + d.w));
-            if (g == j >> 2) diag[j & 3] = r16 >= j ? dot : 0.f;
+            double dot = (d[0] + d[1]) + (d[2] + d[3]);
+            dot += __shfl_xor(dot, 16, 64);
+            dot += __shfl_xor(dot, 32, 64);
+            if (g == j >> 2) diag[j & 3] = r16 >= j ? dot : 0.0;
         }
 #pragma unroll
         for (int s = 0; s < KQ / 4; ++s) {                     // the block's first row: qd is q^ now
@@ -427,7 +440,7 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
                 kc[j * L::KS] = (float)(kc[j * L::KS] * run);
                 run *= ac[j * L::KS];
             }
-            bp[wave * 4 * KQ + c] = (float)run;
+            bp[wave * 4 * KQ + c] = run;
         }
     }
     __syncthreads();
@@ -436,22 +449,21 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
         if (t >= wave || 16 * wave >= n) continue;             // uniform over the wave
 #pragma unroll
         for (int s = 0; s < KQ / 4; ++s) {
-            const float4 x = *reinterpret_cast<const float4*>(ks + (16 * t + r16) * L::KS + 16 * s + 4 * g);
-            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, qd[4 * s], st[t], 0, 0, 0);
-            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, qd[4 * s + 1], st[t], 0, 0, 0);
-            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, qd[4 * s + 2], st[t], 0, 0, 0);
-            st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, qd[4 * s + 3], st[t], 0, 0, 0);
+            const float4 x = *reinterpret_cast<const float4*>(ks + (16 * t + p16) * L::KS + 16 * s + 4 * g);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.x, qd[4 * s], st[t], 0, 0, 0);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.y, qd[4 * s + 1], st[t], 0, 0, 0);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.z, qd[4 * s + 2], st[t], 0, 0, 0);
+            st[t] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.w, qd[4 * s + 3], st[t], 0, 0, 0);
         }
 #pragma unroll
         for (int s = 0; s < KQ / 4; ++s) {
-            const float4 f = *reinterpret_cast<const float4*>(bp + t * 4 * KQ + 16 * s + 4 * g);
-            qd[4 * s] *= f.x; qd[4 * s + 1] *= f.y; qd[4 * s + 2] *= f.z; qd[4 * s + 3] *= f.w;
+            const double* f = bp + t * 4 * KQ + 16 * s + 4 * g;
+            qd[4 * s] *= f[0]; qd[4 * s + 1] *= f[1]; qd[4 * s + 2] *= f[2]; qd[4 * s + 3] *= f[3];
         }
     }
-    // (sums in short chains: the start state's in two, the keys' apart)
-    floatx4 o[NV], o1[NV], ok[NV];
+    doublex4 o[NV];
 #pragma unroll
-    for (int vt = 0; vt < NV; ++vt) o[vt] = o1[vt] = ok[vt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int vt = 0; vt < NV; ++vt) o[vt] = doublex4{0.0, 0.0, 0.0, 0.0};
     // what the chunk's start state gives
 #pragma unroll
     for (int b = 0; b < (KQ + 15) / 16; ++b) {
@@ -463,57 +475,51 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
             ts.template load<float, VEC>(s0 + (int64_t)64 * (b + 1) * dv, dv, min(dk - 64 * (b + 1), 64), 0, dv, 0.f);
 #pragma unroll
         for (int s = 0; s < (KQ < 16 ? KQ : 16); ++s) {
-            const float* sr = as + (16 * (s >> 2) + 4 * g + (s & 3)) * L::VS + r16;
+            const float* sr = as + (16 * (s >> 2) + 4 * g + (s & 3)) * L::VS + p16;
 #pragma unroll
-            for (int vt = 0; vt < NV; ++vt) {
-                floatx4& to = s & 1 ? o1[vt] : o[vt];
-                to = __builtin_amdgcn_mfma_f32_16x16x4f32(sr[16 * vt], qd[(16 * b + s) % KQ], to, 0, 0, 0);
-            }
+            for (int vt = 0; vt < NV; ++vt)
+                o[vt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)sr[16 * vt], qd[(16 * b + s) % KQ], o[vt], 0, 0, 0);
         }
     }
+    // A row meets the later rows of its block with a weight of zero, which an infinity or NaN among their values would turn into
+    // NaN: such a block's rows are summed one by one instead, below.
+    float zero = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int vt = 0; vt < NV; ++vt) zero = fmaf(vs[(16 * wave + 4 * g + r) * L::VS + 16 * vt + r16], 0.f, zero);
+    const bool finite = !__any(!(zero == 0.f));
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        if (t > wave || 16 * wave >= n) continue;
-        const floatx4 p = t == wave ? diag : st[t];
-        if (t == wave) {
-            // A row meets the later rows of its block with a weight of zero, which an infinity or NaN among their values would turn
-            // into NaN: such a block's rows are summed one by one.
-            float finite = 0.f;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int vt = 0; vt < NV; ++vt) finite = fmaf(vs[(16 * t + 4 * g + r) * L::VS + 16 * vt + r16], 0.f, finite);
-            if (__any(!(finite == 0.f))) {
-#pragma unroll 1
-                for (int j4 = 0; j4 < 4; ++j4)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float w = __shfl(p[e], r16 + 16 * j4, 64);
-                        if (4 * j4 + e <= r16)
-#pragma unroll
-                            for (int vt = 0; vt < NV; ++vt)
-#pragma unroll
-                                for (int r = 0; r < 4; ++r) ok[vt][r] = fmaf(w, vs[(16 * t + 4 * j4 + e) * L::VS + 16 * vt + 4 * g + r], ok[vt][r]);
-                        __builtin_amdgcn_sched_barrier(0);   // (one row's values in registers at a time)
-                    }
-                continue;
-            }
-        }
+        if (t > wave || 16 * wave >= n || (t == wave && !finite)) continue;
+        const doublex4 p = t == wave ? diag : st[t];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float* vr = vs + (16 * t + 4 * g + r) * L::VS + r16;
+            const float* vr = vs + (16 * t + 4 * g + r) * L::VS + p16;
 #pragma unroll
-            for (int vt = 0; vt < NV; ++vt) ok[vt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[16 * vt], p[r], ok[vt], 0, 0, 0);
+            for (int vt = 0; vt < NV; ++vt) o[vt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)vr[16 * vt], p[r], o[vt], 0, 0, 0);
         }
     }
+    if (!finite) {
+#pragma unroll 1
+        for (int j4 = 0; j4 < 4; ++j4)
 #pragma unroll
-    for (int vt = 0; vt < NV; ++vt) o[vt] = (o[vt] + o1[vt]) + ok[vt];
+            for (int e = 0; e < 4; ++e) {
+                const double w = __shfl(diag[e], r16 + 16 * j4, 64);
+                if (4 * j4 + e > r16) continue;
+#pragma unroll
+                for (int vt = 0; vt < NV; ++vt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[vt][r] = fma(w, (double)vs[(16 * wave + 4 * j4 + e) * L::VS + 16 * vt + 4 * g + r], o[vt][r]);
+            }
+    }
     // o[vt][r]: value channel 16 vt + 4 g + r of row i
     float ss = 0.f;
+    floatx4 of[NV];
 #pragma unroll
     for (int vt = 0; vt < NV; ++vt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ss = fmaf(o[vt][r], o[vt][r], ss);      // (channels past dv are zeros)
+        for (int r = 0; r < 4; ++r) { of[vt][r] = (float)o[vt][r]; ss = fmaf(of[vt][r], of[vt][r], ss); }      // (channels past dv are zeros)
     ss = rows4_sum(ss);
     if (!row_ok) return;
     const float rms = 1.f / sqrtf(ss / (float)dv + eps);
@@ -524,8 +530,8 @@ __global__ __launch_bounds__(256) void gla_out_kernel(
         const int v0 = 16 * vt + 4 * g;
         if (v0 >= dv) continue;
         const float4 x = gla_piece<T, VEC>(gr, v0, dv, true, 0.f), w = gla_piece<float, false>(gain, v0, dv, true, 0.f);
-        const float y[4] = {o[vt][0] * rms * w.x * (x.x / (1.f + expf(-x.x))), o[vt][1] * rms * w.y * (x.y / (1.f + expf(-x.y))),
-                            o[vt][2] * rms * w.z * (x.z / (1.f + expf(-x.z))), o[vt][3] * rms * w.w * (x.w / (1.f + expf(-x.w)))};
+        const float y[4] = {of[vt][0] * rms * w.x * (x.x / (1.f + expf(-x.x))), of[vt][1] * rms * w.y * (x.y / (1.f + expf(-x.y))),
+                            of[vt][2] * rms * w.z * (x.z / (1.f + expf(-x.z))), of[vt][3] * rms * w.w * (x.w / (1.f + expf(-x.w)))};
         if (VEC) Elem<T>::store4(dst + v0, y);
         else
             for (int r = 0; r < 4 && v0 + r < dv; ++r) Elem<T>::store(dst + v0 + r, y[r]);
@@ -536,7 +542,7 @@ template <typename T, int KQ, bool VEC>
 static int launch_gla_sums(float* U, float* A, const void* k, int64_t ks, const void* v, int64_t vs, const float* z, float inv_tau, const int* item_len,
                            const int* item_tok_off, const int* item_slot, int num_items, unsigned chunks, int heads, int dk, int dv,
                            hipStream_t stream) {
-    constexpr int kLds = (int)sizeof(float) * (2 * 64 * (4 * KQ + 4) + 64 * 68 + 16 * KQ);
+    constexpr int kLds = (int)sizeof(float) * (2 * 64 * (4 * KQ + 4) + 64 * 68 + 32 * KQ);
     ST_CHECK(hipFuncSetAttribute((const void*)gla_sums_kernel<T, KQ, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) == hipSuccess,
              "gla_chunks: cannot raise the LDS limit");
     gla_sums_kernel<T, KQ, VEC><<<dim3(heads, chunks, (dv + 63) / 64), 256, kLds, stream>>>(U, A, (const T*)k, ks, (const T*)v, vs, z, inv_tau, item_len,

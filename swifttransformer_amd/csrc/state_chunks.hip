@@ -34,12 +34,6 @@
 
 namespace st {
 
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-
-// The matrix instruction for doubles (v_mfma_f64_16x16x4_f64) leaves rows g + 4 r of its result with a lane's group g, the one for floats
-// rows 4 g + r; with the first operand's rows dealt like this a lane gets what it gets from the one for floats.
-__device__ inline int double_row(int r16) { return 4 * (r16 & 3) + (r16 >> 2); }
-
 constexpr int kStateShort = 16;      // rows up to which an item is walked row by row
 
 struct StateArgs {
@@ -69,24 +63,6 @@ __device__ inline double state_log_decays(const float* __restrict__ b, int64_t s
     return F;
 }
 
-// e^x for x <= 0 to 2^-31 of itself (the Taylor sum up to r^8 on |r| <= ln(2) / 2), so that a weight is rounded to float once, with
-// all its factors; 0 below e^-200, which is none in float.  Doubles take as long as floats here, and a dozen of them no longer than
-// the library's expf.
-__device__ __forceinline__ double state_exp(double x) {
-    x = x < -200.0 ? -200.0 : x;
-    const double n = rint(x * 1.4426950408889634), r = fma(n, -0.69314718055994531, x);
-    double y = 1.0 / 40320.0;
-    y = fma(y, r, 1.0 / 5040.0);
-    y = fma(y, r, 1.0 / 720.0);
-    y = fma(y, r, 1.0 / 120.0);
-    y = fma(y, r, 1.0 / 24.0);
-    y = fma(y, r, 1.0 / 6.0);
-    y = fma(y, r, 0.5);
-    y = fma(y, r, 1.0);
-    y = fma(y, r, 1.0);
-    return ldexp(y, (int)n);
-}
-
 // U[idx, head] and fall[idx, head].  Grid (heads, chunks, blocks of 64 value channels).  LDS: w doubles [64] | k [64][4 KQ + 4] | v [64][68].
 template <int KQ, bool VEC>
 __global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
@@ -109,8 +85,8 @@ __global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
     if (tid < 64) {
         const double F = state_log_decays(a.gate_b + row0 * a.gate_stride + head, a.gate_stride, n), last = __shfl(F, n - 1, 64);
         const float f = a.gate_a[(row0 + min(tid, n - 1)) * a.gate_stride + head];
-        w[tid] = tid < n ? f * state_exp(last - F) : 0.0;
-        if (blockIdx.z == 0 && tid == 0) a.fall[(int64_t)idx * a.heads + head] = (float)state_exp(last);
+        w[tid] = tid < n ? f * exp_le0_double(last - F) : 0.0;
+        if (blockIdx.z == 0 && tid == 0) a.fall[(int64_t)idx * a.heads + head] = (float)exp_le0_double(last);
     }
     tv.store(vs, VS);
     tk.store(ks, KS);
@@ -317,7 +293,7 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
     ts.template load<VEC>(s0, dv, min(dk, 64), 0, dv);
     __syncthreads();
     const double Fi = sF[i];
-    const double carried = state_exp(Fi);
+    const double carried = exp_le0_double(Fi);
     doublex4 st[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -334,7 +310,7 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int j = 16 * t + 4 * g + r;
-            st[t][r] = j <= i ? st[t][r] * (sa[j] * state_exp(Fi - sF[j])) : 0.0;
+            st[t][r] = j <= i ? st[t][r] * (sa[j] * exp_le0_double(Fi - sF[j])) : 0.0;
         }
     }
     doublex4 o[NV];

@@ -119,3 +119,37 @@ def test_a_number_that_is_not_finite_reaches_no_row_before_it(what, bad):
     assert torch.equal(s[0], s0[0]) and torch.equal(s[1, 1], s0[1, 1])
     hit = s[1, 0] if what == "q" else s[1, 0, :, 5] if what == "v" else s[1, 0, 5]
     assert torch.equal(s[1, 0], s0[1, 0]) if what == "q" else not bool(hit.isfinite().any())
+
+
+@pytest.mark.parametrize("lens,heads,kd,vd,tau", [((2011,), 8, 64, 64, 16.0), ((700, 600, 33), 8, 64, 128, 16.0), ((17,), 16, 64, 64, 4.0),
+                                                  ((33,), 16, 64, 64, 1.0), ((130,), 16, 64, 64, 1.0), ((257, 77), 6, 20, 36, 16.0),
+                                                  ((300,), 4, 128, 128, 16.0), ((1,) * 48, 16, 64, 64, 1.0), ((1,) * 24, 8, 128, 128, 16.0),
+                                                  ((16, 9, 2), 8, 128, 128, 16.0), ((500,), 16, 64, 64, 0.25)])
+def test_sums_are_no_further_from_float64_than_the_scans(lens, heads, kd, vd, tau):
+    """Against decay gates, the kernel that goes row by row, and the norm behind it, on the same numbers."""
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + kd)
+    T, B = sum(lens), len(lens)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    q, k, v, gate, z = rnd(T, heads * kd), rnd(T, heads * kd), rnd(T, heads * vd), rnd(T, heads * vd), rnd(T, heads * kd) * 2
+    state, gain, eps, scale = rnd(B, heads, kd, vd), torch.ones(vd, device=DEV), 1e-5, kd ** -0.5
+    off = [sum(lens[:i]) for i in range(B)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    items, single = (None, i32(list(lens)), i32(off), i32(list(range(B)))), max(lens) == 1
+    s, s0 = state.clone(), state.clone()
+    y = K.gla_chunks(q, k, v, z, tau, s, items, heads, scale, gate, gain, eps, single=single)
+    o = K.gla_scan(q, k, v, K.decay_gate(z.clone(), 1.0 / tau), s0, items, heads, scale, 16 if single else 8)
+    y0 = K.gated_head_norm(o, gate, gain, heads, eps, torch.float32)
+    f = lambda t, w: t.to(F64).view(T, heads, w)
+    q6, k6, v6, g6, a6 = f(q, kd) * scale, f(k, kd), f(v, vd), f(gate, vd), torch.sigmoid(f(z, kd)) ** (1.0 / tau)
+    want, last = torch.empty(T, heads, vd, dtype=F64, device=DEV), state.to(F64)
+    for b in range(B):
+        S = last[b]
+        for t in range(off[b], off[b] + lens[b]):
+            S = a6[t][:, :, None] * S + k6[t][:, :, None] * v6[t][:, None, :]
+            want[t] = (S * q6[t][:, :, None]).sum(1)
+        last[b] = S
+    want = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + eps) * (g6 * torch.sigmoid(g6))
+    err = lambda x, w: float((x.to(F64).view(w.shape) - w).norm() / w.norm())
+    assert err(y, want) <= err(y0, want), (err(y, want), err(y0, want))
+    assert err(s, last) <= err(s0, last), (err(s, last), err(s0, last))
