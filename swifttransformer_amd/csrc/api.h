@@ -150,7 +150,7 @@ int st_concat_cast(void* out, const float* a, int wa, const float* b, int wb, in
                    hipStream_t stream);
 
 // The additive form of st_state_scan over prompts and portions in chunks of 64 rows, for decays gate_b between 0 and 1
-// (csrc/state_chunks.hip); `single` (no item has more than 16 rows): row by row, any decay, no scratch.  Up to 128 key and value channels a
+// (csrc/state_chunks.hip); `single` (for steps of single tokens): row by row, any decay and length, no scratch.  Up to 128 key and value channels a
 // head.  scratch: scratch_chunks >= num_rows / 64 + num_items times heads * (key_dim * value_dim + 1) floats.
 int st_state_chunks(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v,
                     int64_t v_stride, const float* gate_a, const float* gate_b, int64_t gate_stride, const float* skip,

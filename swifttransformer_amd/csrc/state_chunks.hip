@@ -157,15 +157,14 @@ __global__ __launch_bounds__(256) void state_carry_kernel(StateArgs a) {
     *home = S;
 }
 
-// 64 value channels (from vb) of an item of up to kStateShort rows from its slot's state, row by row.  Thread (wave, lane): KQ key
+// 64 value channels (from vb) of up to kStateShort rows of an item from its slot's state, row by row.  Thread (wave, lane): KQ key
 // channels from KQ * wave, value channel vb + lane; the waves' partial read-outs meet in LDS once a row.  (Value channels never meet:
 // a wave with 128 of them holds twice the state and leaves a unit half as many workgroups: 49 against 31 us for 24 items of 32 heads of
 // 128 x 128.)
 template <int KQ>
-__device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int item, int head, int vb) {
+__device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int item, int64_t row0, int n, int head, int vb) {
     constexpr int C = 4 * KQ, V = 64;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = a.dk, dv = a.dv, n = a.item_len[item];
-    const int64_t row0 = a.item_tok_off[item];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = a.dk, dv = a.dv;
     const int group = head / (a.heads / a.qk_heads), col = vb + lane, colc = min(col, dv - 1);
     float* sq = lds;                       // [n][C], keys likewise, zeros past dk
     float* sk = sq + kStateShort * C;
@@ -222,13 +221,17 @@ __device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int i
     }
 }
 
-// Steps of single tokens: grid (heads, items, blocks of 64 value channels), a kernel of its own with few registers.
+// Steps of single tokens: grid (heads, items, blocks of 64 value channels), a kernel of its own with few registers.  (The caller's word
+// that there are no longer items is about speed: they are walked kStateShort rows at a time.)
 template <int KQ>
 __global__ __launch_bounds__(256) void state_walk_kernel(StateArgs a) {
     extern __shared__ __attribute__((aligned(16))) float state_lds[];
-    const int item = blockIdx.y;
-    if (a.item_slot[item] < 0 || a.item_len[item] <= 0 || a.item_len[item] > kStateShort) return;
-    state_walk<KQ>(state_lds, a, item, blockIdx.x, blockIdx.z * 64);
+    const int item = blockIdx.y, len = a.item_len[item];
+    if (a.item_slot[item] < 0) return;
+    for (int r = 0; r < len; r += kStateShort) {
+        if (r > 0) __syncthreads();                            // the rows before have been read
+        state_walk<KQ>(state_lds, a, item, (int64_t)a.item_tok_off[item] + r, min(kStateShort, len - r), blockIdx.x, blockIdx.z * 64);
+    }
 }
 
 // Rows of a chunk, transposed as in gla_chunks.hip and the matrix memory's outputs.  LDS: F doubles [64] | a [64] | k [64][4 KQ + 4],
@@ -252,7 +255,7 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
     if (a.item_len[item] <= kStateShort) {
         for (int vb = 0; vb < a.dv; vb += 64) {
             if (vb > 0) __syncthreads();                       // the rows before have been read
-            state_walk<KQ>(state_lds, a, item, head, vb);
+            state_walk<KQ>(state_lds, a, item, a.item_tok_off[item], a.item_len[item], head, vb);
         }
         return;
     }

@@ -1084,7 +1084,7 @@ def state_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_a: torch.
     rows, any stride; head h reads q/k head h // (heads / qk_heads)); state: float
     [slots, heads, key_dim, value_dim] (slots may be parts of a larger per-slot state).  ``max_item_rows``: a
     bound on the rows of any item where the caller knows one (1 in steps of single tokens; 0: the launch's
-    rows); it sizes the kernel's staging, nothing else.  ``chunks`` (additive; the caller's decays lie between 0 and 1): prompts
+    rows); it chooses the kernel and sizes its staging, and is about speed alone: longer items are computed all the same.  ``chunks`` (additive; the caller's decays lie between 0 and 1): prompts
     and portions go by chunks of 64 rows, up to ``STATE_CHUNK_DIM`` key and value channels a head.  Returns float [T, heads * value_dim]."""
     _token_item, item_len, item_tok_off, item_slot = ctx_arrays
     T = q.shape[0]

@@ -158,3 +158,25 @@ def test_sums_are_no_further_from_float64_than_the_scans(monkeypatch, lens, head
     # (prompts: 0.3 to 0.6 of the scan's; single rows 0.8, with the same state, whose one multiplication and addition are the scan's)
     assert err(y, want) <= err(y0, want), (err(y, want), err(y0, want))
     assert err(s, last) <= err(s0, last), (err(s, last), err(s0, last))
+
+
+@pytest.mark.parametrize("lens,kd,vd", [((40, 1, 17), 64, 64), ((1, 16, 33, 130), 20, 100)])
+def test_the_bound_on_an_items_rows_is_about_speed_alone(lens, kd, vd):
+    """Items longer than the caller's bound come out as without one (the walk's sums and the scan's: the same products, 64 of them in
+    another order)."""
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(kd)
+    heads, T, B = 4, sum(lens), len(lens)
+    x = torch.randn(T, heads * (2 * kd + vd), generator=g).to(DEV)
+    q, k, v = x.split([heads * kd, heads * kd, heads * vd], 1)
+    step = (torch.rand(T, heads, generator=g) * 0.1).to(DEV)
+    decay, state = torch.exp(-4 * step), torch.randn(B, heads, kd, vd, generator=g).to(DEV)
+    items = (None, i32(list(lens)), i32([sum(lens[:i]) for i in range(B)]), i32(list(range(B))[::-1]))
+
+    def run(q, k, v, state, bound):
+        s = state.clone()
+        return K.state_scan(q, k, v, step, decay, s, items, heads, "additive", max_item_rows=bound), s
+
+    (y, s), (y0, s0) = run(q, k, v, state, 1), run(q, k, v, state, 0)
+    ya, sa = run(q.abs(), k.abs(), v.abs(), state.abs(), 0)                    # the sums of magnitudes
+    assert bool(((y - y0).abs() <= 2 * UNIT * ya + 1e-30).all()) and bool(((s - s0).abs() <= 2 * UNIT * sa + 1e-30).all())
