@@ -324,7 +324,8 @@ __device__ __forceinline__ void gla_walk(float* lds, T* __restrict__ out, const 
     }
 }
 
-// Steps of single tokens: grid (heads, items), a kernel of its own, whose few registers leave room for three workgroups a unit.
+// Steps of single tokens: grid (heads, items), a kernel of its own, whose few registers leave room for three workgroups a unit.  (That
+// there are no longer items is about speed: they are walked kGlaShort rows at a time.)
 template <typename T, int KQ, int NV>
 __global__ __launch_bounds__(256, 3) void gla_walk_kernel(
     T* __restrict__ out, const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k, int64_t k_stride, const T* __restrict__ v,
@@ -332,10 +333,13 @@ __global__ __launch_bounds__(256, 3) void gla_walk_kernel(
     const float* __restrict__ gain, const int* __restrict__ item_len, const int* __restrict__ item_tok_off,
     const int* __restrict__ item_slot, int heads, int dk, int dv, float scale, float eps) {
     extern __shared__ __attribute__((aligned(16))) float gla_lds[];
-    const int head = blockIdx.x, item = blockIdx.y, slot = item_slot[item], n = item_len[item];
-    if (slot < 0 || n <= 0 || n > kGlaShort) return;
-    gla_walk<T, KQ, NV>(gla_lds, out, q, q_stride, k, k_stride, v, v_stride, z, inv_tau, state + ((int64_t)slot * heads + head) * dk * dv, gate,
-                        gate_stride, gain, item_tok_off[item], n, heads, head, dk, dv, scale, eps);
+    const int head = blockIdx.x, item = blockIdx.y, slot = item_slot[item], len = item_len[item];
+    if (slot < 0) return;
+    for (int r = 0; r < len; r += kGlaShort) {
+        if (r > 0) __syncthreads();                            // the rows before have been read
+        gla_walk<T, KQ, NV>(gla_lds, out, q, q_stride, k, k_stride, v, v_stride, z, inv_tau, state + ((int64_t)slot * heads + head) * dk * dv, gate,
+                            gate_stride, gain, (int64_t)item_tok_off[item] + r, min(kGlaShort, len - r), heads, head, dk, dv, scale, eps);
+    }
 }
 
 template <int KQ, int NV>
@@ -577,7 +581,7 @@ static int launch_gla_out(void* out, const void* q, int64_t qs, const void* k, i
 using namespace st;
 
 // scratch: float [chunks][heads][key_dim * value_dim] then [chunks][heads][key_dim], chunks = num_rows / 64 + num_items; not needed
-// (may be null) where no item has more than 16 rows, `single`
+// (may be null) for steps of single tokens, `single`
 extern "C" int st_gla_chunks(void* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
                              const float* z, float inv_tau, const void* gate, int64_t gate_stride, const float* gain, float* state, const int* item_len,
                              const int* item_tok_off, const int* item_slot, int num_items, int num_rows, int heads, int key_dim,

@@ -1270,7 +1270,7 @@ GLA_CHUNK_DIM = 128              # key and value channels a head that the chunk 
 def gla_chunks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, logits: torch.Tensor, tau: float, state: torch.Tensor, ctx_arrays, heads: int,
                scale: float, gate: torch.Tensor, gain: torch.Tensor, eps: float, single: bool = False) -> torch.Tensor:
     """``gated_head_norm(gla_scan(.., decay_gate(logits, 1 / tau), ..), gate, gain, ...)``: the recurrence as products within chunks of 64 rows and a carry between
-    chunks, norm and gate in the last kernel; items of up to 16 rows row by row.  ``single``: no item has more than one row.  Up to ``GLA_CHUNK_DIM`` key and value channels
+    chunks, norm and gate in the last kernel; items of up to 16 rows row by row.  ``single``: for steps of single tokens (longer items are computed all the same, row by row).  Up to ``GLA_CHUNK_DIM`` key and value channels
     a head; gate: rows like v's.  Rows of no item are left as they are."""
     _token_item, item_len, item_tok_off, item_slot = ctx_arrays
     T = q.shape[0]

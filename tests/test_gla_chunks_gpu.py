@@ -153,3 +153,22 @@ def test_sums_are_no_further_from_float64_than_the_scans(lens, heads, kd, vd, ta
     err = lambda x, w: float((x.to(F64).view(w.shape) - w).norm() / w.norm())
     assert err(y, want) <= err(y0, want), (err(y, want), err(y0, want))
     assert err(s, last) <= err(s0, last), (err(s, last), err(s0, last))
+
+
+@pytest.mark.parametrize("lens,kd,vd", [((40, 1, 17), 64, 64), ((1, 16, 33, 130), 20, 100), ((50,), 128, 128)])
+def test_items_of_a_step_said_to_be_single_may_be_longer(lens, kd, vd):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(kd)
+    heads, T, B = 3, sum(lens), len(lens)
+    q, k, v, gate, z = (torch.randn(T, heads * w, generator=g).to(DEV) for w in (kd, kd, vd, vd, kd))
+    state, gain = torch.randn(B, heads, kd, vd, generator=g).to(DEV), torch.ones(vd, device=DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    items = (None, i32(list(lens)), i32([sum(lens[:i]) for i in range(B)]), i32(list(range(B))[::-1]))
+
+    def run(single):
+        s = state.clone()
+        return K.gla_chunks(q, k, v, z, 4.0, s, items, heads, kd ** -0.5, gate, gain, 1e-5, single=single), s
+
+    (y, s), (y0, s0) = run(True), run(False)
+    # (the same float sums in another order: 256 roundings, of numbers up to 5 after the norm and 5 of the gate)
+    assert float((y - y0).abs().max()) < 256 * 2.0 ** -24 * 5 * 8 and float((s - s0).norm() / s0.norm()) < 1e-6
