@@ -151,7 +151,7 @@ int st_concat_cast(void* out, const float* a, int wa, const float* b, int wb, in
 
 // The additive form of st_state_scan over prompts and portions in chunks of 64 rows, for decays gate_b between 0 and 1
 // (csrc/state_chunks.hip); `single` (for steps of single tokens): row by row, any decay and length, no scratch.  Up to 128 key and value channels a
-// head.  scratch: scratch_chunks >= num_rows / 64 + num_items times heads * (key_dim * value_dim + 1) floats.
+// head.  scratch: scratch_chunks >= num_rows / 64 + min(num_items, num_rows / 17) times heads * (key_dim * value_dim + 1) floats.
 int st_state_chunks(float* out, const float* q, int64_t q_stride, const float* k, int64_t k_stride, const float* v,
                     int64_t v_stride, const float* gate_a, const float* gate_b, int64_t gate_stride, const float* skip,
                     float* state, int64_t slot_stride, const int* item_len, const int* item_tok_off, const int* item_slot,
@@ -229,8 +229,8 @@ int st_gla_scan(float* o_part, int64_t part_stride, int part_dim, const void* q,
 int st_gla_scan_parts(int key_dim, int part_dim);
 // The same recurrence, the head norm and the gate (as st_gated_head_norm) over prompts and portions, in chunks of 64 rows
 // (csrc/gla_chunks.hip): out [T, heads * value_dim] of `dtype`, rows of no item left as they are.  Up to 128 key and value channels
-// a head.  z [T, heads * key_dim]: the decays' logits, a = sigmoid(z)^inv_tau.  scratch: scratch_chunks >= num_rows / 64 + num_items times heads * key_dim * (value_dim + 1) floats; none where every
-// item has at most one row (`single`).
+// a head.  z [T, heads * key_dim]: the decays' logits, a = sigmoid(z)^inv_tau.  scratch: scratch_chunks >= num_rows / 64 + min(num_items,
+// num_rows / 17) times heads * key_dim * (value_dim + 1) floats; none for steps of single tokens (`single`: row by row).
 int st_gla_chunks(void* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
                   const float* z, float inv_tau, const void* gate, int64_t gate_stride, const float* gain, float* state, const int* item_len,
                   const int* item_tok_off, const int* item_slot, int num_items, int num_rows, int heads, int key_dim,

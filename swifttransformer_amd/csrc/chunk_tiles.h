@@ -7,17 +7,22 @@ namespace st {
 
 constexpr int kChunkRows = 64;       // counted from an item's first row of the step
 
-__device__ inline int chunks_of(int len, int slot, int rows) { return slot >= 0 && len > 0 ? (len + rows - 1) / rows : 0; }
+// an item's chunks: none for items of up to `least` rows, which the kernels that say so take without chunks
+__device__ inline int chunks_of(int len, int slot, int rows, int least = 0) { return slot >= 0 && len > least ? (len + rows - 1) / rows : 0; }
+// at most so many chunks has a step whose items have chunks from `least` + 1 rows on: every item's last one may be a short one
+inline int64_t most_chunks(int64_t rows, int64_t items, int least) {
+    return rows / kChunkRows + (items < rows / (least + 1) ? items : rows / (least + 1));
+}
 
 // The chunk of an item that a global chunk index means; false past the last one (`chunk` is then how far).  Whole waves: a lane an item, so that the items'
 // lengths are one trip to memory and not one after the other (48 rows beside 24 single tokens through gla_chunks: 109 -> 91 us).
 __device__ inline bool find_chunk(int idx, const int* __restrict__ item_len, const int* __restrict__ item_slot, int num_items, int& item,
-                                  int& chunk, int rows = kChunkRows) {
+                                  int& chunk, int rows = kChunkRows, int least = 0) {
     const int lane = threadIdx.x & 63;
     int base = 0;
     for (int b0 = 0; b0 < num_items; b0 += 64) {
         const int b = min(b0 + lane, num_items - 1), len = item_len[b], slot = item_slot[b];
-        const int own = b0 + lane < num_items ? chunks_of(len, slot, rows) : 0;
+        const int own = b0 + lane < num_items ? chunks_of(len, slot, rows, least) : 0;
         int upto = own;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -38,10 +43,11 @@ __device__ inline bool find_chunk(int idx, const int* __restrict__ item_len, con
 }
 
 // the chunks of all items before `item`; whole waves
-__device__ inline int chunks_before(int item, const int* __restrict__ item_len, const int* __restrict__ item_slot, int rows = kChunkRows) {
+__device__ inline int chunks_before(int item, const int* __restrict__ item_len, const int* __restrict__ item_slot, int rows = kChunkRows,
+                                    int least = 0) {
     const int lane = threadIdx.x & 63;
     int sum = 0;
-    for (int b = lane; b < item; b += 64) sum += chunks_of(item_len[b], item_slot[b], rows);
+    for (int b = lane; b < item; b += 64) sum += chunks_of(item_len[b], item_slot[b], rows, least);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
     return __builtin_amdgcn_readfirstlane(sum);

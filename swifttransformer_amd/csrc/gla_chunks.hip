@@ -120,8 +120,7 @@ __global__ __launch_bounds__(256) void gla_sums_kernel(
     extern __shared__ __attribute__((aligned(16))) float gla_lds[];
     const int head = blockIdx.x, idx = blockIdx.y, vb = blockIdx.z * 64, tid = threadIdx.x;
     int item, chunk;
-    if (!find_chunk(idx, item_len, item_slot, num_items, item, chunk)) return;
-    if (item_len[item] <= kGlaShort) return;
+    if (!find_chunk(idx, item_len, item_slot, num_items, item, chunk, kChunkRows, kGlaShort)) return;
     const int n = min(kChunkRows, item_len[item] - chunk * kChunkRows);
     const int64_t row0 = (int64_t)item_tok_off[item] + (int64_t)chunk * kChunkRows;
     constexpr int KS = 4 * KQ + 4, VS = 68;
@@ -202,7 +201,7 @@ __global__ __launch_bounds__(256) void gla_carry_kernel(
     const int e = blockIdx.z * 256 + threadIdx.x;
     const int slot = item_slot[item], len = item_len[item];
     if (slot < 0 || len <= kGlaShort) return;
-    const int base = chunks_before(item, item_len, item_slot);
+    const int base = chunks_before(item, item_len, item_slot, kChunkRows, kGlaShort);
     if (e >= dk * dv) return;
     const int chunks = (len + kChunkRows - 1) / kChunkRows;
     const int64_t plane = (int64_t)dk * dv, first = (int64_t)base * heads + head;
@@ -241,11 +240,12 @@ __global__ __launch_bounds__(256) void gla_carry_kernel(
 // An item of up to kGlaShort rows is walked here from its slot's state instead, row by row, and leaves its state there: 16 x less
 // traffic than a chunk for a single token.  Thread (wave, lane): KQ key channels from KQ * wave, value channels lane (and lane + 64);
 // the waves' partial read-outs meet in LDS once a row.
-template <typename T, int KQ, int NV>
+// LONG: any number of rows, kGlaShort of them in LDS at a time.
+template <typename T, int KQ, int NV, bool LONG>
 __device__ __forceinline__ void gla_walk(float* lds, T* __restrict__ out, const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k,
                                 int64_t k_stride, const T* __restrict__ v, int64_t v_stride, const float* __restrict__ z, float inv_tau,
                                 float* __restrict__ state, const T* __restrict__ gate, int64_t gate_stride, const float* __restrict__ gain,
-                                int64_t row0, int n, int heads, int head, int dk, int dv, float scale, float eps) {
+                                int64_t row0, int rows, int heads, int head, int dk, int dv, float scale, float eps) {
     constexpr int C = 4 * KQ, V = 16 * NV, VL = NV / 4;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float* sq = lds;                       // [n][C], k and a likewise, zeros past dk
@@ -263,44 +263,64 @@ __device__ __forceinline__ void gla_walk(float* lds, T* __restrict__ out, const 
             const float x = state[(int64_t)min(kk, dk - 1) * dv + min(col, dv - 1)];
             S[c][u] = kk < dk && col < dv ? x : 0.f;
         }
-    for (int e = tid; e < n * C; e += 256) {
-        const int j = e / C, c = e - j * C;
-        const int64_t at = (int64_t)head * dk + min(c, dk - 1), row = row0 + j;
-        const float x = Elem<T>::load(q + row * q_stride + at), y = Elem<T>::load(k + row * k_stride + at), f = gla_decay(z[row * heads * dk + at], inv_tau);
-        sq[e] = c < dk ? x * scale : 0.f;
-        sk[e] = c < dk ? y : 0.f;
-        sa[e] = c < dk ? f : 0.f;
-    }
-    for (int e = tid; e < n * V; e += 256) {
-        const int j = e / V, c = e - j * V;
-        const float x = Elem<T>::load(v + (row0 + j) * v_stride + (int64_t)head * dv + min(c, dv - 1));
-        sv[e] = c < dv ? x : 0.f;
-    }
-    __syncthreads();
-    for (int j = 0; j < n; ++j) {
-        float* p = part + (j & 1) * 4 * V;
-        float vv[VL];
-        float4 acc[VL];                    // (sums in short chains)
+    do {
+        const int n = LONG ? min(rows, kGlaShort) : rows;
+        for (int e = tid; e < n * C; e += 256) {
+            const int j = e / C, c = e - j * C;
+            const int64_t at = (int64_t)head * dk + min(c, dk - 1), row = row0 + j;
+            const float x = Elem<T>::load(q + row * q_stride + at), y = Elem<T>::load(k + row * k_stride + at), f = gla_decay(z[row * heads * dk + at], inv_tau);
+            sq[e] = c < dk ? x * scale : 0.f;
+            sk[e] = c < dk ? y : 0.f;
+            sa[e] = c < dk ? f : 0.f;
+        }
+        for (int e = tid; e < n * V; e += 256) {
+            const int j = e / V, c = e - j * V;
+            const float x = Elem<T>::load(v + (row0 + j) * v_stride + (int64_t)head * dv + min(c, dv - 1));
+            sv[e] = c < dv ? x : 0.f;
+        }
+        __syncthreads();
+        for (int j = 0; j < n; ++j) {
+            float* p = part + (j & 1) * 4 * V;
+            float vv[VL];
+            float4 acc[VL];                    // (sums in short chains)
 #pragma unroll
-        for (int u = 0; u < VL; ++u) { vv[u] = sv[j * V + lane + 64 * u]; acc[u] = make_float4(0.f, 0.f, 0.f, 0.f); }
+            for (int u = 0; u < VL; ++u) { vv[u] = sv[j * V + lane + 64 * u]; acc[u] = make_float4(0.f, 0.f, 0.f, 0.f); }
 #pragma unroll
-        for (int c = 0; c < KQ; c += 4) {
-            const float4 q4 = *reinterpret_cast<const float4*>(sq + j * C + wave * KQ + c);
-            const float4 k4 = *reinterpret_cast<const float4*>(sk + j * C + wave * KQ + c);
-            const float4 a4 = *reinterpret_cast<const float4*>(sa + j * C + wave * KQ + c);
+            for (int c = 0; c < KQ; c += 4) {
+                const float4 q4 = *reinterpret_cast<const float4*>(sq + j * C + wave * KQ + c);
+                const float4 k4 = *reinterpret_cast<const float4*>(sk + j * C + wave * KQ + c);
+                const float4 a4 = *reinterpret_cast<const float4*>(sa + j * C + wave * KQ + c);
+#pragma unroll
+                for (int u = 0; u < VL; ++u) {
+                    S[c][u] = fmaf(a4.x, S[c][u], k4.x * vv[u]);         acc[u].x = fmaf(S[c][u], q4.x, acc[u].x);
+                    S[c + 1][u] = fmaf(a4.y, S[c + 1][u], k4.y * vv[u]); acc[u].y = fmaf(S[c + 1][u], q4.y, acc[u].y);
+                    S[c + 2][u] = fmaf(a4.z, S[c + 2][u], k4.z * vv[u]); acc[u].z = fmaf(S[c + 2][u], q4.z, acc[u].z);
+                    S[c + 3][u] = fmaf(a4.w, S[c + 3][u], k4.w * vv[u]); acc[u].w = fmaf(S[c + 3][u], q4.w, acc[u].w);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < VL; ++u) p[wave * V + lane + 64 * u] = (acc[u].x + acc[u].y) + (acc[u].z + acc[u].w);
+            __syncthreads();                   // (the other half of `part` was read before this row's sums were written)
+            if (tid < V) so[j * V + tid] = (p[tid] + p[V + tid]) + (p[2 * V + tid] + p[3 * V + tid]);
+        }
+        __syncthreads();
+        for (int j = wave; j < n; j += 4) {
+            float x[VL], ss = 0.f;
+#pragma unroll
+            for (int u = 0; u < VL; ++u) { x[u] = so[j * V + lane + 64 * u]; ss = fmaf(x[u], x[u], ss); }
+            const float r = 1.f / sqrtf(wave_sum(ss) / (float)dv + eps);
 #pragma unroll
             for (int u = 0; u < VL; ++u) {
-                S[c][u] = fmaf(a4.x, S[c][u], k4.x * vv[u]);         acc[u].x = fmaf(S[c][u], q4.x, acc[u].x);
-                S[c + 1][u] = fmaf(a4.y, S[c + 1][u], k4.y * vv[u]); acc[u].y = fmaf(S[c + 1][u], q4.y, acc[u].y);
-                S[c + 2][u] = fmaf(a4.z, S[c + 2][u], k4.z * vv[u]); acc[u].z = fmaf(S[c + 2][u], q4.z, acc[u].z);
-                S[c + 3][u] = fmaf(a4.w, S[c + 3][u], k4.w * vv[u]); acc[u].w = fmaf(S[c + 3][u], q4.w, acc[u].w);
+                const int col = lane + 64 * u;
+                if (col >= dv) continue;
+                const float y = Elem<T>::load(gate + (row0 + j) * gate_stride + (int64_t)head * dv + col);
+                Elem<T>::store(out + ((row0 + j) * heads + head) * dv + col, x[u] * r * gain[col] * (y / (1.f + expf(-y))));
             }
         }
-#pragma unroll
-        for (int u = 0; u < VL; ++u) p[wave * V + lane + 64 * u] = (acc[u].x + acc[u].y) + (acc[u].z + acc[u].w);
-        __syncthreads();                   // (the other half of `part` was read before this row's sums were written)
-        if (tid < V) so[j * V + tid] = (p[tid] + p[V + tid]) + (p[2 * V + tid] + p[3 * V + tid]);
-    }
+        if (LONG) __syncthreads();             // the rows have been read
+        rows -= kGlaShort;
+        row0 += kGlaShort;
+    } while (LONG && rows > 0);
 #pragma unroll
     for (int c = 0; c < KQ; ++c)
 #pragma unroll
@@ -308,38 +328,25 @@ __device__ __forceinline__ void gla_walk(float* lds, T* __restrict__ out, const 
             const int kk = wave * KQ + c, col = lane + 64 * u;
             if (kk < dk && col < dv) state[(int64_t)kk * dv + col] = S[c][u];
         }
-    __syncthreads();
-    for (int j = wave; j < n; j += 4) {
-        float x[VL], ss = 0.f;
-#pragma unroll
-        for (int u = 0; u < VL; ++u) { x[u] = so[j * V + lane + 64 * u]; ss = fmaf(x[u], x[u], ss); }
-        const float r = 1.f / sqrtf(wave_sum(ss) / (float)dv + eps);
-#pragma unroll
-        for (int u = 0; u < VL; ++u) {
-            const int col = lane + 64 * u;
-            if (col >= dv) continue;
-            const float y = Elem<T>::load(gate + (row0 + j) * gate_stride + (int64_t)head * dv + col);
-            Elem<T>::store(out + ((row0 + j) * heads + head) * dv + col, x[u] * r * gain[col] * (y / (1.f + expf(-y))));
-        }
-    }
 }
 
 // Steps of single tokens: grid (heads, items), a kernel of its own, whose few registers leave room for three workgroups a unit.  (That
-// there are no longer items is about speed: they are walked kGlaShort rows at a time.)
+// there are no longer items is about speed alone: the second walk takes them, at the price of registers in scratch.)
 template <typename T, int KQ, int NV>
-__global__ __launch_bounds__(256, 3) void gla_walk_kernel(
+__global__ __launch_bounds__(256, KQ * NV <= 64 ? 6 : KQ * NV <= 128 ? 4 : 3) void gla_walk_kernel(
     T* __restrict__ out, const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k, int64_t k_stride, const T* __restrict__ v,
     int64_t v_stride, const float* __restrict__ z, float inv_tau, float* __restrict__ state, const T* __restrict__ gate, int64_t gate_stride,
     const float* __restrict__ gain, const int* __restrict__ item_len, const int* __restrict__ item_tok_off,
     const int* __restrict__ item_slot, int heads, int dk, int dv, float scale, float eps) {
     extern __shared__ __attribute__((aligned(16))) float gla_lds[];
     const int head = blockIdx.x, item = blockIdx.y, slot = item_slot[item], len = item_len[item];
-    if (slot < 0) return;
-    for (int r = 0; r < len; r += kGlaShort) {
-        if (r > 0) __syncthreads();                            // the rows before have been read
-        gla_walk<T, KQ, NV>(gla_lds, out, q, q_stride, k, k_stride, v, v_stride, z, inv_tau, state + ((int64_t)slot * heads + head) * dk * dv, gate,
-                            gate_stride, gain, (int64_t)item_tok_off[item] + r, min(kGlaShort, len - r), heads, head, dk, dv, scale, eps);
-    }
+    if (slot < 0 || len <= 0) return;
+    if (len <= kGlaShort)
+        gla_walk<T, KQ, NV, false>(gla_lds, out, q, q_stride, k, k_stride, v, v_stride, z, inv_tau, state + ((int64_t)slot * heads + head) * dk * dv, gate,
+                            gate_stride, gain, item_tok_off[item], len, heads, head, dk, dv, scale, eps);
+    else
+        gla_walk<T, KQ, NV, true>(gla_lds, out, q, q_stride, k, k_stride, v, v_stride, z, inv_tau, state + ((int64_t)slot * heads + head) * dk * dv, gate,
+                            gate_stride, gain, item_tok_off[item], len, heads, head, dk, dv, scale, eps);
 }
 
 template <int KQ, int NV>
@@ -356,18 +363,19 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void gla_out_kern
     T* __restrict__ out, const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k, int64_t k_stride, const T* __restrict__ v,
     int64_t v_stride, const float* __restrict__ z, float inv_tau, const float* __restrict__ S0, float* __restrict__ state, const T* __restrict__ gate, int64_t gate_stride,
     const float* __restrict__ gain, const int* __restrict__ item_len, const int* __restrict__ item_tok_off,
-    const int* __restrict__ item_slot, int num_items, int heads, int dk, int dv, float scale, float eps) {
+    const int* __restrict__ item_slot, int num_items, int chunks, int heads, int dk, int dv, float scale, float eps) {
     extern __shared__ __attribute__((aligned(16))) float gla_lds[];
     using L = GlaOutLds<KQ, NV>;
     const int head = blockIdx.x, idx = blockIdx.y, tid = threadIdx.x;
-    int item, chunk;
-    if (!find_chunk(idx, item_len, item_slot, num_items, item, chunk)) return;
-    if (item_len[item] <= kGlaShort) {
-        gla_walk<T, KQ, NV>(gla_lds, out, q, q_stride, k, k_stride, v, v_stride, z, inv_tau,
+    int item = idx - chunks, chunk;
+    if (item >= 0) {
+        if (item_slot[item] < 0 || item_len[item] <= 0 || item_len[item] > kGlaShort) return;
+        gla_walk<T, KQ, NV, false>(gla_lds, out, q, q_stride, k, k_stride, v, v_stride, z, inv_tau,
                             state + ((int64_t)item_slot[item] * heads + head) * dk * dv, gate, gate_stride, gain, item_tok_off[item],
                             item_len[item], heads, head, dk, dv, scale, eps);
         return;
     }
+    if (!find_chunk(idx, item_len, item_slot, num_items, item, chunk, kChunkRows, kGlaShort)) return;
     const int n = min(kChunkRows, item_len[item] - chunk * kChunkRows);
     const int64_t row0 = (int64_t)item_tok_off[item] + (int64_t)chunk * kChunkRows;
     float* ks = gla_lds;
@@ -569,9 +577,9 @@ static int launch_gla_out(void* out, const void* q, int64_t qs, const void* k, i
     }
     ST_CHECK(hipFuncSetAttribute((const void*)gla_out_kernel<T, KQ, NV, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds) == hipSuccess,
              "gla_chunks: cannot raise the LDS limit");
-    gla_out_kernel<T, KQ, NV, VEC><<<dim3(heads, chunks), 256, kLds, stream>>>((T*)out, (const T*)q, qs, (const T*)k, ks,
+    gla_out_kernel<T, KQ, NV, VEC><<<dim3(heads, chunks + num_items), 256, kLds, stream>>>((T*)out, (const T*)q, qs, (const T*)k, ks,
         (const T*)v, vs, z, inv_tau, S0, state,
-        (const T*)gate, gs, gain, item_len, item_tok_off, item_slot, num_items, heads, dk, dv, scale, eps);
+        (const T*)gate, gs, gain, item_len, item_tok_off, item_slot, num_items, (int)chunks, heads, dk, dv, scale, eps);
     ST_LAUNCH_CHECK("gla_chunks (outputs)");
     return 0;
 }
@@ -580,8 +588,9 @@ static int launch_gla_out(void* out, const void* q, int64_t qs, const void* k, i
 
 using namespace st;
 
-// scratch: float [chunks][heads][key_dim * value_dim] then [chunks][heads][key_dim], chunks = num_rows / 64 + num_items; not needed
-// (may be null) for steps of single tokens, `single`
+// scratch: float [chunks][heads][key_dim * value_dim] then [chunks][heads][key_dim], chunks = num_rows / 64 and one more for each of
+// the items that may have more than 16 rows (num_items, or num_rows / 17 where that is less); may be null where that is none, and for
+// steps of single tokens, `single`
 extern "C" int st_gla_chunks(void* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
                              const float* z, float inv_tau, const void* gate, int64_t gate_stride, const float* gain, float* state, const int* item_len,
                              const int* item_tok_off, const int* item_slot, int num_items, int num_rows, int heads, int key_dim,
@@ -591,10 +600,10 @@ extern "C" int st_gla_chunks(void* out, const void* q, int64_t q_stride, const v
     ST_CHECK(dtype == kF32 || dtype == kBF16, "gla_chunks: unknown dtype %d", dtype);
     ST_CHECK(eps > 0.f, "gla_chunks: eps must be positive");
     if (num_items == 0 || num_rows == 0) return 0;
-    ST_CHECK(out && q && k && v && z && gate && gain && state && item_len && item_tok_off && item_slot && (scratch || single), "gla_chunks: null operand");
-    const int64_t chunks = single ? num_items : num_rows / kChunkRows + num_items;   // (every item's last chunk may be a short one)
-    ST_CHECK(single || scratch_chunks >= chunks, "gla_chunks: scratch for %lld chunks, %lld needed", (long long)scratch_chunks, (long long)chunks);
-    ST_CHECK(chunks <= 65535 && num_items <= 65535, "gla_chunks: too many chunks or items");
+    ST_CHECK(out && q && k && v && z && gate && gain && state && item_len && item_tok_off && item_slot, "gla_chunks: null operand");
+    const int64_t chunks = single ? 0 : most_chunks(num_rows, num_items, kGlaShort);
+    ST_CHECK(chunks == 0 || (scratch && scratch_chunks >= chunks), "gla_chunks: scratch for %lld chunks, %lld needed", (long long)scratch_chunks, (long long)chunks);
+    ST_CHECK(chunks + num_items <= 65535, "gla_chunks: too many chunks or items");
     float* U = scratch;
     float* A = scratch + scratch_chunks * heads * key_dim * value_dim;
     // four numbers at a time: rows and heads start on their size, and the tables on 16 bytes
@@ -613,7 +622,7 @@ extern "C" int st_gla_chunks(void* out, const void* q, int64_t q_stride, const v
         if (dtype == kF32) { if (vec) what(float, __VA_ARGS__, true); else what(float, __VA_ARGS__, false); }      \
         else { if (vec) what(bf16_t, __VA_ARGS__, true); else what(bf16_t, __VA_ARGS__, false); }                  \
     } while (0)
-    if (!single) {
+    if (chunks) {
         if (key_dim <= 64) ST_GLA_T(ST_GLA_SUMS, 16);
         else ST_GLA_T(ST_GLA_SUMS, 32);
         if (rc) return rc;

@@ -47,7 +47,7 @@ struct StateArgs {
     int64_t slot_stride;
     float *U, *fall;                 // [chunks][heads][dk * dv], [chunks][heads]
     const int *item_len, *item_tok_off, *item_slot;
-    int num_items, heads, qk_heads, dk, dv;
+    int num_items, heads, qk_heads, dk, dv, chunks;
 };
 
 // the first wave: F_i of a chunk's n rows; past them the last one's
@@ -69,8 +69,7 @@ __global__ __launch_bounds__(256) void state_sums_kernel(StateArgs a) {
     extern __shared__ __attribute__((aligned(16))) float state_lds[];
     const int head = blockIdx.x, idx = blockIdx.y, vb = blockIdx.z * 64, tid = threadIdx.x;
     int item, chunk;
-    if (!find_chunk(idx, a.item_len, a.item_slot, a.num_items, item, chunk)) return;
-    if (a.item_len[item] <= kStateShort) return;
+    if (!find_chunk(idx, a.item_len, a.item_slot, a.num_items, item, chunk, kChunkRows, kStateShort)) return;
     const int n = min(kChunkRows, a.item_len[item] - chunk * kChunkRows), dk = a.dk, dv = a.dv;
     const int64_t row0 = (int64_t)a.item_tok_off[item] + (int64_t)chunk * kChunkRows;
     const int group = head / (a.heads / a.qk_heads);
@@ -127,7 +126,7 @@ __global__ __launch_bounds__(256) void state_carry_kernel(StateArgs a) {
     const int e = blockIdx.z * 256 + threadIdx.x;
     const int slot = a.item_slot[item], len = a.item_len[item];
     if (slot < 0 || len <= kStateShort) return;
-    const int base = chunks_before(item, a.item_len, a.item_slot), chunks = (len + kChunkRows - 1) / kChunkRows;
+    const int base = chunks_before(item, a.item_len, a.item_slot, kChunkRows, kStateShort), chunks = (len + kChunkRows - 1) / kChunkRows;
     if (e >= a.dk * a.dv) return;
     const int64_t plane = (int64_t)a.dk * a.dv, first = (int64_t)base * a.heads + head;
     float* home = a.state + (int64_t)slot * a.slot_stride + (int64_t)head * plane + e;
@@ -157,14 +156,16 @@ __global__ __launch_bounds__(256) void state_carry_kernel(StateArgs a) {
     *home = S;
 }
 
-// 64 value channels (from vb) of up to kStateShort rows of an item from its slot's state, row by row.  Thread (wave, lane): KQ key
+// 64 value channels (from vb) of an item of up to kStateShort rows from its slot's state, row by row.  Thread (wave, lane): KQ key
 // channels from KQ * wave, value channel vb + lane; the waves' partial read-outs meet in LDS once a row.  (Value channels never meet:
 // a wave with 128 of them holds twice the state and leaves a unit half as many workgroups: 49 against 31 us for 24 items of 32 heads of
 // 128 x 128.)
-template <int KQ>
-__device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int item, int64_t row0, int n, int head, int vb) {
+// LONG: any number of rows, kStateShort of them in LDS at a time.
+template <int KQ, bool LONG>
+__device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int item, int rows, int head, int vb) {
     constexpr int C = 4 * KQ, V = 64;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = a.dk, dv = a.dv;
+    int64_t row0 = a.item_tok_off[item];
     const int group = head / (a.heads / a.qk_heads), col = vb + lane, colc = min(col, dv - 1);
     float* sq = lds;                       // [n][C], keys likewise, zeros past dk
     float* sk = sq + kStateShort * C;
@@ -179,41 +180,47 @@ __device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int i
         const float x = home[(int64_t)min(kk, dk - 1) * dv + colc];
         S[c] = kk < dk && col < dv ? x : 0.f;
     }
-    for (int e = tid; e < n * C; e += 256) {
-        const int j = e / C, c = e - j * C;
-        const int64_t at = (int64_t)group * dk + min(c, dk - 1), row = row0 + j;
-        const float x = a.q[row * a.q_stride + at], y = a.k[row * a.k_stride + at];
-        sq[e] = c < dk ? x : 0.f;
-        sk[e] = c < dk ? y : 0.f;
-    }
-    for (int j = wave; j < n; j += 4) {
-        const float x = a.v[(row0 + j) * a.v_stride + (int64_t)head * dv + colc];
-        sv[j * V + lane] = col < dv ? x : 0.f;
-    }
-    if (tid < n) {
-        sb[tid] = a.gate_b[(row0 + tid) * a.gate_stride + head];
-        sb[kStateShort + tid] = a.gate_a[(row0 + tid) * a.gate_stride + head];
-    }
     const float skip = a.skip ? a.skip[head] : 0.f;
-    __syncthreads();
-    for (int j = 0; j < n; ++j) {
-        float* p = part + (j & 1) * 4 * V;
-        const float b = sb[j], vv = sv[j * V + lane], av = sb[kStateShort + j] * vv;
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};                   // (sums in short chains)
-#pragma unroll
-        for (int c = 0; c < KQ; c += 4) {
-            const float4 q4 = *reinterpret_cast<const float4*>(sq + j * C + wave * KQ + c);
-            const float4 k4 = *reinterpret_cast<const float4*>(sk + j * C + wave * KQ + c);
-            S[c] = fmaf(b, S[c], k4.x * av);         acc[0] = fmaf(S[c], q4.x, acc[0]);
-            S[c + 1] = fmaf(b, S[c + 1], k4.y * av); acc[1] = fmaf(S[c + 1], q4.y, acc[1]);
-            S[c + 2] = fmaf(b, S[c + 2], k4.z * av); acc[2] = fmaf(S[c + 2], q4.z, acc[2]);
-            S[c + 3] = fmaf(b, S[c + 3], k4.w * av); acc[3] = fmaf(S[c + 3], q4.w, acc[3]);
+    do {
+        const int n = LONG ? min(rows, kStateShort) : rows;
+        for (int e = tid; e < n * C; e += 256) {
+            const int j = e / C, c = e - j * C;
+            const int64_t at = (int64_t)group * dk + min(c, dk - 1), row = row0 + j;
+            const float x = a.q[row * a.q_stride + at], y = a.k[row * a.k_stride + at];
+            sq[e] = c < dk ? x : 0.f;
+            sk[e] = c < dk ? y : 0.f;
         }
-        p[wave * V + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        __syncthreads();                   // (the other half of `part` was read before this row's sums were written)
-        if (wave == 0 && col < dv)
-            a.out[((row0 + j) * a.heads + head) * dv + col] = fmaf(skip, vv, (p[lane] + p[V + lane]) + (p[2 * V + lane] + p[3 * V + lane]));
-    }
+        for (int j = wave; j < n; j += 4) {
+            const float x = a.v[(row0 + j) * a.v_stride + (int64_t)head * dv + colc];
+            sv[j * V + lane] = col < dv ? x : 0.f;
+        }
+        if (tid < n) {
+            sb[tid] = a.gate_b[(row0 + tid) * a.gate_stride + head];
+            sb[kStateShort + tid] = a.gate_a[(row0 + tid) * a.gate_stride + head];
+        }
+        __syncthreads();
+        for (int j = 0; j < n; ++j) {
+            float* p = part + (j & 1) * 4 * V;
+            const float b = sb[j], vv = sv[j * V + lane], av = sb[kStateShort + j] * vv;
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};                   // (sums in short chains)
+#pragma unroll
+            for (int c = 0; c < KQ; c += 4) {
+                const float4 q4 = *reinterpret_cast<const float4*>(sq + j * C + wave * KQ + c);
+                const float4 k4 = *reinterpret_cast<const float4*>(sk + j * C + wave * KQ + c);
+                S[c] = fmaf(b, S[c], k4.x * av);         acc[0] = fmaf(S[c], q4.x, acc[0]);
+                S[c + 1] = fmaf(b, S[c + 1], k4.y * av); acc[1] = fmaf(S[c + 1], q4.y, acc[1]);
+                S[c + 2] = fmaf(b, S[c + 2], k4.z * av); acc[2] = fmaf(S[c + 2], q4.z, acc[2]);
+                S[c + 3] = fmaf(b, S[c + 3], k4.w * av); acc[3] = fmaf(S[c + 3], q4.w, acc[3]);
+            }
+            p[wave * V + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            __syncthreads();                   // (the other half of `part` was read before this row's sums were written)
+            if (wave == 0 && col < dv)
+                a.out[((row0 + j) * a.heads + head) * dv + col] = fmaf(skip, vv, (p[lane] + p[V + lane]) + (p[2 * V + lane] + p[3 * V + lane]));
+        }
+        if (LONG) __syncthreads();         // the rows have been read
+        rows -= kStateShort;
+        row0 += kStateShort;
+    } while (LONG && rows > 0);
 #pragma unroll
     for (int c = 0; c < KQ; ++c) {
         const int kk = wave * KQ + c;
@@ -227,11 +234,9 @@ template <int KQ>
 __global__ __launch_bounds__(256) void state_walk_kernel(StateArgs a) {
     extern __shared__ __attribute__((aligned(16))) float state_lds[];
     const int item = blockIdx.y, len = a.item_len[item];
-    if (a.item_slot[item] < 0) return;
-    for (int r = 0; r < len; r += kStateShort) {
-        if (r > 0) __syncthreads();                            // the rows before have been read
-        state_walk<KQ>(state_lds, a, item, (int64_t)a.item_tok_off[item] + r, min(kStateShort, len - r), blockIdx.x, blockIdx.z * 64);
-    }
+    if (a.item_slot[item] < 0 || len <= 0) return;
+    if (len <= kStateShort) state_walk<KQ, false>(state_lds, a, item, len, blockIdx.x, blockIdx.z * 64);
+    else state_walk<KQ, true>(state_lds, a, item, len, blockIdx.x, blockIdx.z * 64);
 }
 
 // Rows of a chunk, transposed as in gla_chunks.hip and the matrix memory's outputs.  LDS: F doubles [64] | a [64] | k [64][4 KQ + 4],
@@ -250,15 +255,16 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
     extern __shared__ __attribute__((aligned(16))) float state_lds[];
     using L = StateOutLds<KQ, NV>;
     const int head = blockIdx.x, idx = blockIdx.y, tid = threadIdx.x;
-    int item, chunk;
-    if (!find_chunk(idx, a.item_len, a.item_slot, a.num_items, item, chunk)) return;
-    if (a.item_len[item] <= kStateShort) {
+    int item = idx - a.chunks, chunk;
+    if (item >= 0) {
+        if (a.item_slot[item] < 0 || a.item_len[item] <= 0 || a.item_len[item] > kStateShort) return;
         for (int vb = 0; vb < a.dv; vb += 64) {
             if (vb > 0) __syncthreads();                       // the rows before have been read
-            state_walk<KQ>(state_lds, a, item, a.item_tok_off[item], a.item_len[item], head, vb);
+            state_walk<KQ, false>(state_lds, a, item, a.item_len[item], head, vb);
         }
         return;
     }
+    if (!find_chunk(idx, a.item_len, a.item_slot, a.num_items, item, chunk, kChunkRows, kStateShort)) return;
     const int n = min(kChunkRows, a.item_len[item] - chunk * kChunkRows), dk = a.dk, dv = a.dv;
     const int64_t row0 = (int64_t)a.item_tok_off[item] + (int64_t)chunk * kChunkRows;
     const int group = head / (a.heads / a.qk_heads);
@@ -388,7 +394,7 @@ __global__ __launch_bounds__(256, KQ == 16 && NV == 4 ? 3 : 1) void state_out_ke
 }
 
 template <int KQ, int NV, bool VEC>
-static int launch_state_chunks(const StateArgs& a, unsigned chunks, bool single, hipStream_t stream) {
+static int launch_state_chunks(const StateArgs& a, bool single, hipStream_t stream) {
     using L = StateOutLds<KQ, NV>;
     if constexpr (KQ == 16) if (single) {
         state_walk_kernel<KQ><<<dim3(a.heads, a.num_items, (a.dv + 63) / 64), 256, L::walk, stream>>>(a);
@@ -399,11 +405,13 @@ static int launch_state_chunks(const StateArgs& a, unsigned chunks, bool single,
     ST_CHECK(hipFuncSetAttribute((const void*)state_sums_kernel<KQ, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kSums) == hipSuccess &&
              hipFuncSetAttribute((const void*)state_out_kernel<KQ, NV, VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, kOut) == hipSuccess,
              "state_chunks: cannot raise the LDS limit");
-    state_sums_kernel<KQ, VEC><<<dim3(a.heads, chunks, (a.dv + 63) / 64), 256, kSums, stream>>>(a);
-    ST_LAUNCH_CHECK("state_chunks (sums)");
-    state_carry_kernel<<<dim3(a.heads, a.num_items, (unsigned)((a.dk * a.dv + 255) / 256)), 256, 0, stream>>>(a);
-    ST_LAUNCH_CHECK("state_chunks (carry)");
-    state_out_kernel<KQ, NV, VEC><<<dim3(a.heads, chunks), 256, kOut, stream>>>(a);
+    if (a.chunks) {
+        state_sums_kernel<KQ, VEC><<<dim3(a.heads, a.chunks, (a.dv + 63) / 64), 256, kSums, stream>>>(a);
+        ST_LAUNCH_CHECK("state_chunks (sums)");
+        state_carry_kernel<<<dim3(a.heads, a.num_items, (unsigned)((a.dk * a.dv + 255) / 256)), 256, 0, stream>>>(a);
+        ST_LAUNCH_CHECK("state_chunks (carry)");
+    }
+    state_out_kernel<KQ, NV, VEC><<<dim3(a.heads, a.chunks + a.num_items), 256, kOut, stream>>>(a);
     ST_LAUNCH_CHECK("state_chunks (outputs)");
     return 0;
 }
@@ -422,22 +430,21 @@ extern "C" int st_state_chunks(float* out, const float* q, int64_t q_stride, con
     ST_CHECK(key_dim <= 128 && value_dim <= 128, "state_chunks: up to 128 key and 128 value channels a head, not %d and %d", key_dim, value_dim);
     ST_CHECK(!single || key_dim <= 64, "state_chunks: steps of single tokens take up to 64 key channels a head, not %d", key_dim);
     if (num_items == 0 || num_rows == 0) return 0;
-    ST_CHECK(out && q && k && v && gate_a && gate_b && state && item_len && item_tok_off && item_slot && (scratch || single),
-             "state_chunks: null operand");
-    const int64_t chunks = single ? num_items : num_rows / kChunkRows + num_items;   // (every item's last chunk may be a short one)
-    ST_CHECK(single || scratch_chunks >= chunks, "state_chunks: scratch for %lld chunks, %lld needed", (long long)scratch_chunks, (long long)chunks);
-    ST_CHECK(chunks <= 65535 && num_items <= 65535, "state_chunks: too many chunks or items");
+    ST_CHECK(out && q && k && v && gate_a && gate_b && state && item_len && item_tok_off && item_slot, "state_chunks: null operand");
+    const int64_t chunks = single ? 0 : most_chunks(num_rows, num_items, kStateShort);
+    ST_CHECK(chunks == 0 || (scratch && scratch_chunks >= chunks), "state_chunks: scratch for %lld chunks, %lld needed", (long long)scratch_chunks, (long long)chunks);
+    ST_CHECK(chunks + num_items <= 65535, "state_chunks: too many chunks or items");
     StateArgs a;
     a.out = out; a.q = q; a.k = k; a.v = v; a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride;
     a.gate_a = gate_a; a.gate_b = gate_b; a.gate_stride = gate_stride; a.skip = skip; a.state = state; a.slot_stride = slot_stride;
     a.U = scratch; a.fall = scratch + scratch_chunks * heads * key_dim * value_dim;
     a.item_len = item_len; a.item_tok_off = item_tok_off; a.item_slot = item_slot; a.num_items = num_items;
-    a.heads = heads; a.qk_heads = qk_heads; a.dk = key_dim; a.dv = value_dim;
+    a.heads = heads; a.qk_heads = qk_heads; a.dk = key_dim; a.dv = value_dim; a.chunks = (int)chunks;
     // four numbers at a time: rows and heads start on their size
     const bool vec = ((key_dim | value_dim) & 3) == 0 && ((q_stride | k_stride | v_stride) & 3) == 0 &&
                      (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out | (uintptr_t)scratch) & 15) == 0;
 #define ST_STATE(KQ, NV) \
-    (vec ? launch_state_chunks<KQ, NV, true>(a, (unsigned)chunks, single != 0, stream) : launch_state_chunks<KQ, NV, false>(a, (unsigned)chunks, single != 0, stream))
+    (vec ? launch_state_chunks<KQ, NV, true>(a, single != 0, stream) : launch_state_chunks<KQ, NV, false>(a, single != 0, stream))
     if (key_dim <= 64) return value_dim <= 64 ? ST_STATE(16, 4) : ST_STATE(16, 8);
     return value_dim <= 64 ? ST_STATE(32, 4) : ST_STATE(32, 8);
 #undef ST_STATE

@@ -1069,6 +1069,12 @@ def _d_state_scan(q, k, v, gate_a, gate_b, state, ctx_arrays, heads, mode, skip=
                      8 * ctx_arrays[2].shape[0] * heads * kd * vd}
 
 
+def _chunk_states(rows: int, items: int) -> int:
+    """How many states the chunk kernels of a recurrence want room for: one a chunk of 64 rows and one more for each of the items that may
+    have more than 16 rows (shorter ones are walked from their slots; csrc/chunk_tiles.h counts the same)."""
+    return rows // 64 + min(items, rows // 17)
+
+
 STATE_CHUNK_DIM = 128            # key and value channels a head that the chunk kernels of the additive recurrence take
 
 
@@ -1113,9 +1119,9 @@ def state_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate_a: torch.
         _need(t, name, torch.int32, (B,))
     out = empty((T, heads * vd), torch.float32, q.device)
     single = max_item_rows == 1
-    n = 0 if single else T // 64 + B
+    n = 0 if single else _chunk_states(T, B)
     if (mode == "additive" and (single or chunks) and max(kd, vd) <= STATE_CHUNK_DIM and (kd <= 64 or not single and
-            T >= tuning.state_chunks_wide_rows + tuning.state_chunks_wide_rows_per_item * B) and n <= 65535):
+            T >= tuning.state_chunks_wide_rows + tuning.state_chunks_wide_rows_per_item * B) and n + B <= 65535):
         scratch = empty((n * heads * (kd * vd + 1),), torch.float32, q.device) if n else None
         _check(_lib().st_state_chunks(_ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(gate_a),
                                       _ptr(gate_b), gate_stride, _ptr(skip), _ptr(state), slot_stride, _ptr(item_len), _ptr(item_tok_off),
@@ -1264,6 +1270,11 @@ def gla_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Ten
 GLA_CHUNK_DIM = 128              # key and value channels a head that the chunk kernels take
 
 
+def gla_chunks_fit(rows: int, items: int, key_dim: int, value_dim: int) -> bool:
+    """Whether ``gla_chunks`` takes a step of these sizes (the scan takes any)."""
+    return max(key_dim, value_dim) <= GLA_CHUNK_DIM and _chunk_states(rows, items) + items <= 65535
+
+
 @_timed("gla_chunks", lambda q, k, v, logits, tau, state, *a, **kw: {
     "rows": q.shape[0], "width": v.shape[1], "flops": 4 * q.shape[0] * v.shape[1] * (q.shape[1] // state.shape[1]),
     "bytes": (2 * q.shape[1] + 3 * v.shape[1]) * q.shape[0] * q.element_size() + logits.numel() * 4})
@@ -1290,7 +1301,7 @@ def gla_chunks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, logits: torch.
     for name, t in (("item_len", item_len), ("item_tok_off", item_tok_off), ("item_slot", item_slot)):
         _need(t, name, torch.int32, (B,))
     out = empty((T, heads * vd), q.dtype, q.device)
-    chunks = 0 if single else T // 64 + B
+    chunks = 0 if single else _chunk_states(T, B)
     scratch = empty((chunks * heads * kd * (vd + 1),), torch.float32, q.device) if chunks else None
     _check(_lib().st_gla_chunks(_ptr(out), _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(logits), 1.0 / float(tau), _ptr(gate),
                                 gate.stride(0), _ptr(gain), _ptr(state), _ptr(item_len), _ptr(item_tok_off), _ptr(item_slot), B, T,

@@ -78,7 +78,7 @@ class GatedLinearAttention(Mixer):
         logits = K.gemm(low, self.w_decay_out, bias=self.b_decay, out_f32=True)
         items = (ctx.token_item, ctx.item_len, ctx.item_tok_off, ctx.item_slot)
         q, k, v, gate = proj[:, :qk], proj[:, qk:2 * qk], proj[:, 2 * qk:2 * qk + vs], proj[:, 2 * qk + vs:]
-        if max(self.key_dim, self.value_dim) <= K.GLA_CHUNK_DIM:
+        if K.gla_chunks_fit(q.shape[0], ctx.item_slot.shape[0], self.key_dim, self.value_dim):
             y = K.gla_chunks(q, k, v, logits, self.tau, cache.state, items, self.num_heads, self.scale, gate, self.gain, self.eps,
                              single=ctx.all_single)
         else:
