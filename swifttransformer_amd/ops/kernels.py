@@ -960,6 +960,17 @@ def _d_sink_attention(q, k_cache, v_cache, token_item, positions, block_table, h
             "elem": k_cache.element_size()}
 
 
+def sink_tile_splits(rows: int, items: int, heads: int, kv_heads: int, key_dim: int, value_dim: int, mixed: bool, span: int) -> int:
+    """Workgroups that share a tile's keys: as many as make the tiles fill the chip (every item's last tile may be a short one, so a
+    single token is a tile too), at least 128 of the ``span`` keys each and 8 at most.  A unit holds one workgroup of a mix or of the
+    largest heads and two of the others.  (The instances of csrc/sink_tiles.hip; figures beside ``tuning.sink_tiles_rows``.)"""
+    wave_heads = 4 if heads // kv_heads % 4 == 0 else 1
+    groups = 1 if mixed else -(-heads // (4 * wave_heads))
+    large = mixed or wave_heads * (8 if value_dim > 64 else 4) >= 32
+    tiles = rows // 16 + items
+    return max(1, min(int((256 if large else 512) / (tiles * groups) + 0.5), span // 128, 8))
+
+
 @_timed("sink_attention", _d_sink_attention)
 def sink_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, token_item: torch.Tensor,
                    positions: torch.Tensor, block_table: torch.Tensor, heads: int, scale: float, *,
@@ -991,16 +1002,13 @@ def sink_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     if out is None:
         out = empty((T, heads * dv), q.dtype, q.device)
     _need(out, "out", q.dtype, (T, heads * dv))
-    # (from 128 rows: 32 heads of 64 with a mix and a window of 1,024 take 21 us by rows and 32 by tiles at 40 rows, 31 and 25 at 130)
-    tiled = (items is not None and T >= 128 and q.dtype == torch.bfloat16 and (q.stride(0) | k_cache.stride(0) | v_cache.stride(0)) % 8 == 0 and
+    tiled = (items is not None and T >= tuning.sink_tiles_rows and q.dtype == torch.bfloat16 and (q.stride(0) | k_cache.stride(0) | v_cache.stride(0)) % 8 == 0 and
              (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr() | out.data_ptr()) % 16 == 0 and
              bool(_lib().st_sink_tiles_fit(heads, nkv, dk, dv, int(head_mix is not None), int(window), int(keep_first),
                                            block_table.shape[1], ps)))
     if tiled:
-        # keys are split where a tile's workgroups (mixed: one, else one for sixteen heads) leave most of the chip idle
-        groups = 1 if head_mix is not None else max(1, heads // 16)
         span = window + keep_first if window > 0 else block_table.shape[1] * ps
-        num_splits = max(1, min(256 // max(1, -(-T // 16) * groups), span // 128, 8))
+        num_splits = sink_tile_splits(T, items[3].shape[0], heads, nkv, dk, dv, head_mix is not None, span)
     part_o = part_ml = None
     if num_splits > 1:
         part_o = empty((T, num_splits, heads * dv), torch.float32, q.device)

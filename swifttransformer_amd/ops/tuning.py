@@ -45,6 +45,13 @@ class Tuning:
     # norm sums).
     gla_part_dim_decode: int = 16
     gla_part_dim_prompt: int = 8
+    # Window attention of bfloat16 rows goes by tiles of 16 rows from so many rows of a step on (csrc/sink_tiles.hip), by rows below.
+    # 32 heads of 64 on 8 key heads, window 1,024, by rows and by tiles in us, mixed and not: a prompt of 64 rows 28 and 29, 24 and 13;
+    # of 128 28 and 35, 24 and 25; of 256 72 and 37, 60 and 27.  Beside single tokens of 900 keys a row costs more by rows than a whole
+    # tile: 64 and a portion of 64 173 and 89, 148 and 52; 100 and 28 173 and 133, 149 and 78.  At 60 keys the same 100 and 28 take 27
+    # and 34, 24 and 24: what the kernel for rows gains there is less than what it loses at long contexts, which a recorded step's host
+    # does not see.
+    sink_tiles_rows: int = 128
     # The additive recurrence of heads with more than 64 key channels goes by chunks from so many rows on, and so many more for
     # each item of the step (figures beside csrc/state_chunks.hip: 32 heads of 128 x 128, one prompt of 64 rows 38 us row by row
     # and 43 by chunks, 96 rows 52 and 44; 104 rows beside 24 single ones 78 and 83, 200 rows 100 and 86).

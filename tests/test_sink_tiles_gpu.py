@@ -18,6 +18,12 @@ DEV, F64 = "cuda", torch.float64
     ((70, 66), (33, 2), 24, 6, 80, 112, 64, 3, True, True),                   # sizes between the instances
     ((160,), (0,), 8, 2, 128, 128, 1, 0, False, False),                       # a row sees itself alone
     ((130,), (0,), 32, 8, 128, 128, 50, 7, True, True),                       # the largest
+    # keys split over workgroups: the sink in the first share, kept and window blocks in different ones, shares without a block
+    ((150, 1), (700, 900), 32, 8, 64, 64, 512, 16, True, True),
+    ((140,), (600,), 8, 2, 64, 64, 300, 20, True, True),
+    ((135, 3), (800, 5), 32, 8, 64, 64, 400, 40, False, False),
+    ((200, 1), (0, 2), 32, 8, 128, 128, 1024, 0, True, True),
+    ((64,) + (1,) * 64, (10,) + tuple(range(300, 364)), 32, 8, 64, 64, 256, 0, False, False),
 ])
 def test_tiles_are_the_attention(lens, starts, H, G, dk, dv, window, keep, sink, mixed):
     from swifttransformer_amd.ops import kernels as K
@@ -39,6 +45,8 @@ def test_tiles_are_the_attention(lens, starts, H, G, dk, dv, window, keep, sink,
     pos = i32([s + i for s, n in zip(starts, lens) for i in range(n)] + [-1, 0])
     items = (item, i32(list(lens) + [0]), i32(off + [0]), i32(list(range(B)) + [-1]))
     scale = dk ** -0.5
+    span = window + keep if window else 8 * table.shape[1]
+    assert (K.sink_tile_splits(T + 2, B + 1, H, G, dk, dv, mixed, span) > 1) == (span >= 256)
     assert T >= 128 and K._lib().st_sink_tiles_fit(H, G, dk, dv, int(mixed), window, keep, table.shape[1], ps)
     args = (q.to(DEV), kc.to(DEV), vc.to(DEV), item, pos, table.to(DEV), H, scale)
     kw = dict(window=window, sink=sink, head_mix=mix.to(DEV) if mixed else None, keep_first=keep)
