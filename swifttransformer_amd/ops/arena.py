@@ -128,6 +128,12 @@ def current() -> Optional[StepArena]:
     return _current
 
 
+def measuring() -> bool:
+    """Whether this run finds out how much room steps need: an operation whose scratch is not largest in the largest step asks for
+    what any step of up to these rows may want."""
+    return _current is not None and _current.measure
+
+
 def empty(shape: Sequence[int], dtype: torch.dtype, device) -> torch.Tensor:
     """An uninitialised tensor for a step's intermediate result: from the step's arena while one
     is in use (``using``), from the ordinary allocator otherwise."""

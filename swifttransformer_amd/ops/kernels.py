@@ -1009,10 +1009,14 @@ def sink_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     if tiled:
         span = window + keep_first if window > 0 else block_table.shape[1] * ps
         num_splits = sink_tile_splits(T, items[3].shape[0], heads, nkv, dk, dv, head_mix is not None, span)
+    parts = (T, num_splits) if num_splits > 1 else None
+    if tiled and arena.measuring():        # (fewer rows may be split more ways)
+        of = [(t, sink_tile_splits(t, 1, heads, nkv, dk, dv, head_mix is not None, span)) for t in range(tuning.sink_tiles_rows, T)]
+        parts = max([parts or (0, 0)] + [x for x in of if x[1] > 1], key=lambda x: x[0] * x[1])
     part_o = part_ml = None
-    if num_splits > 1:
-        part_o = empty((T, num_splits, heads * dv), torch.float32, q.device)
-        part_ml = empty((T, num_splits, heads, 2), torch.float32, q.device)
+    if parts and parts[0]:
+        part_o = empty((*parts, heads * dv), torch.float32, q.device)
+        part_ml = empty((*parts, heads, 2), torch.float32, q.device)
     if tiled:
         _t, item_len, item_tok_off, item_slot = items
         B = item_slot.shape[0]

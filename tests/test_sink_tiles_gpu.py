@@ -182,3 +182,30 @@ def test_sums_before_the_rounding_are_no_further_from_float64_than_the_row_kerne
     err = lambda x: float((x - want).norm() / want.norm())
     # (by a tenth to a half nearer; two bfloat16 numbers a weight: 1.4 to 7 times as far)
     assert err(tiles) <= err(rows), (err(tiles), err(rows))
+
+
+def test_the_arena_has_room_for_the_shares_of_smaller_steps():
+    """Steps of fewer rows split their keys more ways: their partial results fit what was measured on the largest step, which splits none."""
+    from swifttransformer_amd.ops import arena
+    from swifttransformer_amd.ops import kernels as K
+    H, G, d, ps, most = 8, 2, 64, 16, 6144
+    kc = torch.randn(1, G, ps, d, device=DEV).bfloat16()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    table = torch.zeros(1, 64, dtype=torch.int32, device=DEV)
+    a = arena.StepArena(DEV)
+
+    def run(T):
+        item, pos = torch.zeros(T, dtype=torch.int32, device=DEV), torch.arange(T, dtype=torch.int32, device=DEV) % 1024
+        q = torch.zeros(T, H * d, dtype=torch.bfloat16, device=DEV)
+        with arena.using(a):
+            K.sink_attention(q, kc, kc, item, pos, table, H, 1.0, window=1024, items=(item, i32([min(T, 1024)]), i32([0]), i32([0])))
+        torch.cuda.synchronize()
+
+    assert K.sink_tile_splits(most, 1, H, G, d, d, False, 1024) == 1
+    a.measure = True
+    run(most)
+    a.measure = False
+    a.resize(a.peak)
+    for T in (128, 512, 1000, 2048, 2500, 3000, 4000, most):
+        run(T)
+    assert a.overflows == 0
