@@ -664,6 +664,10 @@ __global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
     const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, const int* __restrict__ sorted, const int* __restrict__ tile_expert,
     const float* __restrict__ weights, int max_tiles, int blocks, int top, int N, int K, float limit, float out_scale, int style) {
     constexpr bool UP = KIND == kTiledUp, GATHER = KIND != kTiledDown;
+    // Results that stay float, of tiles of 64 places: sums are carried in double every few steps.  With 7 to 31 pairs an expert the tiles of
+    // 16 were used before, whose waves share the depth: their chains are an eighth as long (2,048 deep: 2.7e-7 off float64 in one chain,
+    // 1.3e-7 in theirs).
+    constexpr bool DOUBLE = KIND == kTiledDown && NJ == 1;
     constexpr int PLACES = 64 * NJ;
     constexpr int BUF = (128 + PLACES) * 8;        // 16-byte pieces a buffer: weight rows, then places
     constexpr int NL = (128 + PLACES) / 32;        // direct loads a wave and step, eight rows each
@@ -714,6 +718,17 @@ __global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+    // (a chain's numbers are `per` steps long, so that it has no more roundings than the shares of the tiles of 16 places)
+    double total[DOUBLE ? 2 : 1][DOUBLE ? NJ : 1][16];
+    const int per = max(1, min(4, K >> 9));
+    int since = 0;
+    if constexpr (DOUBLE)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int q = 0; q < 16; ++q) total[i][j][q] = 0.0;
     // (the swizzle of a lane's rows is that of l32: the rows before it are a multiple of 32)
     const uint4* own = lds + l32 * 8;
     const int swz = swizzle(l32);
@@ -741,6 +756,19 @@ __global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
                 for (int j = 0; j < NJ; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kk & 1][i], b[kk & 1][j], acc[i][j], 0, 0, 0);
         }
+        if constexpr (DOUBLE)
+            if (++since == per || s + 1 == steps) {
+                since = 0;
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) {
+                            total[i][j][q] += (double)acc[i][j][q];
+                            acc[i][j][q] = s + 1 == steps ? (float)total[i][j][q] : 0.f;
+                        }
+            }
     }
     // acc[i][j][q]: weight row wn * 64 + i * 32 + 8 * (q / 4) + 4 * lh + q % 4, place base + (wm * NJ + j) * 32 + l32
     auto store_row = [&](int place, int f, const float* r) {

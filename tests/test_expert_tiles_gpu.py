@@ -78,3 +78,28 @@ def test_tiles_of_64_and_128_places(T, W, F, E, top, style, clamped, same):
     err = (got.double().cpu() - (res.to(F64) + 0.5 * want)).abs()
     assert bool((err[:T - 3] <= bound[:T - 3]).all()), float((err / bound)[:T - 3].max())
     assert torch.equal(got[T - 3:].cpu(), res[T - 3:])
+
+
+@pytest.mark.parametrize("E,W,F,T,top", [(16, 256, 264, 100, 2), (16, 256, 1000, 60, 2), (8, 128, 2048, 64, 2), (4, 128, 8192, 30, 1), (8, 128, 768, 120, 4)])
+def test_sums_of_64_places_are_no_further_from_float64_than_those_of_16(E, W, F, T, top):
+    """The output products of the same rows in tiles of 64 places and of 16, whose waves share the depth in short chains."""
+    from swifttransformer_amd.ops import kernels as K
+    dev, P, lib = "cuda", K._ptr, K._lib()
+    g = torch.Generator(device=dev).manual_seed(F)
+    ids = torch.stack([torch.randperm(E, generator=g, device=dev)[:top] for _ in range(T)]).int().reshape(-1)
+    w = (torch.randn(E, W, F, generator=g, device=dev) * 0.02).bfloat16()
+    rows = torch.randn(T * top, F, generator=g, device=dev).bfloat16()
+    want = torch.stack([w[e].to(torch.float64) @ rows[i].to(torch.float64) for i, e in enumerate(ids.tolist())])
+
+    def err(tile):
+        cap = K.moe_capacity(T, top, E, tile)
+        i32 = lambda n: torch.empty(n, dtype=torch.int32, device=dev)
+        order, place, owner = i32(cap), i32(T * top), i32(cap // tile)
+        K._check(lib.st_moe_align(P(order), P(place), P(owner), P(ids), T * top, E, cap, tile, K._stream()))
+        y = torch.zeros(cap, F, dtype=torch.bfloat16, device=dev)
+        y[place.long()] = rows
+        out = torch.empty(cap, W, device=dev)
+        K._check(lib.st_moe_down(None, None, P(out), P(y), P(w), P(order), P(owner), cap, tile, 2, W, F, 1.0, K.dtype_code(y.dtype), K._stream()))
+        return float((out[place.long()] - want).norm() / want.norm())
+
+    assert err(64) <= err(16), (err(64), err(16))
