@@ -185,41 +185,19 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
         return (mode == 3 ? 1.f / (1.f + expf(-z[e])) : expf(z[e] - m_all) * inv_sum) + correction[e];
     };
     auto weight_of = [&](float v) { return mode == 0 ? 1.f / (1.f + expf(-v)) : mode == 2 ? expf(v - m_all) * inv_sum : v; };
-    if (experts <= 64) {
-        // which experts can still be chosen, a bit each: no list of the chosen ones to walk
-        uint64_t free_ = experts == 64 ? ~0ull : (1ull << experts) - 1;
-        if (mode == 2 && keep < groups) {
-            const uint64_t one_group = per == 64 ? ~0ull : (1ull << per) - 1;
-            free_ = 0;
-            for (int g = 0; g < groups; ++g)
-                if ((open >> g) & 1) free_ |= one_group << (g * per);
+    int chosen[kMaxTop];
+    for (int j = 0; j < top; ++j) {
+        int best = -1;
+        float bv = 0.f;
+        for (int e = 0; e < experts; ++e) {
+            bool taken = mode == 2 && !((open >> (e / per)) & 1);
+            for (int u = 0; u < j; ++u) taken |= chosen[u] == e;
+            const float v = choice(e);
+            if (!taken && (best < 0 || v > bv)) { best = e; bv = v; }
         }
-        for (int j = 0; j < top; ++j) {
-            int best = -1;
-            float bv = 0.f;
-            for (int e = 0; e < experts; ++e) {
-                const float v = choice(e);
-                if (((free_ >> e) & 1) && (best < 0 || v > bv)) { best = e; bv = v; }
-            }
-            free_ &= ~(1ull << best);
-            ids[(int64_t)t * top + j] = best;
-            weights[(int64_t)t * top + j] = weight_of(bv);
-        }
-    } else {
-        int chosen[kMaxTop];
-        for (int j = 0; j < top; ++j) {
-            int best = -1;
-            float bv = 0.f;
-            for (int e = 0; e < experts; ++e) {
-                bool taken = mode == 2 && !((open >> (e / per)) & 1);
-                for (int u = 0; u < j; ++u) taken |= chosen[u] == e;
-                const float v = choice(e);
-                if (!taken && (best < 0 || v > bv)) { best = e; bv = v; }
-            }
-            chosen[j] = best;
-            ids[(int64_t)t * top + j] = best;
-            weights[(int64_t)t * top + j] = weight_of(bv);
-        }
+        chosen[j] = best;
+        ids[(int64_t)t * top + j] = best;
+        weights[(int64_t)t * top + j] = weight_of(bv);
     }
     if (mode == 1) {
         // softmax over the chosen logits alone; the first chosen is the largest
@@ -507,7 +485,8 @@ __global__ __launch_bounds__(256) void moe_up_kernel(
                 }
         }
     };
-    if (vec && RT == 4) batches(Steps<2>());
+    if constexpr (RT == 4 && sizeof(T) == 4)           // (bfloat16 that allows it goes through LDS, below)
+        if (vec) batches(Steps<2>());
     for (; k0 < width; k0 += D) {
         Frag<T> a[RT], bg, bu;
         const int k = k0 + L * g;
@@ -583,7 +562,8 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
                 for (int b = 0; b < RT; ++b) c[b] = Frag<T>::mma(a[u][b], bw[u], c[b]);
         }
     };
-    if (vec && RT == 4) batches(Steps<2>());
+    if constexpr (RT == 4 && sizeof(T) == 4)           // (bfloat16 that allows it goes through LDS, below)
+        if (vec) batches(Steps<2>());
     for (; k0 < inner; k0 += D) {
         Frag<T> a[RT], bw;
         const int k = k0 + L * g;
@@ -620,8 +600,9 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 // lane holds both halves of a result; rows of x are gathered through the sorted list.  GELU: the one input matrix of experts
 // without a gate.  Otherwise: output features of the expert's output matrix over the rows of y.
 //
-// What bounds it: the path from L2 into LDS (about 19 bytes a cycle and unit; the weights' own stream from memory is the floor
-// below it, all experts' matrices whatever the rows).  Workgroups go round the eight dies by their number; here each die takes
+// What bounds it: waiting for the operands' way from L2 into LDS.  It moves about 19 bytes a cycle and unit there, where direct loads
+// alone reach 50: one step's loads are on their way at a time, and the wait before each barrier is for all of them.  (The weights' own
+// stream from memory is the floor below it, all experts' matrices whatever the rows.)  Workgroups go round the eight dies by their number; here each die takes
 // an eighth of the work in the order (expert, weight rows, tile of that expert), so that an expert's matrix passes through one
 // die's L2 once, its tiles next to each other, and a die gets the same number of tiles as any other, however the tokens chose.
 // Measured beside the kernels before it (operands through registers into LDS for 128 places, straight from memory for 64), 16

@@ -1381,14 +1381,12 @@ def latent_write(cache: torch.Tensor, x: torch.Tensor, gain: torch.Tensor, eps: 
 # ---------------------------------------------------------------- routed experts
 def moe_tile(num_tokens: int, top: int, experts: int, staged: bool = False) -> int:
     """Places a tile: 16 for few rows an expert (only the weights' stream counts), 64 or 128 for more.
-    ``staged``: bfloat16 rows in whole 16-byte pieces, whose larger tiles go through LDS.  Up + down of 16
-    experts of 2,048 x 2,048, two a token, us with tiles of 16 / 64 / 128 places: 79 / 89 / 93 at 6 pairs an
-    expert, 79 / 72 at 7, 112 / 93 / 98 at 12, 361 / 122 / 135 at 64, 137 / 137 at 112 (64 / 128),
-    144 / 135 at 128.  Otherwise a tile's weight operands come from memory for four or eight blocks of 16
+    ``staged``: bfloat16 rows in whole 16-byte pieces, whose larger tiles go through LDS (from ``tuning.moe_staged_64_pairs`` and
+    ``moe_staged_128_pairs`` an expert).  Otherwise a tile's weight operands come from memory for four or eight blocks of 16
     rows, which takes some dozens of pairs an expert to pay."""
     pairs = num_tokens * top
     if staged:
-        return 128 if pairs >= 112 * experts else 64 if pairs >= 7 * experts else 16
+        return 128 if pairs >= tuning.moe_staged_128_pairs * experts else 64 if pairs >= tuning.moe_staged_64_pairs * experts else 16
     return 128 if pairs >= 96 * experts else 64 if pairs >= 32 * experts else 16
 
 

@@ -45,6 +45,14 @@ class Tuning:
     # norm sums).
     gla_part_dim_decode: int = 16
     gla_part_dim_prompt: int = 8
+    # Pairs an expert from which bfloat16 experts go in tiles of 64 and of 128 places through LDS instead of 16 (csrc/moe.hip).  All
+    # kernels of a call with tiles of 16 / 64 / 128 places, us: 64 experts of 2,048 x 1,024, four a token, 189 / 177 / 182 at 6 pairs an
+    # expert, 371 / 212 / 221 at 31, 1,088 / 265 / 245 at 100, 1,195 / 278 / 279 at 112; 8 of 4,096 x 4,096, two a token, 177 / 168 / 175
+    # at 6, 437 / 174 / 182 at 31, 1,061 / 266 / 230 at 100, 1,148 / 271 / 232 at 112; up and down alone of 16 of 2,048 x 2,048, two a
+    # token, 79 / 89 / 93 at 6, 112 / 93 / 98 at 12, 361 / 122 / 135 at 64, - / 137 / 137 at 112, - / 144 / 135 at 128.  How tokens spread
+    # over experts moves the lines: tiles of 64 win from 4 to 12 pairs on, of 128 from 100 to 128.
+    moe_staged_64_pairs: int = 7
+    moe_staged_128_pairs: int = 112
     # Window attention of bfloat16 rows goes by tiles of 16 rows from so many rows of a step on (csrc/sink_tiles.hip), by rows below.
     # 32 heads of 64 on 8 key heads, window 1,024, by rows and by tiles in us, mixed and not: a prompt of 64 rows 28 and 29, 24 and 13;
     # of 128 28 and 35, 24 and 25; of 256 72 and 37, 60 and 27.  Beside single tokens of 900 keys a row costs more by rows than a whole
