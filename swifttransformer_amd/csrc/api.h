@@ -267,14 +267,14 @@ int st_moe_route(int* ids, float* weights, const float* logits, int logit_stride
 // Sorts the num_pairs = tokens * top (token, choice) pairs by expert into tiles of `tile` (16, 64 or 128)
 // places that hold one expert's pairs each: sorted[capacity] (pair index, or -1),
 // place_of_pair[num_pairs] (or -1), tile_expert[capacity / tile] (or -1).
-// capacity >= round_up(num_pairs, tile) + tile * experts.  The three calls below take the same `tile`.
+// capacity >= round_up(num_pairs, tile) + tile * experts.  st_moe_up and st_moe_down take the same `tile`.
+int st_moe_align(int* sorted, int* place_of_pair, int* tile_expert, const int* ids, int num_pairs,
+                 int experts, int capacity, int tile, hipStream_t stream);
 // st_moe_route and st_moe_align by one workgroup, for up to 64 tokens of 16 router outputs, 32 of 32 or 16 of 64; `experts` of the
 // outputs have weights.
 int st_moe_route_align(int* ids, float* weights, int* sorted, int* place_of_pair, int* tile_expert, const float* logits,
                        int logit_stride, const int* token_item, const float* correction, float scale, int num_tokens, int outputs,
                        int experts, int top, int mode, int groups, int keep, int capacity, int tile, hipStream_t stream);
-int st_moe_align(int* sorted, int* place_of_pair, int* tile_expert, const int* ids, int num_pairs,
-                 int experts, int capacity, int tile, hipStream_t stream);
 // y[place, f] = g * sigmoid(1.702 g) * (u + 1) with g = min(s * (x_t . Wg[e, f]), limit) and
 // u = clamp(s * (x_t . Wu[e, f]), -limit, limit), for the pair (t, j) at `place`, e its expert and s
 // its weight (style 0); style 1: y[place, f] = silu(x_t . Wg[e, f]) * (x_t . Wu[e, f]), no weight and no

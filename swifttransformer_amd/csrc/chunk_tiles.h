@@ -3,6 +3,8 @@
 
 #include "common.h"
 
+#include <type_traits>
+
 namespace st {
 
 constexpr int kChunkRows = 64;       // counted from an item's first row of the step
@@ -51,6 +53,32 @@ __device__ inline int chunks_before(int item, const int* __restrict__ item_len, 
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
     return __builtin_amdgcn_readfirstlane(sum);
+}
+
+// S <- keep * S + add over an item's chunks: `u` holds an element of the chunks' sums (step floats apart) and receives the state that
+// each chunk starts from, `f` their factors; returns the last S.
+__device__ inline float carry_states(float* __restrict__ u, int64_t u_step, const float* __restrict__ f, int64_t f_step, int chunks, float S) {
+    int c0 = 0;
+    auto batch = [&](auto count) {                             // so many chunks' operands on their way at once
+        constexpr int B = decltype(count)::value;
+        for (; c0 + B <= chunks; c0 += B) {
+            float add[B], keep[B];
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                add[b] = u[(c0 + b) * u_step];
+                keep[b] = f[(c0 + b) * f_step];
+            }
+#pragma unroll
+            for (int b = 0; b < B; ++b) {
+                u[(c0 + b) * u_step] = S;
+                S = fmaf(keep[b], S, add[b]);
+            }
+        }
+    };
+    batch(std::integral_constant<int, 16>());
+    batch(std::integral_constant<int, 4>());
+    batch(std::integral_constant<int, 1>());
+    return S;
 }
 
 typedef double doublex4 __attribute__((ext_vector_type(4)));

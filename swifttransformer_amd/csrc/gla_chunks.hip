@@ -33,7 +33,6 @@
 #include "fragment.h"
 
 #include <cfloat>
-#include <type_traits>
 
 namespace st {
 
@@ -208,28 +207,7 @@ __global__ __launch_bounds__(256) void gla_carry_kernel(
     float* home = state + ((int64_t)slot * heads + head) * plane + e;
     float* u = U + first * plane + e;
     const float* f = A + first * dk + e / dv;
-    float S = *home;
-    int c0 = 0;
-    auto batch = [&](auto count) {                             // so many chunks' operands on their way at once
-        constexpr int B = decltype(count)::value;
-        for (; c0 + B <= chunks; c0 += B) {
-            float add[B], keep[B];
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                add[b] = u[(int64_t)(c0 + b) * heads * plane];
-                keep[b] = f[(int64_t)(c0 + b) * heads * dk];
-            }
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                u[(int64_t)(c0 + b) * heads * plane] = S;
-                S = fmaf(keep[b], S, add[b]);
-            }
-        }
-    };
-    batch(std::integral_constant<int, 16>());
-    batch(std::integral_constant<int, 4>());
-    batch(std::integral_constant<int, 1>());
-    *home = S;
+    *home = carry_states(u, (int64_t)heads * plane, f, (int64_t)heads * dk, chunks, *home);
 }
 
 // Rows of a chunk, transposed as in the matrix memory's outputs: a wave has a block of 16 rows, lane (r16, g) row r16 of it with

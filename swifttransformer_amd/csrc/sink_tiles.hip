@@ -17,8 +17,8 @@
 // heads and rows the other: v_mfma_f32_16x16x4_f32), then every wave takes its own heads back.  Two barriers a block.
 //
 // What bounds it: vector instructions around the products (exponentials, roundings, masks) and, with the mix, its float products
-// (heads^2 multiply-adds a row and key) with two barriers a block and one workgroup a unit.  Rows whose tiles leave units idle have their keys split over workgroups;
-// the row kernel's merge adds them up.
+// (heads^2 multiply-adds a row and key) with two barriers a block and one workgroup a unit.  Rows whose tiles leave units idle have
+// their keys split over workgroups; the row kernel's merge adds them up.
 // Measured beside the row kernel, 32 heads of 64 on 8 key heads, window 1,024: mixed, one prompt of 2,048 rows 755 -> 247 us, three
 // that make 2,048 437 -> 181; not mixed 671 -> 107; 512 rows beside 16 single tokens 225 -> 77; 32 heads of 128 x 128, 1,024 rows,
 // 510 -> 241 (mixed), 454 -> 190.  The sums' distance from float64 before they are rounded to bfloat16: 512 rows behind 600 keys, mixed
@@ -431,9 +431,17 @@ extern "C" int st_sink_tiles(void* out, float* part_o, float* part_ml, const voi
     const int64_t tiles = num_tokens / kSinkRows + num_items + 1;      // (every item's last tile may be a short one; one without a tile)
     ST_CHECK(tiles <= 0x7fffffff, "sink_tiles: too many rows");
     int rc = 0;
-#define ST_SINK(DS, NV, HW)                                                                                         rc = !mix ? launch_sink_tiles<DS, NV, HW, 0>(a, (int)tiles, stream) : heads > 16 ? launch_sink_tiles<DS, NV, HW, 2>(a, (int)tiles, stream) \
-                                                                               : launch_sink_tiles<DS, NV, HW, 1>(a, (int)tiles, stream)
-#define ST_SINK_SIZES(HW)                                                                                           do {                                                                                                                if (key_dim <= 64 && value_dim <= 64) ST_SINK(2, 4, HW);                                                        else if (key_dim <= 64) ST_SINK(2, 8, HW);                                                                      else if (value_dim <= 64) ST_SINK(4, 4, HW);                                                                    else ST_SINK(4, 8, HW);                                                                                     } while (0)
+#define ST_SINK(DS, NV, HW)                                                                                                    \
+    rc = !mix ? launch_sink_tiles<DS, NV, HW, 0>(a, (int)tiles, stream)                                                        \
+       : heads > 16 ? launch_sink_tiles<DS, NV, HW, 2>(a, (int)tiles, stream)                                                  \
+                    : launch_sink_tiles<DS, NV, HW, 1>(a, (int)tiles, stream)
+#define ST_SINK_SIZES(HW)                                                                                                      \
+    do {                                                                                                                       \
+        if (key_dim <= 64 && value_dim <= 64) ST_SINK(2, 4, HW);                                                               \
+        else if (key_dim <= 64) ST_SINK(2, 8, HW);                                                                             \
+        else if (value_dim <= 64) ST_SINK(4, 4, HW);                                                                           \
+        else ST_SINK(4, 8, HW);                                                                                                \
+    } while (0)
     if (sink_tiles_heads(heads, kv_heads, key_dim, value_dim, mix != nullptr) == 4) ST_SINK_SIZES(4);
     else ST_SINK_SIZES(1);
 #undef ST_SINK_SIZES

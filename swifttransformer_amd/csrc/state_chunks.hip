@@ -30,7 +30,6 @@
 #include "chunk_tiles.h"
 #include "fragment.h"
 
-#include <type_traits>
 
 namespace st {
 
@@ -132,28 +131,7 @@ __global__ __launch_bounds__(256) void state_carry_kernel(StateArgs a) {
     float* home = a.state + (int64_t)slot * a.slot_stride + (int64_t)head * plane + e;
     float* u = a.U + first * plane + e;
     const float* f = a.fall + first;
-    float S = *home;
-    int c0 = 0;
-    auto batch = [&](auto count) {                             // so many chunks' operands on their way at once
-        constexpr int B = decltype(count)::value;
-        for (; c0 + B <= chunks; c0 += B) {
-            float add[B], keep[B];
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                add[b] = u[(int64_t)(c0 + b) * a.heads * plane];
-                keep[b] = f[(int64_t)(c0 + b) * a.heads];
-            }
-#pragma unroll
-            for (int b = 0; b < B; ++b) {
-                u[(int64_t)(c0 + b) * a.heads * plane] = S;
-                S = fmaf(keep[b], S, add[b]);
-            }
-        }
-    };
-    batch(std::integral_constant<int, 16>());
-    batch(std::integral_constant<int, 4>());
-    batch(std::integral_constant<int, 1>());
-    *home = S;
+    *home = carry_states(u, (int64_t)a.heads * plane, f, a.heads, chunks, *home);
 }
 
 // 64 value channels (from vb) of an item of up to kStateShort rows from its slot's state, row by row.  Thread (wave, lane): KQ key

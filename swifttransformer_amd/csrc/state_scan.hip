@@ -9,7 +9,8 @@
 // `recurrence_gates` (or one row of constants for every token: a fixed decay a head); q, k, v are float rows; the state is float, lives in the request's slot and is
 // loaded before and stored after the item's rows, so prompts, portions and single tokens take the
 // same route and a position's sums are formed in the same order however the tokens were cut.
-// (The additive form with up to 128 channels a head runs by chunks instead: csrc/state_chunks.hip.)
+// (That is the delta rule, and the additive form of wider heads or few rows.  The additive form with up to 128 channels a head goes by
+// chunks or a walk of its own, csrc/state_chunks.hip, whose sums depend on where a step cut the tokens.)
 //
 // Launch: a two-wave workgroup a (head, block of 16 value channels, item), see the kernel.
 #include "api.h"
