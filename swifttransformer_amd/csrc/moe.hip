@@ -950,7 +950,7 @@ extern "C" int st_moe_route_align(int* ids, float* weights, int* sorted, int* pl
     ST_CHECK(outputs <= 64 && experts >= 1 && experts <= outputs, "moe_route_align: up to 64 router outputs, not %d", outputs);
     ST_CHECK((int64_t)num_tokens * route_lanes(outputs) <= 1024, "moe_route_align: up to %d tokens of %d experts", 1024 / route_lanes(outputs), outputs);
     static_assert(kFusedPairs >= 1024 / 16 * kMaxTop, "the choices of all tokens fit LDS");
-    if (num_tokens == 0) return 0;
+    if (num_tokens == 0) return st_moe_align(sorted, place_of_pair, tile_expert, ids, 0, experts, capacity, tile, stream);
     ST_CHECK(tile == 16 || tile == 64 || tile == 128, "moe_align: tiles of 16, 64 or 128 places, not %d", tile);
     const int num_pairs = num_tokens * top;
     ST_CHECK(capacity % tile == 0 && capacity >= (num_pairs + tile - 1) / tile * tile + tile * experts,

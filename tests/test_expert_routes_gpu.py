@@ -80,3 +80,16 @@ def test_routes_and_lists(T, E, identity, top, mode, groups, keep):
     assert torch.equal(texp[p // tile], ids[real])
     used = int((texp >= 0).sum())
     assert (texp[:used] >= 0).all() and (texp[1:used] >= texp[:used - 1]).all()        # an expert's tiles are neighbours
+
+
+def test_no_token_leaves_no_tile():
+    """Routing and sorting of no token marks every place and tile as empty, as sorting alone does: the products that follow read them."""
+    from swifttransformer_amd.ops import kernels as K
+    E, tile, lib, P = 8, 16, K._lib(), K._ptr
+    cap = K.moe_capacity(0, 2, E, tile)
+    i32 = lambda n: torch.full((n,), 5, dtype=torch.int32, device="cuda")
+    order, place, owner, ids = i32(cap), i32(2), i32(cap // tile), i32(2)
+    wts, logits = torch.ones(2, device="cuda"), torch.zeros(1, E, device="cuda")
+    K._check(lib.st_moe_route_align(P(ids), P(wts), P(order), P(place), P(owner), P(logits), E, None, None, 1.0, 0, E, E, 2, 1, 1, 1, cap, tile,
+                                    K._stream()))
+    assert bool((order == -1).all()) and bool((owner == -1).all())
