@@ -22,10 +22,10 @@
 // LDS.
 //
 // Measured beside decay gates, scan and norm kernel (which sums the scan's planes): one item of 2,011 rows, 32 heads of 64 x 64,
-// 427 -> 99 us (the scan's 2,011 dependent steps; now the carry's 32, and the products at a few workgroups a unit; with everything in
-// float 65); three items of 2,048 rows together 219 -> 107; 32 heads of 128 x 128 637 -> 304; 33 rows 35 -> 31; 512 rows beside 24 single
-// tokens 123 -> 49; 8 single tokens 34 -> 15, 24 of 32 heads of 128 x 128 58 -> 29 us.  Relative distance from float64 behind norm and
-// gate, in float: 2,011 rows outputs 1.5e-7 -> 9.3e-8, state 9.6e-8 -> 6.5e-8; 33 rows 1.4e-7 -> 7.7e-8 and 4.4e-8 -> 3.2e-8; 48 single
+// 427 -> 97 us (the scan's 2,011 dependent steps; now the carry's 32, and the products at a few workgroups a unit; with everything in
+// float 65); three items of 2,048 rows together 219 -> 104; 32 heads of 128 x 128 637 -> 297; 33 rows 35 -> 30; 512 rows beside 24 single
+// tokens 123 -> 48; 8 single tokens 34 -> 14, 24 of 32 heads of 128 x 128 58 -> 29 us.  Relative distance from float64 behind norm and
+// gate, in float: 2,011 rows outputs 1.5e-7 -> 9.3e-8, state 9.6e-8 -> 6.6e-8; 33 rows 1.4e-7 -> 7.7e-8 and 4.4e-8 -> 3.2e-8; 48 single
 // tokens 1.4e-7 -> 1.2e-7 and 3.6e-8 -> 3.5e-8 (with everything in float 1.7e-7 and 9.9e-8, 1.3e-7 and 5.0e-8, 1.4e-7 and 3.9e-8).
 #include "api.h"
 #include "common.h"
@@ -39,21 +39,23 @@ namespace st {
 constexpr int kGlaShort = 16;        // rows up to which an item is walked row by row
 
 // sigmoid(z)^inv_tau = e^(inv_tau (min(z, 0) - log(1 + e^-|z|))), rounded to float once; 1 for the largest float, which stands for
-// rows that do not exist.  log(1 + u) = 2 artanh(u / (2 + u)), nine terms of its series for u up to 1 (the tenth is below 2^-32).  (The
-// library's float functions, off by up to 2^-24 each, take 23 us more for 2,011 rows of 32 heads of 64.)
+// rows that do not exist.  log(1 + u) = 2 artanh(s) = 2 s (1 + s^2 / 3 + ..), s = u / (2 + u) up to 1/3: the sum behind the one, up to s^16
+// (the next term is below 2^-32), is at most 0.04 and float.  (With the exponential of -|z| and that sum in
+// double too 2,011 rows of 32 heads of 64 take 102 us instead of 97, at the same distance from float64; the library's float functions,
+// off by up to 2^-24 each, took 23 us more than the hardware's.)
 __device__ inline float gla_decay(float z, float inv_tau) {
-    const double u = exp_le0_double(-fabs((double)z));
-    const double r0 = __builtin_amdgcn_rcpf((float)(2.0 + u)), s = u * (r0 * fma(-(2.0 + u), r0, 2.0)), s2 = s * s;
-    double y = 1.0 / 17.0;
-    y = fma(y, s2, 1.0 / 15.0);
-    y = fma(y, s2, 1.0 / 13.0);
-    y = fma(y, s2, 1.0 / 11.0);
-    y = fma(y, s2, 1.0 / 9.0);
-    y = fma(y, s2, 1.0 / 7.0);
-    y = fma(y, s2, 1.0 / 5.0);
-    y = fma(y, s2, 1.0 / 3.0);
-    y = fma(y, s2, 1.0);
-    return (float)exp_le0_double(((z < 0.f ? (double)z : 0.0) - 2.0 * s * y) * inv_tau);
+    const double u = exp_le0(-fabsf(z));
+    const double r0 = __builtin_amdgcn_rcpf((float)(2.0 + u)), s = u * (r0 * fma(-(2.0 + u), r0, 2.0));
+    const float s2 = (float)(s * s);
+    float y = 1.f / 17.f;
+    y = fmaf(y, s2, 1.f / 15.f);
+    y = fmaf(y, s2, 1.f / 13.f);
+    y = fmaf(y, s2, 1.f / 11.f);
+    y = fmaf(y, s2, 1.f / 9.f);
+    y = fmaf(y, s2, 1.f / 7.f);
+    y = fmaf(y, s2, 1.f / 5.f);
+    y = fmaf(y, s2, 1.f / 3.f);
+    return (float)exp_le0_double(((z < 0.f ? (double)z : 0.0) - 2.0 * fma(s, (double)(y * s2), s)) * inv_tau);
 }
 
 // four neighbouring numbers of a row as floats, `fill` past its end or where the row does not exist (see load_piece)
