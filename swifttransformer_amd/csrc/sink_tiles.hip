@@ -19,10 +19,10 @@
 // What bounds it: vector instructions around the products (exponentials, roundings, masks) and, with the mix, its float products
 // (heads^2 multiply-adds a row and key) with two barriers a block and one workgroup a unit.  Rows whose tiles leave units idle have
 // their keys split over workgroups; the row kernel's merge adds them up.
-// Measured beside the row kernel, 32 heads of 64 on 8 key heads, window 1,024: mixed, one prompt of 2,048 rows 755 -> 247 us, three
-// that make 2,048 437 -> 181; not mixed 671 -> 107; 512 rows beside 16 single tokens 225 -> 77; 32 heads of 128 x 128, 1,024 rows,
+// Measured beside the row kernel, 32 heads of 64 on 8 key heads, window 1,024: mixed, one prompt of 2,048 rows 736 -> 164 us, 64 single
+// tokens of 900 keys beside 448 rows 314 -> 111; not mixed 628 -> 95 and 268 -> 75; 32 heads of 128 x 128, 1,024 rows,
 // 510 -> 241 (mixed), 454 -> 190.  The sums' distance from float64 before they are rounded to bfloat16: 512 rows behind 600 keys, mixed
-// 3.8e-7 -> 3.3e-7, not mixed 3.0e-7 -> 1.8e-7; with weights of two bfloat16 numbers (230 and 99 us for 2,048 rows) 1.7e-6 and 2.0e-6.
+// 3.8e-7 -> 3.3e-7, not mixed 3.0e-7 -> 1.8e-7; with weights of two bfloat16 numbers, some 7 % faster, 1.7e-6 and 2.0e-6.
 #include "api.h"
 #include "common.h"
 #include "chunk_tiles.h"
