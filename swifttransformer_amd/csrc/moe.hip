@@ -591,24 +591,30 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 }
 
 // ---- prompts in bfloat16: tiles of 64 or 128 places, operands by direct loads into LDS -----------
-// With some dozens of rows and more an expert a tile of 64 NJ places meets 128 rows of its expert's matrix, steps of 64 in depth.
+// With some dozens of rows and more an expert a tile of 64 NJ places meets 64 WN rows of its expert's matrix, steps of 64 in depth.
 // Both operand tiles go from memory into LDS without passing through registers (16 bytes a lane; a row's chunks are rotated by
-// the lane's choice of address, so that the matrix instruction's reads spread over the banks), the next step's into the other of
-// two buffers while this one is multiplied: one barrier a step.  Each of four waves multiplies a 64 x 32 NJ part
-// (v_mfma_f32_32x32x16_bf16), the operands of a product of depth 16 read ahead of the one before.
+// the lane's choice of address, so that the matrix instruction's reads spread over the banks), the two steps after the one that is
+// multiplied on their way into the other two of three buffers: one barrier a step, before which a wave waits for its loads of that step
+// alone.  Each of 2 WN waves multiplies a 64 x 32 NJ part (v_mfma_f32_32x32x16_bf16), the operands of a product of depth 16 read ahead
+// of the one before; the two waves that share weight rows take the tile's blocks of 32 places in turn, and a block without a pair
+// (an expert's last tile) is not multiplied.
 // UP: of every 64 weight rows 32 are inner features of the gate matrix and 32 the same features of the other one, so that a
 // lane holds both halves of a result; rows of x are gathered through the sorted list.  GELU: the one input matrix of experts
 // without a gate.  Otherwise: output features of the expert's output matrix over the rows of y.
 //
-// What bounds it: waiting for the operands' way from L2 into LDS.  It moves about 19 bytes a cycle and unit there, where direct loads
-// alone reach 50: one step's loads are on their way at a time, and the wait before each barrier is for all of them.  (The weights' own
-// stream from memory is the floor below it, all experts' matrices whatever the rows.)  Workgroups go round the eight dies by their number; here each die takes
+// What bounds it: the weights' way from memory, all experts' matrices whatever the rows, and the operands' way from L2 into LDS, which
+// a unit takes at some 25 bytes a clock.  So: tiles of 128 places meet 256 weight rows (a quarter fewer bytes for the same products than
+// 128 rows, 48 KB a step, one workgroup a unit), tiles of 64 meet 128 (two workgroups a unit); and a workgroup begins its depth three
+// steps after its neighbour does, going round, since rows that lie a power of two apart meet in the same memory channels while everyone
+// reads at the same depth.  Workgroups go round the eight dies by their number; here each die takes
 // an eighth of the work in the order (expert, weight rows, tile of that expert), so that an expert's matrix passes through one
 // die's L2 once, its tiles next to each other, and a die gets the same number of tiles as any other, however the tokens chose.
-// Measured beside the kernels before it (operands through registers into LDS for 128 places, straight from memory for 64), 16
-// experts of 2,048 x 2,048, two a token, up + down: 2,011 tokens 299 -> 201 us, 1,024 tokens 257 -> 135, 512 tokens (tiles of 64)
-// 319 -> 122, 256 tokens 223 -> 100 us; 14 experts of 4,096 x 4,096 at 2,048 tokens 1,034 -> 660 us.  Tried and no better: 256
-// weight rows a workgroup (four waves of 128 x 64, or eight waves), steps of 32 in depth in three to five buffers.
+// Measured on weights that no cache holds, up + down, beside the kernel before it (128 rows, the next step's loads alone on their way,
+// all beginning at depth 0): 16 experts of 2,048 x 2,048, two a token, 2,011 tokens 220 -> 204 us, 1,024 tokens 145 -> 128, 753 tokens
+// (tiles of 64) 138 -> 127, 128 tokens 106 -> 81; 14 experts of 4,096 x 4,096, 2,048 tokens 663 -> 613, 951 tokens 430 -> 390.  Tiles of
+// 64 on 256 rows: 145 us at 753 tokens.  Tried and no better: 256 places a tile (at 753 tokens 187 us), two buffers for 256 rows (156),
+// four and five for 128 rows, workgroups that stay and take the next item while the last one's results are stored (no gain), loads of
+// one word a line that bring the weights into L2 two steps earlier (+ 25 %), streaming loads (twice as slow where tiles share weights).
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 #define ST_LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
 #define ST_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void*)(p))
@@ -639,8 +645,9 @@ __device__ inline bool moe_work_item(int& tile, int& block, int& expert, const i
 }
 
 enum TiledKind : int { kTiledDown = 0, kTiledUp = 1, kTiledGelu = 2 };
-template <int KIND, int NJ>
-__global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
+
+template <int KIND, int WN, int NJ>
+__global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void moe_tiled_kernel(
     bf16_t* __restrict__ y_out, float* out, const float* residual, float* __restrict__ pair_out, const bf16_t* __restrict__ a_rows,
     const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, const int* __restrict__ sorted, const int* __restrict__ tile_expert,
     const float* __restrict__ weights, int max_tiles, int blocks, int top, int N, int K, float limit, float out_scale, int style) {
@@ -649,109 +656,126 @@ __global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
     // 16 were used before, whose waves share the depth: their chains are an eighth as long (2,048 deep: 2.7e-7 off float64 in one chain,
     // 1.3e-7 in theirs).
     constexpr bool DOUBLE = KIND == kTiledDown && NJ == 1;
-    constexpr int PLACES = 64 * NJ;
-    constexpr int BUF = (128 + PLACES) * 8;        // 16-byte pieces a buffer: weight rows, then places
-    constexpr int NL = (128 + PLACES) / 32;        // direct loads a wave and step, eight rows each
-    __shared__ uint4 lds[2 * BUF];
+    constexpr int WAVES = 2 * WN, ROWS = 64 * WN, PLACES = 64 * NJ, AHEAD = 2;      // steps on their way
+    constexpr int BUF = (ROWS + PLACES) * 8;               // 16-byte pieces a buffer: weight rows, then places
+    constexpr int NW = ROWS / (8 * WAVES), NP = PLACES / (8 * WAVES), NL = NW + NP;      // direct loads a wave and step, eight rows each
+    __shared__ uint4 lds[(AHEAD + 1) * BUF];
     int tile, block, e;
     if (!moe_work_item(tile, block, e, tile_expert, max_tiles, blocks)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave & 1, wm = wave >> 1, l32 = lane & 31, lh = lane >> 5;
-    const int base = tile * PLACES, n0 = block * (UP ? 64 : 128);
-    // Load t of a wave brings rows 8 (wave + 4 t) on, a lane 16 bytes of row + lane / 8: piece lane % 8 of the row's place in
-    // LDS, which is the chunk that the row's swizzle puts there, the same for all t.  Rows past the matrix and places without a
-    // pair stand for row 0: their results are not stored, or stored as zeros.
+    const int wn = wave % WN, wm = wave / WN, l32 = lane & 31, lh = lane >> 5;
+    const int base = tile * PLACES, n0 = block * (UP ? ROWS / 2 : ROWS);
+    int pair[NJ], full = 0;                        // the pairs of the lane's columns of results; how many of the wave's blocks hold one
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        pair[j] = sorted[base + (2 * j + wm) * 32 + l32];
+        full += __ballot(pair[j] >= 0) != 0;       // (an expert's pairs come first in its tiles)
+    }
+    // Load t of a wave brings rows 8 (wave + WAVES t) on, a lane 16 bytes of row + lane / 8: piece lane % 8 of the row's place in
+    // LDS, which is the chunk that the row's swizzle puts there, the same for all t.  Rows past the matrix stand for row 0 and places
+    // without a pair for a row that is there: their results are not stored, or stored as zeros.
     const int chunk = (lane & 7) ^ swizzle(8 * wave + (lane >> 3));
     const bf16_t* src[NL];
 #pragma unroll
     for (int t = 0; t < NL; ++t) {
-        const int row = 8 * (wave + 4 * t) + (lane >> 3);
-        if (t < 4) {
+        const int row = 8 * (wave + WAVES * t) + (lane >> 3);
+        if (t < NW) {
             const int n = UP ? n0 + (row >> 6) * 32 + (row & 31) : n0 + row;
             const bf16_t* m = UP && ((row >> 5) & 1) ? w1 : w0;
             src[t] = m + ((int64_t)e * N + (n < N ? n : 0)) * K;
         } else {
-            const int place = base + row - 128, p = sorted[place];
-            src[t] = GATHER ? a_rows + (int64_t)(p >= 0 ? p / top : 0) * K : a_rows + (int64_t)place * K;
+            const int p = sorted[base + row - ROWS];
+            src[t] = a_rows + (GATHER ? (int64_t)(p >= 0 ? p / top : 0) : (int64_t)base + (p >= 0 ? row - ROWS : 0)) * K;
         }
         src[t] += chunk * 8;
     }
-    const int whole = K >> 6, steps = (K + 63) >> 6;
-    auto stage = [&](int s) {
-        uint4* dst = lds + (s & 1) * BUF + wave * 64;
-        if (s < whole) {
+    const int whole = K >> 6, steps = (K + 63) >> 6, begin = block * 3 % steps;
+    auto stage = [&](int s, int buf) {
+        int k = s + begin;
+        if (k >= steps) k -= steps;
+        uint4* dst = lds + buf * BUF + wave * 64;
+        if (k < whole) {
 #pragma unroll
             for (int t = 0; t < NL; ++t)
-                __builtin_amdgcn_global_load_lds(ST_GLOBAL_PTR(src[t] + s * 64), ST_LDS_PTR(void, dst + t * 256), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds(ST_GLOBAL_PTR(src[t] + k * 64), ST_LDS_PTR(void, dst + t * 64 * WAVES), 16, 0, 0);
         } else {                                   // the last, shorter step: zeros past the depth
-            const bool in = s * 64 + chunk * 8 < K;
+            const bool in = k * 64 + chunk * 8 < K;
 #pragma unroll
             for (int t = 0; t < NL; ++t) {
-                const uint4 v = *reinterpret_cast<const uint4*>(src[t] + (in ? s * 64 : -chunk * 8));
-                dst[t * 256 + lane] = in ? v : make_uint4(0, 0, 0, 0);
+                const uint4 v = *reinterpret_cast<const uint4*>(src[t] + (in ? k * 64 : -chunk * 8));
+                dst[t * 64 * WAVES + lane] = in ? v : make_uint4(0, 0, 0, 0);
             }
         }
     };
+    // (the swizzle of a lane's rows is that of l32: the rows before it are a multiple of 32)
+    const uint4* own = lds + l32 * 8;
+    const int swz = swizzle(l32);
     floatx16 acc[2][NJ];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
-    // (a chain's numbers are `per` steps long, so that it has no more roundings than the shares of the tiles of 16 places)
+            for (int q = 0; q < 16; ++q) acc[a][j][q] = 0.f;
     double total[DOUBLE ? 2 : 1][DOUBLE ? NJ : 1][16];
+    // (a chain's numbers are `per` steps long, so that it has no more roundings than the shares of the tiles of 16 places)
     const int per = max(1, min(4, K >> 9));
     int since = 0;
     if constexpr (DOUBLE)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                for (int q = 0; q < 16; ++q) total[i][j][q] = 0.0;
-    // (the swizzle of a lane's rows is that of l32: the rows before it are a multiple of 32)
-    const uint4* own = lds + l32 * 8;
-    const int swz = swizzle(l32);
+                for (int q = 0; q < 16; ++q) total[a][j][q] = 0.0;
     bf16x8 a[2][2], b[2][NJ];
-    auto fetch = [&](int buf, int kk) {            // the operands of a product of depth 16
-        const uint4* at = own + buf * BUF + ((kk * 2 + lh) ^ swz);
+    auto fetch = [&](auto blocks32, int cur, int kk) {              // the operands of a product of depth 16
+        const uint4* at = own + cur * BUF + ((kk * 2 + lh) ^ swz);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) a[kk & 1][i] = __builtin_bit_cast(bf16x8, at[(wn * 64 + i * 32) * 8]);
+        for (int q = 0; q < 2; ++q) a[kk & 1][q] = __builtin_bit_cast(bf16x8, at[(wn * 64 + q * 32) * 8]);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) b[kk & 1][j] = __builtin_bit_cast(bf16x8, at[(128 + (wm * NJ + j) * 32) * 8]);
+        for (int j = 0; j < decltype(blocks32)::value; ++j) b[kk & 1][j] = __builtin_bit_cast(bf16x8, at[(ROWS + (j * 2 + wm) * 32) * 8]);
     };
-    stage(0);
-    for (int s = 0; s < steps; ++s) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // this wave's loads of this step have landed
-        __syncthreads();                                             // everyone's have, and the other buffer has been read
-        fetch(s & 1, 0);
-        if (s + 1 < steps) stage(s + 1);
+    auto multiply = [&](auto blocks32, int cur) {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
-            if (kk < 3) fetch(s & 1, kk + 1);
+            if (kk < 3) fetch(blocks32, cur, kk + 1);
             __builtin_amdgcn_sched_barrier(0);     // (the next operands are on their way before these are multiplied)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int j = 0; j < NJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kk & 1][i], b[kk & 1][j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < decltype(blocks32)::value; ++j)
+                    acc[q][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kk & 1][q], b[kk & 1][j], acc[q][j], 0, 0, 0);
         }
+    };
+    stage(0, 0);
+    if (steps > 1) stage(1, 1);
+    for (int s = 0, cur = 0; s < steps; ++s) {
+        // This wave's loads of the step have landed, those of the steps after it may be on their way; then everyone's have, and the
+        // buffer of the step before has been read.
+        if (s + AHEAD > steps) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((AHEAD - 1) * NL) : "memory");
+        if (full == NJ) fetch(Steps<NJ>(), cur, 0);
+        else if (NJ > 1 && full > 0) fetch(Steps<1>(), cur, 0);
+        if (s + AHEAD < steps) stage(s + AHEAD, cur == 0 ? AHEAD : cur - 1);
+        if (full == NJ) multiply(Steps<NJ>(), cur);
+        else if (NJ > 1 && full > 0) multiply(Steps<1>(), cur);
+        cur = cur == AHEAD ? 0 : cur + 1;
         if constexpr (DOUBLE)
             if (++since == per || s + 1 == steps) {
                 since = 0;
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int q = 0; q < 2; ++q)
 #pragma unroll
                     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-                        for (int q = 0; q < 16; ++q) {
-                            total[i][j][q] += (double)acc[i][j][q];
-                            acc[i][j][q] = s + 1 == steps ? (float)total[i][j][q] : 0.f;
+                        for (int u = 0; u < 16; ++u) {
+                            total[q][j][u] += (double)acc[q][j][u];
+                            acc[q][j][u] = s + 1 == steps ? (float)total[q][j][u] : 0.f;
                         }
             }
     }
-    // acc[i][j][q]: weight row wn * 64 + i * 32 + 8 * (q / 4) + 4 * lh + q % 4, place base + (wm * NJ + j) * 32 + l32
+    // acc[q][j][u]: weight row wn * 64 + q * 32 + 8 * (u / 4) + 4 * lh + u % 4, place base + (2 * j + wm) * 32 + l32
     auto store_row = [&](int place, int f, const float* r) {
         bf16_t* dst = y_out + (int64_t)place * N + f;
         if (f + 3 < N && (N & 3) == 0) Elem<bf16_t>::store4(dst, r);
@@ -760,8 +784,8 @@ __global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
     };
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        const int place = base + (wm * NJ + j) * 32 + l32;
-        const int p = sorted[place];
+        const int place = base + (j * 2 + wm) * 32 + l32;
+        const int p = pair[j];
         if (UP) {
             const float scale = p >= 0 && style == 0 ? weights[p] : 1.f;
 #pragma unroll
@@ -784,32 +808,32 @@ __global__ __launch_bounds__(256, 2) void moe_tiled_kernel(
             }
         } else if (KIND == kTiledGelu) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int q = 0; q < 2; ++q)
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) {
-                    const int f = n0 + wn * 64 + i * 32 + 8 * q4 + 4 * lh;
+                    const int f = n0 + wn * 64 + q * 32 + 8 * q4 + 4 * lh;
                     if (f >= N) continue;
                     float r[4];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) r[u] = p >= 0 ? apply_activation(kActGeluErf, acc[i][j][4 * q4 + u]) : 0.f;
+                    for (int u = 0; u < 4; ++u) r[u] = p >= 0 ? apply_activation(kActGeluErf, acc[q][j][4 * q4 + u]) : 0.f;
                     store_row(place, f, r);
                 }
         } else {
             if (p < 0) continue;
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int q = 0; q < 2; ++q)
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) {
-                    const int n = n0 + wn * 64 + i * 32 + 8 * q4 + 4 * lh;
+                    const int n = n0 + wn * 64 + q * 32 + 8 * q4 + 4 * lh;
                     if (pair_out && (N & 3) == 0 && n + 3 < N) {
                         *reinterpret_cast<float4*>(pair_out + (int64_t)place * N + n) = make_float4(
-                            acc[i][j][4 * q4], acc[i][j][4 * q4 + 1], acc[i][j][4 * q4 + 2], acc[i][j][4 * q4 + 3]);
+                            acc[q][j][4 * q4], acc[q][j][4 * q4 + 1], acc[q][j][4 * q4 + 2], acc[q][j][4 * q4 + 3]);
                         continue;
                     }
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
                         if (n + u >= N) continue;
-                        const float v = acc[i][j][4 * q4 + u];
+                        const float v = acc[q][j][4 * q4 + u];
                         if (pair_out) pair_out[(int64_t)place * N + n + u] = v;
                         else {
                             const int64_t at = (int64_t)p * N + n + u;       // one expert a token: p is the token
@@ -825,14 +849,15 @@ template <int KIND>
 static int launch_tiled(bf16_t* y, float* out, const float* residual, float* pair_out, const void* a_rows, const void* w0,
                         const void* w1, const int* sorted, const int* tile_expert, const float* weights, int capacity, int tile, int top,
                         int N, int K, float limit, float out_scale, int style, hipStream_t stream) {
-    const int features = KIND == kTiledUp ? 64 : 128, tiles = capacity / tile, blocks = (N + features - 1) / features;
+    const int rows = tile == 64 ? 128 : 256, features = KIND == kTiledUp ? rows / 2 : rows;
+    const int tiles = capacity / tile, blocks = (N + features - 1) / features;
     ST_CHECK((int64_t)tiles * blocks < (1ll << 30), "moe: too many tiles");
     const unsigned grid = (unsigned)((tiles * blocks + 7) / 8 * 8);
     if (tile == 64)
-        moe_tiled_kernel<KIND, 1><<<grid, 256, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
+        moe_tiled_kernel<KIND, 2, 1><<<grid, 256, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
             (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
     else
-        moe_tiled_kernel<KIND, 2><<<grid, 256, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
+        moe_tiled_kernel<KIND, 4, 2><<<grid, 512, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
             (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
     ST_LAUNCH_CHECK("moe (tiled)");
     return 0;

@@ -103,3 +103,28 @@ def test_sums_of_64_places_are_no_further_from_float64_than_those_of_16(E, W, F,
         return float((out[place.long()] - want).norm() / want.norm())
 
     assert err(64) <= err(16), (err(64), err(16))
+
+
+@pytest.mark.parametrize("W,F", [(64, 128), (128, 136), (192, 256), (200, 264), (320, 520)])      # depths of 1 to 5 steps, 4 of them part of a step
+@pytest.mark.parametrize("counts", [(1, 127, 0, 260), (32, 33, 64, 300), (65, 96, 97, 200), (128, 129, 160, 31)])
+def test_last_tiles_that_are_partly_empty(W, F, counts):
+    """Experts with chosen numbers of rows (one choice a token), around every block of 32 places of their last tile of 128."""
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator().manual_seed(W + sum(counts))
+    E, T = len(counts), sum(counts)
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).bfloat16().to(F64)
+    x, wg, wu, wd = rnd(T, W), rnd(E, F, W, std=W ** -0.5), rnd(E, F, W, std=W ** -0.5), rnd(E, W, F, std=F ** -0.5)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)]
+    z = torch.full((T, E), -4.0)
+    z[torch.arange(T), ids] = 4.0
+    dev = lambda t, d=torch.bfloat16: t.to("cuda").to(d)
+    res = torch.randn(T, W, generator=g)
+    for top in (1, 2):                                         # straight into the stream; a row a pair (the second choice: expert 0 or 1)
+        ids2 = torch.topk(z, top, dim=1).indices
+        wts = torch.softmax(z.to(F64).gather(1, ids2), 1)
+        want, size = _experts(x, ids2, wts, wg, wu, wd, "silu", False, 0.0)
+        got = K.routed_experts(dev(x), dev(z, torch.float32), dev(wg), dev(wu), dev(wd), dev(res, torch.float32), top=top, style="softmax_output")
+        assert K.moe_tile(T, top, E, True) == (128 if top * T >= 112 * E else 64)
+        # an expert's inner values are rounded to bfloat16 once (by 2^-8 of each at most); every sum is float
+        err = (got.double().cpu() - (res.to(F64) + want)).abs()
+        assert bool((err <= (2.0 ** -8 + 1e-4) * size + 1e-5).all()), float((err / size).max())
