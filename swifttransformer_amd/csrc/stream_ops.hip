@@ -21,26 +21,52 @@
 
 namespace st {
 
-template <typename T>
+// V columns a thread (4: 16-byte accesses); a workgroup takes 256 V columns of one row.  1,024 rows of 2,048 into the storage type, by
+// element and by four: 8.8 and 6.0 us.
+template <typename T, int V>
 __global__ __launch_bounds__(256) void dynamic_tanh_kernel(
     T* __restrict__ out_t, float* __restrict__ out32, const float* __restrict__ x, const int* __restrict__ rows,
     const float* __restrict__ w, const float* __restrict__ b, const float* __restrict__ alpha,
     const float* __restrict__ base, const float* __restrict__ w2, const float* __restrict__ b2,
-    const float* __restrict__ alpha2, int width, int64_t total) {
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int64_t r = idx / width;
-    const int c = (int)(idx - r * width);
+    const float* __restrict__ alpha2, int width) {
+    const int64_t r = blockIdx.x;
+    const int c = (blockIdx.y * 256 + threadIdx.x) * V;
+    if (c >= width) return;
     int64_t src = r;
     if (rows) {
         src = rows[r];
         if (src < 0) return;                              // a padding entry
     }
-    float y = tanhf(alpha[0] * x[src * width + c]) * w[c] + (b ? b[c] : 0.f);
-    if (base) y += base[idx];
-    if (out32) out32[idx] = y;
-    if (w2) y = tanhf(alpha2[0] * y) * w2[c] + (b2 ? b2[c] : 0.f);     // the next norm, of the sum just made
-    if (out_t) Elem<T>::store(out_t + idx, y);
+    const int64_t idx = r * width + c;
+    auto load = [](const float* p, float* v) {
+        if (V == 4) Elem<float>::load_vec(p, v);
+        else v[0] = p[0];
+    };
+    float y[V], g[V], s[V], g2[V], s2[V], on[V];
+    load(x + src * width + c, y);
+    load(w + c, g);
+    if (b) load(b + c, s);
+    if (base) load(base + idx, on);
+    if (w2) load(w2 + c, g2);
+    if (b2) load(b2 + c, s2);
+    const float a = alpha[0], a2 = w2 ? alpha2[0] : 0.f;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        y[u] = tanhf(a * y[u]) * g[u] + (b ? s[u] : 0.f);
+        if (base) y[u] += on[u];
+    }
+    if (out32) {
+        if (V == 4) Elem<float>::store_vec(out32 + idx, y);
+        else out32[idx] = y[0];
+    }
+    if (w2) {                                             // the next norm, of the sum just made
+#pragma unroll
+        for (int u = 0; u < V; ++u) y[u] = tanhf(a2 * y[u]) * g2[u] + (b2 ? s2[u] : 0.f);
+    }
+    if (out_t) {
+        if (V == 4) Elem<T>::store4(out_t + idx, y);
+        else Elem<T>::store(out_t + idx, y[0]);
+    }
 }
 
 // logits through a factor and a smooth limit: cap * tanh(x * scale / cap)
@@ -156,13 +182,18 @@ extern "C" int st_dynamic_tanh(void* out_t, float* out32, const float* x, const 
     if (num_rows == 0) return 0;
     ST_CHECK(x && w && alpha && (out_t || out32), "dynamic_tanh: null operand");
     ST_CHECK(!w2 || (alpha2 && out_t), "dynamic_tanh: a second norm needs its alpha and the storage-type output");
-    const int64_t total = (int64_t)num_rows * width;
-    const unsigned grid = (unsigned)((total + 255) / 256);
-    if (dtype == kF32)
-        dynamic_tanh_kernel<float><<<grid, 256, 0, stream>>>((float*)out_t, out32, x, rows, w, b, alpha, base, w2, b2, alpha2, width, total);
-    else if (dtype == kBF16)
-        dynamic_tanh_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)out_t, out32, x, rows, w, b, alpha, base, w2, b2, alpha2, width, total);
-    else ST_CHECK(false, "dynamic_tanh: unknown dtype %d", dtype);
+    ST_CHECK(dtype == kF32 || dtype == kBF16, "dynamic_tanh: unknown dtype %d", dtype);
+    const uintptr_t align = (uintptr_t)out32 | (uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)base | (uintptr_t)w2 | (uintptr_t)b2;
+    const bool four = width % 4 == 0 && (align & 15) == 0 && (uintptr_t)out_t % (dtype == kF32 ? 16 : 8) == 0;
+    const int span = four ? 1024 : 256;
+    const int64_t blocks = ((int64_t)width + span - 1) / span;
+    ST_CHECK(blocks <= 65535, "dynamic_tanh: rows of %d are too wide", width);
+    const dim3 grid((unsigned)num_rows, (unsigned)blocks);
+#define ST_DT(T, V)                                                                                             \
+    dynamic_tanh_kernel<T, V><<<grid, 256, 0, stream>>>((T*)out_t, out32, x, rows, w, b, alpha, base, w2, b2, alpha2, width)
+    if (dtype == kF32) { if (four) ST_DT(float, 4); else ST_DT(float, 1); }
+    else { if (four) ST_DT(bf16_t, 4); else ST_DT(bf16_t, 1); }
+#undef ST_DT
     ST_LAUNCH_CHECK("dynamic_tanh");
     return 0;
 }
@@ -208,6 +239,8 @@ extern "C" int st_token_side(float* x, const int* token_ids, const int* token_it
     ST_CHECK(lds <= 60 * 1024, "token_side: a row of %d and a gated vector of %d do not fit the LDS", width, dim);
     if (num_rows == 0) return 0;
     ST_CHECK(x && token_ids && table && w_gate && w_proj && gain, "token_side: null operand");
+    const int vec = dtype == kF32 ? 4 : 8;
+    const bool aligned = width % vec == 0 && dim % vec == 0 && (uintptr_t)w_gate % 16 == 0 && (uintptr_t)w_proj % 16 == 0;
     const int threads = num_rows <= 256 ? 1024 : 256;
     const int vec = dtype == kF32 ? 4 : 8;
     const bool aligned = width % vec == 0 && dim % vec == 0 && (uintptr_t)w_gate % 16 == 0 && (uintptr_t)w_proj % 16 == 0;
