@@ -239,8 +239,6 @@ extern "C" int st_token_side(float* x, const int* token_ids, const int* token_it
     ST_CHECK(lds <= 60 * 1024, "token_side: a row of %d and a gated vector of %d do not fit the LDS", width, dim);
     if (num_rows == 0) return 0;
     ST_CHECK(x && token_ids && table && w_gate && w_proj && gain, "token_side: null operand");
-    const int vec = dtype == kF32 ? 4 : 8;
-    const bool aligned = width % vec == 0 && dim % vec == 0 && (uintptr_t)w_gate % 16 == 0 && (uintptr_t)w_proj % 16 == 0;
     const int threads = num_rows <= 256 ? 1024 : 256;
     const int vec = dtype == kF32 ? 4 : 8;
     const bool aligned = width % vec == 0 && dim % vec == 0 && (uintptr_t)w_gate % 16 == 0 && (uintptr_t)w_proj % 16 == 0;
