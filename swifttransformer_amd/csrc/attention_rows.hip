@@ -300,6 +300,9 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
 }
 
 // out[t,h,:] = sum_s w_s * part_o[ri,h,s,:] / sum_s w_s,  w_s = exp(lse_s - max lse)
+// What bounds it: trips to memory one after the other.  A lane a split forms the weights, and the partial results are asked for eight
+// splits at a time without waiting for them (one row of 12 heads, 16 splits: 6.9 us with the splits one by one, 4.8 us; sums in the
+// same order).
 template <typename T>
 __global__ __launch_bounds__(64) void attn_merge_kernel(
     T* __restrict__ out, const float* __restrict__ part_o, const float* __restrict__ part_lse,
@@ -307,25 +310,45 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(
     int64_t gate_stride) {
     const int64_t row = blockIdx.x;   // ri * num_q_heads + h
     const int64_t ri = row / num_q_heads, h = row - ri * num_q_heads;
-    if (row_ids && row_ids[ri] < 0) return;        // padding entry: its partial results were never written
-    const int64_t t = row_ids ? row_ids[ri] : ri, orow = t * num_q_heads + h;
-    const float gate = head_gate ? gate_factor(head_gate[t * gate_stride + h]) : 1.f;
     const float* lse = part_lse + row * num_splits;
-    float M = -INFINITY;
-    for (int s = 0; s < num_splits; ++s) M = fmaxf(M, lse[s]);
-    for (int d = threadIdx.x; d < head_dim; d += blockDim.x) {
+    const float* parts = part_o + row * num_splits * head_dim;
+    const int lane = threadIdx.x, t_id = row_ids ? row_ids[ri] : 0;
+    constexpr int U = 8;
+    const bool few = num_splits <= 64;
+    const float own = lse[min(lane, num_splits - 1)];          // (with up to 64 splits: lane s has that of split s)
+    float first[U];                                            // the first columns' first partial results
+#pragma unroll
+    for (int u = 0; u < U; ++u) first[u] = parts[(int64_t)min(u, num_splits - 1) * head_dim + min(lane, head_dim - 1)];
+    if (t_id < 0) return;             // padding entry: its partial results were never written
+    const int64_t t = row_ids ? t_id : ri, orow = t * num_q_heads + h;
+    const float gate = head_gate ? gate_factor(head_gate[t * gate_stride + h]) : 1.f;
+    float M = own;
+    for (int s = 64 + lane; s < num_splits; s += 64) M = fmaxf(M, lse[s]);
+    M = wave_max(M);
+    const float weight = own > -INFINITY ? expf(own - M) : 0.f;
+    for (int d0 = 0; d0 < head_dim; d0 += 64) {
+        const int d = min(d0 + lane, head_dim - 1);
         float W = 0.f, o = 0.f;
-        if (M > -INFINITY) {
-            for (int s = 0; s < num_splits; ++s) {
-                const float ls = lse[s];
-                if (ls > -INFINITY) {
-                    const float w = expf(ls - M);
-                    W += w;
-                    o += w * part_o[(row * num_splits + s) * head_dim + d];
+        for (int s0 = 0; s0 < num_splits; s0 += U) {
+            float v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                v[u] = d0 == 0 && s0 == 0 ? first[u] : parts[(int64_t)min(s0 + u, num_splits - 1) * head_dim + d];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (s0 + u >= num_splits) break;
+                float w;
+                if (few) {
+                    w = __shfl(weight, s0 + u, 64);
+                } else {
+                    const float ls = lse[s0 + u];
+                    w = ls > -INFINITY ? expf(ls - M) : 0.f;
                 }
+                W += w;
+                if (w > 0.f) o += w * v[u];          // (no weight: nothing to add, whatever lies there)
             }
         }
-        Elem<T>::store(out + orow * head_dim + d, W > 0.f ? o / W * gate : 0.f);
+        if (d0 + lane < head_dim) Elem<T>::store(out + orow * head_dim + d, W > 0.f ? o / W * gate : 0.f);
     }
 }
 

@@ -237,7 +237,9 @@ class DecoderModel:
             # the head's kernel normalises the wanted rows itself and finds their best tokens
             y_t, fused_best = self.final_norm.as_input(x32, rows), best
         elif self.final_norm is not None:
-            (y_t, _), fused_best = self.final_norm.forward(x32, out_t=True, rows=rows), None
+            # (a norm that the head's kernel does not know: the kernel finds the best tokens all the same)
+            offers = getattr(self.head, "offers_best", None)
+            (y_t, _), fused_best = self.final_norm.forward(x32, out_t=True, rows=rows), best if offers is not None and offers(n) else None
         else:
             y32 = K.empty((n, self.hidden_size), torch.float32, x32.device)
             K.lookup(rows, x32, out_f32=y32)

@@ -163,9 +163,15 @@ class LMHead(Part):
         return (self.logit_scale > 0 and not self.projected and hasattr(norm, "as_input") and getattr(norm, "width", None) == self.embed_dim
                 and K.wide_offered(rows, self.vocab_size, self.embed_dim, self.dtype))
 
+    def offers_best(self, rows: int) -> bool:
+        """Whether ``forward`` of that many normalised rows reports the rows' best outputs.  (Not through a limit: it may make two
+        different outputs equal, and the best is then the lower index.)"""
+        return (self.logit_scale > 0 and self.softcap == 0 and not self.projected
+                and K.wide_offered(rows, self.vocab_size, self.embed_dim, self.dtype))
+
     def forward(self, y_t, best: Optional[torch.Tensor] = None) -> torch.Tensor:
         """float32 logits [rows, vocab] of ``y_t``: normalised rows, or (where ``takes_norm``) what a
-        norm's ``as_input`` returned.  ``best`` (int32 [rows], where ``takes_norm``): receives every
+        norm's ``as_input`` returned.  ``best`` (int32 [rows], where ``takes_norm`` or ``offers_best``): receives every
         row's best output, the lowest index on ties."""
         if self.projected:
             y_t = K.gemm(y_t, self.w_out)

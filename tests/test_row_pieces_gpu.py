@@ -1,0 +1,75 @@
+"""Row kernels that take several columns and rows a thread, beside the same kernels on operands that no wide access fits: the same bits."""
+import pytest
+import torch
+
+from test_zimorax_gpu import DEV, DTYPES, items_ctx
+
+pytestmark = pytest.mark.gpu
+
+
+def _shifted(t):
+    """The same values, contiguous, four bytes (two in bfloat16) past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)[1:1 + t.numel()].view(t.shape)
+    return flat.copy_(t)
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("in_dtype,out_dtype", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("width,lens", [(4, (70,)), (1028, (1, 2, 3, 61)), (8, (5, 1, 1, 1, 64, 2)), (2048, (63,)), (260, (1, 1, 1))])
+def test_token_conv_in_pieces_of_four(taps, in_dtype, out_dtype, width, lens):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(width + taps)
+    T = sum(lens) + 1                                          # and a padding row
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    wide = rnd(T, width + 5).to(in_dtype)
+    x = torch.empty(T, width + 8, dtype=in_dtype, device=DEV)[:, 4:4 + width].copy_(wide[:, 1:1 + width])
+    w, bias, state = rnd(width, taps), rnd(width), rnd(len(lens), taps - 1, width)
+    ti, ln, off, sl = items_ctx(list(lens), list(range(len(lens)))[::-1])
+    ti = torch.cat([ti, torch.full((1,), -1, dtype=torch.int32, device=DEV)])
+    for kw in ({}, {"add_input": False, "bias": bias, "activation": "silu"}):
+        s1, s2 = state.clone(), state.clone()
+        four = K.token_conv(x, w, s1, (ti, ln, off, sl), out_dtype, **kw)
+        one = K.token_conv(wide[:, 1:1 + width], w, s2, (ti, ln, off, sl), out_dtype, **kw)
+        assert torch.equal(four, one) and torch.equal(s1, s2)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("rows,width", [(1, 4), (3, 1024), (70, 1028), (2, 2052)])
+def test_dynamic_tanh_and_concat_cast_in_pieces_of_four(dtype, rows, width):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(width)
+    dt = DTYPES[dtype]
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, base, w, b, w2, b2, alpha = rnd(rows, width), rnd(rows, width), rnd(width), rnd(width), rnd(width), rnd(width), rnd(1)
+    picked = torch.randint(-1, rows, (rows + 2,), generator=g, device=DEV, dtype=torch.int32)
+
+    def run(shift):
+        f = _shifted if shift else (lambda t: t)
+        outs = [torch.full((rows, width), 3.0, device=DEV), torch.full((rows, width), 3.0, device=DEV, dtype=dt),
+                torch.full((rows + 2, width), 3.0, device=DEV, dtype=dt)]
+        K.dynamic_tanh(f(x), w, b, alpha, out_f32=outs[0], out_t=outs[1], base=base, then=(w2, b2, alpha))
+        K.dynamic_tanh(f(x), w, None, alpha, out_t=outs[2], rows=picked)
+        return outs + [K.concat_cast(f(x), base, dt)]
+    for four, one in zip(run(False), run(True)):
+        assert torch.equal(four, one)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("heads,hd,splits,gated", [(12, 64, 16, False), (3, 16, 2, True), (2, 80, 9, True), (1, 256, 70, False), (4, 128, 64, True)])
+def test_split_attention_merged_by_lanes(dtype, heads, hd, splits, gated):
+    """Rows whose keys are shared out over many splits, some of them empty (3 to 90 keys on up to 70 splits), against one split."""
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(splits)
+    dt, ps, lens = DTYPES[dtype], 16, (3, 90, 17)
+    B = len(lens)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    kc, vc = rnd(8 * B, heads, ps, hd).to(dt), rnd(8 * B, heads, ps, hd).to(dt)
+    bt = torch.arange(8 * B, device=DEV, dtype=torch.int32).view(B, 8)
+    q, item = rnd(B, heads * hd).to(dt), torch.arange(B, device=DEV, dtype=torch.int32)
+    pos = torch.tensor(lens, device=DEV, dtype=torch.int32) - 1
+    kw = {"head_gate": rnd(B, heads)} if gated else {}
+    one = K.attention_rows(q, kc, vc, item, pos, bt, heads, hd ** -0.5, num_splits=1, **kw)
+    many = K.attention_rows(q, kc, vc, item, pos, bt, heads, hd ** -0.5, num_splits=splits, **kw)
+    # float sums of up to 90 weights in another order, then one rounding to the storage type (2^-9 of a value up to twice)
+    tol = 1e-5 if dt == torch.float32 else 2.0 ** -8
+    assert bool(((one.float() - many.float()).abs() <= tol * one.float().abs() + 1e-5).all())
