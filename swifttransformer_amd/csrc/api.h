@@ -374,6 +374,7 @@ int st_latent_inputs(void* cq, int cq_width, const float* gain_q, int q_rank, vo
                      const int* block_table, int max_pages, int page_size, int num_tokens, float eps, int dtype,
                      hipStream_t stream);
 int st_latent_max_entry();
+int st_latent_tiles_fit(int heads, int entry, int page_size, int max_pages, int rot_half);
 int st_latent_tiles(void* out, const void* q, int64_t q_stride, const void* cache, int64_t page_stride, const int* tile_item,
                     const int* tile_q0, int num_tiles, const int* item_tok_off, const int* item_start, const int* item_len,
                     const int* block_table, const float* sink, const float* freq, int max_pages, int page_size, int heads,

@@ -720,13 +720,18 @@ static size_t latent_turn_bytes(const LatentArgs& a, bool tiles, int rows) {
 }
 
 template <bool TILES, int HDP, int QT, int NKT, int RW, int KW>
-static int launch_latent(const LatentArgs& a, int list, hipStream_t stream) {
-    auto kernel = latent_attn_kernel<TILES, HDP, QT, NKT, RW, KW>;
+static size_t latent_lds(const LatentArgs& a) {
     constexpr size_t bufs = (size_t)KW * 2 * 16 * NKT * HDP * 64;
     constexpr size_t merge = (size_t)(KW - 1) * RW * 64 * QT * (2 + 8 * HDP) * sizeof(float);
+    const size_t table = (size_t)latent_table(a, TILES, 16 * NKT) * sizeof(int) + latent_turn_bytes(a, TILES, RW * QT * 16);
+    return bufs + table > merge ? bufs + table : merge;
+}
+
+template <bool TILES, int HDP, int QT, int NKT, int RW, int KW>
+static int launch_latent(const LatentArgs& a, int list, hipStream_t stream) {
+    auto kernel = latent_attn_kernel<TILES, HDP, QT, NKT, RW, KW>;
     constexpr int rows = RW * QT * 16;
-    const size_t table = (size_t)latent_table(a, TILES, 16 * NKT) * sizeof(int) + latent_turn_bytes(a, TILES, rows);
-    const size_t lds = bufs + table > merge ? bufs + table : merge;
+    const size_t lds = latent_lds<TILES, HDP, QT, NKT, RW, KW>(a);
     if (latent_raise_lds(reinterpret_cast<const void*>(kernel), lds)) return 1;
     const int x = ((TILES ? kTileTokens : 1) * a.heads + rows - 1) / rows;
     LatentArgs args = a;
@@ -770,10 +775,16 @@ static int latent_dispatch(const LatentArgs& a, int list, int dtype, hipStream_t
     // (an entry runs in the next larger instance, its missing chunks zeros in LDS)
     const int hdp = (a.entry + 31) / 32;
     // tiles: four waves of 16 rows, blocks of 64 keys (32 where entries are large); rows: one or two waves of 16 rows,
-    // four (two) shares of the keys, blocks of 32 keys
+    // four (two) shares of the keys, blocks of 32 keys.  Tiles whose workgroups are fewer than one and a half times the compute units
+    // (and whose page lists leave the room) share out their keys over two groups of waves: entries of 160, one item from position 0,
+    // without and with, us: 64 tokens of 32 heads behind 1,500 others (32 workgroups) 53 and 37, 512 tokens (256) 22 and 18, 1,024 of 16
+    // heads and 192 (256) 43 and 31; 1,024 of 32 heads (512) 40 and 43.
+    const bool half_empty = 2ll * list * ((kTileTokens * (int64_t)a.heads + 63) / 64) < 3 * device_compute_units();
 #define ST_LT(H)                                                                                                       \
     if (hdp <= H) {                                                                                                    \
-        if constexpr (TILES) return launch_latent<TILES, H, 1, 4, 4, 1>(a, list, stream);                              \
+        if constexpr (TILES)                                                                                           \
+            return half_empty && latent_lds<TILES, H, 1, 4, 4, 2>(a) <= kLatentMaxLds                                  \
+                       ? launch_latent<TILES, H, 1, 4, 4, 2>(a, list, stream) : launch_latent<TILES, H, 1, 4, 4, 1>(a, list, stream); \
         else return a.heads <= 16 ? launch_latent<TILES, H, 1, 2, 1, 4>(a, list, stream) : launch_latent<TILES, H, 1, 2, 2, 4>(a, list, stream); \
     }
 #define ST_LB(H)                                                                                                       \
@@ -788,6 +799,14 @@ static int latent_dispatch(const LatentArgs& a, int list, int dtype, hipStream_t
 }
 
 extern "C" int st_latent_max_entry() { return kLatentMaxEntry; }
+
+// Whether bfloat16 tiles of entries of up to 256 dims leave room for page lists this long.
+extern "C" int st_latent_tiles_fit(int heads, int entry, int page_size, int max_pages, int rot_half) {
+    if (heads <= 0 || entry <= 0 || entry % 16 || entry > 256 || page_size <= 0 || max_pages <= 0 || rot_half < 0) return 0;
+    LatentArgs a = {};
+    a.heads = heads; a.entry = entry; a.page_size = page_size; a.max_pages = max_pages; a.rot_half = rot_half; a.num_splits = 1;
+    return latent_lds<true, 8, 1, 4, 4, 1>(a) <= kLatentMaxLds ? 1 : 0;
+}
 
 // Common arguments of both forms: q [tokens, heads, entry] with rows of q_stride elements; cache [pages, page_size, entry];
 // out_dim: dims of a result (a multiple of 16, at most entry); rot_off / rot_half / freq / rot_mult: pairs (rot_off + 2i,

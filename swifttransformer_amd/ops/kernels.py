@@ -113,6 +113,7 @@ def _lib():
         lib.st_latent_inputs.argtypes = [_c_p, _c_int, _c_p, _c_int, _c_p, _c_i64, _c_p, _c_int, _c_int, _c_int, _c_p, _c_int,
                                          _c_f, _c_int, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_f, _c_int,
                                          _c_p]
+        lib.st_latent_tiles_fit.argtypes = [_c_int] * 5
         lib.st_latent_tiles.argtypes = [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_int, _c_p, _c_p, _c_p, _c_p, _c_p,
                                         _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _c_int,
                                         _c_int, _c_p]
@@ -2011,6 +2012,11 @@ def delta_rule(proj: torch.Tensor, taps_w: torch.Tensor, a_log: torch.Tensor, dt
 def latent_max_entry() -> int:
     """The largest cached entry (a multiple of 16) that the latent attention kernels take."""
     return int(_lib().st_latent_max_entry())
+
+
+def latent_tiles_fit(heads: int, entry: int, page_size: int, max_pages: int, turned_pairs: int = 0) -> bool:
+    """Whether ``latent_tiles`` of bfloat16 takes entries of this size (up to 256) with block tables this wide."""
+    return bool(_lib().st_latent_tiles_fit(int(heads), int(entry), int(page_size), int(max_pages), int(turned_pairs)))
 
 
 class LatentShape:

@@ -28,7 +28,7 @@ import torch
 
 from ..ops import kernels as K
 from ..weights.loader import TensorSpec
-from .attention import PagedAttention
+from .attention import PagedAttention, plan_tiles
 from .base import CacheNeed
 from .position import rotary_frequencies
 
@@ -114,6 +114,31 @@ class LatentAttention(PagedAttention):
 
     accepts_norm = False
 
+    def _latent_tiles(self, page_size: int, max_pages: int) -> bool:
+        """Whether prompts go through the tiles made for a latent cache, which read an entry once for scores and sums.  Entries of up
+        to 128 stay with the paged kernels (2,011 tokens of 32 heads, entries of 128: 63 us there in tiles of 128 rows, 65 by latent
+        tiles; 300 tokens of 12 heads, 96: 8 and 11); above, the paged kernel is the general one (entries of 160, 1,024 tokens of 32
+        heads 59 and 40 us, 753 behind 1,024 others 85 and 48, 112 tokens 9.1 and 9.3; entries of 256 105 and 59)."""
+        half = self.rot_dim // 2 if self._turns_in_tiles() else 0
+        return (self.dtype == torch.bfloat16 and self.entry > 128 and not self._biased()
+                and K.latent_tiles_fit(self.num_heads, self.entry, page_size, max_pages, half))
+
+    def _biased(self) -> bool:
+        return self.position is not None and getattr(self.position, "biases_scores", False)      # (the latent kernel knows no slopes)
+
+    def _turns_in_tiles(self) -> bool:
+        return self.rot_dim > 0 and self.rank % 8 == 0       # (the kernel turns whole pieces of 8)
+
+    def plan_key(self):
+        return ("latent_attention_tiles", self.tile_min_len, self.num_heads, self.entry, self.dtype, self._turns_in_tiles(), self.rot_dim, self._biased())
+
+    def step_planner(self):
+        def planner(items, info):
+            choose = lambda rows: (K.PREFILL_TILE if self._biased() or self._latent_tiles(info.page_size, info.max_pages) else
+                                   K.prefill_tile_rows(self.entry, info.page_size, info.max_pages, self.num_heads, rows, self.dtype))
+            return plan_tiles(items, self.tile_min_len, choose, bucketed=info.bucketed)
+        return self.plan_key(), planner
+
     def forward(self, x_t: torch.Tensor, residual32: Optional[torch.Tensor], ctx, cache, write: bool = True,
                 norm=None) -> torch.Tensor:
         if write != self.own_latent:
@@ -123,7 +148,24 @@ class LatentAttention(PagedAttention):
             K.latent_write(cache.k, raw, self.gain, self.eps, ctx.token_item, ctx.positions,
                            ctx.block_tables[cache.group], tail=self.rot_dim, tail_freq=self.freq, tail_mult=self.rot_mult)
         q = K.gemm(x_t, self.w_q)
-        if self.rot_dim:
+        plan, bt = ctx.plans.get(self.plan_key()), ctx.block_tables[cache.group]
+        tiles = plan is not None and K.prefill_available() and self._latent_tiles(cache.k.shape[2], bt.shape[1])
+        # (the tiles turn the queries themselves, unless rows of another kernel need them turned too)
+        inside = tiles and plan.host["num_short_rows"] == 0 and self._turns_in_tiles()
+        if self.rot_dim and not inside:
             K.rotary(q, None, self.entry, self.freq, self.rot_mult, ctx.positions, offset=self.rank, interleaved=True)
-        o = self.attend(q, ctx, cache, unmerged_ok=True)
+        if not tiles:
+            o = self.attend(q, ctx, cache, unmerged_ok=True)
+        else:
+            o = K.empty((q.shape[0], self.q_size), self.dtype, q.device)
+            # (whole entries as results: the output matrix has zeros for the turned part)
+            shape = K.LatentShape(self.num_heads, self.entry, self.entry, self.scale, self.rank if inside else 0,
+                                  self.freq if inside else None, self.rot_mult, None, self.window)
+            K.latent_tiles(q, cache.k, plan.arrays["tile_item"], plan.arrays["tile_q0"], ctx.item_tok_off, ctx.item_start,
+                           ctx.item_len, bt, shape, o)
+            n = plan.host["num_short_rows"]
+            if n > 0:
+                splits, waves = self._shape_row_kernel(ctx, n)
+                K.attention_rows(q, cache.k, cache.v, ctx.token_item, ctx.positions, bt, self.num_heads, self.scale,
+                                 window=self.window, row_ids=plan.arrays["short_rows"], num_splits=splits, num_waves=waves, out=o)
         return K.gemm(o, self.w_out, residual=residual32, out_f32=True, out_scale=self.residual_scale)
