@@ -268,6 +268,11 @@ int st_moe_route(int* ids, float* weights, const float* logits, int logit_stride
 // places that hold one expert's pairs each: sorted[capacity] (pair index, or -1),
 // place_of_pair[num_pairs] (or -1), tile_expert[capacity / tile] (or -1).
 // capacity >= round_up(num_pairs, tile) + tile * experts.  st_moe_up and st_moe_down take the same `tile`.
+int st_moe_router_align_offered(int num_tokens, int w_rows, int outputs, int width, int dtype);
+int st_moe_router_align(int* ids, float* weights, int* sorted, int* place_of_pair, int* tile_expert, const void* x, const void* w,
+                        const float* bias, int width, int w_rows, const int* token_item, const float* correction, float scale,
+                        int num_tokens, int outputs, int experts, int top, int mode, int groups, int keep, int capacity, int tile,
+                        hipStream_t stream);
 int st_moe_align(int* sorted, int* place_of_pair, int* tile_expert, const int* ids, int num_pairs,
                  int experts, int capacity, int tile, hipStream_t stream);
 // st_moe_route and st_moe_align by one workgroup, for up to 64 tokens of 16 router outputs, 32 of 32 or 16 of 64; `experts` of the

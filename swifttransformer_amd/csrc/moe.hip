@@ -302,6 +302,88 @@ __global__ __launch_bounds__(1024) void moe_route_align_kernel(
     moe_align(sorted, place_of_pair, tile_expert, s_ids, num_tokens * r.top, real, capacity, tile, s_count, s_offset);
 }
 
+// The same behind the router's own product, for the fewest rows: one workgroup forms the logits (each wave a share of the depth, its
+// operands straight from memory in the matrix instruction's layout, all on their way at once; the shares meet in LDS), routes and sorts.
+// What bounds it: trips to memory, the operands' and then the routing's own chain; a product kernel of its own adds another launch and a
+// trip for its logits.  One row of 768, 16 outputs: with the product apart 2.7 and 4.5 us, so 6.2; a step of fiterax-125m 1.1 % shorter.  RB x CB blocks of 16 rows and 16 outputs.
+template <int RB, int CB, int G>
+__global__ __launch_bounds__(1024) void moe_router_align_kernel(
+    int* __restrict__ ids, float* __restrict__ weights, int* __restrict__ sorted, int* __restrict__ place_of_pair,
+    int* __restrict__ tile_expert, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias, int num_tokens,
+    int width, int w_rows, RouteRule r, int real, int capacity, int tile) {
+    constexpr int D = Frag<bf16_t>::kDepth, WAVES = 16, U = 4;
+    __shared__ __attribute__((aligned(16))) float part[WAVES * RB * CB * 256];
+    __shared__ float z[RB * 16 * CB * 16];
+    __shared__ int s_ids[kFusedPairs], s_count[64], s_offset[65];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, r16 = lane & 15;
+    const bf16_t *xr[RB], *wr[CB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) xr[i] = x + (int64_t)min(i * 16 + r16, num_tokens - 1) * width;
+#pragma unroll
+    for (int i = 0; i < CB; ++i) wr[i] = w + (int64_t)min(i * 16 + r16, w_rows - 1) * width;
+    floatx4 acc[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int steps = (width + D - 1) / D, share = (steps + WAVES - 1) / WAVES;
+    int k = wave * share * D;
+    const int end = min(width, k + share * D);
+    auto multiply = [&](const Frag<bf16_t>* a, const Frag<bf16_t>* b) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j) acc[i][j] = Frag<bf16_t>::mma(a[i], b[j], acc[i][j]);
+    };
+    for (; k + U * D <= end; k += U * D) {
+        Frag<bf16_t> a[U][RB], b[U][CB];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int j = 0; j < CB; ++j) b[u][j].load_whole(wr[j] + k + u * D + 8 * g);
+#pragma unroll
+            for (int i = 0; i < RB; ++i) a[u][i].load_whole(xr[i] + k + u * D + 8 * g);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) multiply(a[u], b[u]);
+    }
+    for (; k < end; k += D) {
+        Frag<bf16_t> a[RB], b[CB];
+#pragma unroll
+        for (int j = 0; j < CB; ++j) b[j].load(wr[j], k + 8 * g, width, true, true);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) a[i].load(xr[i], k + 8 * g, width, true, true);
+        multiply(a, b);
+    }
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) *reinterpret_cast<floatx4*>(part + ((wave * RB + i) * CB + j) * 256 + lane * 4) = acc[i][j];
+    __syncthreads();
+    if (tid < RB * CB * 256) {
+        const int block = tid >> 8, row = (tid >> 4) & 15, f = tid & 15, n = block % CB * 16 + f;
+        const int from = block * 256 + ((row >> 2) * 16 + f) * 4 + (row & 3);
+        float sum = 0.f;
+#pragma unroll
+        for (int q = 0; q < WAVES; ++q) sum += part[q * RB * CB * 256 + from];
+        if (bias && n < r.experts) sum += bias[n];
+        z[(block / CB * 16 + row) * (CB * 16) + n] = sum;
+    }
+    __syncthreads();
+    const int e = tid & (G - 1), t = tid / G, tc = min(t, num_tokens - 1);
+    int id;
+    float weight;
+    route_token<G>(id, weight, z + tc * (CB * 16), r);
+    if (t < num_tokens && e < r.top) {
+        const bool none = r.token_item && r.token_item[t] < 0;
+        s_ids[t * r.top + e] = none ? -1 : id;
+        ids[t * r.top + e] = none ? -1 : id;
+        weights[t * r.top + e] = none ? 0.f : weight;
+    }
+    moe_align(sorted, place_of_pair, tile_expert, s_ids, num_tokens * r.top, real, capacity, tile, s_count, s_offset);
+}
+
 // ---- few rows an expert: tiles of 16 places, where only the weights' stream counts.  A workgroup takes 16 features; its
 // four waves share the depth, so that a wave's part is one or a few batches of loads that are all on their way at once and
 // that the waves' rows, which lie a whole row of weights apart, start at different offsets (equal offsets meet in the
@@ -991,6 +1073,45 @@ extern "C" int st_moe_route_align(int* ids, float* weights, int* sorted, int* pl
     else if (outputs <= 32) launch(Steps<32>());
     else launch(Steps<64>());
     ST_LAUNCH_CHECK("moe_route_align");
+    return 0;
+}
+
+// Whether st_moe_router_align takes the product too: up to 32 rows of 16 outputs or 16 of 32, and operands that one workgroup brings in
+// little more than a trip to memory (8 rows of 2,048 and 16 outputs, 96 KB: 11.8 us apart, 10.0 so; beyond, product and routing by kernels of
+// their own are as fast or faster).
+constexpr int64_t kRouterAlignBytes = 128 * 1024;
+extern "C" int st_moe_router_align_offered(int num_tokens, int w_rows, int outputs, int width, int dtype) {
+    return dtype == kBF16 && num_tokens >= 1 && outputs >= 1 && w_rows >= outputs && width >= 8 && width % 8 == 0 &&
+           ((num_tokens <= 32 && outputs <= 16) || (num_tokens <= 16 && outputs <= 32)) &&
+           ((int64_t)num_tokens + w_rows) * width * 2 <= kRouterAlignBytes ? 1 : 0;
+}
+
+// st_moe_route_align of the logits x [num_tokens, width] . w [w_rows, width]^T (+ bias), in bfloat16.
+extern "C" int st_moe_router_align(int* ids, float* weights, int* sorted, int* place_of_pair, int* tile_expert, const void* x, const void* w,
+                                   const float* bias, int width, int w_rows, const int* token_item, const float* correction, float scale,
+                                   int num_tokens, int outputs, int experts, int top, int mode, int groups, int keep, int capacity, int tile,
+                                   hipStream_t stream) {
+    if (mode != 2) groups = keep = 1;
+    static const float some = 0.f;                 // (check_route asks for logits)
+    if (const int rc = check_route(&some, outputs, correction, num_tokens, outputs, top, mode, groups, keep)) return rc;
+    ST_CHECK(st_moe_router_align_offered(num_tokens, w_rows, outputs, width, kBF16), "moe_router_align: not for %d rows of %d and %d outputs",
+             num_tokens, width, outputs);
+    ST_CHECK(experts >= 1 && experts <= outputs, "moe_router_align: %d experts of %d outputs", experts, outputs);
+    ST_CHECK(tile == 16 || tile == 64 || tile == 128, "moe_align: tiles of 16, 64 or 128 places, not %d", tile);
+    const int num_pairs = num_tokens * top;
+    ST_CHECK(capacity % tile == 0 && capacity >= (num_pairs + tile - 1) / tile * tile + tile * experts,
+             "moe_align: %d places do not hold %d pairs of %d experts in tiles of %d", capacity, num_pairs, experts, tile);
+    ST_CHECK(ids && weights && sorted && place_of_pair && tile_expert && x && w, "moe_router_align: null operand");
+    ST_CHECK((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "moe_router_align: rows are 16-byte aligned");
+    const RouteRule r{token_item, correction, scale, outputs, top, mode, groups, keep};
+#define ST_RA(RB, CB, G)                                                                                              \
+    moe_router_align_kernel<RB, CB, G><<<1, 1024, 0, stream>>>(ids, weights, sorted, place_of_pair, tile_expert, (const bf16_t*)x,   \
+        (const bf16_t*)w, bias, num_tokens, width, w_rows, r, experts, capacity, tile)
+    if (outputs > 16) ST_RA(1, 2, 32);
+    else if (num_tokens > 16) ST_RA(2, 1, 16);
+    else ST_RA(1, 1, 16);
+#undef ST_RA
+    ST_LAUNCH_CHECK("moe_router_align");
     return 0;
 }
 

@@ -5,7 +5,7 @@ from __future__ import annotations
 
 import ctypes
 import os
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -103,6 +103,8 @@ def _lib():
                                         _c_int, _c_int, _c_f, _c_int, _c_p, _c_f, _c_int, _c_p]
         lib.st_moe_route_align.argtypes = [_c_p] * 6 + [_c_int, _c_p, _c_p, _c_f] + [_c_int] * 9 + [_c_p]
         lib.st_moe_route.argtypes = [_c_p, _c_p, _c_p, _c_int, _c_p, _c_p, _c_f, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_p]
+        lib.st_moe_router_align_offered.argtypes = [_c_int] * 5
+        lib.st_moe_router_align.argtypes = [_c_p] * 8 + [_c_int, _c_int, _c_p, _c_p, _c_f] + [_c_int] * 9 + [_c_p]
         lib.st_moe_align.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_p]
         lib.st_moe_up.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                   _c_f, _c_int, _c_int, _c_p]
@@ -1396,6 +1398,12 @@ def moe_routes_at_once(num_tokens: int, outputs: int) -> bool:
     return outputs <= 64 and num_tokens * (16 if outputs <= 16 else 32 if outputs <= 32 else 64) <= 1024
 
 
+def moe_routes_by_matrix(x: torch.Tensor, w_router: torch.Tensor, outputs: int) -> bool:
+    """Whether ``routed_experts`` takes the router's matrix itself for these rows: few bfloat16 rows and few outputs."""
+    return (x.data_ptr() % 16 == 0 and w_router.data_ptr() % 16 == 0 and
+            bool(_lib().st_moe_router_align_offered(x.shape[0], w_router.shape[0], int(outputs), x.shape[1], dtype_code(x.dtype))))
+
+
 def moe_capacity(num_tokens: int, top: int, experts: int, tile: int) -> int:
     """Places of the sorted pair list: every expert's pairs start a tile of their own."""
     return -(-num_tokens * top // tile) * tile + tile * experts
@@ -1416,7 +1424,7 @@ def routed_experts(x: torch.Tensor, logits: torch.Tensor, w_gate: Optional[torch
                    out_scale: float = 1.0, token_item: Optional[torch.Tensor] = None,
                    style: str = "scaled_input", groups: int = 1, keep: int = 1,
                    correction: Optional[torch.Tensor] = None, scale: float = 1.0, identity: int = 0,
-                   clamped: bool = False) -> torch.Tensor:
+                   clamped: bool = False, router: Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]] = None) -> torch.Tensor:
     """residual <- residual + out_scale * sum over a row's ``top`` best experts e (by ``logits``) of
     Wd[e] y with y = g * sigmoid(1.702 g) * (u + 1), g = min(s * Wg[e] x, limit),
     u = clamp(s * Wu[e] x, -limit, limit), s = sigmoid(logit of e).  In place on ``residual``
@@ -1439,15 +1447,25 @@ def routed_experts(x: torch.Tensor, logits: torch.Tensor, w_gate: Optional[torch
 
     ``w_gate`` None (not in the first style): experts without a gate, Wd[e] gelu(Wu[e] x), the exact GELU.
 
+    ``router`` (matrix [rows, width], bias or None; ``logits`` None, where ``moe_routes_by_matrix``): the logits are the product of x
+    with the matrix's first rows, formed by the kernel that routes.
+
     x: [T, width]; logits: float [T, experts + identity] (rows may be longer and of any stride); w_gate, w_up: [experts, inner, width]; w_down:
     [experts, width, inner].  Rows whose ``token_item`` is negative are left as they are."""
     T, W = x.shape
     E, F, _ = w_up.shape
     _need(x, "x", w_up.dtype, (T, W))
     outputs = E + int(identity)
-    _need(logits, "logits", torch.float32, (T, logits.shape[1]), contiguous=False)
-    if logits.shape[1] < outputs or logits.stride(1) != 1:
-        raise KernelError(f"logits: dense rows of {outputs}")
+    if (router is None) == (logits is None):
+        raise KernelError("routed_experts: logits or the router's matrix")
+    if router is not None:
+        _need(router[0], "router", x.dtype, (router[0].shape[0], W))
+        if router[1] is not None:
+            _need(router[1], "router bias", torch.float32, (router[0].shape[0],))
+    else:
+        _need(logits, "logits", torch.float32, (T, logits.shape[1]), contiguous=False)
+        if logits.shape[1] < outputs or logits.stride(1) != 1:
+            raise KernelError(f"logits: dense rows of {outputs}")
     if w_gate is not None:
         _need(w_gate, "w_gate", w_up.dtype, (E, F, W))
     _need(w_up, "w_up", None, (E, F, W))
@@ -1481,13 +1499,18 @@ def routed_experts(x: torch.Tensor, logits: torch.Tensor, w_gate: Optional[torch
     place = empty((T * top,), torch.int32, dev)
     tile_expert = empty((cap // tile,), torch.int32, dev)
     y = empty((cap, F), x.dtype, dev)
-    stride = logits.stride(0) if T > 1 else logits.shape[1]
     corr = _ptr(correction) if mode >= 3 else None
-    if moe_routes_at_once(T, outputs):
+    if router is not None:
+        _check(lib.st_moe_router_align(_ptr(ids), _ptr(wts), _ptr(sorted_pairs), _ptr(place), _ptr(tile_expert), _ptr(x), _ptr(router[0]),
+                                       _ptr(router[1]), W, router[0].shape[0], _ptr(token_item), corr, float(scale), T, outputs, E, int(top),
+                                       mode, int(groups), int(keep), cap, tile, st))
+    elif moe_routes_at_once(T, outputs):
+        stride = logits.stride(0) if T > 1 else logits.shape[1]
         _check(lib.st_moe_route_align(_ptr(ids), _ptr(wts), _ptr(sorted_pairs), _ptr(place), _ptr(tile_expert), _ptr(logits), stride,
                                       _ptr(token_item), corr, float(scale), T, outputs, E, int(top), mode, int(groups), int(keep), cap,
                                       tile, st))
     else:
+        stride = logits.stride(0) if T > 1 else logits.shape[1]
         _check(lib.st_moe_route(_ptr(ids), _ptr(wts), _ptr(logits), stride, _ptr(token_item), corr, float(scale), T, outputs, int(top),
                                 mode, int(groups), int(keep), st))
         _check(lib.st_moe_align(_ptr(sorted_pairs), _ptr(place), _ptr(tile_expert), _ptr(ids), T * top, E, cap, tile, st))

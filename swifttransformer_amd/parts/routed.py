@@ -116,8 +116,10 @@ class RoutedExperts(Part):
         self.correction = tensors[self.name("correction")].contiguous() if self.corrected else None
 
     def forward(self, x_t: torch.Tensor, residual32: torch.Tensor, ctx) -> torch.Tensor:
-        logits = K.gemm(x_t, self.w_router, bias=self.b_router, out_f32=True)
+        by_matrix = K.moe_routes_by_matrix(x_t, self.w_router, self.outputs)
+        logits = None if by_matrix else K.gemm(x_t, self.w_router, bias=self.b_router, out_f32=True)
         return K.routed_experts(x_t, logits, self.w_gate, self.w_up, self.w_down, residual32, top=self.top,
                                 limit=self.limit, out_scale=self.residual_scale, token_item=ctx.token_item,
                                 style=self.style, groups=self.groups, keep=self.keep, correction=self.correction, scale=self.scale,
-                                identity=self.identity, clamped=self.clamped)
+                                identity=self.identity, clamped=self.clamped,
+                                router=(self.w_router, self.b_router) if by_matrix else None)

@@ -93,3 +93,52 @@ def test_no_token_leaves_no_tile():
     K._check(lib.st_moe_route_align(P(ids), P(wts), P(order), P(place), P(owner), P(logits), E, None, None, 1.0, 0, E, E, 2, 1, 1, 1, cap, tile,
                                     K._stream()))
     assert bool((order == -1).all()) and bool((owner == -1).all())
+
+
+@pytest.mark.parametrize("T,W,E,identity,top,mode,groups,keep,biased", [
+    (1, 768, 16, 0, 2, 3, 1, 1, False), (16, 8, 5, 0, 2, 1, 1, 1, True), (17, 1024, 16, 0, 2, 2, 4, 2, False), (32, 1000, 14, 2, 2, 4, 1, 1, False),
+    (16, 1096, 32, 0, 3, 0, 1, 1, True), (3, 40, 17, 0, 4, 1, 1, 1, False), (8, 2048, 16, 0, 2, 2, 4, 2, False)])
+def test_the_routers_product_and_its_routes_in_one_kernel(T, W, E, identity, top, mode, groups, keep, biased):
+    """Whole numbers, whose products and sums are exact: the same choices, weights and places per expert as from the logits themselves."""
+    from swifttransformer_amd.ops import kernels as K
+    lib, ptr = K._lib(), K._ptr
+    g = torch.Generator().manual_seed(T + W)
+    out = E + identity
+    rows = -(-out // 8) * 8
+    x = torch.randint(-2, 3, (T, W), generator=g).float() * (torch.rand(T, W, generator=g) < 8 / W)        # (logits of some units)
+    w = torch.randint(-3, 4, (rows, W), generator=g).float()
+    bias = torch.randint(-2, 3, (rows,), generator=g).float() / 4 if biased else None
+    z = x @ w.T + (bias if biased else 0)
+    correction = torch.randn(out, generator=g) * 0.2
+    item = torch.zeros(T, dtype=torch.int32)
+    if T > 4:
+        item[T - 2] = -1
+    cap = K.moe_capacity(T, top, E, 16)
+    dev = lambda t, d: t.to("cuda").to(d)
+    xd, wd, zd, cd, it = dev(x, torch.bfloat16), dev(w, torch.bfloat16), dev(z, torch.float32), dev(correction, torch.float32), item.to("cuda")
+    bd = dev(bias, torch.float32) if biased else None
+    assert K.moe_routes_by_matrix(xd, wd, out)
+
+    def run(by_matrix):
+        i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+        ids, srt, place, texp, wts = i32(T * top), i32(cap), i32(T * top), i32(cap // 16), torch.full((T * top,), -7.0, device="cuda")
+        tail = (T, out, E, top, mode, groups, keep, cap, 16, K._stream())
+        if by_matrix:
+            K._check(lib.st_moe_router_align(ptr(ids), ptr(wts), ptr(srt), ptr(place), ptr(texp), ptr(xd), ptr(wd), ptr(bd), W, rows, ptr(it), ptr(cd),
+                                             1.5, *tail))
+        else:
+            K._check(lib.st_moe_route_align(ptr(ids), ptr(wts), ptr(srt), ptr(place), ptr(texp), ptr(zd), rows, ptr(it), ptr(cd), 1.5, *tail))
+        return [t.cpu() for t in (ids, wts, texp, srt, place)]
+    (ids, wts, texp, srt, place), (ids0, wts0, texp0, srt0, _p) = run(True), run(False)
+    assert torch.equal(ids, ids0) and torch.equal(wts, wts0) and torch.equal(texp, texp0)
+    assert torch.equal(srt.view(-1, 16).sort(1).values, srt0.view(-1, 16).sort(1).values)       # (places within a tile are in any order)
+    real = (ids >= 0) & (ids < E)
+    assert torch.equal(srt[place[real].long()], torch.arange(T * top, dtype=torch.int32)[real]) and bool((place[~real] == -1).all())
+
+
+def test_larger_routers_keep_kernels_of_their_own():
+    from swifttransformer_amd.ops import kernels as K
+    offered = lambda T, W, out, dt=torch.bfloat16: K.moe_routes_by_matrix(torch.empty(T, W, dtype=dt, device="cuda"),
+                                                                          torch.empty(-(-out // 8) * 8, W, dtype=dt, device="cuda"), out)
+    assert offered(16, 2048, 16) and not offered(17, 2048, 16) and not offered(33, 64, 16) and not offered(17, 64, 17)
+    assert not offered(1, 64, 33) and not offered(1, 60, 16) and not offered(1, 64, 16, torch.float32) and not offered(0, 64, 16)
