@@ -73,3 +73,28 @@ def test_split_attention_merged_by_lanes(dtype, heads, hd, splits, gated):
     # float sums of up to 90 weights in another order, then one rounding to the storage type (2^-9 of a value up to twice)
     tol = 1e-5 if dt == torch.float32 else 2.0 ** -8
     assert bool(((one.float() - many.float()).abs() <= tol * one.float().abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("heads,kv_heads,hd", [(1, 1, 16), (32, 8, 64), (33, 3, 64), (12, 12, 80), (32, 32, 128), (16, 17, 64)])
+def test_normed_queries_and_keys_in_pieces(dtype, heads, kv_heads, hd):
+    """Rows in registers (up to 4,096 numbers) beside the same rows past a 16-byte boundary, which go a number at a time, with padding rows."""
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(heads + hd)
+    dt, ps, T = DTYPES[dtype], 16, 5
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    qk, gq, gk = rnd(T, (heads + kv_heads) * hd), rnd(heads * hd), rnd(kv_heads * hd)
+    item = torch.tensor([0, 1, -1, 0, 1], dtype=torch.int32, device=DEV)
+    pos = torch.tensor([0, 17, 3, 1, -1], dtype=torch.int32, device=DEV)
+    bt = torch.tensor([[2, 0], [1, 3]], dtype=torch.int32, device=DEV)
+    res = []
+    for shift in (False, True):
+        k, v = torch.full((4, kv_heads, ps, hd), 7.0, dtype=dt, device=DEV), torch.full((4, kv_heads, ps, hd), 7.0, dtype=dt, device=DEV)
+        f = _shifted if shift else (lambda t: t)
+        q = K.qk_norm_write(qk, f(gq), f(gk), 1e-5, heads, kv_heads, hd, k, v, item, pos, bt, write=True)
+        res.append((q.clone(), k, v))
+    # two float sums of up to 4,096 squares in different orders, then one rounding (to either side of a half at most)
+    tol = 2e-6 if dt == torch.float32 else 2.0 ** -7
+    for a, b in zip(*res):
+        assert bool(((a.float() - b.float()).abs() <= tol * b.float().abs()).all())
+    assert torch.equal(res[0][2], res[1][2])
