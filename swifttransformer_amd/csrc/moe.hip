@@ -453,11 +453,11 @@ __global__ __launch_bounds__(256) void moe_up_few_kernel(
     int top, int width, int inner, float limit, int style, int vec) {
     constexpr int MATS = GATED ? 2 : 1;
     __shared__ __attribute__((aligned(16))) float lds[4 * MATS * 256];
-    const int tile = blockIdx.x, e = tile_expert[tile];
+    // (the tile's pairs are asked for beside its expert: one trip to memory before the weights', not two)
+    const int tile = blockIdx.x, r16 = threadIdx.x & 15, f0 = blockIdx.y * 16, base = tile * kRows;
+    const int e = tile_expert[tile], pair = sorted[base + r16], p = sorted[base + (threadIdx.x >> 4)];
     if (e < 0) return;
-    const int r16 = threadIdx.x & 15, f0 = blockIdx.y * 16, base = tile * kRows;
     const int64_t feature = (int64_t)e * inner + min(f0 + r16, inner - 1);
-    const int pair = sorted[base + r16];
     const T* wr[MATS];
     wr[0] = w_up + feature * width;
     if (GATED) wr[MATS - 1] = w_gate + feature * width;
@@ -469,7 +469,6 @@ __global__ __launch_bounds__(256) void moe_up_few_kernel(
     moe_sum_shares<MATS>(sum, acc, lds);
     const int place = base + (threadIdx.x >> 4), f = f0 + r16;
     if (f >= inner) return;
-    const int p = sorted[place];
     float out = 0.f;
     if (p >= 0 && !GATED) {
         out = apply_activation(kActGeluErf, sum[0]);
@@ -492,16 +491,15 @@ __global__ __launch_bounds__(256) void moe_down_few_kernel(
     const int* __restrict__ sorted, const int* __restrict__ tile_expert, int top, int width, int inner, float out_scale,
     int vec) {
     __shared__ __attribute__((aligned(16))) float lds[4 * 256];
-    const int tile = blockIdx.x, e = tile_expert[tile];
+    const int tile = blockIdx.x, r16 = threadIdx.x & 15, n0 = blockIdx.y * 16, base = tile * kRows;
+    const int e = tile_expert[tile], p = sorted[base + (threadIdx.x >> 4)];
     if (e < 0) return;
-    const int r16 = threadIdx.x & 15, n0 = blockIdx.y * 16, base = tile * kRows;
     const T* wr[1] = {w_down + ((int64_t)e * width + min(n0 + r16, width - 1)) * inner};
     floatx4 acc[1] = {floatx4{0.f, 0.f, 0.f, 0.f}};
     moe_depth_share<T, 1>(acc, y + (int64_t)(base + r16) * inner, wr, inner, vec);
     float sum[1];
     moe_sum_shares<1>(sum, acc, lds);
     const int place = base + (threadIdx.x >> 4), n = n0 + r16;
-    const int p = sorted[place];
     if (n >= width || p < 0) return;
     if (pair_out) {
         pair_out[(int64_t)place * width + n] = sum[0];
