@@ -30,42 +30,42 @@ __global__ __launch_bounds__(256) void dynamic_tanh_kernel(
     const float* __restrict__ base, const float* __restrict__ w2, const float* __restrict__ b2,
     const float* __restrict__ alpha2, int width) {
     const int64_t r = blockIdx.x;
-    const int c = (blockIdx.y * 256 + threadIdx.x) * V;
-    if (c >= width) return;
     int64_t src = r;
     if (rows) {
         src = rows[r];
         if (src < 0) return;                              // a padding entry
     }
-    const int64_t idx = r * width + c;
     auto load = [](const float* p, float* v) {
         if (V == 4) Elem<float>::load_vec(p, v);
         else v[0] = p[0];
     };
-    float y[V], g[V], s[V], g2[V], s2[V], on[V];
-    load(x + src * width + c, y);
-    load(w + c, g);
-    if (b) load(b + c, s);
-    if (base) load(base + idx, on);
-    if (w2) load(w2 + c, g2);
-    if (b2) load(b2 + c, s2);
-    const float a = alpha[0], a2 = w2 ? alpha2[0] : 0.f;
+    for (int64_t c = ((int64_t)blockIdx.y * 256 + threadIdx.x) * V; c < width; c += (int64_t)gridDim.y * 256 * V) {
+        const int64_t idx = r * width + c;
+        float y[V], g[V], s[V], g2[V], s2[V], on[V];
+        load(x + src * width + c, y);
+        load(w + c, g);
+        if (b) load(b + c, s);
+        if (base) load(base + idx, on);
+        if (w2) load(w2 + c, g2);
+        if (b2) load(b2 + c, s2);
+        const float a = alpha[0], a2 = w2 ? alpha2[0] : 0.f;
 #pragma unroll
-    for (int u = 0; u < V; ++u) {
-        y[u] = tanhf(a * y[u]) * g[u] + (b ? s[u] : 0.f);
-        if (base) y[u] += on[u];
-    }
-    if (out32) {
-        if (V == 4) Elem<float>::store_vec(out32 + idx, y);
-        else out32[idx] = y[0];
-    }
-    if (w2) {                                             // the next norm, of the sum just made
+        for (int u = 0; u < V; ++u) {
+            y[u] = tanhf(a * y[u]) * g[u] + (b ? s[u] : 0.f);
+            if (base) y[u] += on[u];
+        }
+        if (out32) {
+            if (V == 4) Elem<float>::store_vec(out32 + idx, y);
+            else out32[idx] = y[0];
+        }
+        if (w2) {                                             // the next norm, of the sum just made
 #pragma unroll
-        for (int u = 0; u < V; ++u) y[u] = tanhf(a2 * y[u]) * g2[u] + (b2 ? s2[u] : 0.f);
-    }
-    if (out_t) {
-        if (V == 4) Elem<T>::store4(out_t + idx, y);
-        else Elem<T>::store(out_t + idx, y[0]);
+            for (int u = 0; u < V; ++u) y[u] = tanhf(a2 * y[u]) * g2[u] + (b2 ? s2[u] : 0.f);
+        }
+        if (out_t) {
+            if (V == 4) Elem<T>::store4(out_t + idx, y);
+            else Elem<T>::store(out_t + idx, y[0]);
+        }
     }
 }
 
@@ -187,8 +187,7 @@ extern "C" int st_dynamic_tanh(void* out_t, float* out32, const float* x, const 
     const bool four = width % 4 == 0 && (align & 15) == 0 && (uintptr_t)out_t % (dtype == kF32 ? 16 : 8) == 0;
     const int span = four ? 1024 : 256;
     const int64_t blocks = ((int64_t)width + span - 1) / span;
-    ST_CHECK(blocks <= 65535, "dynamic_tanh: rows of %d are too wide", width);
-    const dim3 grid((unsigned)num_rows, (unsigned)blocks);
+    const dim3 grid((unsigned)num_rows, (unsigned)(blocks < 65535 ? blocks : 65535));
 #define ST_DT(T, V)                                                                                             \
     dynamic_tanh_kernel<T, V><<<grid, 256, 0, stream>>>((T*)out_t, out32, x, rows, w, b, alpha, base, w2, b2, alpha2, width)
     if (dtype == kF32) { if (four) ST_DT(float, 4); else ST_DT(float, 1); }
