@@ -164,9 +164,9 @@ class LMHead(Part):
                 and K.wide_offered(rows, self.vocab_size, self.embed_dim, self.dtype))
 
     def offers_best(self, rows: int) -> bool:
-        """Whether ``forward`` of that many normalised rows reports the rows' best outputs.  (Not through a limit: it may make two
-        different outputs equal, and the best is then the lower index.)"""
-        return (self.logit_scale > 0 and self.softcap == 0 and not self.projected
+        """Whether ``forward`` of that many normalised rows reports the rows' best outputs.  (Not through a factor or a limit: they may
+        make two different outputs equal, and the best is then the lower index.)"""
+        return (self.logit_scale == 1.0 and self.softcap == 0 and not self.projected
                 and K.wide_offered(rows, self.vocab_size, self.embed_dim, self.dtype))
 
     def forward(self, y_t, best: Optional[torch.Tensor] = None) -> torch.Tensor:
