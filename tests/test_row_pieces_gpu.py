@@ -98,3 +98,21 @@ def test_normed_queries_and_keys_in_pieces(dtype, heads, kv_heads, hd):
     for a, b in zip(*res):
         assert bool(((a.float() - b.float()).abs() <= tol * b.float().abs()).all())
     assert torch.equal(res[0][2], res[1][2])
+
+
+@pytest.mark.parametrize("streams", [1, 4, 5])
+@pytest.mark.parametrize("rows,width", [(1, 4), (3, 1028), (2, 2048), (2, 8196), (300, 516)])
+def test_streams_written_by_as_many_threads_as_columns(streams, rows, width):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(width + streams)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, y, mix, b, a2, gain = rnd(rows, streams, width), rnd(rows, width), rnd(streams, streams), rnd(streams), rnd(streams), rnd(width)
+    new = torch.einsum("rsw,st->rtw", x.double(), mix.double()) + b.double()[None, :, None] * y.double()[:, None]
+    size = torch.einsum("rsw,st->rtw", x.double().abs(), mix.double().abs()) + (b.double()[None, :, None] * y.double()[:, None]).abs()
+    u, u_size = torch.einsum("rtw,t->rw", new, a2.double()), torch.einsum("rtw,t->rw", size, a2.double().abs())
+    norm = torch.sqrt(u.square().mean(1, keepdim=True) + 1e-5)
+    got = x.clone().view(rows, streams * width)
+    out = K.streams_write(got, y, mix, b, then=(a2, gain, 1e-5), out_dtype=torch.float32)
+    # chains of a few float operations a number; the norm's sum of squares adds its own few roundings, relative
+    assert bool(((got.view_as(x).double() - new).abs() <= 1e-6 * size + 1e-30).all())
+    assert bool(((out.double() - u / norm * gain.double()).abs() <= (2e-6 * u_size + 2e-5 * u.abs()) / norm * gain.double().abs() + 1e-30).all())
