@@ -326,6 +326,7 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(
     for (int s = 64 + lane; s < num_splits; s += 64) M = fmaxf(M, lse[s]);
     M = wave_max(M);
     const float weight = own > -INFINITY ? expf(own - M) : 0.f;
+    const uint64_t held = __ballot(own > -INFINITY);           // the splits that hold a key
     for (int d0 = 0; d0 < head_dim; d0 += 64) {
         const int d = min(d0 + lane, head_dim - 1);
         float W = 0.f, o = 0.f;
@@ -338,14 +339,21 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(
             for (int u = 0; u < U; ++u) {
                 if (s0 + u >= num_splits) break;
                 float w;
+                bool holds;
                 if (few) {
                     w = __shfl(weight, s0 + u, 64);
+                    holds = (held >> (s0 + u)) & 1;
                 } else {
                     const float ls = lse[s0 + u];
-                    w = ls > -INFINITY ? expf(ls - M) : 0.f;
+                    holds = ls > -INFINITY;
+                    w = holds ? expf(ls - M) : 0.f;
                 }
-                W += w;
-                if (w > 0.f) o += w * v[u];          // (no weight: nothing to add, whatever lies there)
+                // (an empty split adds nothing, whatever lies there; one with keys adds its result also where its weight is down to
+                // zero: a NaN or an infinity among the values of visible keys reaches the result, as it does without splits)
+                if (holds) {
+                    W += w;
+                    o += w * v[u];
+                }
             }
         }
         if (d0 + lane < head_dim) Elem<T>::store(out + orow * head_dim + d, W > 0.f ? o / W * gate : 0.f);

@@ -76,6 +76,26 @@ def test_split_attention_merged_by_lanes(dtype, heads, hd, splits, gated):
 
 
 @pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("splits", [1, 4, 64, 70])
+def test_a_value_that_is_no_number_reaches_the_result_of_every_split(dtype, splits):
+    """A visible key whose weight is down to zero beside another split's, with a NaN or an infinity in its value (zero times either is NaN):
+    the result shows it however many splits the keys are shared out over, and splits without a key show nothing."""
+    from swifttransformer_amd.ops import kernels as K
+    dt, ps, hd, n = DTYPES[dtype], 16, 64, 80
+    q = torch.zeros(1, hd, device=DEV, dtype=dt)
+    q[0, 0] = 1.0
+    kc, vc = torch.zeros(6, 1, ps, hd, device=DEV, dtype=dt), torch.ones(6, 1, ps, hd, device=DEV, dtype=dt)
+    kc[4, 0, 15, 0] = 4000.0                                   # the last key has all of the weight
+    vc[0, 0, 3, 5], vc[1, 0, 7, 9] = float("nan"), float("inf")
+    kc[5], vc[5] = float("nan"), float("nan")                  # nobody's page
+    bt = torch.arange(6, device=DEV, dtype=torch.int32).view(1, 6)
+    item, pos = torch.zeros(1, dtype=torch.int32, device=DEV), torch.full((1,), n - 1, dtype=torch.int32, device=DEV)
+    out = K.attention_rows(q, kc, vc, item, pos, bt, 1, 1.0, num_splits=splits)[0]
+    bad = torch.isnan(out).nonzero().flatten().tolist()
+    assert bad == [5, 9] and bool((out[~torch.isnan(out)] == 1.0).all())
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
 @pytest.mark.parametrize("heads,kv_heads,hd", [(1, 1, 16), (32, 8, 64), (33, 3, 64), (12, 12, 80), (32, 32, 128), (16, 17, 64)])
 def test_normed_queries_and_keys_in_pieces(dtype, heads, kv_heads, hd):
     """Rows in registers (up to 4,096 numbers) beside the same rows past a 16-byte boundary, which go a number at a time, with padding rows."""
