@@ -383,7 +383,7 @@ int st_latent_tiles_fit(int heads, int entry, int page_size, int max_pages, int 
 int st_latent_tiles(void* out, const void* q, int64_t q_stride, const void* cache, int64_t page_stride, const int* tile_item,
                     const int* tile_q0, int num_tiles, const int* item_tok_off, const int* item_start, const int* item_len,
                     const int* block_table, const float* sink, const float* freq, int max_pages, int page_size, int heads,
-                    int entry, int out_dim, int rot_off, int rot_half, float rot_mult, float scale, int window, int dtype,
+                    int entry, int out_dim, int rot_off, int rot_half, float rot_mult, float scale, int window, int float_sum, int dtype,
                     hipStream_t stream);
 int st_latent_rows(float* part_o, float* part_lse, const void* q, int64_t q_stride, const void* cache, int64_t page_stride,
                    const int* row_ids, const int* token_item, const int* positions, int num_rows, int num_splits,

@@ -136,8 +136,11 @@ __device__ inline float lo_half(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ inline float hi_half(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
 
 // HDP: 32-wide steps over the entry; QT: subtiles of 16 rows a wave; NKT: 16-key subtiles of a block; RW: waves over the
-// rows; KW: groups of RW waves, each with its own share of the key blocks and its own LDS, merged at the end.
-template <bool TILES, int HDP, int QT, int NKT, int RW, int KW>
+// rows; KW: groups of RW waves, each with its own share of the key blocks and its own LDS, merged at the end.  FS: the normaliser sums
+// the weights as they are (float, a lane's own keys), else as they are rounded for the product (one more row of the product).  What was
+// attention in a kernel that sums floats keeps them: entries of 160, 1,024 tokens of 32 heads 42.8 us, rounded 39.6, off float64 by 1.91e-3
+// and 1.90e-3.
+template <bool TILES, int HDP, int QT, int NKT, int RW, int KW, bool FS>
 __global__ __launch_bounds__(64 * RW * KW) void latent_attn_kernel(const LatentArgs a) {
     constexpr int CH = 4 * HDP, ROWB = CH * 16, DK = 16 * NKT, DT = 2 * HDP, ROWS = RW * QT * 16, BUF = DK * ROWB;
     constexpr int NI = DK * CH / (64 * RW);          // direct loads (1 KB each) a wave and block
@@ -239,14 +242,15 @@ __global__ __launch_bounds__(64 * RW * KW) void latent_attn_kernel(const LatentA
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) voff[dt] = vrow * ROWB + (((2 * dt + ((r16 & 3) >> 1)) ^ sw_v) << 4) + ((r16 & 1) << 3);
 
-    // running maximum (log2 units, from a finite floor), accumulators, and the normaliser as one more row of the product
+    // running maximum (log2 units, from a finite floor), accumulators, and the normaliser: as one more row of the product, or (FS) this
+    // lane's share of it in the first number
     float ms[QT];
     floatx4 acc[QT][DT], accl[QT];
     const bool with_sink = a.sink && part == 0 && (TILES || blockIdx.z == 0);
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         ms[t] = with_sink ? a.sink[qhead[t]] * kLog2e : -1.0e30f;
-        const float one = with_sink ? 1.f : 0.f;
+        const float one = with_sink && (!FS || g == 0) ? 1.f : 0.f;          // (the sink's share is one lane's)
         accl[t] = floatx4{one, one, one, one};
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) acc[t][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -312,6 +316,7 @@ __global__ __launch_bounds__(64 * RW * KW) void latent_attn_kernel(const LatentA
                 for (int dt = 0; dt < DT; ++dt) acc[t][dt] *= alpha;
                 accl[t] *= alpha;
             }
+            float psum = 0.f;
 #pragma unroll
             for (int u = 0; u < NKT / 2; ++u) {
                 uint32_t packed[4];
@@ -319,17 +324,21 @@ __global__ __launch_bounds__(64 * RW * KW) void latent_attn_kernel(const LatentA
                 for (int half = 0; half < 2; ++half) {
                     float p[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(fmaf(st[t][2 * u + half][r], sl, -mc));
+                    for (int r = 0; r < 4; ++r) {
+                        p[r] = __builtin_amdgcn_exp2f(fmaf(st[t][2 * u + half][r], sl, -mc));
+                        if (FS) psum += p[r];
+                    }
                     packed[2 * half] = pack_bf16x2(p[0], p[1]);
                     packed[2 * half + 1] = pack_bf16x2(p[2], p[3]);
                 }
                 pf[t][u] = __builtin_bit_cast(bf16x8, make_uint4(packed[0], packed[1], packed[2], packed[3]));
             }
+            if (FS) accl[t][0] += psum;
         }
 #pragma unroll
         for (int u = 0; u < NKT / 2; ++u) {
 #pragma unroll
-            for (int t = 0; t < QT; ++t) accl[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[t][u], accl[t], 0, 0, 0);
+            for (int t = 0; t < QT && !FS; ++t) accl[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pf[t][u], accl[t], 0, 0, 0);
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
                 if (16 * dt >= a.out_dim) continue;  // uniform
@@ -402,8 +411,9 @@ __global__ __launch_bounds__(64 * RW * KW) void latent_attn_kernel(const LatentA
     // acc[t][dt][r] = O[this lane's row of subtile t][dim 16 dt + 4 g + r]
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
+        const float lsum = FS ? rows4_sum(accl[t][0]) : accl[t][0];
         if (!qvalid[t]) continue;
-        const float lsum = accl[t][0], inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+        const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
         if (TILES) {
             bf16_t* orow = reinterpret_cast<bf16_t*>(a.out) + ((rows.token0 + qpos[t] - rows.pos0) * a.heads + qhead[t]) * a.out_dim;
 #pragma unroll
@@ -727,9 +737,9 @@ static size_t latent_lds(const LatentArgs& a) {
     return bufs + table > merge ? bufs + table : merge;
 }
 
-template <bool TILES, int HDP, int QT, int NKT, int RW, int KW>
+template <bool TILES, int HDP, int QT, int NKT, int RW, int KW, bool FS = false>
 static int launch_latent(const LatentArgs& a, int list, hipStream_t stream) {
-    auto kernel = latent_attn_kernel<TILES, HDP, QT, NKT, RW, KW>;
+    auto kernel = latent_attn_kernel<TILES, HDP, QT, NKT, RW, KW, FS>;
     constexpr int rows = RW * QT * 16;
     const size_t lds = latent_lds<TILES, HDP, QT, NKT, RW, KW>(a);
     if (latent_raise_lds(reinterpret_cast<const void*>(kernel), lds)) return 1;
@@ -764,7 +774,7 @@ static int launch_latent_f32(const LatentArgs& a, int list, hipStream_t stream) 
 }
 
 template <bool TILES>
-static int latent_dispatch(const LatentArgs& a, int list, int dtype, hipStream_t stream) {
+static int latent_dispatch(const LatentArgs& a, int list, bool float_sum, int dtype, hipStream_t stream) {
     if (dtype == kF32) {
         const int et = (a.entry + 15) / 16;
 #define ST_LF(E) if (et <= E) return launch_latent_f32<TILES, E>(a, list, stream)
@@ -782,6 +792,11 @@ static int latent_dispatch(const LatentArgs& a, int list, int dtype, hipStream_t
     const bool half_empty = 2ll * list * ((kTileTokens * (int64_t)a.heads + 63) / 64) < 3 * device_compute_units();
 #define ST_LT(H)                                                                                                       \
     if (hdp <= H) {                                                                                                    \
+        if constexpr (TILES && H >= 5) {                                                                               \
+            if (float_sum)                                                                                             \
+                return half_empty && latent_lds<TILES, H, 1, 4, 4, 2>(a) <= kLatentMaxLds                              \
+                           ? launch_latent<TILES, H, 1, 4, 4, 2, true>(a, list, stream) : launch_latent<TILES, H, 1, 4, 4, 1, true>(a, list, stream); \
+        }                                                                                                              \
         if constexpr (TILES)                                                                                           \
             return half_empty && latent_lds<TILES, H, 1, 4, 4, 2>(a) <= kLatentMaxLds                                  \
                        ? launch_latent<TILES, H, 1, 4, 4, 2>(a, list, stream) : launch_latent<TILES, H, 1, 4, 4, 1>(a, list, stream); \
@@ -839,20 +854,23 @@ static int latent_args(LatentArgs& a, const void* q, int64_t q_stride, const voi
 }
 
 // Tile i: tokens [tile_q0[i], + 64) of item tile_item[i] (-1: skipped).  out [tokens, heads, out_dim], the storage type.
+// float_sum: bfloat16 weights meet the entries, but the normaliser is the sum of the weights before they are rounded (entries of 129 to
+// 256 dims; float tiles always do).
 extern "C" int st_latent_tiles(void* out, const void* q, int64_t q_stride, const void* cache, int64_t page_stride,
                                const int* tile_item, const int* tile_q0, int num_tiles, const int* item_tok_off,
                                const int* item_start, const int* item_len, const int* block_table, const float* sink,
                                const float* freq, int max_pages, int page_size, int heads, int entry, int out_dim, int rot_off,
-                               int rot_half, float rot_mult, float scale, int window, int dtype, hipStream_t stream) {
+                               int rot_half, float rot_mult, float scale, int window, int float_sum, int dtype, hipStream_t stream) {
     LatentArgs a = {};
     if (latent_args(a, q, q_stride, cache, page_stride, block_table, sink, freq, max_pages, page_size, heads, entry, out_dim,
                     rot_off, rot_half, rot_mult, scale, window, dtype)) return 1;
+    ST_CHECK(!float_sum || dtype == kF32 || (entry > 128 && entry <= 256), "latent_attention: float normalisers for entries of 129 to 256 dims, not %d", entry);
     ST_CHECK(num_tiles >= 0 && num_tiles <= 65535, "latent_attention: %d tiles", num_tiles);
     if (num_tiles == 0) return 0;
     ST_CHECK(out && tile_item && tile_q0 && item_tok_off && item_start && item_len && ((uintptr_t)out & 15) == 0, "latent_attention: null operand");
     a.out = out; a.tile_item = tile_item; a.tile_q0 = tile_q0; a.item_tok_off = item_tok_off; a.item_start = item_start;
     a.item_len = item_len;
-    return latent_dispatch<true>(a, num_tiles, dtype, stream);
+    return latent_dispatch<true>(a, num_tiles, float_sum != 0, dtype, stream);
 }
 
 // List entry i: batch row row_ids[i] (null: i; -1: skipped).  part_o [list, heads, splits, out_dim], part_lse [list, heads,
@@ -870,7 +888,7 @@ extern "C" int st_latent_rows(float* part_o, float* part_lse, const void* q, int
     ST_CHECK(part_o && part_lse && token_item && positions && ((uintptr_t)part_o & 15) == 0, "latent_attention: null operand");
     a.part_o = part_o; a.part_lse = part_lse; a.row_ids = row_ids; a.token_item = token_item; a.positions = positions;
     a.num_splits = num_splits;
-    return latent_dispatch<false>(a, num_rows, dtype, stream);
+    return latent_dispatch<false>(a, num_rows, false, dtype, stream);
 }
 
 extern "C" int st_latent_merge(void* out, const float* part_o, const float* part_lse, const int* row_ids, int num_rows, int heads,

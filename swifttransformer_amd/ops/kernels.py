@@ -118,7 +118,7 @@ def _lib():
         lib.st_latent_tiles_fit.argtypes = [_c_int] * 5
         lib.st_latent_tiles.argtypes = [_c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_int, _c_p, _c_p, _c_p, _c_p, _c_p,
                                         _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _c_int,
-                                        _c_int, _c_p]
+                                        _c_int, _c_int, _c_p]
         lib.st_latent_rows.argtypes = [_c_p, _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_int, _c_int, _c_p, _c_p,
                                        _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_f, _c_int,
                                        _c_int, _c_p]
@@ -2045,10 +2045,12 @@ def latent_tiles_fit(heads: int, entry: int, page_size: int, max_pages: int, tur
 class LatentShape:
     """How a latent cache and its queries are laid out: ``entry`` dims a cached vector and query head, of which the first
     ``out_dim`` make the result; pairs (rot_off + 2i, rot_off + 2i + 1) of a query turn by position * freq[i] (``freq``
-    float on the device, or None); ``sink`` float [heads] or None; ``window`` > 0: the last positions only."""
+    float on the device, or None); ``sink`` float [heads] or None; ``window`` > 0: the last positions only.  ``float_sum`` (tiles of
+    bfloat16 entries of 129 to 256 dims): the softmax's normaliser sums the weights before they are rounded to meet the entries."""
 
     def __init__(self, heads: int, entry: int, out_dim: int, scale: float, rot_off: int = 0, freq: Optional[torch.Tensor] = None,
-                 rot_mult: float = 1.0, sink: Optional[torch.Tensor] = None, window: int = 0):
+                 rot_mult: float = 1.0, sink: Optional[torch.Tensor] = None, window: int = 0, float_sum: bool = False):
+        self.float_sum = bool(float_sum)
         self.heads, self.entry, self.out_dim, self.scale = int(heads), int(entry), int(out_dim), float(scale)
         self.rot_off, self.freq, self.rot_mult, self.sink, self.window = int(rot_off), freq, float(rot_mult), sink, int(window)
 
@@ -2135,7 +2137,7 @@ def latent_tiles(q: torch.Tensor, cache: torch.Tensor, tile_item: torch.Tensor, 
         _need(t, name, torch.int32, (B,))
     _need(out, "out", q.dtype, (q.shape[0], sh.heads * sh.out_dim))
     _check(_lib().st_latent_tiles(_ptr(out), *head, _ptr(tile_item), _ptr(tile_q0), n, _ptr(item_tok_off), _ptr(item_start),
-                                  _ptr(item_len), *tail))
+                                  _ptr(item_len), *tail[:-2], int(sh.float_sum), *tail[-2:]))
 
 
 @_timed("latent_rows", lambda q, cache, token_item, positions, block_table, sh, num_splits=1, row_ids=None: {

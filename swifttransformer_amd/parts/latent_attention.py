@@ -160,7 +160,7 @@ class LatentAttention(PagedAttention):
             o = K.empty((q.shape[0], self.q_size), self.dtype, q.device)
             # (whole entries as results: the output matrix has zeros for the turned part)
             shape = K.LatentShape(self.num_heads, self.entry, self.entry, self.scale, self.rank if inside else 0,
-                                  self.freq if inside else None, self.rot_mult, None, self.window)
+                                  self.freq if inside else None, self.rot_mult, None, self.window, float_sum=True)
             K.latent_tiles(q, cache.k, plan.arrays["tile_item"], plan.arrays["tile_q0"], ctx.item_tok_off, ctx.item_start,
                            ctx.item_len, bt, shape, o)
             n = plan.host["num_short_rows"]

@@ -34,6 +34,45 @@ def test_tiles_of_latent_entries(heads, entry, window, start, tokens):
     assert bool((err <= 2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-4).all()), float((err / size).max())
 
 
+@pytest.mark.parametrize("heads,entry,tokens", [(4, 160, 64), (32, 144, 1000), (6, 256, 40)])       # two groups of waves, one, two
+def test_the_normaliser_is_the_sum_of_unrounded_weights(heads, entry, tokens):
+    """A coordinate that only the first key's entry has, whose weight is exactly one: its result is one over the normaliser, and nothing
+    but the result's own rounding separates it from float64."""
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(heads + entry)
+    ps, start = 16, 70
+    n = start + tokens
+    pages = -(-n // ps)
+    cache = torch.zeros(pages * ps, entry, device=DEV)
+    cache[0, 0], cache[1:, 1] = 1.0, -1.0                      # scores: the first key's 0, all others' -a
+    cache = cache.view(pages, 1, ps, entry).bfloat16()
+    q = torch.zeros(tokens, heads, entry, device=DEV)
+    q[..., 1] = 0.01 + torch.rand(tokens, heads, generator=g, device=DEV)
+    q = q.view(tokens, -1).bfloat16()
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    q0 = list(range(0, tokens, 64))
+    out = torch.empty(tokens, heads * entry, dtype=torch.bfloat16, device=DEV)
+    bt = torch.arange(pages, device=DEV, dtype=torch.int32).view(1, -1)
+    K.latent_tiles(q, cache, i32(*([0] * len(q0))), i32(*q0), i32(0), i32(start), i32(tokens), bt,
+                   K.LatentShape(heads, entry, entry, 1.0, float_sum=True), out)
+    a = q.view(tokens, heads, entry)[..., 1].to(F64)
+    others = torch.arange(start, n, device=DEV, dtype=F64)[:, None]                # keys beside the first one
+    want = 1.0 / (1.0 + others * torch.exp(-a))
+    err = (out.view(tokens, heads, entry)[..., 0].to(F64) - want).abs() / want
+    # the rounding of the result, up to 1,070 float additions and the hardware's exponentials; equal weights rounded to bfloat16 would all
+    # be off to the same side, by up to 2^-8 more
+    assert float(err.max()) <= 2.0 ** -8 + 1100 * 2.0 ** -24, float(err.max())
+
+
+def test_float_normalisers_are_offered_for_large_entries_alone():
+    from swifttransformer_amd.ops import kernels as K
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    cache, q = torch.zeros(1, 1, 16, 128, device=DEV).bfloat16(), torch.zeros(4, 128, device=DEV).bfloat16()
+    with pytest.raises(K.KernelError, match="float normalisers"):
+        K.latent_tiles(q, cache, i32(0), i32(0), i32(0), i32(0), i32(4), i32(0).view(1, 1), K.LatentShape(1, 128, 128, 1.0, float_sum=True),
+                       torch.empty_like(q))
+
+
 def test_wide_block_tables_do_not_fit():
     from swifttransformer_amd.ops import kernels as K
     assert K.latent_tiles_fit(32, 160, 16, 128, 16) and K.latent_tiles_fit(32, 256, 16, 2048, 16)
