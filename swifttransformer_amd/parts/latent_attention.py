@@ -118,9 +118,10 @@ class LatentAttention(PagedAttention):
         """Whether prompts go through the tiles made for a latent cache, which read an entry once for scores and sums.  Entries of up
         to 128 stay with the paged kernels (2,011 tokens of 32 heads, entries of 128: 63 us there in tiles of 128 rows, 65 by latent
         tiles; 300 tokens of 12 heads, 96: 8 and 11); above, the paged kernel is the general one (entries of 160, 1,024 tokens of 32
-        heads 59 and 40 us, 753 behind 1,024 others 85 and 48, 112 tokens 9.1 and 9.3; entries of 256 105 and 59)."""
+        heads 59 and 40 us, 753 behind 1,024 others 85 and 48, 112 tokens 9.1 and 9.3; entries of 256 105 and 59).  The latent kernel
+        knows windows and no chunks (a window below zero)."""
         half = self.rot_dim // 2 if self._turns_in_tiles() else 0
-        return (self.dtype == torch.bfloat16 and self.entry > 128 and not self._biased()
+        return (self.dtype == torch.bfloat16 and self.entry > 128 and self.window >= 0 and not self._biased()
                 and K.latent_tiles_fit(self.num_heads, self.entry, page_size, max_pages, half))
 
     def _biased(self) -> bool:
@@ -130,7 +131,8 @@ class LatentAttention(PagedAttention):
         return self.rot_dim > 0 and self.rank % 8 == 0       # (the kernel turns whole pieces of 8)
 
     def plan_key(self):
-        return ("latent_attention_tiles", self.tile_min_len, self.num_heads, self.entry, self.dtype, self._turns_in_tiles(), self.rot_dim, self._biased())
+        return ("latent_attention_tiles", self.tile_min_len, self.num_heads, self.entry, self.dtype, self._turns_in_tiles(), self.rot_dim,
+                self.window < 0, self._biased())
 
     def step_planner(self):
         def planner(items, info):
