@@ -151,7 +151,9 @@ class LatentAttention(PagedAttention):
                            ctx.block_tables[cache.group], tail=self.rot_dim, tail_freq=self.freq, tail_mult=self.rot_mult)
         q = K.gemm(x_t, self.w_q)
         plan, bt = ctx.plans.get(self.plan_key()), ctx.block_tables[cache.group]
-        tiles = plan is not None and K.prefill_available() and self._latent_tiles(cache.k.shape[2], bt.shape[1])
+        # (a plan of 128 rows a tile is not for the latent tiles, which take 64)
+        tiles = (plan is not None and plan.host["tile_rows"] == K.PREFILL_TILE and K.prefill_available()
+                 and self._latent_tiles(cache.k.shape[2], bt.shape[1]))
         # (the tiles turn the queries themselves, unless rows of another kernel need them turned too)
         inside = tiles and plan.host["num_short_rows"] == 0 and self._turns_in_tiles()
         if self.rot_dim and not inside:

@@ -72,6 +72,23 @@ def test_large_entries_in_the_mixer(monkeypatch, rank, rot, window):
     assert inside == ([] if window < 0 else [turns, turns, False, False, turns])
 
 
+def test_a_plan_of_other_tiles_is_not_read_as_one_of_64_rows():
+    from swifttransformer_amd.engine.batch import StepItem
+    from swifttransformer_amd.ops import kernels as K
+    from swifttransformer_amd.parts.attention import plan_tiles
+    from swifttransformer_amd.cache.device import CacheView
+    from swifttransformer_amd.parts.base import StepPlan
+    part, _w, _c = _mixer(128, 32, 0)
+    items = [StepItem(0, 0, list(range(130)), [], {0: list(range(9))})]
+    ctx = ctx_for(items, page_size=16, parts=[part])
+    plan = plan_tiles(items, 8, 128)
+    arrays = {k: torch.from_numpy(v).to(DEV) for k, v in plan.arrays.items()}
+    ctx.plans[part.plan_key()] = StepPlan(arrays, plan.host)
+    pool = torch.zeros((9, 1, 16, part.entry), dtype=BF16, device=DEV)
+    with pytest.raises(K.KernelError, match="128 rows"):
+        part.forward(torch.randn(130, 64, device=DEV).to(BF16), torch.zeros(130, 64, device=DEV), ctx, CacheView(0, 0, k=pool, v=pool))
+
+
 CONFIGS = {
     "rank 128": [tiny._with(tiny._latent(4, 24, 32, 16, 128, 0.3, window=70), tiny._moe(4, 2, 24)),
                  tiny._with(tiny._latent(4, 24, 32, 16, 128, 0.3), None)],
