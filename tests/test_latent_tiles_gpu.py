@@ -64,6 +64,52 @@ def test_the_normaliser_is_the_sum_of_unrounded_weights(heads, entry, tokens):
     assert float(err.max()) <= 2.0 ** -8 + 1100 * 2.0 ** -24, float(err.max())
 
 
+# a launch of few tiles shares out their keys over two groups of waves; with many (here: entries that are skipped), or with page lists that leave
+# no room for two groups' blocks, one group goes through all of a tile's keys
+@pytest.mark.parametrize("skipped,long_list", [(0, False), (400, False), (0, True)])
+@pytest.mark.parametrize("entry,heads,rot_off,pairs,window,scale,float_sum", [
+    (64, 5, 40, 9, 0, 0.2, False), (128, 3, 96, 16, 70, -0.1, False), (160, 4, 128, 16, 0, 0.1, True), (144, 6, 136, 4, 33, -0.15, True),
+    (192, 2, 0, 5, 100, 0.1, True), (256, 3, 240, 8, 0, 0.08, True), (160, 4, 128, 16, 40, 0.1, False)])
+def test_tiles_with_turned_pairs_sinks_and_windows(entry, heads, rot_off, pairs, window, scale, float_sum, skipped, long_list):
+    from swifttransformer_amd.ops import kernels as K
+    g = torch.Generator(device=DEV).manual_seed(entry + heads)
+    ps, start, tokens = 16, 90, 150
+    n, out_dim = start + tokens, entry - 16
+    pages = -(-n // ps)
+    listed = {64: 35000, 128: 30000, 256: 20000}.get(entry, 24000) if long_list else pages
+    cache = torch.randn(pages + 1, 1, ps, entry, generator=g, device=DEV).bfloat16()
+    cache[-1] = float("nan")                                   # nobody's page, listed behind the request's own
+    order = torch.randperm(pages, generator=g, device=DEV).int()
+    bt = torch.full((1, listed), pages, dtype=torch.int32, device=DEV)
+    bt[0, :pages] = order
+    q = torch.randn(tokens, heads, entry, generator=g, device=DEV).bfloat16()
+    freq = torch.rand(pairs, generator=g, device=DEV)
+    sink = torch.randn(heads, generator=g, device=DEV)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    q0 = [0] * skipped + list(range(0, tokens, 64))
+    item = [-1] * skipped + [0] * (len(q0) - skipped)
+    out = torch.empty(tokens, heads * out_dim, dtype=torch.bfloat16, device=DEV)
+    K.latent_tiles(q.view(tokens, -1), cache, i32(*item), i32(*q0), i32(0), i32(start), i32(tokens), bt,
+                   K.LatentShape(heads, entry, out_dim, scale, rot_off, freq, 1.25, sink, window, float_sum), out)
+    keys = cache[order.long()].reshape(-1, entry)[:n].to(F64)
+    i, j = torch.arange(start, n, device=DEV)[:, None], torch.arange(n, device=DEV)[None]
+    seen = (j <= i) & ((i - j < window) if window else torch.ones_like(j, dtype=torch.bool))
+    angle = (torch.arange(start, n, device=DEV).float()[:, None] * freq[None]).to(F64)[:, None]          # (float angles)
+    c, s = torch.cos(angle) * 1.25, torch.sin(angle) * 1.25
+    turned = q.to(F64)
+    even, odd = turned[..., rot_off:rot_off + 2 * pairs:2].clone(), turned[..., rot_off + 1:rot_off + 2 * pairs:2].clone()
+    turned[..., rot_off:rot_off + 2 * pairs:2], turned[..., rot_off + 1:rot_off + 2 * pairs:2] = even * c - odd * s, odd * c + even * s
+    turned = turned.bfloat16().to(F64)
+    z = torch.matmul(turned.transpose(0, 1), keys.T) * scale
+    z = torch.cat([z.masked_fill(~seen[None], float("-inf")), sink.to(F64)[:, None, None].expand(heads, tokens, 1)], 2)
+    p = torch.softmax(z, -1)[..., :-1]
+    want, size = torch.matmul(p, keys[:, :out_dim]).transpose(0, 1), torch.matmul(p, keys[:, :out_dim].abs()).transpose(0, 1)
+    # a weight is rounded to bfloat16 (2^-8 at most) and so is the result; a turned number may be rounded to the other side than here (2^-8 of
+    # up to 6, against a key of up to 5, times the scale: a score off by 0.12 |scale|)
+    err = (out.view(tokens, heads, out_dim).to(F64) - want).abs()
+    assert bool((err <= (2.0 ** -8 + 0.24 * abs(scale)) * size + 2.0 ** -8 * want.abs() + 1e-4).all()), float((err / size).max())
+
+
 def test_float_normalisers_are_offered_for_large_entries_alone():
     from swifttransformer_amd.ops import kernels as K
     i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)
