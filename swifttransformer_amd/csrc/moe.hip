@@ -673,8 +673,8 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 // ---- prompts in bfloat16: tiles of 64 or 128 places, operands by direct loads into LDS -----------
 // With some dozens of rows and more an expert a tile of 64 NJ places meets 64 WN rows of its expert's matrix, steps of 64 in depth.
 // Both operand tiles go from memory into LDS without passing through registers (16 bytes a lane; a row's chunks are rotated by
-// the lane's choice of address, so that the matrix instruction's reads spread over the banks), the two steps after the one that is
-// multiplied on their way into the other two of three buffers: one barrier a step, before which a wave waits for its loads of that step
+// the lane's choice of address, so that the matrix instruction's reads spread over the banks), the AHEAD steps (1 or 2) after the one that is
+// multiplied on their way into the other buffers: one barrier a step, before which a wave waits for its loads of that step
 // alone.  Each of 2 WN waves multiplies a 64 x 32 NJ part (v_mfma_f32_32x32x16_bf16), the operands of a product of depth 16 read ahead
 // of the one before; the two waves that share weight rows take the tile's blocks of 32 places in turn, and a block without a pair
 // (an expert's last tile) is not multiplied.
@@ -684,7 +684,7 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 //
 // What bounds it: the weights' way from memory, all experts' matrices whatever the rows, and the operands' way from L2 into LDS, which
 // a unit takes at some 25 bytes a clock.  So: tiles of 128 places meet 256 weight rows (a quarter fewer bytes for the same products than
-// 128 rows, 48 KB a step, one workgroup a unit), tiles of 64 meet 128 (two workgroups a unit); and a workgroup begins its depth three
+// 128 rows, 48 KB a step, one workgroup a unit) unless that leaves units idle (the launch says where), tiles of 64 meet 128 (two workgroups a unit); and a workgroup begins its depth three
 // steps after its neighbour does, going round, since rows that lie a power of two apart meet in the same memory channels while everyone
 // reads at the same depth.  Workgroups go round the eight dies by their number; here each die takes
 // an eighth of the work in the order (expert, weight rows, tile of that expert), so that an expert's matrix passes through one
@@ -726,8 +726,9 @@ __device__ inline bool moe_work_item(int& tile, int& block, int& expert, const i
 
 enum TiledKind : int { kTiledDown = 0, kTiledUp = 1, kTiledGelu = 2 };
 
-template <int KIND, int WN, int NJ>
-__global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void moe_tiled_kernel(
+// AHEAD: steps on their way beside the one that is multiplied
+template <int KIND, int WN, int NJ, int AHEAD>
+__global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 1) void moe_tiled_kernel(
     bf16_t* __restrict__ y_out, float* out, const float* residual, float* __restrict__ pair_out, const bf16_t* __restrict__ a_rows,
     const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, const int* __restrict__ sorted, const int* __restrict__ tile_expert,
     const float* __restrict__ weights, int max_tiles, int blocks, int top, int N, int K, float limit, float out_scale, int style) {
@@ -736,7 +737,7 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void moe_tiled_kernel(
     // 16 were used before, whose waves share the depth: their chains are an eighth as long (2,048 deep: 2.7e-7 off float64 in one chain,
     // 1.3e-7 in theirs).
     constexpr bool DOUBLE = KIND == kTiledDown && NJ == 1;
-    constexpr int WAVES = 2 * WN, ROWS = 64 * WN, PLACES = 64 * NJ, AHEAD = 2;      // steps on their way
+    constexpr int WAVES = 2 * WN, ROWS = 64 * WN, PLACES = 64 * NJ;
     constexpr int BUF = (ROWS + PLACES) * 8;               // 16-byte pieces a buffer: weight rows, then places
     constexpr int NW = ROWS / (8 * WAVES), NP = PLACES / (8 * WAVES), NL = NW + NP;      // direct loads a wave and step, eight rows each
     __shared__ uint4 lds[(AHEAD + 1) * BUF];
@@ -829,7 +830,7 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void moe_tiled_kernel(
         }
     };
     stage(0, 0);
-    if (steps > 1) stage(1, 1);
+    if (AHEAD > 1 && steps > 1) stage(1, 1);
     for (int s = 0, cur = 0; s < steps; ++s) {
         // This wave's loads of the step have landed, those of the steps after it may be on their way; then everyone's have, and the
         // buffer of the step before has been read.
@@ -929,16 +930,33 @@ template <int KIND>
 static int launch_tiled(bf16_t* y, float* out, const float* residual, float* pair_out, const void* a_rows, const void* w0,
                         const void* w1, const int* sorted, const int* tile_expert, const float* weights, int capacity, int tile, int top,
                         int N, int K, float limit, float out_scale, int style, hipStream_t stream) {
-    const int rows = tile == 64 ? 128 : 256, features = KIND == kTiledUp ? rows / 2 : rows;
-    const int tiles = capacity / tile, blocks = (N + features - 1) / features;
-    ST_CHECK((int64_t)tiles * blocks < (1ll << 30), "moe: too many tiles");
-    const unsigned grid = (unsigned)((tiles * blocks + 7) / 8 * 8);
-    if (tile == 64)
-        moe_tiled_kernel<KIND, 2, 1><<<grid, 256, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
-            (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
-    else
-        moe_tiled_kernel<KIND, 4, 2><<<grid, 512, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0,
-            (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
+    const int tiles = capacity / tile;
+    const auto launch = [&](auto wn, auto nj, auto ahead) {
+        constexpr int WN = decltype(wn)::value, NJ = decltype(nj)::value, AHEAD = decltype(ahead)::value;
+        const int features = KIND == kTiledUp ? 32 * WN : 64 * WN, blocks = (N + features - 1) / features;
+        ST_CHECK((int64_t)tiles * blocks < (1ll << 30), "moe: too many tiles");
+        const unsigned grid = (unsigned)((tiles * blocks + 7) / 8 * 8);
+        moe_tiled_kernel<KIND, WN, NJ, AHEAD><<<grid, 128 * WN, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows,
+            (const bf16_t*)w0, (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
+        return 0;
+    };
+    int rc;
+    if (tile == 64) {
+        rc = launch(Steps<2>(), Steps<1>(), Steps<2>());
+    } else {
+        // Tiles of 128 places meet 256 weight rows where that still fills the chip, else 128.  A list has fewer tiles than places for them
+        // (an expert's last tile is counted whole, and one more for each expert): from two thirds on, with 112 pairs an expert and more.
+        // Workgroups of 128 rows that are a compute unit's only one bring two steps ahead; where some units may get a second, one (two
+        // buffers: two workgroups a unit have room).  Output products, us, with 256 rows, 128 and two steps, 128 and one step (workgroups
+        // of 128 rows in the list): 16 experts of 768 x 768, 896 tokens (138) 19.3, 15.4, 16.1; 2,048 tokens (252) 20.1, 16.9, 17.1;
+        // 8 of 3,072 x 768, 448 tokens (60) 56.0, 43.6, 50.3; 16 of 1,024 x 1,024, 1,600 tokens (264) 23.4, 34.5, 23.2; 16 of 1,536 x
+        // 1,536, 2,048 tokens (444) 36.3, 50.6, 40.4; of 2,048 x 2,048, 896 tokens (384) 44.2, 61.5, 45.7.
+        const int features = KIND == kTiledUp ? 64 : 128, units = device_compute_units();
+        const int64_t narrow = (int64_t)tiles * ((N + features - 1) / features);
+        rc = narrow <= units ? launch(Steps<2>(), Steps<2>(), Steps<2>())
+             : 7 * narrow <= 10 * (int64_t)units ? launch(Steps<2>(), Steps<2>(), Steps<1>()) : launch(Steps<4>(), Steps<2>(), Steps<2>());
+    }
+    if (rc) return rc;
     ST_LAUNCH_CHECK("moe (tiled)");
     return 0;
 }

@@ -128,3 +128,35 @@ def test_last_tiles_that_are_partly_empty(W, F, counts):
         # an expert's inner values are rounded to bfloat16 once (by 2^-8 of each at most); every sum is float
         err = (got.double().cpu() - (res.to(F64) + want)).abs()
         assert bool((err <= (2.0 ** -8 + 1e-4) * size + 1e-5).all()), float((err / size).max())
+
+
+@pytest.mark.parametrize("W,F,up,down", [
+    (840, 440, "one", "one"), (1160, 648, "wide", "wide"), (64, 712, "wide", "two"), (1224, 64, "two", "wide"), (128, 392, "one", "two"),
+    (776, 136, "two", "one"), (1096, 712, "wide", "wide")])
+@pytest.mark.parametrize("unit", ["silu", "gelu"])
+def test_tiles_of_128_places_on_as_many_weight_rows_as_fill_the_chip(W, F, up, down, unit):
+    """24 experts with chosen numbers of rows: 256 weight rows a workgroup ("wide"), or 128 with one or two steps of loads ahead; depths of 1
+    to 20 steps, whole and not, feature counts that leave part of a block."""
+    from swifttransformer_amd.ops import kernels as K
+    counts = (1, 127, 0, 260, 32, 33, 64, 300, 65, 96, 97, 200, 128, 129, 160, 31, 256, 255, 2, 180, 140, 111, 63, 190)
+    g = torch.Generator().manual_seed(W + F)
+    E, T = len(counts), sum(counts)
+    cap = K.moe_capacity(T, 1, E, 128)
+    assert K.moe_tile(T, 1, E, True) == 128
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    form = lambda blocks: "two" if cap // 128 * blocks <= units else "one" if 7 * (cap // 128) * blocks <= 10 * units else "wide"
+    if unit == "silu":
+        assert (form(-(-F // 64)), form(-(-W // 128))) == (up, down)
+    rnd = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).bfloat16().to(F64)
+    x, wu, wd = rnd(T, W), rnd(E, F, W, std=W ** -0.5), rnd(E, W, F, std=F ** -0.5)
+    wg = rnd(E, F, W, std=W ** -0.5) if unit == "silu" else None
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)]
+    z = torch.full((T, E), -4.0)
+    z[torch.arange(T), ids] = 4.0
+    dev = lambda t, d=torch.bfloat16: None if t is None else t.to("cuda").to(d)
+    res = torch.randn(T, W, generator=g)
+    want, size = _experts(x, ids[:, None], torch.ones(T, 1, dtype=F64), wg, wu, wd, unit, False, 0.0)
+    got = K.routed_experts(dev(x), dev(z, torch.float32), dev(wg), dev(wu), dev(wd), dev(res, torch.float32), top=1, style="softmax_output")
+    # an expert's inner values are rounded to bfloat16 once (by 2^-8 of each at most); every sum is float
+    err = (got.double().cpu() - (res.to(F64) + want)).abs()
+    assert bool((err <= (2.0 ** -8 + 1e-4) * size + 1e-5).all()), float((err / size).max())
