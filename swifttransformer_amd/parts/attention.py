@@ -175,11 +175,7 @@ class PagedAttention(Mixer):
             # others waiting.  Workgroups of half the keys even that out (batch 10, 11, 17, 18: +2 to
             # 3 % a step; nothing where the last round is fuller).
             splits = 2
-        # Eight waves where rows and heads leave a workgroup a unit and its keys whole: a unit with a long row beside others that have
-        # finished then has twice the bytes on their way (8 rows of 32 heads, 300 to 1,990 keys, OPT-1.3B sizes: a step 1,653 -> 1,606 us;
-        # rows of one length 4,969 and 4,967 tokens/s).  With the keys split, what more waves gain at long contexts is less than what
-        # their merge costs at short ones (one row of 12 heads, 97 keys: 384 and 391 us).
-        return max(1, splits), 8 if splits <= 1 and groups <= units else 4
+        return max(1, splits), 4
 
     def attend(self, qkv: torch.Tensor, ctx, cache, unmerged_ok: bool = False):
         """Attention of every row of ``qkv`` [T, q+2kv] over ``cache`` (already holding the rows' keys).
