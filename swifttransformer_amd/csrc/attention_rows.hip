@@ -374,12 +374,8 @@ static int launch_rows(void* out, float* part_o, float* part_lse, const void* q,
     while (lpk < need) lpk <<= 1;
     ST_CHECK(lpk <= 64, "attention: head_dim %d is too large for this kernel (at most %d)",
              head_dim, 64 * VEC);
-    const auto lds_bytes = [&](int waves) {
-        const int G = waves * (64 / lpk);
-        return (size_t)(2 * G + G * head_dim + 16 + max_pages) * sizeof(float);
-    };
-    if (num_waves > 4 && lds_bytes(num_waves) > 64 * 1024) num_waves = 4;      // (long page lists leave room for four waves' results only)
-    const size_t lds = lds_bytes(num_waves);
+    const int G = num_waves * (64 / lpk);
+    const size_t lds = (size_t)(2 * G + G * head_dim + 16 + max_pages) * sizeof(float);
     dim3 grid(num_q_heads, num_tokens, num_splits);
 #define ST_ROWS(L)                                                                              \
     attn_rows_kernel<T, L><<<grid, num_waves * 64, lds, stream>>>((T*)out, part_o, part_lse, (const T*)q,  \
