@@ -785,11 +785,16 @@ static int latent_dispatch(const LatentArgs& a, int list, bool float_sum, int dt
     // (an entry runs in the next larger instance, its missing chunks zeros in LDS)
     const int hdp = (a.entry + 31) / 32;
     // tiles: four waves of 16 rows, blocks of 64 keys (32 where entries are large); rows: one or two waves of 16 rows,
-    // four (two) shares of the keys, blocks of 32 keys.  Tiles whose workgroups are fewer than one and a half times the compute units
-    // (and whose page lists leave the room) share out their keys over two groups of waves: entries of 160, one item from position 0,
-    // without and with, us: 64 tokens of 32 heads behind 1,500 others (32 workgroups) 53 and 37, 512 tokens (256) 22 and 18, 1,024 of 16
-    // heads and 192 (256) 43 and 31; 1,024 of 32 heads (512) 40 and 43.
-    const bool half_empty = 2ll * list * ((kTileTokens * (int64_t)a.heads + 63) / 64) < 3 * device_compute_units();
+    // four (two) shares of the keys, blocks of 32 keys.  Tiles whose workgroups are few (and whose page lists leave the room) share out their
+    // keys over two groups of waves.  Entries of up to 128: up to one and a half times the compute units (entries of 128, 32 heads, 700
+    // tokens, 350 workgroups: one group 23.4 us, two 19.2; behind a window of 256 15.2 and 14.8).  Above, such a workgroup has a unit to
+    // itself: up to as many as units (entries of 160, 64 tokens of 32 heads behind 1,500 others, 32 workgroups, 53 and 37 us; 512 tokens,
+    // 256, 23.0 and 18.0), and to one and a half times as many where tiles read all keys before them, the heavy ones first (12 heads,
+    // 1,984 tokens, 372 workgroups, 70.6 and 50.3; 32 heads, 576 tokens behind 1,000 others, 288, 58.5 and 59.3; 64 heads, 300 behind 500,
+    // 320, 33.3 and 37.3), not where a window makes them even (12 heads, 1,984 tokens, window 256, 19.8 and 27.4).  1,024 tokens of 32
+    // heads, 512 workgroups: 40 and 43.
+    const int64_t groups = (int64_t)list * ((kTileTokens * (int64_t)a.heads + 63) / 64), units = device_compute_units();
+    const bool half_empty = hdp <= 4 || a.window == 0 ? 2 * groups <= 3 * units : groups <= units;
 #define ST_LT(H)                                                                                                       \
     if (hdp <= H) {                                                                                                    \
         if constexpr (TILES && H >= 5) {                                                                               \

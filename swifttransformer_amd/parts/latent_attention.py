@@ -115,14 +115,25 @@ class LatentAttention(PagedAttention):
     accepts_norm = False
 
     def _latent_tiles(self, page_size: int, max_pages: int) -> bool:
-        """Whether prompts go through the tiles made for a latent cache, which read an entry once for scores and sums.  Entries of up
+        """Whether prompts can go through the tiles made for a latent cache, which read an entry once for scores and sums.  Entries of up
         to 128 stay with the paged kernels (2,011 tokens of 32 heads, entries of 128: 63 us there in tiles of 128 rows, 65 by latent
-        tiles; 300 tokens of 12 heads, 96: 8 and 11); above, the paged kernel is the general one (entries of 160, 1,024 tokens of 32
-        heads 59 and 40 us, 753 behind 1,024 others 85 and 48, 112 tokens 9.1 and 9.3; entries of 256 105 and 59).  The latent kernel
-        knows windows and no chunks (a window below zero)."""
+        tiles; 300 tokens of 12 heads, 96: 8 and 11); above, the paged kernel is the general one.  The latent kernel knows windows and no
+        chunks (a window below zero)."""
         half = self.rot_dim // 2 if self._turns_in_tiles() else 0
         return (self.dtype == torch.bfloat16 and self.entry > 128 and self.window >= 0 and not self._biased()
                 and K.latent_tiles_fit(self.num_heads, self.entry, page_size, max_pages, half))
+
+    def _least_keys(self, inside: bool) -> int:
+        """Keys of a step's longest tile from which the latent tiles are no slower.  They take longer to begin (their buffers hold two blocks
+        of keys) and less a block, and they turn the queries themselves (``inside``), which the paged kernel leaves to one of its own.
+        32 heads, paged kernel (with the turn) and latent tiles, us: entries of 160 8 tokens 9.5 and 9.1, 1,024 tokens 61.2 and 41.2, 64
+        behind 1,000 others 43.2 and 29.6; of 192 16 tokens 10.0 and 11.1, 100 tokens 12.0 and 11.9; of 256 64 tokens 11.8 and 13.3, 100
+        tokens 14.9 and 14.2, 1,024 tokens 107 and 64.  Turned by a kernel of its own for both: entries of 144 [300, 200] tokens 18.9 and
+        19.3, 16 tokens behind a window of 256 15.2 and 16.2, 512 behind 1,024 47.4 and 39.8; of 160 100 tokens 11.3 and 11.7, 256 tokens
+        16.8 and 14.7; of 256 100 tokens 14.9 and 15.4, 256 tokens 25.0 and 19.7."""
+        if inside:
+            return 0 if self.entry <= 160 else 96
+        return 384 if self.entry <= 144 else 256
 
     def _biased(self) -> bool:
         return self.position is not None and getattr(self.position, "biases_scores", False)      # (the latent kernel knows no slopes)
@@ -132,14 +143,24 @@ class LatentAttention(PagedAttention):
 
     def plan_key(self):
         return ("latent_attention_tiles", self.tile_min_len, self.num_heads, self.entry, self.dtype, self._turns_in_tiles(), self.rot_dim,
-                self.window < 0, self._biased())
+                self.window if self.entry > 128 else min(self.window, 0), self._biased())
 
     def step_planner(self):
         def planner(items, info):
-            choose = lambda rows: (K.PREFILL_TILE if self._biased() or self._latent_tiles(info.page_size, info.max_pages) else
+            latent = self._latent_tiles(info.page_size, info.max_pages)
+            choose = lambda rows: (K.PREFILL_TILE if self._biased() or latent else
                                    K.prefill_tile_rows(self.entry, info.page_size, info.max_pages, self.num_heads, rows, self.dtype))
-            return plan_tiles(items, self.tile_min_len, choose, bucketed=info.bucketed)
+            plan = plan_tiles(items, self.tile_min_len, choose, bucketed=info.bucketed)
+            if plan is not None and latent:
+                ends = [it.start + len(it.tokens) for it in items if len(it.tokens) >= self.tile_min_len]
+                keys = max(min(n, self.window + K.PREFILL_TILE) if self.window else n for n in ends)
+                plan.host["latent_tiles"] = int(keys >= self._least_keys(self._turns_inside(plan)))
+            return plan
         return self.plan_key(), planner
+
+    def _turns_inside(self, plan) -> bool:
+        """Whether the latent tiles turn a step's queries: where they can, and no row of another kernel needs them turned too."""
+        return self._turns_in_tiles() and plan.host["num_short_rows"] == 0
 
     def forward(self, x_t: torch.Tensor, residual32: Optional[torch.Tensor], ctx, cache, write: bool = True,
                 norm=None) -> torch.Tensor:
@@ -152,10 +173,9 @@ class LatentAttention(PagedAttention):
         q = K.gemm(x_t, self.w_q)
         plan, bt = ctx.plans.get(self.plan_key()), ctx.block_tables[cache.group]
         # (a plan of 128 rows a tile is not for the latent tiles, which take 64)
-        tiles = (plan is not None and plan.host["tile_rows"] == K.PREFILL_TILE and K.prefill_available()
-                 and self._latent_tiles(cache.k.shape[2], bt.shape[1]))
-        # (the tiles turn the queries themselves, unless rows of another kernel need them turned too)
-        inside = tiles and plan.host["num_short_rows"] == 0 and self._turns_in_tiles()
+        tiles = (plan is not None and plan.host.get("latent_tiles", 0) and plan.host["tile_rows"] == K.PREFILL_TILE
+                 and K.prefill_available() and self._latent_tiles(cache.k.shape[2], bt.shape[1]))
+        inside = tiles and self._turns_inside(plan)
         if self.rot_dim and not inside:
             K.rotary(q, None, self.entry, self.freq, self.rot_mult, ctx.positions, offset=self.rank, interleaved=True)
         if not tiles:

@@ -51,25 +51,30 @@ def test_large_entries_in_the_mixer(monkeypatch, rank, rot, window):
     inside = []
     tiles = K.latent_tiles
     monkeypatch.setattr(K, "latent_tiles", lambda *a: (inside.append(a[8].freq is not None), tiles(*a)))
-    n, ps = 150, 16
+    n, ps = 460, 16
     x = {s: torch.randn(n, 64, generator=torch.Generator().manual_seed(s)).to(BF16) for s in (0, 1)}
     res = {s: torch.randn(n, 64, generator=torch.Generator().manual_seed(7 + s)) for s in (0, 1)}
     ref = {s: res[s].to(F64) + plain.latent_attention(x[s].to(F64), w, "m", c, 1e-5) for s in (0, 1)}
-    pool = torch.full((24, 1, ps, part.entry), float("nan"), dtype=BF16, device=DEV)
+    pool = torch.full((64, 1, ps, part.entry), float("nan"), dtype=BF16, device=DEV)
     cache = CacheView(0, 0, k=pool, v=pool)
-    pages = {0: [3, 9, 1, 12, 5, 0, 22, 17, 16, 4], 1: [7, 2, 19, 14, 11, 6, 8, 10, 20, 13]}
-    done = {0: 0, 1: 0}
-    # alone; a portion beside the other's portion; single tokens beside a portion; single tokens alone; the rest
-    for step in ([(0, 70)], [(1, 64), (0, 9)], [(0, 1), (1, 33)], [(1, 1), (0, 20)], [(0, 1), (1, 1)], [(0, 49), (1, 51)]):
+    order = torch.randperm(64, generator=torch.Generator().manual_seed(3)).tolist()
+    pages = {0: order[:29], 1: order[29:58]}
+    done, expected = {0: 0, 1: 0}, []
+    least = (0 if part.entry <= 160 else 96) if rot and rank % 8 == 0 else None, 384 if part.entry <= 144 else 256
+    # alone, few keys and many; beside the other's portion; single tokens beside a portion; single tokens alone; the rest
+    for step in ([(0, 70)], [(0, 300)], [(1, 380), (0, 9)], [(0, 1), (1, 33)], [(1, 1), (0, 40)], [(0, 1), (1, 1)], [(0, 39), (1, 45)]):
         items = [StepItem(s, done[s], list(range(m)), [], {0: pages[s]}) for s, m in step]
-        ctx = ctx_for(items, page_size=ps, parts=[part])
+        ctx = ctx_for(items, page_size=ps, max_pages=32, parts=[part])
         part_of = lambda v: torch.cat([v[s][done[s]:done[s] + m] for s, m in step])
         out = part.forward(part_of(x).to(DEV), part_of(res).to(DEV), ctx, cache)
         check(out, part_of(ref).numpy(), BF16, f"rank {rank} rot {rot} window {window} step {step}")
         for s, m in step:
             done[s] += m
-    turns = rot > 0 and rank % 8 == 0
-    assert inside == ([] if window < 0 else [turns, turns, False, False, turns])
+        long = [done[s] if window == 0 else min(done[s], window + 64) for s, m in step if m >= 8]
+        turned = least[0] is not None and all(m >= 8 for _, m in step)
+        if long and window >= 0 and max(long) >= least[0 if turned else 1]:
+            expected.append(turned)
+    assert inside == expected
 
 
 def test_a_plan_of_other_tiles_is_not_read_as_one_of_64_rows():
@@ -82,6 +87,7 @@ def test_a_plan_of_other_tiles_is_not_read_as_one_of_64_rows():
     items = [StepItem(0, 0, list(range(130)), [], {0: list(range(9))})]
     ctx = ctx_for(items, page_size=16, parts=[part])
     plan = plan_tiles(items, 8, 128)
+    plan.host["latent_tiles"] = 1
     arrays = {k: torch.from_numpy(v).to(DEV) for k, v in plan.arrays.items()}
     ctx.plans[part.plan_key()] = StepPlan(arrays, plan.host)
     pool = torch.zeros((9, 1, 16, part.entry), dtype=BF16, device=DEV)
@@ -104,17 +110,17 @@ def test_models_with_large_entries_against_the_plain_one(tmp_path, monkeypatch, 
     cfg = {"architecture": "Gisedra", "vocab": 97, "width": 64, "max_positions": 512, "norm": {"eps": 1e-6}, "layers": CONFIGS[name]}
     folder = tiny.write_folder(cfg, str(tmp_path / "m"), 5)
     cfg, w = plain.load_folder(folder)
-    seqs = {r: tiny.prompt(150, 97, i) for i, r in enumerate("ab")}
+    seqs = {r: tiny.prompt(450, 97, i) for i, r in enumerate("ab")}
     refs = {r: plain.logits(cfg, w, s).numpy() for r, s in seqs.items()}
     calls = []
     tiles = K.latent_tiles
     monkeypatch.setattr(K, "latent_tiles", lambda *a: (calls.append(1), tiles(*a)))
-    runner = make_runner(folder, "bfloat16", 16, 24, record_after=recording, max_seqs=2)
+    runner = make_runner(folder, "bfloat16", 16, 60, record_after=recording, max_seqs=2)
     what = f"{name} recording {recording}"
     for _ in range(2):                                # the second time on pages used before, and from recordings
-        run_schedule(runner, seqs, refs, [[("a", 150)], [("b", 150)]], "bfloat16", what + " whole")
-        run_schedule(runner, seqs, refs, [[("a", 64)], [("a", 1), ("b", 77)], [("b", 1), ("a", 20)], [("a", 1), ("b", 1)], [("a", 64), ("b", 71)]],
-                     "bfloat16", what + " portions beside decoded tokens")
+        run_schedule(runner, seqs, refs, [[("a", 225)], [("a", 225)], [("b", 225)], [("b", 225)]], "bfloat16", what + " alone")
+        run_schedule(runner, seqs, refs, [[("a", 60)], [("a", 1), ("b", 230)], [("b", 1), ("a", 240)], [("a", 1), ("b", 190)], [("a", 1), ("b", 1)],
+                                          [("a", 147), ("b", 28)]], "bfloat16", what + " portions beside decoded tokens")
     assert calls
     if recording == 1:
         assert runner.graph_replays == runner.steps_run, "a step ran unrecorded"
