@@ -303,7 +303,8 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
 // What bounds it: trips to memory one after the other.  A lane a split forms the weights, and the partial results are asked for eight
 // splits at a time without waiting for them (one row of 12 heads, 16 splits: 6.9 us with the splits one by one, 4.8 us; sums in the
 // same order).
-template <typename T>
+// U: splits asked for at a time (a row of few splits has no more).
+template <typename T, int U>
 __global__ __launch_bounds__(64) void attn_merge_kernel(
     T* __restrict__ out, const float* __restrict__ part_o, const float* __restrict__ part_lse,
     const int* __restrict__ row_ids, int num_q_heads, int head_dim, int num_splits, const float* __restrict__ head_gate,
@@ -313,7 +314,6 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(
     const float* lse = part_lse + row * num_splits;
     const float* parts = part_o + row * num_splits * head_dim;
     const int lane = threadIdx.x, t_id = row_ids ? row_ids[ri] : 0;
-    constexpr int U = 8;
     const bool few = num_splits <= 64;
     const float own = lse[min(lane, num_splits - 1)];          // (with up to 64 splits: lane s has that of split s)
     float first[U];                                            // the first columns' first partial results
@@ -394,9 +394,10 @@ static int launch_rows(void* out, float* part_o, float* part_lse, const void* q,
 #undef ST_ROWS
     ST_LAUNCH_CHECK("attn_rows");
     if (num_splits > 1 && out) {      // without `out` the caller merges the partial results itself
-        attn_merge_kernel<T><<<num_tokens * num_q_heads, 64, 0, stream>>>((T*)out, part_o, part_lse,
-                                                                          row_ids, num_q_heads, head_dim,
-                                                                          num_splits, head_gate, gate_stride);
+#define ST_MERGE(U) attn_merge_kernel<T, U><<<num_tokens * num_q_heads, 64, 0, stream>>>((T*)out, part_o, part_lse, row_ids, num_q_heads, \
+                                                                                     head_dim, num_splits, head_gate, gate_stride)
+        if (num_splits <= 2) ST_MERGE(2); else if (num_splits <= 4) ST_MERGE(4); else ST_MERGE(8);
+#undef ST_MERGE
         ST_LAUNCH_CHECK("attn_merge");
     }
     return 0;
