@@ -153,7 +153,9 @@ extern "C" int st_token_conv(void* out, const void* x, int64_t x_stride, int in_
              "token_conv: unknown dtype %d -> %d", in_dtype, out_dtype);
     if (num_tokens == 0) return 0;
     // Four channels a thread where every row of x, of the state and of the filters starts on a whole piece; filters of 2 to 4 taps, which
-    // all mixers and streams here have.  Four rows a thread from 64 rows on (below that threads are what is missing).
+    // all mixers and streams here have.  Four rows a thread where that still gives every compute unit a workgroup: with fewer, threads are
+    // what is missing (100 rows of 2,048 channels, 4 taps, by element 5.5 us, four rows a thread 6.4, one row 5.0; 505 rows of 768 6.1, 6.8 and
+    // 5.1).  One row or two go by element (one of 2,048, 2 taps, 4.2 and 4.5; eight 4.2 and 4.3, 4 taps 4.8 and 4.7).
     const int in_bytes = in_dtype == kF32 ? 16 : 8, out_bytes = out_dtype == kF32 ? 16 : 8;
     const bool four = channels % 4 == 0 && x_stride % 4 == 0 && slot_stride % 4 == 0 && (uintptr_t)x % in_bytes == 0 &&
                       (uintptr_t)out % out_bytes == 0 && (((uintptr_t)w | (uintptr_t)bias | (uintptr_t)state) & 15) == 0;
@@ -163,8 +165,9 @@ extern "C" int st_token_conv(void* out, const void* x, int64_t x_stride, int in_
         add_input, activation)
 #define ST_CONV_TAPS(TI, TO, ROWS)                                                                              \
     do { if (taps == 2) ST_CONV4(TI, TO, 2, ROWS); else if (taps == 3) ST_CONV4(TI, TO, 3, ROWS); else ST_CONV4(TI, TO, 4, ROWS); } while (0)
-#define ST_CONV_ROWS(TI, TO) do { if (num_tokens >= 64) ST_CONV_TAPS(TI, TO, 4); else ST_CONV_TAPS(TI, TO, 1); } while (0)
-    if (four && taps >= 2 && taps <= 4) {
+#define ST_CONV_ROWS(TI, TO) do { if (four_rows) ST_CONV_TAPS(TI, TO, 4); else ST_CONV_TAPS(TI, TO, 1); } while (0)
+    const bool four_rows = ((int64_t)num_tokens + 3) / 4 * ((channels + 1023) / 1024) >= device_compute_units();
+    if (four && num_tokens > 2 && taps >= 2 && taps <= 4) {
         if (in_dtype == kF32 && out_dtype == kF32) ST_CONV_ROWS(float, float);
         else if (in_dtype == kF32) ST_CONV_ROWS(float, bf16_t);
         else if (out_dtype == kF32) ST_CONV_ROWS(bf16_t, float);

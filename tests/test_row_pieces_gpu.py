@@ -136,3 +136,25 @@ def test_streams_written_by_as_many_threads_as_columns(streams, rows, width):
     # chains of a few float operations a number; the norm's sum of squares adds its own few roundings, relative
     assert bool(((got.view_as(x).double() - new).abs() <= 1e-6 * size + 1e-30).all())
     assert bool(((out.double() - u / norm * gain.double()).abs() <= (2e-6 * u_size + 2e-5 * u.abs()) / norm * gain.double().abs() + 1e-30).all())
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("in_dtype,out_dtype", [(torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("width,lens", [(1028, (1, 2, 3, 1, 514)), (516, (1029,)), (2052, (200, 1, 1, 1, 139, 3))])
+def test_token_conv_with_four_rows_a_thread(taps, in_dtype, out_dtype, width, lens):
+    """Rows enough for every compute unit, items that begin anywhere in a thread's four rows, a last group that is not whole, a padding row."""
+    from swifttransformer_amd.ops import kernels as K
+    T = sum(lens) + 1
+    assert -(-T // 4) * -(-width // 1024) >= torch.cuda.get_device_properties(0).multi_processor_count
+    g = torch.Generator(device=DEV).manual_seed(width + taps)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    wide = rnd(T, width + 5).to(in_dtype)
+    x = torch.empty(T, width + 8, dtype=in_dtype, device=DEV)[:, 4:4 + width].copy_(wide[:, 1:1 + width])
+    w, bias, state = rnd(width, taps), rnd(width), rnd(len(lens), taps - 1, width)
+    ti, ln, off, sl = items_ctx(list(lens), list(range(len(lens)))[::-1])
+    ti = torch.cat([ti, torch.full((1,), -1, dtype=torch.int32, device=DEV)])
+    for kw in ({}, {"add_input": False, "bias": bias, "activation": "silu"}):
+        s1, s2 = state.clone(), state.clone()
+        four = K.token_conv(x, w, s1, (ti, ln, off, sl), out_dtype, **kw)
+        one = K.token_conv(wide[:, 1:1 + width], w, s2, (ti, ln, off, sl), out_dtype, **kw)
+        assert torch.equal(four, one) and torch.equal(s1, s2)
