@@ -158,3 +158,25 @@ def test_token_conv_with_four_rows_a_thread(taps, in_dtype, out_dtype, width, le
         four = K.token_conv(x, w, s1, (ti, ln, off, sl), out_dtype, **kw)
         one = K.token_conv(wide[:, 1:1 + width], w, s2, (ti, ln, off, sl), out_dtype, **kw)
         assert torch.equal(four, one) and torch.equal(s1, s2)
+
+
+@pytest.mark.parametrize("dtype", list(DTYPES))
+@pytest.mark.parametrize("rows,width", [(130, 2052), (300, 516), (257, 4)])
+def test_dynamic_tanh_of_many_rows_in_pieces_of_four(dtype, rows, width):
+    from swifttransformer_amd.ops import kernels as K
+    assert rows * -(-width // 1024) > torch.cuda.get_device_properties(0).multi_processor_count
+    g = torch.Generator(device=DEV).manual_seed(width)
+    dt = DTYPES[dtype]
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, base, w, b, w2, b2, alpha = rnd(rows, width), rnd(rows, width), rnd(width), rnd(width), rnd(width), rnd(width), rnd(1)
+    picked = torch.randint(-1, rows, (rows + 2,), generator=g, device=DEV, dtype=torch.int32)
+
+    def run(shift):
+        f = _shifted if shift else (lambda t: t)
+        outs = [torch.full((rows, width), 3.0, device=DEV), torch.full((rows, width), 3.0, device=DEV, dtype=dt),
+                torch.full((rows + 2, width), 3.0, device=DEV, dtype=dt)]
+        K.dynamic_tanh(f(x), w, b, alpha, out_f32=outs[0], out_t=outs[1], base=base, then=(w2, b2, alpha))
+        K.dynamic_tanh(f(x), w, None, alpha, out_t=outs[2], rows=picked)
+        return outs
+    for four, one in zip(run(False), run(True)):
+        assert torch.equal(four, one)
