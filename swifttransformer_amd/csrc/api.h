@@ -261,18 +261,14 @@ int st_latent_write(void* cache, int64_t page_stride, const float* x, int64_t x_
 // the chosen logits alone, mode 2 each chosen expert's share of the softmax over all experts, where only the
 // experts of the `keep` best of `groups` equal groups of neighbours (a group's rank: its largest logit) can be
 // chosen, mode 3 the sigmoid of each chosen logit over the chosen sigmoids' sum (+ 1e-20), times `scale`, where the
-// choice goes by sigmoid + correction [experts] (else null).  Rows whose item is -1 get ids of -1.
+// choice goes by sigmoid + correction [experts] (else null), mode 4 each chosen expert's share of the softmax over all experts, where the
+// choice goes by share + correction.  Rows whose item is -1 get ids of -1.
 int st_moe_route(int* ids, float* weights, const float* logits, int logit_stride, const int* token_item, const float* correction,
                  float scale, int num_tokens, int experts, int top, int mode, int groups, int keep, hipStream_t stream);
 // Sorts the num_pairs = tokens * top (token, choice) pairs by expert into tiles of `tile` (16, 64 or 128)
 // places that hold one expert's pairs each: sorted[capacity] (pair index, or -1),
 // place_of_pair[num_pairs] (or -1), tile_expert[capacity / tile] (or -1).
 // capacity >= round_up(num_pairs, tile) + tile * experts.  st_moe_up and st_moe_down take the same `tile`.
-int st_moe_router_align_offered(int num_tokens, int w_rows, int outputs, int width, int dtype);
-int st_moe_router_align(int* ids, float* weights, int* sorted, int* place_of_pair, int* tile_expert, const void* x, const void* w,
-                        const float* bias, int width, int w_rows, const int* token_item, const float* correction, float scale,
-                        int num_tokens, int outputs, int experts, int top, int mode, int groups, int keep, int capacity, int tile,
-                        hipStream_t stream);
 int st_moe_align(int* sorted, int* place_of_pair, int* tile_expert, const int* ids, int num_pairs,
                  int experts, int capacity, int tile, hipStream_t stream);
 // st_moe_route and st_moe_align by one workgroup, for up to 64 tokens of 16 router outputs, 32 of 32 or 16 of 64; `experts` of the
@@ -280,6 +276,12 @@ int st_moe_align(int* sorted, int* place_of_pair, int* tile_expert, const int* i
 int st_moe_route_align(int* ids, float* weights, int* sorted, int* place_of_pair, int* tile_expert, const float* logits,
                        int logit_stride, const int* token_item, const float* correction, float scale, int num_tokens, int outputs,
                        int experts, int top, int mode, int groups, int keep, int capacity, int tile, hipStream_t stream);
+// st_moe_route_align of the logits x [num_tokens, width] . w [w_rows, width]^T (+ bias [w_rows]), bfloat16 operands; where offered.
+int st_moe_router_align_offered(int num_tokens, int w_rows, int outputs, int width, int dtype);
+int st_moe_router_align(int* ids, float* weights, int* sorted, int* place_of_pair, int* tile_expert, const void* x, const void* w,
+                        const float* bias, int width, int w_rows, const int* token_item, const float* correction, float scale,
+                        int num_tokens, int outputs, int experts, int top, int mode, int groups, int keep, int capacity, int tile,
+                        hipStream_t stream);
 // y[place, f] = g * sigmoid(1.702 g) * (u + 1) with g = min(s * (x_t . Wg[e, f]), limit) and
 // u = clamp(s * (x_t . Wu[e, f]), -limit, limit), for the pair (t, j) at `place`, e its expert and s
 // its weight (style 0); style 1: y[place, f] = silu(x_t . Wg[e, f]) * (x_t . Wu[e, f]), no weight and no
@@ -379,6 +381,7 @@ int st_latent_inputs(void* cq, int cq_width, const float* gain_q, int q_rank, vo
                      const int* block_table, int max_pages, int page_size, int num_tokens, float eps, int dtype,
                      hipStream_t stream);
 int st_latent_max_entry();
+// Whether bfloat16 tiles of entries of up to 256 dims leave room in LDS for page lists of max_pages.
 int st_latent_tiles_fit(int heads, int entry, int page_size, int max_pages, int rot_half);
 int st_latent_tiles(void* out, const void* q, int64_t q_stride, const void* cache, int64_t page_stride, const int* tile_item,
                     const int* tile_q0, int num_tiles, const int* item_tok_off, const int* item_start, const int* item_len,

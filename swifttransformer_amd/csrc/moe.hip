@@ -305,7 +305,8 @@ __global__ __launch_bounds__(1024) void moe_route_align_kernel(
 // The same behind the router's own product, for the fewest rows: one workgroup forms the logits (each wave a share of the depth, its
 // operands straight from memory in the matrix instruction's layout, all on their way at once; the shares meet in LDS), routes and sorts.
 // What bounds it: trips to memory, the operands' and then the routing's own chain; a product kernel of its own adds another launch and a
-// trip for its logits.  One row of 768, 16 outputs: with the product apart 2.7 and 4.5 us, so 6.2; a step of fiterax-125m 1.1 % shorter.  RB x CB blocks of 16 rows and 16 outputs.
+// trip for its logits.  One row of 768, 16 outputs: with the product apart 2.7 and 4.5 us, so 6.2; a step of fiterax-125m 1.1 % shorter.
+// RB x CB blocks of 16 rows and 16 outputs.
 template <int RB, int CB, int G>
 __global__ __launch_bounds__(1024) void moe_router_align_kernel(
     int* __restrict__ ids, float* __restrict__ weights, int* __restrict__ sorted, int* __restrict__ place_of_pair,
@@ -1018,8 +1019,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
 
 using namespace st;
 
-static int check_route(const float* logits, int logit_stride, const float* correction, int num_tokens, int experts, int top, int mode,
-                       int groups, int keep) {
+static int check_route(const float* correction, int num_tokens, int experts, int top, int mode, int groups, int keep) {
     ST_CHECK(mode >= 0 && mode <= 4, "moe_route: mode 0 (sigmoid of each), 1 (softmax over the chosen), 2 (softmax "
              "over all, the choice within the best groups), 3 (sigmoids over their sum, a corrected choice) or 4 (softmax over "
              "all, a corrected choice)");
@@ -1031,7 +1031,13 @@ static int check_route(const float* logits, int logit_stride, const float* corre
              experts / groups);
     ST_CHECK(top >= 1 && top <= kMaxTop && top <= experts, "moe_route: 1 to %d experts a token (of %d), not %d",
              kMaxTop, experts, top);
-    ST_CHECK(logits && logit_stride >= experts, "moe_route: null operand or short rows");
+    return 0;
+}
+
+static int check_places(int num_pairs, int experts, int capacity, int tile) {
+    ST_CHECK(tile == 16 || tile == 64 || tile == 128, "moe_align: tiles of 16, 64 or 128 places, not %d", tile);
+    ST_CHECK(capacity % tile == 0 && capacity >= (num_pairs + tile - 1) / tile * tile + tile * experts,
+             "moe_align: %d places do not hold %d pairs of %d experts in tiles of %d", capacity, num_pairs, experts, tile);
     return 0;
 }
 
@@ -1039,7 +1045,8 @@ extern "C" int st_moe_route(int* ids, float* weights, const float* logits, int l
                             const float* correction, float scale, int num_tokens, int experts, int top, int mode, int groups, int keep,
                             hipStream_t stream) {
     if (mode != 2) groups = keep = 1;
-    if (const int rc = check_route(logits, logit_stride, correction, num_tokens, experts, top, mode, groups, keep)) return rc;
+    if (const int rc = check_route(correction, num_tokens, experts, top, mode, groups, keep)) return rc;
+    ST_CHECK(logits && logit_stride >= experts, "moe_route: null operand or short rows");
     ST_CHECK(ids && weights, "moe_route: null operand");
     if (num_tokens == 0) return 0;
     if (experts <= 64) {
@@ -1069,15 +1076,13 @@ extern "C" int st_moe_route_align(int* ids, float* weights, int* sorted, int* pl
                                   int logit_stride, const int* token_item, const float* correction, float scale, int num_tokens, int outputs,
                                   int experts, int top, int mode, int groups, int keep, int capacity, int tile, hipStream_t stream) {
     if (mode != 2) groups = keep = 1;
-    if (const int rc = check_route(logits, logit_stride, correction, num_tokens, outputs, top, mode, groups, keep)) return rc;
+    if (const int rc = check_route(correction, num_tokens, outputs, top, mode, groups, keep)) return rc;
+    ST_CHECK(logits && logit_stride >= outputs, "moe_route: null operand or short rows");
     ST_CHECK(outputs <= 64 && experts >= 1 && experts <= outputs, "moe_route_align: up to 64 router outputs, not %d", outputs);
     ST_CHECK((int64_t)num_tokens * route_lanes(outputs) <= 1024, "moe_route_align: up to %d tokens of %d experts", 1024 / route_lanes(outputs), outputs);
     static_assert(kFusedPairs >= 1024 / 16 * kMaxTop, "the choices of all tokens fit LDS");
     if (num_tokens == 0) return st_moe_align(sorted, place_of_pair, tile_expert, ids, 0, experts, capacity, tile, stream);
-    ST_CHECK(tile == 16 || tile == 64 || tile == 128, "moe_align: tiles of 16, 64 or 128 places, not %d", tile);
-    const int num_pairs = num_tokens * top;
-    ST_CHECK(capacity % tile == 0 && capacity >= (num_pairs + tile - 1) / tile * tile + tile * experts,
-             "moe_align: %d places do not hold %d pairs of %d experts in tiles of %d", capacity, num_pairs, experts, tile);
+    if (const int rc = check_places(num_tokens * top, experts, capacity, tile)) return rc;
     ST_CHECK(ids && weights && sorted && place_of_pair && tile_expert, "moe_route_align: null operand");
     const RouteRule r{token_item, correction, scale, outputs, top, mode, groups, keep};
     const auto launch = [&](auto lanes) {
@@ -1108,15 +1113,11 @@ extern "C" int st_moe_router_align(int* ids, float* weights, int* sorted, int* p
                                    int num_tokens, int outputs, int experts, int top, int mode, int groups, int keep, int capacity, int tile,
                                    hipStream_t stream) {
     if (mode != 2) groups = keep = 1;
-    static const float some = 0.f;                 // (check_route asks for logits)
-    if (const int rc = check_route(&some, outputs, correction, num_tokens, outputs, top, mode, groups, keep)) return rc;
+    if (const int rc = check_route(correction, num_tokens, outputs, top, mode, groups, keep)) return rc;
     ST_CHECK(st_moe_router_align_offered(num_tokens, w_rows, outputs, width, kBF16), "moe_router_align: not for %d rows of %d and %d outputs",
              num_tokens, width, outputs);
     ST_CHECK(experts >= 1 && experts <= outputs, "moe_router_align: %d experts of %d outputs", experts, outputs);
-    ST_CHECK(tile == 16 || tile == 64 || tile == 128, "moe_align: tiles of 16, 64 or 128 places, not %d", tile);
-    const int num_pairs = num_tokens * top;
-    ST_CHECK(capacity % tile == 0 && capacity >= (num_pairs + tile - 1) / tile * tile + tile * experts,
-             "moe_align: %d places do not hold %d pairs of %d experts in tiles of %d", capacity, num_pairs, experts, tile);
+    if (const int rc = check_places(num_tokens * top, experts, capacity, tile)) return rc;
     ST_CHECK(ids && weights && sorted && place_of_pair && tile_expert && x && w, "moe_router_align: null operand");
     ST_CHECK((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "moe_router_align: rows are 16-byte aligned");
     const RouteRule r{token_item, correction, scale, outputs, top, mode, groups, keep};
@@ -1133,11 +1134,8 @@ extern "C" int st_moe_router_align(int* ids, float* weights, int* sorted, int* p
 
 extern "C" int st_moe_align(int* sorted, int* place_of_pair, int* tile_expert, const int* ids, int num_pairs,
                             int experts, int capacity, int tile, hipStream_t stream) {
-    const int kTile = tile;
     ST_CHECK(num_pairs >= 0 && experts > 0 && experts <= 4096, "moe_align: bad sizes (up to 4096 experts)");
-    ST_CHECK(tile == 16 || tile == 64 || tile == 128, "moe_align: tiles of 16, 64 or 128 places, not %d", tile);
-    ST_CHECK(capacity % kTile == 0 && capacity >= (num_pairs + kTile - 1) / kTile * kTile + kTile * experts,
-             "moe_align: %d places do not hold %d pairs of %d experts in tiles of %d", capacity, num_pairs, experts, kTile);
+    if (const int rc = check_places(num_pairs, experts, capacity, tile)) return rc;
     ST_CHECK(sorted && place_of_pair && tile_expert && ids, "moe_align: null operand");
     moe_align_kernel<<<1, 1024, (2 * experts + 1) * sizeof(int), stream>>>(sorted, place_of_pair, tile_expert, ids,
                                                                           num_pairs, experts, capacity, tile);
