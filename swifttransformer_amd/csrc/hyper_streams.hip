@@ -13,6 +13,8 @@
 #include "api.h"
 #include "common.h"
 
+#include <type_traits>
+
 namespace st {
 
 constexpr int kMaxStreams = 16;
@@ -108,11 +110,83 @@ __global__ __launch_bounds__(256) void streams_read_kernel(
                         eps, red);
 }
 
-// A row's first columns, y and the next norm's gains are asked for beside the mixing matrix, before anything is waited for, and few rows take as
-// many threads as have four columns each: what bounds them is trips to memory one after the other (8 rows of 4 streams of 2,048: with 256
-// threads and each load where it is used 5.4 us, so 4.8).
 template <typename T, int S, bool VEC>
-__global__ __launch_bounds__(1024) void streams_write_kernel(
+__global__ __launch_bounds__(256) void streams_write_kernel(
+    float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ mix, const float* __restrict__ b,
+    T* __restrict__ out_t, const float* __restrict__ a2, const float* __restrict__ gain2, int streams_rt, int width,
+    float eps2) {
+    const int streams = S ? S : streams_rt;
+    extern __shared__ float4 u4[];
+    float* u = reinterpret_cast<float*>(u4);
+    __shared__ float red[16];
+    __shared__ float s_mix[kMaxStreams * kMaxStreams], s_b[kMaxStreams], s_a2[kMaxStreams];
+    const int64_t row = blockIdx.x;
+    for (int i = threadIdx.x; i < streams * streams; i += 256) s_mix[i] = mix[i];
+    if ((int)threadIdx.x < streams) {
+        s_b[threadIdx.x] = b[threadIdx.x];
+        s_a2[threadIdx.x] = a2 ? a2[threadIdx.x] : 0.f;
+    }
+    __syncthreads();
+    float* xr = x + row * streams * width;
+    const float* yr = y + row * width;
+    float ss = 0.f;
+    if (VEC) {
+        for (int c = threadIdx.x * 4; c < width; c += 1024) {
+            float4 old[S ? S : kMaxStreams];
+#pragma unroll
+            for (int s = 0; s < streams; ++s) old[s] = *reinterpret_cast<const float4*>(xr + (int64_t)s * width + c);
+            const float4 yv = *reinterpret_cast<const float4*>(yr + c);
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int t = 0; t < streams; ++t) {
+                const float bt = s_b[t];
+                float4 nv = make_float4(bt * yv.x, bt * yv.y, bt * yv.z, bt * yv.w);
+#pragma unroll
+                for (int s = 0; s < streams; ++s) {
+                    const float m = s_mix[s * streams + t];
+                    nv.x = fmaf(m, old[s].x, nv.x); nv.y = fmaf(m, old[s].y, nv.y);
+                    nv.z = fmaf(m, old[s].z, nv.z); nv.w = fmaf(m, old[s].w, nv.w);
+                }
+                *reinterpret_cast<float4*>(xr + (int64_t)t * width + c) = nv;
+                const float at = s_a2[t];
+                v.x = fmaf(at, nv.x, v.x); v.y = fmaf(at, nv.y, v.y); v.z = fmaf(at, nv.z, v.z); v.w = fmaf(at, nv.w, v.w);
+            }
+            if (out_t) {
+                *reinterpret_cast<float4*>(u + c) = v;
+                ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
+            }
+        }
+    } else {
+        for (int c = threadIdx.x; c < width; c += 256) {
+            float old[S ? S : kMaxStreams];
+#pragma unroll
+            for (int s = 0; s < streams; ++s) old[s] = xr[(int64_t)s * width + c];
+            const float yv = yr[c];
+            float v = 0.f;
+#pragma unroll
+            for (int t = 0; t < streams; ++t) {
+                float nv = s_b[t] * yv;
+#pragma unroll
+                for (int s = 0; s < streams; ++s) nv = fmaf(s_mix[s * streams + t], old[s], nv);
+                xr[(int64_t)t * width + c] = nv;
+                v = fmaf(s_a2[t], nv, v);
+            }
+            if (out_t) {
+                u[c] = v;
+                ss = fmaf(v, v, ss);
+            }
+        }
+    }
+    if (out_t) finish_read<T, VEC>(out_t + row * width, nullptr, u, gain2, ss, width, eps2, red);
+}
+
+// Few rows of whole 16-byte pieces: as many threads as have four columns each, and a row's first columns, y and the next norm's gains are asked
+// for beside the mixing matrix, before anything is waited for: what bounds them is trips to memory one after the other (8 rows of 4
+// streams of 2,048 with the next read: with 256 threads and each load where it is used 4.1 us, so 3.5).  Not for six or eight streams, whose
+// numbers do not fit the registers of that many threads (8 rows of 8 streams of 2,048 5.2 us above, 8.2 so), nor for more rows than
+// compute units (300 rows of one stream of 4,096 5.3 and 5.7, of four 9.7 either way).
+template <typename T, int S>
+__global__ __launch_bounds__(1024) void streams_write_few_kernel(
     float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ mix, const float* __restrict__ b,
     T* __restrict__ out_t, const float* __restrict__ a2, const float* __restrict__ gain2, int streams_rt, int width,
     float eps2) {
@@ -135,7 +209,7 @@ __global__ __launch_bounds__(1024) void streams_write_kernel(
         yv = *reinterpret_cast<const float4*>(yr + c);
         if (out_t && gain2) gain = *reinterpret_cast<const float4*>(gain2 + c);
     };
-    if (VEC && tid * 4 < width) load(tid * 4);
+    if (tid * 4 < width) load(tid * 4);
     if (tid < streams * streams) s_mix[tid] = own_mix;
     if (tid < streams) {
         s_b[tid] = own_b;
@@ -143,62 +217,37 @@ __global__ __launch_bounds__(1024) void streams_write_kernel(
     }
     __syncthreads();
     float ss = 0.f;
-    if (VEC) {
-        for (int c = tid * 4; c < width; c += blockDim.x * 4) {
-            if (c != tid * 4) load(c);
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int c = tid * 4; c < width; c += blockDim.x * 4) {
+        if (c != tid * 4) load(c);
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-            for (int t = 0; t < streams; ++t) {
-                const float bt = s_b[t];
-                float4 nv = make_float4(bt * yv.x, bt * yv.y, bt * yv.z, bt * yv.w);
+        for (int t = 0; t < streams; ++t) {
+            const float bt = s_b[t];
+            float4 nv = make_float4(bt * yv.x, bt * yv.y, bt * yv.z, bt * yv.w);
 #pragma unroll
-                for (int s = 0; s < streams; ++s) {
-                    const float m = s_mix[s * streams + t];
-                    nv.x = fmaf(m, old[s].x, nv.x); nv.y = fmaf(m, old[s].y, nv.y);
-                    nv.z = fmaf(m, old[s].z, nv.z); nv.w = fmaf(m, old[s].w, nv.w);
-                }
-                *reinterpret_cast<float4*>(xr + (int64_t)t * width + c) = nv;
-                const float at = s_a2[t];
-                v.x = fmaf(at, nv.x, v.x); v.y = fmaf(at, nv.y, v.y); v.z = fmaf(at, nv.z, v.z); v.w = fmaf(at, nv.w, v.w);
+            for (int s = 0; s < streams; ++s) {
+                const float m = s_mix[s * streams + t];
+                nv.x = fmaf(m, old[s].x, nv.x); nv.y = fmaf(m, old[s].y, nv.y);
+                nv.z = fmaf(m, old[s].z, nv.z); nv.w = fmaf(m, old[s].w, nv.w);
             }
-            if (out_t) {
-                *reinterpret_cast<float4*>(u + c) = v;
-                ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
-            }
+            *reinterpret_cast<float4*>(xr + (int64_t)t * width + c) = nv;
+            const float at = s_a2[t];
+            v.x = fmaf(at, nv.x, v.x); v.y = fmaf(at, nv.y, v.y); v.z = fmaf(at, nv.z, v.z); v.w = fmaf(at, nv.w, v.w);
         }
         if (out_t) {
-            const float n = block_sum(ss, red), r = eps2 > 0.f ? 1.f / sqrtf(n / (float)width + eps2) : 1.f;
-            for (int c = tid * 4; c < width; c += blockDim.x * 4) {
-                const float4 uv = *reinterpret_cast<const float4*>(u + c);
-                if (gain2 && width > (int)blockDim.x * 4) gain = *reinterpret_cast<const float4*>(gain2 + c);
-                const float v[4] = {uv.x * r * gain.x, uv.y * r * gain.y, uv.z * r * gain.z, uv.w * r * gain.w};
-                Elem<T>::store4(out_t + row * width + c, v);
-            }
-        }
-        return;
-    }
-    {
-        for (int c = threadIdx.x; c < width; c += 256) {
-            float old[S ? S : kMaxStreams];
-#pragma unroll
-            for (int s = 0; s < streams; ++s) old[s] = xr[(int64_t)s * width + c];
-            const float yv = yr[c];
-            float v = 0.f;
-#pragma unroll
-            for (int t = 0; t < streams; ++t) {
-                float nv = s_b[t] * yv;
-#pragma unroll
-                for (int s = 0; s < streams; ++s) nv = fmaf(s_mix[s * streams + t], old[s], nv);
-                xr[(int64_t)t * width + c] = nv;
-                v = fmaf(s_a2[t], nv, v);
-            }
-            if (out_t) {
-                u[c] = v;
-                ss = fmaf(v, v, ss);
-            }
+            *reinterpret_cast<float4*>(u + c) = v;
+            ss = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, ss))));
         }
     }
-    if (out_t) finish_read<T, VEC>(out_t + row * width, nullptr, u, gain2, ss, width, eps2, red);
+    if (out_t) {
+        const float n = block_sum(ss, red), r = eps2 > 0.f ? 1.f / sqrtf(n / (float)width + eps2) : 1.f;
+        for (int c = tid * 4; c < width; c += blockDim.x * 4) {
+            const float4 uv = *reinterpret_cast<const float4*>(u + c);
+            if (gain2 && width > (int)blockDim.x * 4) gain = *reinterpret_cast<const float4*>(gain2 + c);
+            const float v[4] = {uv.x * r * gain.x, uv.y * r * gain.y, uv.z * r * gain.z, uv.w * r * gain.w};
+            Elem<T>::store4(out_t + row * width + c, v);
+        }
+    }
 }
 
 }  // namespace st
@@ -278,21 +327,26 @@ extern "C" int st_streams_write(float* x, const float* y, const float* mix, cons
     ST_CHECK(!out_t || a2, "streams_write: a following read needs its weights");
     const size_t lds = out_t ? (size_t)width * 4 : 0;
     ST_CHECK(dtype == kF32 || dtype == kBF16, "streams_write: unknown dtype %d", dtype);
-#define ST_WRITE_V(S, V)                                                                                                 \
-    do {                                                                                                             \
-        if (dtype == kF32)                                                                                           \
-            streams_write_kernel<float, S, V><<<num_rows, threads, lds, stream>>>(x, y, mix, b, (float*)out_t, a2, gain2, \
-                                                                              streams, width, eps2);                 \
-        else                                                                                                         \
-            streams_write_kernel<bf16_t, S, V><<<num_rows, threads, lds, stream>>>(x, y, mix, b, (bf16_t*)out_t, a2,      \
-                                                                               gain2, streams, width, eps2);         \
-    } while (0)
     const bool vec = width % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) |
                                          reinterpret_cast<uintptr_t>(out_t) | reinterpret_cast<uintptr_t>(gain2)) & 15) == 0;
-    // (more rows than compute units fill the chip with 256 threads each)
-    const int columns = (width / 4 + 255) / 256 * 256;
-    const int threads = !vec || num_rows > device_compute_units() ? 256 : columns < 1024 ? columns : 1024;
-#define ST_WRITE(S) do { if (vec) ST_WRITE_V(S, true); else ST_WRITE_V(S, false); } while (0)
+    const int columns = (width / 4 + 255) / 256 * 256, threads = columns < 1024 ? columns : 1024;
+    const bool few = vec && num_rows <= device_compute_units();
+    const auto launch = [&](auto known, auto* out) {
+        constexpr int S = decltype(known)::value;
+        using T = std::remove_pointer_t<decltype(out)>;
+        const auto run = [&](auto kernel, int count) {
+            kernel<<<num_rows, count, lds, stream>>>(x, y, mix, b, out, a2, gain2, streams, width, eps2);
+        };
+        if constexpr (S <= 4)
+            if (few) return run(streams_write_few_kernel<T, S>, threads);
+        if (vec) run(streams_write_kernel<T, S, true>, 256);
+        else run(streams_write_kernel<T, S, false>, 256);
+    };
+#define ST_WRITE(S)                                                                                                  \
+    do {                                                                                                             \
+        if (dtype == kF32) launch(std::integral_constant<int, S>(), (float*)out_t);                                  \
+        else launch(std::integral_constant<int, S>(), (bf16_t*)out_t);                                               \
+    } while (0)
     switch (streams) {
         case 1: ST_WRITE(1); break;
         case 2: ST_WRITE(2); break;
@@ -303,7 +357,6 @@ extern "C" int st_streams_write(float* x, const float* y, const float* mix, cons
         default: ST_WRITE(0); break;
     }
 #undef ST_WRITE
-#undef ST_WRITE_V
     ST_LAUNCH_CHECK("streams_write");
     return 0;
 }

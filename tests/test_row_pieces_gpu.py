@@ -120,7 +120,7 @@ def test_normed_queries_and_keys_in_pieces(dtype, heads, kv_heads, hd):
     assert torch.equal(res[0][2], res[1][2])
 
 
-@pytest.mark.parametrize("streams", [1, 4, 5])
+@pytest.mark.parametrize("streams", [1, 4, 5, 6, 8])        # (six and eight with 256 threads whatever the rows)
 @pytest.mark.parametrize("rows,width", [(1, 4), (3, 1028), (2, 2048), (2, 8196), (300, 516)])
 def test_streams_written_by_as_many_threads_as_columns(streams, rows, width):
     from swifttransformer_amd.ops import kernels as K
