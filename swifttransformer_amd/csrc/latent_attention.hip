@@ -138,8 +138,8 @@ __device__ inline float hi_half(uint32_t w) { return __uint_as_float(w & 0xffff0
 // HDP: 32-wide steps over the entry; QT: subtiles of 16 rows a wave; NKT: 16-key subtiles of a block; RW: waves over the
 // rows; KW: groups of RW waves, each with its own share of the key blocks and its own LDS, merged at the end.  FS: the normaliser sums
 // the weights as they are (float, a lane's own keys), else as they are rounded for the product (one more row of the product).  What was
-// attention in a kernel that sums floats keeps them: entries of 160, 1,024 tokens of 32 heads 42.8 us, rounded 39.6, off float64 by 1.91e-3
-// and 1.90e-3.
+// attention in a kernel that sums floats keeps them: entries of 160, 1,024 tokens of 32 heads 41.1 us, rounded 38.1, off float64 by 1.913e-3
+// and 1.900e-3 (the kernel before 56.3 us, 1.901e-3).
 template <bool TILES, int HDP, int QT, int NKT, int RW, int KW, bool FS>
 __global__ __launch_bounds__(64 * RW * KW) void latent_attn_kernel(const LatentArgs a) {
     constexpr int CH = 4 * HDP, ROWB = CH * 16, DK = 16 * NKT, DT = 2 * HDP, ROWS = RW * QT * 16, BUF = DK * ROWB;

@@ -46,11 +46,13 @@ class Tuning:
     gla_part_dim_decode: int = 16
     gla_part_dim_prompt: int = 8
     # Pairs an expert from which bfloat16 experts go in tiles of 64 and of 128 places through LDS instead of 16 (csrc/moe.hip).  All
-    # kernels of a call with tiles of 16 / 64 / 128 places, us: 64 experts of 2,048 x 1,024, four a token, 189 / 177 / 182 at 6 pairs an
-    # expert, 371 / 212 / 221 at 31, 1,088 / 265 / 245 at 100, 1,195 / 278 / 279 at 112; 8 of 4,096 x 4,096, two a token, 177 / 168 / 175
-    # at 6, 437 / 174 / 182 at 31, 1,061 / 266 / 230 at 100, 1,148 / 271 / 232 at 112; up and down alone of 16 of 2,048 x 2,048, two a
-    # token, 79 / 89 / 93 at 6, 112 / 93 / 98 at 12, 361 / 122 / 135 at 64, - / 137 / 137 at 112, - / 144 / 135 at 128.  How tokens spread
-    # over experts moves the lines: tiles of 64 win from 4 to 12 pairs on, of 128 from 100 to 128.
+    # kernels of a call with tiles of 16 / 64 / 128 places, us: 64 experts of 2,048 x 1,024, four a token, 188 / 171 / 177 at 6 pairs an
+    # expert, 374 / 182 / 188 at 31, 1,092 / 258 / 226 at 100, 1,173 / 276 / 265 at 112; 8 of 4,096 x 4,096, two a token, 181 / 176 / 204
+    # at 6, 445 / 180 / 205 at 31, 1,105 / 231 / 221 at 100, 1,138 / 274 / 271 at 112; 16 of 2,048 x 2,048, two a token, 100 / 94 / 109 at
+    # 6, 376 / 124 / 116 at 64, 592 / 129 / 123 at 112, - / 197 / 166 at 200; of 1,024 x 1,024 37 / 36 / 45 at 6, 164 / 47 / 57 at 112, - / 70 / 63
+    # at 200; of 768 x 768 30 / 31 / 35 at 6, 106 / 42 / 47 at 112, - / 56 / 52 at 200; 8 of 768 x 768 23 / 28 / 33 at 6, 29 / 30 / 34 at 20, 61 /
+    # 32 / 42 at 112, - / 39 / 44 at 200.  How large the matrices are moves the lines: tiles of 64 win from 4 to 20 pairs on, of 128 from 64 to
+    # 200 and more.
     moe_staged_64_pairs: int = 7
     moe_staged_128_pairs: int = 112
     # Window attention of bfloat16 rows goes by tiles of 16 rows from so many rows of a step on (csrc/sink_tiles.hip), by rows below.

@@ -29,7 +29,8 @@ def test_tiles_of_latent_entries(heads, entry, window, start, tokens):
     s = torch.matmul(q.view(tokens, heads, entry).to(F64).transpose(0, 1), keys.T) * scale
     p = torch.softmax(s.masked_fill(~seen[None], float("-inf")), -1)
     want, size = torch.matmul(p, keys).transpose(0, 1), torch.matmul(p, keys.abs()).transpose(0, 1)
-    # weights are rounded to bfloat16 before they meet the entries and are summed as rounded (2^-9 each way), the result once (2^-9)
+    # weights are rounded to bfloat16 before they meet the entries (by 2^-8 at most) and summed as rounded, which takes the mean of their
+    # errors out again; the result is rounded once (2^-8)
     err = (out.view(tokens, heads, entry).to(F64) - want).abs()
     assert bool((err <= 2.0 ** -8 * size + 2.0 ** -8 * want.abs() + 1e-4).all()), float((err / size).max())
 
