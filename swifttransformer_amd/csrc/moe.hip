@@ -675,8 +675,8 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 // With some dozens of rows and more an expert a tile of 64 NJ places meets 64 WN rows of its expert's matrix, steps of 64 in depth.
 // Both operand tiles go from memory into LDS without passing through registers (16 bytes a lane; a row's chunks are rotated by
 // the lane's choice of address, so that the matrix instruction's reads spread over the banks), the AHEAD steps (1 or 2) after the one that is
-// multiplied on their way into the other buffers: one barrier a step, before which a wave waits for its loads of that step
-// alone.  Each of 2 WN waves multiplies a 64 x 32 NJ part (v_mfma_f32_32x32x16_bf16), the operands of a product of depth 16 read ahead
+// multiplied on their way into the other buffers: one barrier a step, before the last quarter of the step's products, whose operands are read
+// by then; a wave waits there for its loads of the next step alone, and that step's first operands are read under the quarter that is left.  Each of 2 WN waves multiplies a 64 x 32 NJ part (v_mfma_f32_32x32x16_bf16), the operands of a product of depth 16 read ahead
 // of the one before; the two waves that share weight rows take the tile's blocks of 32 places in turn, and a block without a pair
 // (an expert's last tile) is not multiplied.
 // UP: of every 64 weight rows 32 are inner features of the gate matrix and 32 the same features of the other one, so that a
@@ -693,7 +693,11 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 // Measured on weights that no cache holds, up + down, beside the kernel before it (128 rows, the next step's loads alone on their way,
 // all beginning at depth 0): 16 experts of 2,048 x 2,048, two a token, 2,011 tokens 220 -> 204 us, 1,024 tokens 145 -> 128, 753 tokens
 // (tiles of 64) 138 -> 127, 128 tokens 106 -> 81; 14 experts of 4,096 x 4,096, 2,048 tokens 663 -> 613, 951 tokens 430 -> 390.  Tiles of
-// 64 on 256 rows: 145 us at 753 tokens.  Tried and no better: 256 places a tile (at 753 tokens 187 us), two buffers for 256 rows (156),
+// 64 on 256 rows: 145 us at 753 tokens.  With the meeting before a step's last quarter instead of between two steps: 2,011 tokens
+// 219 -> 205 us, 1,024 tokens 129 -> 123; 4,096 x 4,096, 2,048 tokens 656 -> 619, 951 tokens 395 -> 386; tiles of 64 within 2 %.
+// (2,011 tokens before: 153 us with the loads taken out, 176 with the products taken out; 205 on matrices stored in the order of the tiles.)
+// Tried and no better: 256 places a tile (at 753 tokens 187 us; as the loop is now 195 to 199 at 2,011, 173 at 753, 413 at 951 of 4,096),
+// 128 weight rows on 256 places (220 at 2,011), four waves with 128 weight rows each (206), two buffers for 256 rows (156),
 // four and five for 128 rows, workgroups that stay and take the next item while the last one's results are stored (no gain), loads of
 // one word a line that bring the weights into L2 two steps earlier (+ 25 %), streaming loads (twice as slow where tiles share weights).
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -811,52 +815,70 @@ __global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 
 #pragma unroll
                 for (int q = 0; q < 16; ++q) total[a][j][q] = 0.0;
     bf16x8 a[2][2], b[2][NJ];
-    auto fetch = [&](auto blocks32, int cur, int kk) {              // the operands of a product of depth 16
-        const uint4* at = own + cur * BUF + ((kk * 2 + lh) ^ swz);
+    auto walk = [&](auto blocks32) {                                // over the depth; the wave's blocks of 32 places that hold a pair
+        constexpr int B = decltype(blocks32)::value;
+        auto fetch = [&](int cur, int kk) {                         // the operands of a product of depth 16
+            if constexpr (B > 0) {
+                const uint4* at = own + cur * BUF + ((kk * 2 + lh) ^ swz);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) a[kk & 1][q] = __builtin_bit_cast(bf16x8, at[(wn * 64 + q * 32) * 8]);
+                for (int q = 0; q < 2; ++q) a[kk & 1][q] = __builtin_bit_cast(bf16x8, at[(wn * 64 + q * 32) * 8]);
 #pragma unroll
-        for (int j = 0; j < decltype(blocks32)::value; ++j) b[kk & 1][j] = __builtin_bit_cast(bf16x8, at[(ROWS + (j * 2 + wm) * 32) * 8]);
-    };
-    auto multiply = [&](auto blocks32, int cur) {
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            if (kk < 3) fetch(blocks32, cur, kk + 1);
+                for (int j = 0; j < B; ++j) b[kk & 1][j] = __builtin_bit_cast(bf16x8, at[(ROWS + (j * 2 + wm) * 32) * 8]);
+            }
+        };
+        auto multiply = [&](int kk) {
             __builtin_amdgcn_sched_barrier(0);     // (the next operands are on their way before these are multiplied)
 #pragma unroll
             for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int j = 0; j < decltype(blocks32)::value; ++j)
+                for (int j = 0; j < B; ++j)
                     acc[q][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kk & 1][q], b[kk & 1][j], acc[q][j], 0, 0, 0);
+        };
+        // This wave's loads of step s have landed, those of the AHEAD - 1 steps after it may be on their way, and its reads of the step
+        // before are done; then everyone's are, and that step's buffer may be filled again.
+        auto meet = [&](int s) {
+            if (s + AHEAD > steps) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((AHEAD - 1) * NL) : "memory");
+        };
+        stage(0, 0);
+        if (AHEAD > 1 && steps > 1) stage(1, 1);
+        meet(0);
+        fetch(0, 0);
+        if (AHEAD < steps) stage(AHEAD, AHEAD);
+        for (int s = 0, cur = 0; s < steps; ++s) {
+            const int next = cur == AHEAD ? 0 : cur + 1;
+#pragma unroll
+            for (int kk = 0; kk < 3; ++kk) {
+                fetch(cur, kk + 1);
+                multiply(kk);
+            }
+            // the waves meet before the step's last products, whose operands are in registers: those cover the way to the next step's first
+            if (s + 1 < steps) {
+                __builtin_amdgcn_sched_barrier(0);
+                meet(s + 1);
+                fetch(next, 0);
+                if (s + 1 + AHEAD < steps) stage(s + 1 + AHEAD, cur);
+            }
+            multiply(3);
+            cur = next;
+            if constexpr (DOUBLE)
+                if (++since == per || s + 1 == steps) {
+                    since = 0;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                            for (int u = 0; u < 16; ++u) {
+                                total[q][j][u] += (double)acc[q][j][u];
+                                acc[q][j][u] = s + 1 == steps ? (float)total[q][j][u] : 0.f;
+                            }
+                }
         }
     };
-    stage(0, 0);
-    if (AHEAD > 1 && steps > 1) stage(1, 1);
-    for (int s = 0, cur = 0; s < steps; ++s) {
-        // This wave's loads of the step have landed, those of the steps after it may be on their way; then everyone's have, and the
-        // buffer of the step before has been read.
-        if (s + AHEAD > steps) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((AHEAD - 1) * NL) : "memory");
-        if (full == NJ) fetch(Steps<NJ>(), cur, 0);
-        else if (NJ > 1 && full > 0) fetch(Steps<1>(), cur, 0);
-        if (s + AHEAD < steps) stage(s + AHEAD, cur == 0 ? AHEAD : cur - 1);
-        if (full == NJ) multiply(Steps<NJ>(), cur);
-        else if (NJ > 1 && full > 0) multiply(Steps<1>(), cur);
-        cur = cur == AHEAD ? 0 : cur + 1;
-        if constexpr (DOUBLE)
-            if (++since == per || s + 1 == steps) {
-                since = 0;
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-                        for (int u = 0; u < 16; ++u) {
-                            total[q][j][u] += (double)acc[q][j][u];
-                            acc[q][j][u] = s + 1 == steps ? (float)total[q][j][u] : 0.f;
-                        }
-            }
-    }
+    if (full == NJ) walk(Steps<NJ>());
+    else if (NJ > 1 && full > 0) walk(Steps<1>());
+    else walk(Steps<0>());
     // acc[q][j][u]: weight row wn * 64 + q * 32 + 8 * (u / 4) + 4 * lh + u % 4, place base + (2 * j + wm) * 32 + l32
     auto store_row = [&](int place, int f, const float* r) {
         bf16_t* dst = y_out + (int64_t)place * N + f;
