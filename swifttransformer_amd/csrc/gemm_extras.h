@@ -62,6 +62,9 @@ extern "C" struct StGemmExtras {
     float out_scale;
     // != 0: the bias is added after the factor, out = residual + out_scale * x W^T + bias (no activation)
     int bias_unscaled;
+    // float products: room for partial sums (st_gemm_scratch floats make the best split of them), or null
+    float* scratch;
+    int64_t scratch_floats;
 };
 
 namespace st {

@@ -4,6 +4,7 @@ is no alternative implementation behind these functions."""
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional, Tuple
 
@@ -53,6 +54,7 @@ def _lib():
         lib.st_gemm_can_fuse_norm.argtypes = [_c_int, _c_int, _c_int, _c_int]
         lib.st_gemm_wide_offered.argtypes = [_c_int, _c_int, _c_int, _c_int]
         lib.st_gemm_can_fuse_merge.argtypes = [_c_int] * 7
+        lib.st_gemm_scratch.argtypes, lib.st_gemm_scratch.restype = [_c_int] * 4, _c_i64
         lib.st_gemm_library_tuning.argtypes = [_c_int]
         lib.st_attn_rows_gated.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_p,
                                            _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_f,
@@ -323,7 +325,7 @@ class _GemmExtras(ctypes.Structure):
                 ("mg_o", _c_p), ("mg_lse", _c_p), ("mg_splits", _c_int), ("mg_heads", _c_int),
                 ("mg_head_dim", _c_int), ("_pad2", _c_int),
                 ("ln_rows", _c_p), ("best_ids", _c_p), ("best_val", _c_p), ("best_idx", _c_p),
-                ("out_scale", _c_f), ("bias_unscaled", _c_int)]
+                ("out_scale", _c_f), ("bias_unscaled", _c_int), ("scratch", _c_p), ("scratch_floats", _c_i64)]
 
 
 class KvScatter:
@@ -417,6 +419,14 @@ def wide_offered(M: int, N: int, K: int, dtype: torch.dtype) -> bool:
     rows and a very wide matrix (an output head): the kernel that takes a ``NormInput`` with a row
     index and fills ``best``."""
     return bool(_lib().st_gemm_wide_offered(M, N, K, dtype_code(dtype)))
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_scratch(M: int, N: int, K: int, code: int, most: bool) -> int:
+    """Floats of scratch that a product of M rows asks for; ``most``: that one of any number of rows up to M may ask for (it
+    depends on the tiles of 128 rows)."""
+    of = list(range(128, M, 128)) + [M] if most else [M]
+    return max(_lib().st_gemm_scratch(m, N, K, code) for m in of)
 
 
 # functions of the products' epilogues and of ``activation_multiply``, by the C interface's number
@@ -531,6 +541,13 @@ def gemm(x, w: torch.Tensor, *, bias: Optional[torch.Tensor] = None,
         idx = empty((n_scratch,), torch.int32, device)
         keep += [val, idx]
         ex.best_ids, ex.best_val, ex.best_idx = _ptr(best), _ptr(val), _ptr(idx)
+    scratch = _gemm_scratch(M, N, K, code, arena.measuring()) if code == F32 and M and algo in (0, 3) else 0
+    if scratch:
+        if ex is None:
+            ex = _GemmExtras()
+        room = empty((scratch,), torch.float32, device)
+        keep.append(room)
+        ex.scratch, ex.scratch_floats = _ptr(room), scratch
     if float(out_scale) != 1.0:
         if ex is None:
             ex = _GemmExtras()

@@ -1,0 +1,138 @@
+"""Float products on the bfloat16 matrix cores (csrc/gemm_f32.hip) against float64.
+
+Bound of an element's error: every 32 in depth take 2 x 6 roundings of a running sum in each of two chains, and what is left of
+the depth one a number; a rounding is at most 2^-24 of a sum that never exceeds S = sum |x| |w|; the products left out are at most
+2^-23 of S; the merge of chains and splits, bias, residual and factor add a dozen more."""
+import pytest
+import torch
+
+from swifttransformer_amd.ops import arena
+from swifttransformer_amd.ops import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(M, N, D, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed + M * 7 + N * 3 + D)
+    x = torch.empty(M, D, device="cuda").normal_(0, 1, generator=g)
+    w = torch.empty(N, D, device="cuda").normal_(0, 0.05, generator=g)
+    return x, w, g
+
+
+def check(y, x, w, bias=None, residual=None, scale=1.0, extra=0.0):
+    ref = x.double() @ w.double().T
+    size = x.double().abs() @ w.double().abs().T
+    if bias is not None:
+        ref, size = ref + bias.double(), size + bias.double().abs()
+    ref, size = ref * scale, size * abs(scale)
+    if residual is not None:
+        ref, size = ref + residual.double(), size + residual.double().abs()
+    D = x.shape[1]
+    roundings = 6 * (D // 32) * 2 / 2 + D % 32 + 12
+    bound = (roundings * 2.0 ** -24 + 2.0 ** -23) * size
+    over = ((y.double() - ref).abs() > bound + extra)
+    assert not bool(over.any()), float(((y.double() - ref).abs() / bound).max())
+
+
+# edges of the 128 x 128 tiles, depths that are no whole steps of 32, tiles in whole rounds, split ones and both (256 compute units)
+@pytest.mark.parametrize("M,N,D", [(1, 4, 4), (3, 12, 28), (127, 132, 32), (128, 128, 36), (129, 124, 64), (200, 260, 100), (96, 512, 96),
+                                   (257, 1028, 516), (701, 6144, 512), (1000, 4100, 1000), (130, 2048, 4096)])
+def test_shapes(M, N, D):
+    x, w, g = operands(M, N, D)
+    bias = torch.empty(N, device="cuda").normal_(0, 1, generator=g)
+    check(K.gemm(x, w, algo=3), x, w)
+    check(K.gemm(x, w, bias=bias, algo=3), x, w, bias=bias)
+
+
+def test_chosen_and_closer_than_the_library():
+    """The rule sends a prompt's product here; it is closer to float64 than the library's float product."""
+    x, w, _ = operands(701, 2048, 2048)
+    assert K._gemm_scratch(701, 2048, 2048, 0, False) > 0 and K._gemm_scratch(64, 2048, 2048, 0, False) == 0
+    ref = x.double() @ w.double().T
+    own, lib = K.gemm(x, w), K.gemm(x, w, algo=2)
+    assert torch.equal(own, K.gemm(x, w, algo=3)) and torch.equal(own, K.gemm(x, w))
+    assert float((own - ref).norm()) < float((lib - ref).norm())
+
+
+def test_most_scratch_of_smaller_steps():
+    assert K._gemm_scratch(1024, 2048, 2048, 0, True) >= max(K._gemm_scratch(m, 2048, 2048, 0, False) for m in range(1, 1025))
+    assert not arena.measuring()
+
+
+@pytest.mark.parametrize("M,N", [(300, 256), (701, 2048)])
+def test_epilogues(M, N):
+    x, w, g = operands(M, N, 512)
+    bias = torch.empty(N, device="cuda").normal_(0, 1, generator=g)
+    residual = torch.empty(M, N, device="cuda").normal_(0, 1, generator=g)
+    plain = K.gemm(x, w, algo=3)
+    check(K.gemm(x, w, bias=bias, residual=residual, out_scale=0.5, algo=3), x, w, bias, residual, 0.5)
+    check(K.gemm(x, w, residual=residual, algo=3), x, w, residual=residual)
+    assert torch.equal(K.gemm(x, w, activation="relu", algo=3), plain.clamp(min=0))
+    y = K.gemm(x, w, bias=bias, activation="gelu", algo=3)
+    z = x.double() @ w.double().T + bias.double()
+    want = 0.5 * z * (1 + torch.erf(z / 2 ** 0.5))
+    assert float((y - want).abs().max()) <= 1e-5 * float(z.abs().max())
+    unscaled = K.gemm(x, w, bias=bias, out_scale=0.5, bias_unscaled=True, algo=3)
+    check(unscaled, x, w * 0.5, bias=bias)
+
+
+@pytest.mark.parametrize("M", [130, 701])
+def test_pages(M):
+    """A fused query, key and value product writes its pages as the library's product and the page write do."""
+    heads, hd, page, D = 4, 32, 8, 256
+    N = 3 * heads * hd
+    x, w, _ = operands(M, N, D)
+    pages = -(-M // page) + 2
+    table = torch.randperm(pages, device="cuda").int()[None].contiguous()
+    item = torch.zeros(M, dtype=torch.int32, device="cuda")
+    item[5] = -1                                                    # a padding row
+    pos = torch.arange(M, dtype=torch.int32, device="cuda")
+    made = []
+    for algo in (2, 3):
+        kc, vc = (torch.zeros(pages, heads, page, hd, device="cuda") for _ in range(2))
+        y = K.gemm(x, w, algo=algo, kv_scatter=K.KvScatter(kc, vc, item, pos, table, heads * hd))
+        made.append((y, kc, vc))
+    check(made[1][0], x, w)
+    at = (table[0].long()[pos.long() // page], pos.long() % page)
+    rows = torch.arange(M, device="cuda") != 5
+    for c, part in ((made[1][1], made[1][0][:, heads * hd:2 * heads * hd]), (made[1][2], made[1][0][:, 2 * heads * hd:])):
+        assert torch.equal(c[at[0], :, at[1]].reshape(M, -1)[rows], part[rows])
+        assert bool((c[at[0][5], :, at[1][5]] == 0).all())
+    assert torch.equal(made[0][1] != 0, made[1][1] != 0)
+
+
+def test_numbers_that_parts_do_not_hold():
+    """Infinities, NaN, numbers past bfloat16's largest and tiny ones give what float products give, and other rows are as without."""
+    M, N, D = 300, 256, 200
+    x, w, _ = operands(M, N, D)
+    clean = K.gemm(x, w, algo=3)
+    inf, big = float("inf"), 3.4e38
+    x[3, 7], x[70, 0], x[140, 199], x[200, 5] = inf, -inf, float("nan"), big
+    w[9, 5] = 0.0
+    x[250] *= 2.0 ** -120
+    y = K.gemm(x, w, algo=3)
+    ref = x.double() @ w.double().T
+    for r in (3, 70):
+        assert torch.equal(y[r], ref[r].float())
+    assert bool(torch.isnan(y[140]).all())
+    held = ref[200].abs() < 3e38
+    size = x[200].double().abs() @ w.double().abs().T
+    assert bool(((y[200].double() - ref[200]).abs()[held] <= 2.0 ** -20 * size[held]).all())
+    size = x[250].double().abs() @ w.double().abs().T
+    assert bool(((y[250].double() - ref[250]).abs() <= 2.0 ** -16 * size + 2.0 ** -140).all())
+    rows = torch.ones(M, dtype=torch.bool, device="cuda")
+    rows[[3, 70, 140, 200, 250]] = False
+    keep = torch.ones(N, dtype=torch.bool, device="cuda")
+    keep[9] = False
+    check(y[rows], x[rows], w)
+    assert bool(torch.isfinite(clean).all())
+
+
+def test_rows_off_16_bytes_go_to_the_library():
+    buf, _, _ = operands(1, 1, 701 * 2048 + 1)
+    w = operands(4, 2048, 2048)[1]
+    x = buf[0, 1:].view(701, 2048)
+    assert x.data_ptr() % 16 == 4
+    before = K.gemm_path_counts()["library"]
+    check(K.gemm(x, w), x, w)
+    assert K.gemm_path_counts()["library"] == before + 1
