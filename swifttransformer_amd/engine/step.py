@@ -12,7 +12,7 @@ Steps are launch-bound below some hundreds of tokens: some two hundred kernels w
 launches cost the host more than they cost the device.  A step is therefore recorded
 once per shape as a HIP graph over fixed index buffers and replayed; the kernels and
 the cache are the same as in the unrecorded path.  Steps of single tokens (decoding)
-are recorded per batch-size bucket at their first use; steps of any other composition
+are recorded per batch-size bucket, for short contexts and for all, at their first use; steps of any other composition
 (prompt portions, alone or beside decode tokens) per (padded token count, lengths of the
 parts' work lists) once that shape has come up ``record_after`` times; their final norm
 and head run after the replay on the rows that are wanted, so the number of wanted rows
@@ -101,7 +101,8 @@ class ModelRunner:
         self.cache = DeviceCache(self.manager, model.dtype, self.device, fill=cache_fill)
         self.paged_group_ids = [g.index for g in self.manager.paged_groups]
         self.steps_run = 0
-        self._recorded: Dict[int, _RecordedStep] = {}
+        self._recorded_spans: Dict[Tuple[int, int], _RecordedStep] = {}      # by rows and longest context
+        self._recorded: Dict[int, _RecordedStep] = {}                        # of these the last one used, by rows
         self._recorded_general: Dict[tuple, _RecordedStep] = {}
         self._seen: Dict[tuple, int] = {}
         self.record_after = int(tuning.record_after if record_after is None else record_after)
@@ -172,7 +173,7 @@ class ModelRunner:
         call it while the pool is free.  Returns the number of recordings made."""
         if not self.use_graphs:
             return 0
-        before = len(self._recorded) + len(self._recorded_general)
+        before = len(self._recorded_spans) + len(self._recorded_general)
         keep, self.record_after = self.record_after, 1
         try:
             for n in prompt_tokens:
@@ -193,13 +194,14 @@ class ModelRunner:
                         self.admit(r)
                         done.append(r)
                     self.step([StepEntry(r, [0], [0]) for r in ids])
+                    self._decode_step(b, self.model.max_positions)       # (that one was for short contexts, where there is one)
                 finally:
                     for r in done:
                         self.finish(r)
         finally:
             self.record_after = keep
         torch.cuda.synchronize(self.device)
-        return len(self._recorded) + len(self._recorded_general) - before
+        return len(self._recorded_spans) + len(self._recorded_general) - before
 
     # --------------------------------------------------------------------- step
     def item(self, req_id: Hashable, start: int, tokens: Sequence[int], want: Sequence[int]) -> StepItem:
@@ -282,16 +284,29 @@ class ModelRunner:
             b <<= 1
         return min(b, self.cache_param.max_seqs)
 
-    def _record(self, capacity: int) -> _RecordedStep:
+    def _decode_span(self, longest: int) -> int:
+        """The longest context that the recorded step of requests with contexts of up to ``longest`` tokens is made for:
+        ``tuning.short_span`` or all that the model allows.  The parts shape their attention by it (``ctx.max_kv_len``)."""
+        short = tuning.short_span
+        return short if self.paged_group_ids and longest <= short < self.model.max_positions else self.model.max_positions
+
+    def _decode_step(self, n: int, longest: int) -> _RecordedStep:
+        """The recorded step of ``n`` single tokens whose contexts, the tokens included, are up to ``longest`` long."""
+        cap, span = self._bucket(n), self._decode_span(longest)
+        rec = self._recorded_spans.get((cap, span))
+        if rec is None:
+            rec = self._recorded_spans[cap, span] = self._record(cap, span)
+        self._recorded[cap] = rec
+        return rec
+
+    def _record(self, capacity: int, span: int) -> _RecordedStep:
         buffers = DecodeBuffers(capacity, self.paged_group_ids, self.max_pages_per_seq,
-                                self.cache_param.page_size, self.device, self.model.max_positions)
+                                self.cache_param.page_size, self.device, span)
         # one unrecorded run on padding rows first: loads code objects, sizes the allocator, and
         # has the library's products of this row count timed and chosen
         # The rows' best tokens are left where the next step's token ids are read: a step that
         # decodes greedily from what the step before it chose needs no copy between the two.
-        rec = self._capture(buffers, tune=True, best=buffers.ctx.token_ids)
-        self._recorded[capacity] = rec
-        return rec
+        return self._capture(buffers, tune=True, best=buffers.ctx.token_ids)
 
     def _capture(self, buffers, tune: bool, layers_only: bool = False,
                  best: Optional[torch.Tensor] = None) -> _RecordedStep:
@@ -393,8 +408,7 @@ class ModelRunner:
         for rc, st in zip(rcs, starts):
             if st + 1 > rc.length or st + 1 > self.model.max_positions:
                 raise ValueError(f"position {st} is not reserved")
-        cap = self._bucket(B)
-        rec = self._recorded.get(cap) or self._record(cap)
+        rec = self._decode_step(B, max(starts) + 1)
         slots = np.fromiter((rc.slot for rc in rcs), dtype=np.int64, count=B)
         rec.buffers.fill(None, np.asarray(starts, dtype=np.int32), slots.astype(np.int32),
                          {g: self.manager.table_array[g][slots] for g in self.paged_group_ids})
@@ -411,8 +425,7 @@ class ModelRunner:
         check_items(items, self.paged_group_ids, self.cache_param.page_size, self.model.vocab_size,
                     self.model.max_positions)
         B = len(items)
-        cap = self._bucket(B)
-        rec = self._recorded.get(cap) or self._record(cap)
+        rec = self._decode_step(B, max(it.start for it in items) + 1)
         slots = np.fromiter((it.slot for it in items), dtype=np.int64, count=B)
         rec.buffers.fill(np.fromiter((it.tokens[0] for it in items), dtype=np.int32, count=B),
                          np.fromiter((it.start for it in items), dtype=np.int32, count=B),
