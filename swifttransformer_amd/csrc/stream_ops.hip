@@ -19,6 +19,8 @@
 #include "api.h"
 #include "common.h"
 
+#include <type_traits>
+
 namespace st {
 
 // V columns a thread (4: 16-byte accesses); a workgroup takes 256 V columns of one row.  1,024 rows of 2,048 into the storage type, by
@@ -170,6 +172,127 @@ __global__ __launch_bounds__(1024) void token_side_kernel(
     for (int c = threadIdx.x; c < width; c += threads) xr[c] += xs[c] * r * gain[c];
 }
 
+// The same for more bfloat16 rows than there are compute units: a workgroup two rows, so that G and P pass from the L2 to a compute unit
+// once for both (a row a workgroup: 128 KB a row at 2,048 columns, 134 MB for 1,024 rows).  Everything that is read, the rows, G (a wave a
+// feature), P, the table's entries and the gains, is asked for before anything waits: one trip to memory.  What bounds it then is the LDS, from
+// which every wave reads the rows.  us, a row a workgroup of 256 threads and this, columns of 2,048: 300 rows 11.0 and 6.8, 512 11.4 and 7.3, 768
+// 12.5 and 10.9, 1,024 13.5 and 11.5, 2,048 23.1 and 21.2.  Four rows a workgroup: 12.2 at 512, 14.1 at 1,024.  NC: columns a thread.
+template <int NC>
+__global__ __launch_bounds__(1024) void token_side_rows_kernel(
+    float* __restrict__ x, const int* __restrict__ token_ids, const int* __restrict__ token_item, const bf16_t* __restrict__ table,
+    int64_t table_stride, int vocab, const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_proj, const float* __restrict__ gain,
+    int num_rows, int dim, int width, float eps) {
+    constexpr int R = 2;
+    constexpr int DIM = 16, V = Elem<bf16_t>::kVec, NV = 2 * NC;         // NV: pieces of eight columns of G a lane
+    extern __shared__ __attribute__((aligned(16))) float side_rows_lds[];
+    __shared__ __attribute__((aligned(16))) float gs[R][DIM], red[16][R];
+    float* xs = side_rows_lds;                                           // [R][width]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row0 = blockIdx.x * R, quads = width >> 2;
+    // a row's quads of numbers in LDS: the even ones, then the odd ones (a lane reads two neighbouring ones)
+    const auto place = [&](int r, int q) { return r * quads + (q & 1) * (quads >> 1) + (q >> 1); };
+    // (rows past the last stand for it)
+    constexpr int XV = (NC + 1) / 2;                                     // quads a thread: half of the workgroup a row
+    const int half = tid >> 9, first = tid & 511;
+    const float* xr = x + (int64_t)min(row0 + half, num_rows - 1) * width;
+    float4 xv[XV];
+#pragma unroll
+    for (int i = 0; i < XV; ++i) xv[i] = *reinterpret_cast<const float4*>(xr + 4 * min(first + 512 * i, quads - 1));
+    uint4 g[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const int c = (lane + 64 * v) * V;
+        g[v] = *reinterpret_cast<const uint4*>(w_gate + (int64_t)min(wave, dim - 1) * width + (c < width ? c : 0));
+    }
+    float e = 0.f;                                                       // lane r: row r's entry of the wave's feature
+    if (lane < R && row0 + lane < num_rows && wave < dim) {
+        const int tok = token_ids[row0 + lane];
+        if (tok >= 0 && tok < vocab) e = Elem<bf16_t>::load(table + (int64_t)tok * table_stride + wave);
+    }
+    uint4 p[NC][DIM / V];
+    float gn[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        const int c = min(tid + 1024 * i, width - 1);
+#pragma unroll
+        for (int h = 0; h < DIM / V; ++h)
+            p[i][h] = h * V < dim ? *reinterpret_cast<const uint4*>(w_proj + (int64_t)c * dim + h * V) : make_uint4(0, 0, 0, 0);
+        gn[i] = gain[c];
+    }
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {
+        if (first + 512 * i < quads) reinterpret_cast<float4*>(xs)[place(half, first + 512 * i)] = xv[i];
+    }
+    __syncthreads();
+    float sum[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) sum[r] = 0.f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const int c = (lane + 64 * v) * V;
+        if (c >= width) continue;
+        float w[V];
+        Elem<bf16_t>::unpack(g[v], w);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float4 lo = reinterpret_cast<const float4*>(xs)[place(r, c >> 2)], hi = reinterpret_cast<const float4*>(xs)[place(r, (c >> 2) + 1)];
+            sum[r] = fmaf(w[0], lo.x, sum[r]); sum[r] = fmaf(w[1], lo.y, sum[r]); sum[r] = fmaf(w[2], lo.z, sum[r]); sum[r] = fmaf(w[3], lo.w, sum[r]);
+            sum[r] = fmaf(w[4], hi.x, sum[r]); sum[r] = fmaf(w[5], hi.y, sum[r]); sum[r] = fmaf(w[6], hi.z, sum[r]); sum[r] = fmaf(w[7], hi.w, sum[r]);
+        }
+    }
+    float own = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        sum[r] = wave_sum(sum[r]);
+        if (lane == r) own = sum[r];
+    }
+    if (lane < R) gs[lane][wave] = wave < dim ? apply_activation(kActGeluTanh, own) * e : 0.f;
+    __syncthreads();
+    float y[R][NC], ss[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) ss[r] = 0.f;
+    float w[NC][DIM];
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int h = 0; h < DIM / V; ++h) Elem<bf16_t>::unpack(p[i][h], w[i] + h * V);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) y[r][i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < DIM; j += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(&gs[r][j]);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                y[r][i] = fmaf(w[i][j], v.x, y[r][i]); y[r][i] = fmaf(w[i][j + 1], v.y, y[r][i]);
+                y[r][i] = fmaf(w[i][j + 2], v.z, y[r][i]); y[r][i] = fmaf(w[i][j + 3], v.w, y[r][i]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+            if (tid + 1024 * i < width) ss[r] = fmaf(y[r][i], y[r][i], ss[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        ss[r] = wave_sum(ss[r]);
+        if (lane == 0) red[wave][r] = ss[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (row0 + r >= num_rows || (token_item && token_item[row0 + r] < 0)) continue;      // past the last row, or a padding row
+        float total = 0.f;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) total += red[w][r];
+        const float scale = 1.f / sqrtf(total / (float)width + eps);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const int c = tid + 1024 * i;
+            if (c < width) x[(int64_t)(row0 + r) * width + c] = xs[place(r, c >> 2) * 4 + (c & 3)] + y[r][i] * scale * gn[i];
+        }
+    }
+}
+
 }  // namespace st
 
 using namespace st;
@@ -244,6 +367,23 @@ extern "C" int st_token_side(float* x, const int* token_ids, const int* token_it
     const int threads = num_rows <= 256 ? 1024 : 256;
     const int vec = dtype == kF32 ? 4 : 8;
     const bool aligned = width % vec == 0 && dim % vec == 0 && (uintptr_t)w_gate % 16 == 0 && (uintptr_t)w_proj % 16 == 0;
+    // Two rows a workgroup up to two rounds of rows a unit, and beyond that where the rows are neither so short that their weights are not what
+    // counts nor so long that few of their workgroups run at once (us, a row a workgroup and two: 600 rows of 768 7.3 and 7.6, 1,024 8.2 and
+    // 8.3; 600 of 2,560 13.6 and 18.7, 1,024 of 4,096 22.6 and 24.3; but 300 of 4,096 18.4 and 12.1, of 768 7.0 and 5.4).
+    const int units = device_compute_units();
+    if (dtype == kBF16 && aligned && dim <= 16 && width <= 4096 && (uintptr_t)x % 16 == 0 && num_rows > 256 &&
+        (num_rows <= 2 * units || (width > 1024 && width <= 2048))) {
+        const auto launch = [&](auto columns) {
+            token_side_rows_kernel<decltype(columns)::value><<<(unsigned)((num_rows + 1) / 2), 1024, sizeof(float) * 2 * width, stream>>>(
+                x, token_ids, token_item, (const bf16_t*)table, table_stride, vocab, (const bf16_t*)w_gate, (const bf16_t*)w_proj, gain, num_rows,
+                dim, width, eps);
+        };
+        if (width <= 1024) launch(std::integral_constant<int, 1>());
+        else if (width <= 2048) launch(std::integral_constant<int, 2>());
+        else launch(std::integral_constant<int, 4>());
+        ST_LAUNCH_CHECK("token_side");
+        return 0;
+    }
 #define ST_SIDE(T, VEC)                                                                                          \
     token_side_kernel<T, VEC><<<(unsigned)num_rows, threads, lds, stream>>>(                                         \
         x, token_ids, token_item, (const T*)table, table_stride, vocab, (const T*)w_gate, (const T*)w_proj, gain, dim, \
