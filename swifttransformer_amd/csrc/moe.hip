@@ -493,11 +493,12 @@ __global__ __launch_bounds__(256) void moe_down_few_kernel(
     int vec) {
     __shared__ __attribute__((aligned(16))) float lds[4 * 256];
     const int tile = blockIdx.x, r16 = threadIdx.x & 15, n0 = blockIdx.y * 16, base = tile * kRows;
-    const int e = tile_expert[tile], p = sorted[base + (threadIdx.x >> 4)];
+    const int e = tile_expert[tile], p = sorted[base + (threadIdx.x >> 4)], pair = sorted[base + r16];
     if (e < 0) return;
     const T* wr[1] = {w_down + ((int64_t)e * width + min(n0 + r16, width - 1)) * inner};
     floatx4 acc[1] = {floatx4{0.f, 0.f, 0.f, 0.f}};
-    moe_depth_share<T, 1>(acc, y + (int64_t)(base + r16) * inner, wr, inner, vec);
+    // (places without a pair stand for the tile's first, which has one: a tile of few pairs reads few rows)
+    moe_depth_share<T, 1>(acc, y + (int64_t)(base + (pair >= 0 ? r16 : 0)) * inner, wr, inner, vec);
     float sum[1];
     moe_sum_shares<1>(sum, acc, lds);
     const int place = base + (threadIdx.x >> 4), n = n0 + r16;
