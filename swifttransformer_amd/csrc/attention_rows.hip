@@ -99,6 +99,33 @@ __device__ inline float group_sum(float s) {
     return s;
 }
 
+// The sum (or, MAX, the largest) of a value over the lanes that differ by O, where the lanes O apart from each other's are already
+// alike or distinct by it alone: turns of 32, 16 (row swaps), 8, 4, 2, 1 (rotations within 16 lanes), from the largest down to any of them.
+template <int O, bool MAX>
+__device__ inline float across(float x) {
+    float a, b;
+    if (O >= 16) {
+        const uint32_t u = __float_as_uint(x);
+        const auto v = O == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        a = __uint_as_float(v[0]); b = __uint_as_float(v[1]);
+    } else {
+        a = x;
+        b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + (O >= 16 ? 1 : O), 0xF, 0xF, false));
+    }
+    return MAX ? fmaxf(a, b) : a + b;
+}
+// over the 64 / LPK lanes that are `lane % LPK` alike
+template <int LPK, bool MAX>
+__device__ inline float across_groups(float x) {
+    if (LPK <= 32) x = across<32, MAX>(x);
+    if (LPK <= 16) x = across<16, MAX>(x);
+    if (LPK <= 8) x = across<8, MAX>(x);
+    if (LPK <= 4) x = across<4, MAX>(x);
+    if (LPK <= 2) x = across<2, MAX>(x);
+    if (LPK <= 1) x = across<1, MAX>(x);
+    return x;
+}
+
 template <typename T, int LPK>
 __global__ __launch_bounds__(512) void attn_rows_kernel(
     T* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_lse,
@@ -113,11 +140,10 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
     const int G = (blockDim.x >> 6) * KPW;  // lane groups in the workgroup (4 or 8 waves)
     constexpr bool ACC = sizeof(T) == 4;    // float path: accurate expf
     extern __shared__ float lds[];
-    float* s_m = lds;                       // [G]
-    float* s_l = lds + G;                   // [G]
-    float* s_acc = lds + 2 * G;             // [G][head_dim]
-    float* s_red = lds + 2 * G + G * head_dim;   // [16] per-wave partial results of the final merge
-    int* s_bt = reinterpret_cast<int*>(s_red + 16);   // [max_pages] pages of this request
+    float* s_m = lds;                       // [8] the waves' maxima,
+    float* s_l = lds + 8;                   // [8] normalisers
+    float* s_acc = lds + 16;                // [waves][head_dim] and sums
+    int* s_bt = reinterpret_cast<int*>(s_acc + (blockDim.x >> 6) * head_dim);   // [max_pages] pages of this request
 
     const int h = blockIdx.x, ri = blockIdx.y, split = blockIdx.z;
     const int t = row_ids ? row_ids[ri] : ri;      // batch row of this query
@@ -172,6 +198,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
     // a position encoding may add slope * (key position - query position) to this head's scores
     const float slope = head_slopes ? head_slopes[h] : 0.f;
     const float inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;   // scores pass through softcap * tanh(s / softcap)
+    const float gate_logit = head_gate && num_splits == 1 ? head_gate[(int64_t)t * gate_stride + h] : 0.f;
     __syncthreads();
 
     float m = -INFINITY, l = 0.f, acc[VEC];
@@ -254,40 +281,30 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
         }
     }
 
-    if (sub == 0) { s_m[gi] = m; s_l[gi] = l; }
-    if (dvalid) {
+    // Merge of the groups: a wave's by moves between its lanes, to their common maximum, then the waves' through LDS.  (By way of LDS alone,
+    // a slot a group: three barriers and a chain over up to 64 slots.)
+    const float wm = across_groups<LPK, true>(m);
+    const float own = m > -INFINITY ? exp_<ACC>(m - wm) : 0.f;
+    l = across_groups<LPK, false>(l * own);
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) s_acc[gi * head_dim + d0 + i] = acc[i];
+    for (int i = 0; i < VEC; ++i) acc[i] = across_groups<LPK, false>(acc[i] * own);
+    if (lane == 0) { s_m[wave] = wm; s_l[wave] = l; }
+    if (g == 0 && dvalid) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) s_acc[wave * head_dim + d0 + i] = acc[i];
     }
     __syncthreads();
-
-    // merge of the groups: common maximum, one weight per group, then the weighted sums
     const int nwaves = blockDim.x >> 6;
-    float mx = -INFINITY;
-    for (int i = threadIdx.x; i < G; i += blockDim.x) mx = fmaxf(mx, s_m[i]);
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
-    if (lane == 0) s_red[wave] = mx;
-    __syncthreads();
     float M = -INFINITY;
-    for (int w = 0; w < nwaves; ++w) M = fmaxf(M, s_red[w]);
-    float lsum = 0.f;
-    for (int i = threadIdx.x; i < G; i += blockDim.x) {
-        const float mi = s_m[i];
-        const float w = mi > -INFINITY ? exp_<ACC>(mi - M) : 0.f;
-        s_m[i] = w;                                      // the group's weight takes its maximum's place
-        lsum += w * s_l[i];
-    }
-    lsum = wave_sum(lsum);
-    if (lane == 0) s_red[8 + wave] = lsum;
-    __syncthreads();
-    float L = 0.f;
-    for (int w = 0; w < nwaves; ++w) L += s_red[8 + w];
-    const float gate = head_gate && num_splits == 1 ? gate_factor(head_gate[(int64_t)t * gate_stride + h]) : 1.f;
+    for (int w = 0; w < nwaves; ++w) M = fmaxf(M, s_m[w]);
+    const float gate = head_gate && num_splits == 1 ? gate_factor(gate_logit) : 1.f;
     for (int d = threadIdx.x; d < head_dim; d += blockDim.x) {
-        float o = 0.f;
-#pragma unroll 4
-        for (int i = 0; i < G; ++i) o = fmaf(s_m[i], s_acc[i * head_dim + d], o);
+        float o = 0.f, L = 0.f;
+        for (int w = 0; w < nwaves; ++w) {
+            const float part = s_m[w] > -INFINITY ? exp_<ACC>(s_m[w] - M) : 0.f;
+            L = fmaf(part, s_l[w], L);
+            o = fmaf(part, s_acc[w * head_dim + d], o);
+        }
         const float res = L > 0.f ? o / L : 0.f;
         if (num_splits == 1) {
             Elem<T>::store(out + ((int64_t)t * num_q_heads + h) * head_dim + d, res * gate);
