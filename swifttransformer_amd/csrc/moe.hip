@@ -386,7 +386,7 @@ __global__ __launch_bounds__(1024) void moe_router_align_kernel(
 }
 
 // ---- few rows an expert: tiles of 16 places, where only the weights' stream counts.  A workgroup takes 16 features; its
-// four waves share the depth, so that a wave's part is one or a few batches of loads that are all on their way at once and
+// four waves (of a choice) share the depth, so that a wave's part is one or a few batches of loads that are all on their way at once and
 // that the waves' rows, which lie a whole row of weights apart, start at different offsets (equal offsets meet in the
 // same memory channels); the waves' sums meet in LDS.  The addresses of rows and features that do not exist stand for
 // row and feature 0: their results are not stored.
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(1024) void moe_router_align_kernel(
 template <typename T, int MATS>
 __device__ inline void moe_depth_share(floatx4* acc, const T* xr, const T* const* wr, int K, int vec) {
     constexpr int D = Frag<T>::kDepth, L = Frag<T>::kLane;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, g = lane >> 4;
     const int steps = (K + D - 1) / D, share = (steps + 3) / 4;
     int k0 = wave * share * D;
     const int end = min(K, k0 + share * D);
@@ -514,6 +514,47 @@ __global__ __launch_bounds__(256) void moe_down_few_kernel(
         const int64_t at = (int64_t)p * width + n;
         out[at] = fmaf(out_scale, sum[0], residual[at]);
     }
+}
+
+// The output product of one or two tokens with the sum over their choices: four waves a choice, whose sums meet in LDS in the order of the
+// choices, so that neither the pairs' results nor a kernel that adds them stand between (the same numbers to the last bit).  Tokens do
+// not share an expert's weights, so no more than two.  grid (ceil(width / 16), tokens), 256 threads a choice.
+template <typename T>
+__global__ __launch_bounds__(1024) void moe_down_sum_kernel(
+    float* out, const float* residual, const T* __restrict__ y, const T* __restrict__ w_down, const int* __restrict__ place_of_pair,
+    const float* __restrict__ weights, const int* __restrict__ ids, const T* __restrict__ x, int experts, int top, int width, int inner,
+    float out_scale, int vec) {
+    __shared__ float lds[16][16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, n0 = blockIdx.x * 16;
+    const int64_t pair0 = (int64_t)blockIdx.y * top, at = (int64_t)blockIdx.y * width + min(n0 + r16, width - 1);
+    const int place = place_of_pair[pair0 + (wave >> 2)], id = ids[pair0 + (wave >> 2)];
+    // what the sum needs beside the products (by the lanes of the first wave that form it)
+    const float base = residual && wave == 0 ? residual[at] : 0.f, own = x && wave == 0 ? Elem<T>::load(x + at) : 0.f;
+    const float weight = weights && wave == 0 && lane < top ? weights[pair0 + lane] : 1.f;
+    const int held = wave == 0 && lane < top ? place_of_pair[pair0 + lane] : -1, chosen = wave == 0 && lane < top ? ids[pair0 + lane] : -1;
+    if (place >= 0) {
+        const T* wr[1] = {w_down + ((int64_t)id * width + min(n0 + r16, width - 1)) * inner};
+        floatx4 acc[1] = {floatx4{0.f, 0.f, 0.f, 0.f}};
+        moe_depth_share<T, 1>(acc, y + (int64_t)place * inner, wr, inner, vec);
+        if (lane < 16) lds[wave][lane] = acc[0][0];        // (all rows of the block are the pair's)
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float sum = 0.f;
+    bool any = false;
+    for (int j = 0; j < top; ++j) {
+        const float w = __shfl(weight, j, 64);
+        const bool here = __shfl(held, j, 64) >= 0, identity = x && __shfl(chosen, j, 64) >= experts;
+        float r = 0.f;
+        if (here)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r += lds[j * 4 + q][r16];
+        if (here || identity) {
+            sum = fmaf(w, identity ? own : r, sum);
+            any = true;
+        }
+    }
+    if (lane < 16 && n0 + lane < width) out[at] = any ? fmaf(out_scale, sum, base) : base;
 }
 
 // grid (tiles, ceil(inner / 64)); wave w of the workgroup takes inner features f0 + 16 w .. +15 of
@@ -1266,6 +1307,29 @@ extern "C" int st_moe_down(float* out, const float* residual, float* pair_out, c
 
 // ids and x (both or neither): a choice of `experts` or above is an identity expert, whose result is the token's row of x
 // [tokens, width] in the storage type.
+// Whether st_moe_down_sum takes so many tokens and choices.
+extern "C" int st_moe_down_sum_offered(int num_tokens, int top) { return num_tokens <= 2 && top >= 1 && top <= 4; }
+
+// st_moe_down (into the pairs' results) and st_moe_combine at once, for the tokens of tiles of 16 places.
+extern "C" int st_moe_down_sum(float* out, const float* residual, const void* y, const void* w_down, const int* place_of_pair,
+                               const float* weights, const int* ids, const void* x, int experts, int num_tokens, int top, int width, int inner,
+                               float out_scale, int dtype, hipStream_t stream) {
+    ST_CHECK(num_tokens >= 0 && width > 0 && inner > 0, "moe_down_sum: bad sizes");
+    ST_CHECK(st_moe_down_sum_offered(num_tokens, top), "moe_down_sum: one or two tokens of up to four choices, not %d of %d", num_tokens, top);
+    ST_CHECK(out && y && w_down && place_of_pair && ids, "moe_down_sum: null operand");
+    ST_CHECK(dtype == kF32 || dtype == kBF16, "moe_down_sum: unknown dtype %d", dtype);
+    if (num_tokens == 0) return 0;
+    const int vec = rows_vectorised(y, w_down, nullptr, inner, dtype);
+    const dim3 grid((width + 15) / 16, num_tokens);
+#define ST_MDS(T)                                                                                                        \
+    moe_down_sum_kernel<T><<<grid, 256 * top, 0, stream>>>(out, residual, (const T*)y, (const T*)w_down, place_of_pair, weights, ids, \
+                                                           (const T*)x, experts, top, width, inner, out_scale, vec)
+    if (dtype == kF32) ST_MDS(float); else ST_MDS(bf16_t);
+#undef ST_MDS
+    ST_LAUNCH_CHECK("moe_down_sum");
+    return 0;
+}
+
 extern "C" int st_moe_combine(float* out, const float* residual, const float* pair_out, const int* place_of_pair,
                               const float* weights, const int* ids, const void* x, int experts, int num_tokens, int top,
                               int width, float out_scale, int dtype, hipStream_t stream) {
