@@ -206,14 +206,51 @@ __device__ __forceinline__ void state_walk(float* lds, const StateArgs& a, int i
     }
 }
 
+// One row, the same numbers as state_walk's: everything that is read is asked for before anything waits (state, query, key, value and gates
+// one after the other were four trips to memory: 8 rows of 4 heads of 64 x 128 4.9 -> 3.4 us, 48 of 32 heads of 64 x 64 11.5 -> 8.1).
+template <int KQ>
+__device__ __forceinline__ void state_row(float* lds, const StateArgs& a, int64_t row, int slot, int head, int vb) {
+    constexpr int C = 4 * KQ, V = 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dk = a.dk, dv = a.dv;
+    const int group = head / (a.heads / a.qk_heads), col = vb + lane, colc = min(col, dv - 1);
+    float* sq = lds;                       // [C], and the keys
+    float* part = sq + 2 * C;              // [4][V]
+    float* home = a.state + (int64_t)slot * a.slot_stride + (int64_t)head * dk * dv;
+    // a thread's channel of the query (the first C threads) or of the key
+    const int c = tid < C ? tid : tid - C, in = tid < 2 * C && c < dk;
+    const float* from = tid < C ? a.q + row * a.q_stride : a.k + row * a.k_stride;
+    const float x = from[(int64_t)group * dk + (in ? c : 0)];
+    const float v = a.v[row * a.v_stride + (int64_t)head * dv + colc];
+    const float b = a.gate_b[row * a.gate_stride + head], ga = a.gate_a[row * a.gate_stride + head], skip = a.skip ? a.skip[head] : 0.f;
+    float S[KQ];
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) S[i] = home[(int64_t)min(wave * KQ + i, dk - 1) * dv + colc];
+    if (tid < 2 * C) sq[tid] = in ? x : 0.f;
+    __syncthreads();
+    const float vv = col < dv ? v : 0.f, av = ga * vv;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) {
+        const int kk = wave * KQ + i;
+        S[i] = fmaf(b, kk < dk && col < dv ? S[i] : 0.f, sq[C + kk] * av);
+        acc[i & 3] = fmaf(S[i], sq[kk], acc[i & 3]);
+        if (kk < dk && col < dv) home[(int64_t)kk * dv + col] = S[i];
+    }
+    part[wave * V + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    __syncthreads();
+    if (wave == 0 && col < dv)
+        a.out[(row * a.heads + head) * dv + col] = fmaf(skip, vv, (part[lane] + part[V + lane]) + (part[2 * V + lane] + part[3 * V + lane]));
+}
+
 // Steps of single tokens: grid (heads, items, blocks of 64 value channels), a kernel of its own with few registers.  (The caller's word
 // that there are no longer items is about speed: they are walked kStateShort rows at a time.)
 template <int KQ>
 __global__ __launch_bounds__(256) void state_walk_kernel(StateArgs a) {
     extern __shared__ __attribute__((aligned(16))) float state_lds[];
-    const int item = blockIdx.y, len = a.item_len[item];
-    if (a.item_slot[item] < 0 || len <= 0) return;
-    if (len <= kStateShort) state_walk<KQ, false>(state_lds, a, item, len, blockIdx.x, blockIdx.z * 64);
+    const int item = blockIdx.y, len = a.item_len[item], slot = a.item_slot[item], row = a.item_tok_off[item];
+    if (slot < 0 || len <= 0) return;
+    if (len == 1) state_row<KQ>(state_lds, a, row, slot, blockIdx.x, blockIdx.z * 64);
+    else if (len <= kStateShort) state_walk<KQ, false>(state_lds, a, item, len, blockIdx.x, blockIdx.z * 64);
     else state_walk<KQ, true>(state_lds, a, item, len, blockIdx.x, blockIdx.z * 64);
 }
 
