@@ -271,8 +271,10 @@ static void launch_activation_multiply(void* out, int64_t out_stride, const void
                                        int64_t b_stride, int rows, int width, int kind, hipStream_t stream) {
     constexpr int V = Elem<T>::kVec;
     const uintptr_t align = (uintptr_t)out | (uintptr_t)a | (uintptr_t)b;
+    // (where a thread a number leaves no unit more than a workgroup it is the faster one: eight functions in a row take longer than the
+    // trip to memory; 8 rows of 4,096, GELU, 3.2 -> 2.1 us, SiLU 3.0 -> 2.1)
     const bool vec = width % V == 0 && out_stride % V == 0 && a_stride % V == 0 && (!b || b_stride % V == 0) &&
-                     (align & 15) == 0;
+                     (align & 15) == 0 && (int64_t)rows * width > 256 * (int64_t)device_compute_units();
     const int64_t work = (int64_t)rows * (vec ? width / V : width);
     const int64_t want = (work + 255) / 256, most = (int64_t)device_compute_units() * 16;
     const unsigned grid = (unsigned)(want < most ? want : most);
