@@ -1034,12 +1034,12 @@ static int launch_tiled(bf16_t* y, float* out, const float* residual, float* pai
 // V columns a thread and turn (4: 16-byte accesses).  x (or null): the tokens' own vectors, the results of the identity
 // experts, whose numbers are `experts` and above.
 template <typename T, int V>
-__global__ __launch_bounds__(256) void moe_combine_kernel(
+__global__ __launch_bounds__(1024) void moe_combine_kernel(
     float* out, const float* residual, const float* __restrict__ pair_out,
     const int* __restrict__ place_of_pair, const float* __restrict__ weights, const int* __restrict__ ids,
     const T* __restrict__ x, int experts, int top, int width, float out_scale) {
     const int t = blockIdx.x;
-    for (int n = threadIdx.x * V; n < width; n += 256 * V) {
+    for (int n = threadIdx.x * V; n < width; n += blockDim.x * V) {
         float sum[V], base[V], own[V];
         bool any = false;
         const int64_t at = (int64_t)t * width + n;
@@ -1338,8 +1338,12 @@ extern "C" int st_moe_combine(float* out, const float* residual, const float* pa
     ST_CHECK(dtype == kF32 || dtype == kBF16, "moe_combine: unknown dtype %d", dtype);
     if (num_tokens == 0) return 0;
     const bool vec = width % 4 == 0 && (((uintptr_t)out | (uintptr_t)residual | (uintptr_t)pair_out) & 15) == 0;
+    // a turn is two trips to memory (a choice's place, then its result): few rows have a thread for every piece, up to 1,024 (us, 256 threads
+    // and so: 8 rows of 2,048 2.7 and 2.15, 24 of 4,096 4.0 and 2.5, 256 of 2,048 3.0 and 2.5)
+    int threads = 256;
+    while (num_tokens <= device_compute_units() && threads < 1024 && threads * (vec ? 4 : 1) < width) threads <<= 1;
 #define ST_MC(T, V)                                                                                                    \
-    moe_combine_kernel<T, V><<<num_tokens, 256, 0, stream>>>(out, residual, pair_out, place_of_pair, weights, ids, (const T*)x, \
+    moe_combine_kernel<T, V><<<num_tokens, threads, 0, stream>>>(out, residual, pair_out, place_of_pair, weights, ids, (const T*)x, \
                                                              experts, top, width, out_scale)
     if (dtype == kF32) { if (vec) ST_MC(float, 4); else ST_MC(float, 1); }
     else { if (vec) ST_MC(bf16_t, 4); else ST_MC(bf16_t, 1); }
