@@ -32,8 +32,8 @@ class Tuning:
     # Decode steps of requests with contexts of up to this many tokens have recordings of their own: where few rows' keys are
     # split until there is a workgroup for every compute unit, one row of 12 heads of 64 takes (attention and output projection, us)
     # 8.8 whole and 12.5 in 16 splits that a kernel merges at 57 keys, 11.0 and 12.8 at 300, 12.4 and 12.9 at 500; merged by the
-    # projection itself, in 8 splits, 10.2 at 97 keys (whole 8.9), 10.5 at 300.
-    short_span: int = 256
+    # projection itself, in 8 splits, 10.2 at 97 keys (whole 8.9), 10.5 at 300 (whole 11.0): the two meet at about 210.
+    short_span: int = 192
     # A step that is not plain decoding is recorded when its shape comes up for this many-th time.
     record_after: int = 2
     # Recordings of up to this many rows have the vendor library's kernels timed (20 to 100 ms a

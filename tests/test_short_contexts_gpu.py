@@ -59,18 +59,20 @@ def test_tokens_chosen_on_the_device_cross_over(model):
 
 
 def test_warm_up_records_both(model):
+    from swifttransformer_amd.ops.tuning import tuning
     runner = make_runner(model[0], torch.float32, 16, num_pages=40, max_seqs=2)
     assert runner.warm_up([], [1, 2]) == 4
-    assert set(runner._recorded_spans) == {(b, s) for b in (1, 2) for s in (256, 1024)}
+    assert set(runner._recorded_spans) == {(b, s) for b in (1, 2) for s in (tuning.short_span, 1024)}
     assert runner.warm_up([], [1, 2]) == 0
 
 
 def test_models_no_longer_than_short_contexts_have_one(tmp_path):
     from swifttransformer_amd.engine.step import StepEntry
     from swifttransformer_amd.config import OptHyperParam
+    from swifttransformer_amd.ops.tuning import tuning
     from swifttransformer_amd.weights import write_random_model
-    d = write_random_model(OptHyperParam(**dict(CFG, max_position_embeddings=256)).validate(), str(tmp_path / "m"), seed=3)
+    d = write_random_model(OptHyperParam(**dict(CFG, max_position_embeddings=tuning.short_span)).validate(), str(tmp_path / "m"), seed=3)
     runner = make_runner(d, torch.float32, 16, num_pages=8, max_seqs=1)
     runner.admit(0)
     runner.step([StepEntry(0, [5], [0])])
-    assert set(runner._recorded_spans) == {(1, 256)}
+    assert set(runner._recorded_spans) == {(1, tuning.short_span)}
