@@ -275,7 +275,7 @@ extern "C" int st_gemm_library_rule(int min_rows, int64_t min_weights, int min_d
 }
 
 // Calls of st_gemm per kernel family since the last reset (order of st::GemmPath); returns the
-// number of families.  `out` may be null.
+// number of families.  `out` may be null.  (The products of gemm_f32_split are in none of them: which they are follows from the sizes, f32_split_pays.)
 extern "C" int st_gemm_path_counts(uint64_t* out, int reset) {
     for (int i = 0; i < kNumGemmPaths; ++i) {
         const uint64_t v = reset ? g_path_counts[i].exchange(0) : g_path_counts[i].load();

@@ -56,7 +56,7 @@ class StepContext:
     host_item_slot: List[int] = field(default_factory=list)
     # True when the step is recorded once and replayed: nothing may depend on the values
     # of this step (lengths, slots); kernels size their work for `max_kv_len` = the longest
-    # sequence the model allows
+    # context that the recording serves (`tuning.short_span`, or all that the model allows)
     static_shapes: bool = False
     # the model's position encoding, for mixers to call its ``rotate`` (set by the model)
     position: Optional[object] = None

@@ -164,7 +164,7 @@ class PagedAttention(Mixer):
         (row, head, split); when rows * heads alone does not fill the chip, a row's keys are
         split over workgroups (merged by a second kernel), at least tuning.min_keys_per_split keys
         each.  ctx.max_kv_len is the longest sequence of this step, or, for a recorded step,
-        the longest the model allows: then the shape depends on the batch size alone."""
+        the longest context that the recording serves: then the shape depends on the recording and the batch size alone."""
         span = self.key_span(ctx)
         groups = max(1, rows * self.num_heads)
         units = _target_workgroups()

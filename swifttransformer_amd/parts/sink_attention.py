@@ -94,8 +94,8 @@ class SinkAttention(Mixer):
 
     def _splits(self, ctx, rows: int) -> int:
         """Workgroups a row: a row's keys are split when the rows alone leave most of the chip idle (decoded
-        tokens).  For a recorded step ``ctx.max_kv_len`` is the longest sequence the model allows, so the
-        shape depends on the number of rows alone."""
+        tokens).  For a recorded step ``ctx.max_kv_len`` is the longest context that the recording
+        serves, so the shape depends on the recording and the number of rows alone."""
         span = ctx.max_kv_len if self.window <= 0 else min(ctx.max_kv_len, self.window)
         blocks = max(1, -(-span // 64))
         return max(1, min(256 // max(rows, 1), blocks, 16))

@@ -96,8 +96,8 @@ class GatedWindowAttention(Mixer):
         return parts
 
     def _splits(self, ctx, rows: int) -> int:
-        """Workgroups a row (see ``SinkAttention._splits``): a function of the rows and, for recorded
-        steps, of nothing else."""
+        """Workgroups a row (see ``SinkAttention._splits``): for recorded steps a function of the rows
+        and the recording alone."""
         span = ctx.max_kv_len if self.window <= 0 else min(ctx.max_kv_len, self.window + self.keep_first)
         blocks = max(1, -(-span // 64))
         return max(1, min(256 // max(rows, 1), blocks, 16))
