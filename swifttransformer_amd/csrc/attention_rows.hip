@@ -281,29 +281,31 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
         }
     }
 
-    // Merge of the groups: a wave's by moves between its lanes, to their common maximum, then the waves' through LDS.  (By way of LDS alone,
-    // a slot a group: three barriers and a chain over up to 64 slots.)
+    // Merge of the groups: the workgroup's maximum, then a wave's groups by moves between its lanes, each with one weight to that maximum
+    // (to the wave's first and from there to the workgroup's, a barrier less, rounds two weights), then the waves' through LDS.  (By way of
+    // LDS alone, a slot a group: three barriers and a chain over up to 64 slots.)
     const float wm = across_groups<LPK, true>(m);
-    const float own = m > -INFINITY ? exp_<ACC>(m - wm) : 0.f;
+    const int nwaves = blockDim.x >> 6;
+    if (lane == 0) s_m[wave] = wm;
+    __syncthreads();
+    float M = -INFINITY;
+    for (int w = 0; w < nwaves; ++w) M = fmaxf(M, s_m[w]);
+    const float own = m > -INFINITY ? exp_<ACC>(m - M) : 0.f;
     l = across_groups<LPK, false>(l * own);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) acc[i] = across_groups<LPK, false>(acc[i] * own);
-    if (lane == 0) { s_m[wave] = wm; s_l[wave] = l; }
+    if (lane == 0) s_l[wave] = l;
     if (g == 0 && dvalid) {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) s_acc[wave * head_dim + d0 + i] = acc[i];
     }
     __syncthreads();
-    const int nwaves = blockDim.x >> 6;
-    float M = -INFINITY;
-    for (int w = 0; w < nwaves; ++w) M = fmaxf(M, s_m[w]);
     const float gate = head_gate && num_splits == 1 ? gate_factor(gate_logit) : 1.f;
     for (int d = threadIdx.x; d < head_dim; d += blockDim.x) {
         float o = 0.f, L = 0.f;
         for (int w = 0; w < nwaves; ++w) {
-            const float part = s_m[w] > -INFINITY ? exp_<ACC>(s_m[w] - M) : 0.f;
-            L = fmaf(part, s_l[w], L);
-            o = fmaf(part, s_acc[w * head_dim + d], o);
+            L += s_l[w];
+            o += s_acc[w * head_dim + d];
         }
         const float res = L > 0.f ? o / L : 0.f;
         if (num_splits == 1) {
