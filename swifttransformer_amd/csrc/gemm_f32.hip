@@ -9,9 +9,13 @@
 // Measured against float64 (x normal, W normal of 0.02): 701 x 6,144 x 2,048 4.7e-7 where the library's float product has 8.1e-7,
 // 701 x 2,048 x 8,192 4.6e-7 and 1.6e-6, 1,500 x 2,560 x 10,240 1.2e-6 and 1.8e-6; never more at 96 rows and above.
 //
-// Where the parts do not do, a block of 64 x 64 is formed again by float products: infinities, NaN and numbers that round past
-// bfloat16's largest make a NaN of products that float would not (infinity times a part that is zero), so a sum that is not finite;
-// of numbers below 2^-109 the last part loses bits (bfloat16's least number is 2^-133), so a sum below 2^-90 that is not zero.
+// Where the parts do not do, a block of 64 x 64 is formed again by float products:
+// - A row of either matrix holds a number that is more than its three parts.  bfloat16's least number is 2^-133, so numbers below 2^-109 may
+//   be, whatever they are multiplied by.  The third part is the upper half of what the first two leave, and the row is marked if a lower half
+//   is not zero (one instruction for two numbers; 701 x 6,144 x 2,048 takes 3 % longer for it).
+// - A sum is not finite: infinities, NaN and numbers that round past bfloat16's largest make a NaN of products that float would not
+//   (infinity times a part that is zero).
+// - A sum is below 2^-90 and not zero: products of small parts may be below float's least number where the whole product is not.
 //
 // What bounds it: the chip's power, more than its matrix cores (six products a float product, 1.0 to 1.2 PFLOP/s of them where a large
 // bfloat16 product reaches 1.6): the same launch takes 381 us on normal numbers and 320 on zeros, 290 without loads, 270 with products
@@ -74,6 +78,7 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
     float* __restrict__ out, const float* __restrict__ x, const float* __restrict__ w, const float* bias, const float* residual,
     float* __restrict__ part, int M, int N, int K, int act, int tiles_m, int tiles, int whole, int splits, const StGemmExtras ex) {
     __shared__ uint4 lds[kBufs][kParts][2 * kTile * 4];   // rows of W, then rows of x: four pieces of eight in depth each
+    __shared__ int s_lost[2 * kTile];                     // of these rows: whether they hold a number that is more than its parts
     int tile, split = 0;
     if ((int)blockIdx.x < whole) {
         tile = by_die(blockIdx.x, whole);
@@ -106,11 +111,17 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
     };
     // Part `i` % 12 / 4 of numbers 2 (i % 4) and the next of row `i` / 12; a row's pieces go to LDS when they are whole, rotated by row / 4:
     // 16 neighbouring rows' like pieces lie in different banks.
-    uint32_t piece[kParts][4];
+    uint32_t piece[kParts][4], lost[2] = {0, 0};     // (lower halves: of what the parts leave of the row of W, of x)
     auto take = [&](auto parity, int i, int buf) {
         constexpr int P = decltype(parity)::value;
         float4& v = raw[P][i / 12][i % 4 / 2];
-        piece[i % 12 / 4][i % 4] = i % 2 ? split_off(v.z, v.w) : split_off(v.x, v.y);
+        if (i % 12 / 4 < kParts - 1) {
+            piece[i % 12 / 4][i % 4] = i % 2 ? split_off(v.z, v.w) : split_off(v.x, v.y);
+        } else {
+            const uint32_t lo = __float_as_uint(i % 2 ? v.z : v.x), hi = __float_as_uint(i % 2 ? v.w : v.y);
+            piece[i % 12 / 4][i % 4] = __builtin_amdgcn_perm(hi, lo, 0x07060302);      // the upper halves of both
+            lost[i / 12] |= lo | hi;
+        }
         if (i % 12 == 11)
 #pragma unroll
             for (int q = 0; q < kParts; ++q)
@@ -176,7 +187,14 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
         step(even, s);
         if (s + 1 < end) step(odd, s + 1);
     }
-    // the halves' sums meet in LDS
+    // a row's four threads mark it; the halves' sums meet in LDS
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        int bits = (int)(lost[i] & 0xffffu);
+        bits |= __shfl_xor(bits, 1, 64);
+        bits |= __shfl_xor(bits, 2, 64);
+        if (j == 0) s_lost[kTile * i + row] = bits;
+    }
     float4* other = reinterpret_cast<float4*>(lds);
     if (half)
 #pragma unroll
@@ -189,7 +207,7 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
                         make_float4(acc[q][r][4 * u4], acc[q][r][4 * u4 + 1], acc[q][r][4 * u4 + 2], acc[q][r][4 * u4 + 3]);
     __syncthreads();
     if (half) return;
-    bool sound = true;
+    uint32_t most = 0, least = 0xffffffffu;          // of the sums' sizes, as whole numbers; of those that are not zero, less one
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
@@ -197,15 +215,17 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
 #pragma unroll
             for (int u4 = 0; u4 < 4; ++u4) {
                 const float4 v = other[((wave * 4 + q * 2 + r) * 4 + u4) * 64 + lane];
-                acc[q][r][4 * u4] += v.x; acc[q][r][4 * u4 + 1] += v.y; acc[q][r][4 * u4 + 2] += v.z; acc[q][r][4 * u4 + 3] += v.w;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float size = fabsf(acc[q][r][4 * u4 + i]);
-                    sound = sound && size < INFINITY && (size >= 0x1p-90f || size == 0.f);
+                    const float sum = acc[q][r][4 * u4 + i] + (&v.x)[i];
+                    const uint32_t size = __float_as_uint(sum) & 0x7fffffffu;
+                    acc[q][r][4 * u4 + i] = sum;
+                    most = max(most, size);
+                    least = min(least, size - 1);
                 }
             }
     // numbers k0 .. k1-1 of the depth as float products, straight from memory (a lane brings every other four of a row's numbers):
-    // what is left of the depth behind whole steps, and everything again where a sum says that the parts did not do
+    // what is left of the depth behind whole steps, and everything again where the parts do not do
     auto plain = [&](int k0, int k1) {
         const float *wr[2], *xr[2];
 #pragma unroll
@@ -229,7 +249,8 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
                         acc[q][r] = __builtin_amdgcn_mfma_f32_32x32x2f32((&wv[q].x)[i], (&xv[r].x)[i], acc[q][r], 0, 0, 0);
         }
     };
-    if (__any(!sound)) {
+    constexpr uint32_t kInf = 0x7f800000u, kSmall = 0x12800000u;     // infinity, 2^-90
+    if (__any(s_lost[wn * 64 + lane] | s_lost[kTile + wm * 64 + lane] || most >= kInf || least < kSmall - 1)) {
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll

@@ -119,13 +119,35 @@ def test_numbers_that_parts_do_not_hold():
     size = x[200].double().abs() @ w.double().abs().T
     assert bool(((y[200].double() - ref[200]).abs()[held] <= 2.0 ** -20 * size[held]).all())
     size = x[250].double().abs() @ w.double().abs().T
-    assert bool(((y[250].double() - ref[250]).abs() <= 2.0 ** -16 * size + 2.0 ** -140).all())
+    assert bool(((y[250].double() - ref[250]).abs() <= (D + 12) * 2.0 ** -24 * size + D * 2.0 ** -149).all())
     rows = torch.ones(M, dtype=torch.bool, device="cuda")
     rows[[3, 70, 140, 200, 250]] = False
     keep = torch.ones(N, dtype=torch.bool, device="cuda")
     keep[9] = False
     check(y[rows], x[rows], w)
     assert bool(torch.isfinite(clean).all())
+
+
+# (splits: 701 rows of 2,048 x 2,048 are 96 tiles, parted over the depth; 300 of 256 x 200 are whole)
+@pytest.mark.parametrize("M,N,D", [(300, 256, 200), (701, 2048, 2048)])
+@pytest.mark.parametrize("tiny,large", [(-120, 40), (-130, 60), (-140, 60), (-136, 0), (-110, 100)])
+def test_tiny_numbers_with_large_ones(M, N, D, tiny, large):
+    """Numbers that three bfloat16 numbers do not hold, in rows of x and of W, times numbers that make ordinary sums of them: no further off
+    than D roundings of a float sum."""
+    x, w, g = operands(M, N, D)
+    normal = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).double()
+    x[5], x[M - 2] = (normal(D) * 2.0 ** tiny).float(), torch.where(torch.arange(D, device="cuda") == D - 40, 2.0 ** tiny * 1.2345678, 0.0)
+    w[7], w[130] = (normal(D) * 2.0 ** large).float(), 2.0 ** large
+    w[3], x[131] = (normal(D) * 2.0 ** tiny).float(), 2.0 ** large
+    # some rows, all of x and all of W (sums that look ordinary everywhere)
+    for a, b in ((x, w), ((normal(M, D) * 2.0 ** tiny).float(), (normal(N, D) * 2.0 ** large).float()),
+                 ((normal(M, D) * 2.0 ** large).float(), (normal(N, D) * 2.0 ** tiny).float())):
+        y = K.gemm(a, b, algo=3)
+        ref, size = a.double() @ b.double().T, a.double().abs() @ b.double().abs().T
+        over = (y.double() - ref).abs() > (D + 12) * 2.0 ** -24 * size + D * 2.0 ** -149
+        held = ref.abs() < 2.0 ** 128                               # (large ones among themselves may be past float's range)
+        assert not bool((over & held).any()), (over & held).nonzero()[:4].tolist()
+        assert not bool(torch.isfinite(y[~held]).any())
 
 
 def test_rows_off_16_bytes_go_to_the_library():
