@@ -9,13 +9,14 @@
 // Measured against float64 (x normal, W normal of 0.02): 701 x 6,144 x 2,048 4.7e-7 where the library's float product has 8.1e-7,
 // 701 x 2,048 x 8,192 4.6e-7 and 1.6e-6, 1,500 x 2,560 x 10,240 1.2e-6 and 1.8e-6; never more at 96 rows and above.
 //
-// Where the parts do not do, a block of 64 x 64 is formed again by float products:
-// - A row of either matrix holds a number that is more than its three parts.  bfloat16's least number is 2^-133, so numbers below 2^-109 may
+// Where the parts do not do, a result is formed again by float products (a block of 64 x 64 at once; the others of the block keep theirs, so
+// that no row's numbers change what another row gets):
+// - Its row of either matrix holds a number that is more than its three parts.  bfloat16's least number is 2^-133, so numbers below 2^-109 may
 //   be, whatever they are multiplied by.  The third part is the upper half of what the first two leave, and the row is marked if a lower half
 //   is not zero (one instruction for two numbers; 701 x 6,144 x 2,048 takes 3 % longer for it).
-// - A sum is not finite: infinities, NaN and numbers that round past bfloat16's largest make a NaN of products that float would not
+// - Its sum is not finite: infinities, NaN and numbers that round past bfloat16's largest make a NaN of products that float would not
 //   (infinity times a part that is zero).
-// - A sum is below 2^-90 and not zero: products of small parts may be below float's least number where the whole product is not.
+// - Its sum is below 2^-90 and not zero: products of small parts may be below float's least number where the whole product is not.
 //
 // What bounds it: the chip's power, more than its matrix cores (six products a float product, 1.0 to 1.2 PFLOP/s of them where a large
 // bfloat16 product reaches 1.6): the same launch takes 381 us on normal numbers and 320 on zeros, 290 without loads, 270 with products
@@ -224,9 +225,10 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
                     least = min(least, size - 1);
                 }
             }
-    // numbers k0 .. k1-1 of the depth as float products, straight from memory (a lane brings every other four of a row's numbers):
-    // what is left of the depth behind whole steps, and everything again where the parts do not do
-    auto plain = [&](int k0, int k1) {
+    // acc[q][r][u]: feature n0 + wn * 64 + q * 32 + 8 * (u / 4) + 4 * lh + u % 4 of row m0 + wm * 64 + r * 32 + l32.
+    // Numbers k0 .. k1-1 of the depth as float products, straight from memory (a lane brings every other four of a row's numbers):
+    // what is left of the depth behind whole steps, and everything again where the parts do not do.
+    auto plain = [&](floatx16 (&to)[2][2], int k0, int k1) {
         const float *wr[2], *xr[2];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -246,21 +248,33 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
                 for (int q = 0; q < 2; ++q)
 #pragma unroll
                     for (int r = 0; r < 2; ++r)
-                        acc[q][r] = __builtin_amdgcn_mfma_f32_32x32x2f32((&wv[q].x)[i], (&xv[r].x)[i], acc[q][r], 0, 0, 0);
+                        to[q][r] = __builtin_amdgcn_mfma_f32_32x32x2f32((&wv[q].x)[i], (&xv[r].x)[i], to[q][r], 0, 0, 0);
         }
     };
     constexpr uint32_t kInf = 0x7f800000u, kSmall = 0x12800000u;     // infinity, 2^-90
     if (__any(s_lost[wn * 64 + lane] | s_lost[kTile + wm * 64 + lane] || most >= kInf || least < kSmall - 1)) {
+        floatx16 again[2][2];
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int r = 0; r < 2; ++r)
 #pragma unroll
-                for (int u = 0; u < 16; ++u) acc[q][r][u] = 0.f;
-        plain(begin * kStep, end * kStep);
+                for (int u = 0; u < 16; ++u) again[q][r][u] = 0.f;
+        plain(again, begin * kStep, end * kStep);
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int u = 0; u < 16; ++u) {
+                    const uint32_t size = __float_as_uint(acc[q][r][u]) & 0x7fffffffu;
+                    if (s_lost[kTile + wm * 64 + r * 32 + l32] | s_lost[wn * 64 + q * 32 + 8 * (u / 4) + 4 * lh + u % 4] || size >= kInf ||
+                        size - 1 < kSmall - 1)
+                        acc[q][r][u] = again[q][r][u];
+                }
     }
-    if (end == steps && steps * kStep < K) plain(steps * kStep, K);
-    // acc[q][r][u]: feature n0 + wn * 64 + q * 32 + 8 * (u / 4) + 4 * lh + u % 4 of row m0 + wm * 64 + r * 32 + l32.  What is added to them is
+    if (end == steps && steps * kStep < K) plain(acc, steps * kStep, K);
+    // What is added to the results is
     // asked for before the first is stored: one trip to memory a row of the block, not one a store.
 #pragma unroll
     for (int r = 0; r < 2; ++r) {

@@ -150,6 +150,20 @@ def test_tiny_numbers_with_large_ones(M, N, D, tiny, large):
         assert not bool(torch.isfinite(y[~held]).any())
 
 
+@pytest.mark.parametrize("M,N,D", [(300, 256, 200), (701, 2048, 2048)])
+def test_rows_do_not_change_each_other(M, N, D):
+    """Infinities, NaN, numbers past bfloat16's largest and tiny ones in some rows of x: the others' results stay the same to the last bit."""
+    x, w, _ = operands(M, N, D)
+    clean = K.gemm(x, w, algo=3)
+    x[3, 7], x[70, 0], x[140, D - 1], x[200, 5], x[201, 3] = float("inf"), -float("inf"), float("nan"), 3.4e38, 1e-42
+    x[250] *= 2.0 ** -120
+    rows = torch.ones(M, dtype=torch.bool, device="cuda")
+    rows[[3, 70, 140, 200, 201, 250]] = False
+    y = K.gemm(x, w, algo=3)
+    assert torch.equal(y[rows], clean[rows])
+    assert not torch.equal(y[201], clean[201])
+
+
 def test_rows_off_16_bytes_go_to_the_library():
     buf, _, _ = operands(1, 1, 701 * 2048 + 1)
     w = operands(4, 2048, 2048)[1]
