@@ -2,12 +2,15 @@
 // x[M,K], W[N,K] contiguous along K, float in and out.
 //
 // A float has 24 significant bits and a bfloat16 eight, so a float is the sum of three bfloat16 numbers, a = a0 + a1 + a2, exactly
-// (each the rounded rest of the ones before it; a1 is at most 2^-8 of a, a2 2^-16).  Of the nine products of two such sums six are
+// (each the rounded rest of the ones before it; a1 is at most 2^-9 of a, a2 2^-18).  Of the nine products of two such sums six are
 // formed, a0 b0, a0 b1, a1 b0, a0 b2, a1 b1 and a2 b0, each exact in the matrix cores, whose sums are float; the three left out are
-// together at most 2^-23 of |a b| and 2^-26 as a rule, the size of a float product's own rounding.  16 in depth then take six roundings
-// of a sum where the float matrix instruction takes four or eight, in chains half as long (two groups of waves share the depth).
-// Measured against float64 (x normal, W normal of 0.02): 701 x 6,144 x 2,048 4.7e-7 where the library's float product has 8.1e-7,
-// 701 x 2,048 x 8,192 4.6e-7 and 1.6e-6, 1,500 x 2,560 x 10,240 1.2e-6 and 1.8e-6; never more at 96 rows and above.
+// together at most 2^-25.9 of |a b|, a quarter of a float product's own rounding.  a0 b0 has a sum of its own and the five small ones
+// another, 2^-8 of it, which meet at the end: a product then takes one rounding of a running sum at full size, as with float products, and
+// 16 products in depth share one where the float matrix instruction takes four or eight.  (One sum for all six: six roundings, and more
+// error than float products where most of x is zero, 1.2 times at 10 % and 1.6 at 0.2 % of 701 x 6,144 x 2,048, at the same speed.)
+// Error against float64 (x normal, W normal of 0.02), the library's float product and this: 701 x 6,144 x 2,048 8.1e-7 and 1.8e-7, with 1 % of x
+// not zero 8.5e-8 and 3.9e-8, with 0.2 % 4.4e-8 and 3.0e-8; 701 x 2,048 x 8,192 1.6e-6 and 1.7e-7, 1.6e-7 and 5.7e-8, 7.7e-8 and 5.2e-8;
+// 1,500 x 2,560 x 2,560 9.1e-7 and 2.1e-7, 9.4e-8 and 3.8e-8, 4.8e-8 and 2.8e-8.
 //
 // Where the parts do not do, a result is formed again by float products (a block of 64 x 64 at once; the others of the block keep theirs, so
 // that no row's numbers change what another row gets):
@@ -19,11 +22,12 @@
 // - Its sum is below 2^-90 and not zero: products of small parts may be below float's least number where the whole product is not.
 //
 // What bounds it: the chip's power, more than its matrix cores (six products a float product, 1.0 to 1.2 PFLOP/s of them where a large
-// bfloat16 product reaches 1.6): the same launch takes 381 us on normal numbers and 320 on zeros, 290 without loads, 270 with products
-// and LDS reads alone (2,048 x 8,192 x 2,048).  So every number is split once a workgroup, by all waves, between the products (a step's products and
-// splitting one after the other, by waves in turn or all alike: 392 and 383 us), and what is multiplied next is read from LDS a step ahead.
-// us, the library's best of 32 and this: 701 rows of 6,144 x 2,048 145 and 113, of 2,048 x 8,192 185 and 145, 1,500 rows of 2,560 x 2,560
-// 158 and 109, of 768 x 3,072 66 and 52.
+// bfloat16 product reaches 1.6): with one sum for all six the same launch took 381 us on normal numbers and 320 on zeros, 290 without loads,
+// 270 with products and LDS reads alone (2,048 x 8,192 x 2,048).  So every number is split once a workgroup, by all waves, between the
+// products (a step's products and splitting one after the other, by waves in turn or all alike: 392 and 383 us), and what is multiplied next is
+// read from LDS while there are products left that do not need the registers.
+// us, the library's best of 32 and this: 701 rows of 6,144 x 2,048 143 and 120, of 2,048 x 8,192 184 and 160, 1,500 rows of 2,560 x 2,560
+// 154 and 116, of 768 x 3,072 64 and 57.
 //
 // Reference: cuBLAS calls (src/csrc/util/cublas_wrapper.cc:29).
 #include "common.h"
@@ -132,24 +136,19 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
 #pragma unroll
         for (int i = 0; i < 24; ++i) take(parity, i, buf);
     };
-    floatx16 acc[2][2];
+    floatx16 acc[2][2], low[2][2];                   // the sums of a0 b0; of the other products
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int u = 0; u < 16; ++u) acc[a][b][u] = 0.f;
-    bf16x8 a[2][2][kParts], b[2][2][kParts];         // operands of a step of either parity
+            for (int u = 0; u < 16; ++u) acc[a][b][u] = low[a][b][u] = 0.f;
+    bf16x8 a[2][kParts], b[2][kParts];               // a step's operands
     const int at = l32 * 4 + ((half * 2 + lh) ^ ((l32 >> 2) & 3));
-    auto fetch = [&](auto parity, int buf) {
-        constexpr int P = decltype(parity)::value;
+    auto fetch = [&](bf16x8 (&to)[2][kParts], int p, int buf) {
 #pragma unroll
-        for (int p = 0; p < kParts; ++p)
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                a[P][q][p] = __builtin_bit_cast(bf16x8, lds[buf][p][(wn * 64 + q * 32) * 4 + at]);
-                b[P][q][p] = __builtin_bit_cast(bf16x8, lds[buf][p][(kTile + wm * 64 + q * 32) * 4 + at]);
-            }
+        for (int q = 0; q < 2; ++q)
+            to[q][p] = __builtin_bit_cast(bf16x8, lds[buf][p][((&to == &a ? wn * 64 : kTile + wm * 64) + q * 32) * 4 + at]);
     };
     // this wave's pieces are in LDS and its operands in registers; then everyone's are (loads from memory may be on their way)
     auto meet = [&] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
@@ -163,21 +162,33 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
         park(odd, 1);
         load(odd, begin + 3);
         meet();
-        fetch(even, 0);
+#pragma unroll
+        for (int p = 0; p < kParts; ++p) {
+            fetch(a, p, 0);
+            fetch(b, p, 0);
+        }
     }
     // Each of a step's 24 products, which the matrix core takes 32 cycles for, goes with a piece of the splitting of the step after next.
+    // An operand is read for the next step when it has had its last product of this one, four products or more ahead of its first there.
     int buf = 0;                                     // of step s
     auto step = [&](auto parity, int s) {
-        constexpr int P = decltype(parity)::value;
-        constexpr int kA[6] = {2, 1, 0, 1, 0, 0}, kB[6] = {0, 1, 2, 0, 1, 0};
+        constexpr int kA[6] = {1, 1, 2, 0, 0, 0}, kB[6] = {1, 0, 0, 1, 0, 2};
         const int next = buf == kBufs - 1 ? 0 : buf + 1, free = next == kBufs - 1 ? 0 : next + 1;
-        fetch(std::integral_constant<int, 1 - P>(), next);
 #pragma unroll
         for (int i = 0; i < 24; ++i) {
             const int t = i >> 2, q = (i >> 1) & 1, r = i & 1;
+            floatx16& sum = kA[t] + kB[t] ? low[q][r] : acc[q][r];
             __builtin_amdgcn_sched_barrier(0);
-            acc[q][r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[P][q][kA[t]], b[P][r][kB[t]], acc[q][r], 0, 0, 0);
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[q][kA[t]], b[r][kB[t]], sum, 0, 0, 0);
             take(parity, i, free);
+            if (i == 7) fetch(a, 1, next);
+            if (i == 11) fetch(a, 2, next);
+            if (i == 15) fetch(b, 1, next);
+            if (i == 19) fetch(b, 0, next);
+            if (i == 23) {
+                fetch(a, 0, next);
+                fetch(b, 2, next);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
         load(parity, s + 4);
@@ -196,16 +207,18 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
         bits |= __shfl_xor(bits, 2, 64);
         if (j == 0) s_lost[kTile * i + row] = bits;
     }
-    float4* other = reinterpret_cast<float4*>(lds);
+    float4* other = reinterpret_cast<float4*>(lds) + (wave & 3) * 2048 + lane;       // [4 waves][16 fours of acc and of low][64 lanes]
     if (half)
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int r = 0; r < 2; ++r)
 #pragma unroll
-                for (int u4 = 0; u4 < 4; ++u4)
-                    other[(((wave & 3) * 4 + q * 2 + r) * 4 + u4) * 64 + lane] =
-                        make_float4(acc[q][r][4 * u4], acc[q][r][4 * u4 + 1], acc[q][r][4 * u4 + 2], acc[q][r][4 * u4 + 3]);
+                for (int u4 = 0; u4 < 4; ++u4) {
+                    const floatx16 &h = acc[q][r], &l = low[q][r];
+                    other[((q * 2 + r) * 4 + u4) * 128] = make_float4(h[4 * u4], h[4 * u4 + 1], h[4 * u4 + 2], h[4 * u4 + 3]);
+                    other[((q * 2 + r) * 4 + u4) * 128 + 64] = make_float4(l[4 * u4], l[4 * u4 + 1], l[4 * u4 + 2], l[4 * u4 + 3]);
+                }
     __syncthreads();
     if (half) return;
     uint32_t most = 0, least = 0xffffffffu;          // of the sums' sizes, as whole numbers; of those that are not zero, less one
@@ -215,10 +228,10 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
         for (int r = 0; r < 2; ++r)
 #pragma unroll
             for (int u4 = 0; u4 < 4; ++u4) {
-                const float4 v = other[((wave * 4 + q * 2 + r) * 4 + u4) * 64 + lane];
+                const float4 h = other[((q * 2 + r) * 4 + u4) * 128], l = other[((q * 2 + r) * 4 + u4) * 128 + 64];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float sum = acc[q][r][4 * u4 + i] + (&v.x)[i];
+                    const float sum = (acc[q][r][4 * u4 + i] + (&h.x)[i]) + (low[q][r][4 * u4 + i] + (&l.x)[i]);
                     const uint32_t size = __float_as_uint(sum) & 0x7fffffffu;
                     acc[q][r][4 * u4 + i] = sum;
                     most = max(most, size);
