@@ -209,8 +209,11 @@ extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bia
     ST_CHECK(algo != 2 || library_can, "gemm: the library path has no activation %d before a residual sum", act);
     if (dtype == kF32 && (algo == 0 ? f32_split_pays(M, N, K) : algo == 3 && f32_split_can(M, N, K)) && (!ex.k_cache || (ex.q_size | ex.page_stride) % 4 == 0) &&
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out) |
-          reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(ex.scratch) | reinterpret_cast<uintptr_t>(ex.k_cache) | reinterpret_cast<uintptr_t>(ex.v_cache)) & 15) == 0)
-        return gemm_f32_split((float*)out, (const float*)x, (const float*)w, bias, residual, M, N, K, act, ex, stream);
+          reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(ex.scratch) | reinterpret_cast<uintptr_t>(ex.k_cache) | reinterpret_cast<uintptr_t>(ex.v_cache)) & 15) == 0) {
+        const int rc = gemm_f32_split((float*)out, (const float*)x, (const float*)w, bias, residual, M, N, K, act, ex, stream);
+        if (rc == 0) count_gemm_path(kPathSplitF32);
+        return rc;
+    }
     const bool to_library = algo == 2 || (algo == 0 && !ex.ln_x && !ex.mg_o && library_can &&
         (dtype == kF32 || M >= g_library_min_rows ||
          ((int64_t)N * K >= g_library_min_weights && K >= g_library_min_depth)));
@@ -275,7 +278,7 @@ extern "C" int st_gemm_library_rule(int min_rows, int64_t min_weights, int min_d
 }
 
 // Calls of st_gemm per kernel family since the last reset (order of st::GemmPath); returns the
-// number of families.  `out` may be null.  (The products of gemm_f32_split are in none of them: which they are follows from the sizes, f32_split_pays.)
+// number of families.  `out` may be null.
 extern "C" int st_gemm_path_counts(uint64_t* out, int reset) {
     for (int i = 0; i < kNumGemmPaths; ++i) {
         const uint64_t v = reset ? g_path_counts[i].exchange(0) : g_path_counts[i].load();

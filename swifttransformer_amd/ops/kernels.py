@@ -383,7 +383,7 @@ class tuned_products:
 
 
 GEMM_PATHS = ("library", "generic_f32", "generic_bf16", "resident", "resident_norm", "resident_merge",
-              "resident_staged", "skinny16", "skinny32", "skinny64", "tiled_mfma", "wide")
+              "resident_staged", "skinny16", "skinny32", "skinny64", "tiled_mfma", "wide", "split_f32")
 
 
 def gemm_path_counts(reset: bool = False) -> dict:

@@ -50,7 +50,9 @@ def test_chosen_and_closer_than_the_library():
     x, w, _ = operands(701, 2048, 2048)
     assert K._gemm_scratch(701, 2048, 2048, 0, False) > 0 and K._gemm_scratch(64, 2048, 2048, 0, False) == 0
     ref = x.double() @ w.double().T
+    K.gemm_path_counts(reset=True)
     own, lib = K.gemm(x, w), K.gemm(x, w, algo=2)
+    assert {n: c for n, c in K.gemm_path_counts().items() if c} == {"split_f32": 1, "library": 1}
     assert torch.equal(own, K.gemm(x, w, algo=3)) and torch.equal(own, K.gemm(x, w))
     assert float((own - ref).norm()) < float((lib - ref).norm())
 
