@@ -51,7 +51,7 @@ int st_gemm_wide_workgroups(int mode);
 int st_gemm_can_fuse_norm(int M, int N, int K, int dtype);
 int st_gemm_wide_offered(int M, int N, int K, int dtype);
 int st_gemm_wide_groups();
-int64_t st_gemm_scratch(int M, int N, int K, int dtype);
+int64_t st_gemm_scratch(int M, int N, int K, int dtype, int algo);
 int st_gemm_can_fuse_merge(int M, int N, int K, int splits, int heads, int head_dim, int dtype);
 
 // window > 0: a row reads the last `window` positions; window < 0: the positions of its own chunk of -window

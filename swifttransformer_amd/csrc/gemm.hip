@@ -106,16 +106,13 @@ int gemm_wide(float* out, const bf16_t* x, const bf16_t* w, const float* bias, i
               const StGemmExtras& ex, hipStream_t stream);
 int gemm_library(void* out, const void* x, const void* w, const float* bias, const float* residual,
                  int M, int N, int K, int act, int out_f32, int dtype, float alpha, hipStream_t stream, bool* handled);
+bool gemm_f32_split_pays(int M, int N, int K);
 int64_t gemm_f32_split_scratch(int M, int N, int K);
 int gemm_f32_split(float* out, const float* x, const float* w, const float* bias, const float* residual, int M, int N, int K, int act,
                    const StGemmExtras& ex, hipStream_t stream);
 
-// Float products that gemm_f32_split takes, and those it is asked for (the others go to the library): most of a tile's 128 rows, and enough
-// tiles or depth to fill the chip.  us, the library's best of 32 and gemm_f32_split, by rows x features x depth: 2.1e9 of them (128 x
-// 8,192 x 2,048) 37 and 39, (512 x 2,048 x 2,048) 38 and 37, 2.5e9 (200 x 6,144 x 2,048) 53 and 51, (384 x 2,560 x 2,560) 45 and 42,
-// 3.4e9 (200 x 2,048 x 8,192) 70 and 55; 1.6e9 (701 x 3,072 x 768) 36 and 39; 96 rows of 2,560 x 10,240 (2.5e9) 59 either way, 64 59 and 344.
+// Float products that gemm_f32_split takes
 static bool f32_split_can(int M, int N, int K) { return N % 4 == 0 && K % 4 == 0 && M >= 1; }
-static bool f32_split_pays(int M, int N, int K) { return f32_split_can(M, N, K) && M >= 96 && (int64_t)M * N * K >= 2500000000ll; }
 
 // Float products of prompts go to gemm_f32_split, others to the library when it has a kernel (the other float kernel here is the
 // plain tiled one).  For bfloat16:
@@ -207,9 +204,13 @@ extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bia
     const bool in_epilogue = activation_in_library(act);
     const bool library_can = (in_epilogue || !residual) && (!scaled || (act == 0 && (!bias || ex.bias_unscaled)));
     ST_CHECK(algo != 2 || library_can, "gemm: the library path has no activation %d before a residual sum", act);
-    if (dtype == kF32 && (algo == 0 ? f32_split_pays(M, N, K) : algo == 3 && f32_split_can(M, N, K)) && (!ex.k_cache || (ex.q_size | ex.page_stride) % 4 == 0) &&
+    // (without the scratch for its best split a product may take several times as long: those that are not asked for go to the library)
+    if (dtype == kF32 && f32_split_can(M, N, K) &&
+        (algo == 3 || (algo == 0 && gemm_f32_split_pays(M, N, K) && (ex.scratch ? ex.scratch_floats : 0) >= gemm_f32_split_scratch(M, N, K))) &&
+        (!ex.k_cache || (ex.q_size | ex.page_stride) % 4 == 0) &&
         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out) |
-          reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(ex.scratch) | reinterpret_cast<uintptr_t>(ex.k_cache) | reinterpret_cast<uintptr_t>(ex.v_cache)) & 15) == 0) {
+          reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(ex.scratch) |
+          reinterpret_cast<uintptr_t>(ex.k_cache) | reinterpret_cast<uintptr_t>(ex.v_cache)) & 15) == 0) {
         const int rc = gemm_f32_split((float*)out, (const float*)x, (const float*)w, bias, residual, M, N, K, act, ex, stream);
         if (rc == 0) count_gemm_path(kPathSplitF32);
         return rc;
@@ -257,9 +258,11 @@ extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bia
     return 0;
 }
 
-// Floats of scratch (StGemmExtras::scratch) that a product asks for; it runs without too, with fewer workgroups at its end.
-extern "C" int64_t st_gemm_scratch(int M, int N, int K, int dtype) {
-    return dtype == kF32 && f32_split_pays(M, N, K) ? gemm_f32_split_scratch(M, N, K) : 0;
+// Floats of scratch (StGemmExtras::scratch) that a product asks for, by algo (0 or 3): with less, one of algo 0 goes to the library, one of
+// algo 3 runs with fewer workgroups at its end.
+extern "C" int64_t st_gemm_scratch(int M, int N, int K, int dtype, int algo) {
+    if (dtype != kF32 || !f32_split_can(M, N, K) || !(algo == 3 || (algo == 0 && gemm_f32_split_pays(M, N, K)))) return 0;
+    return gemm_f32_split_scratch(M, N, K);
 }
 
 // The rule by which bfloat16 products go to the vendor library: from `min_rows` rows on, and below

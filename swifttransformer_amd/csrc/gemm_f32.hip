@@ -339,8 +339,8 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(
 }
 
 // How a product is dealt out: `whole` tiles by workgroups of their own (whole rounds of a workgroup a compute unit), the rest by
-// `splits` workgroups each.
-struct Deal { int tiles_m, tiles, whole, splits; };
+// `splits` workgroups each; the longest that a compute unit has to do are `steps` steps of a tile.
+struct Deal { int tiles_m, tiles, whole, splits, steps; };
 
 Deal deal(int M, int N, int K) {
     Deal d;
@@ -358,10 +358,14 @@ Deal deal(int M, int N, int K) {
         const double cost = (double)((rest * s + units - 1) / units) * share + rest * s * 0.033 + 4;
         if (cost < best) { best = cost; d.splits = s; }
     }
+    d.steps = d.tiles / units * steps + (rest * d.splits + units - 1) / units * ((steps + d.splits - 1) / d.splits);
     return d;
 }
 
 }  // namespace
+
+// Whether a product is faster here than in the library: most of a tile's 128 rows, and enough tiles or depth to fill the chip.
+bool gemm_f32_split_pays(int M, int N, int K) { return M >= 96 && (int64_t)M * N * K >= 2500000000ll; }
 
 // Floats of scratch with which gemm_f32_split deals its tiles out best (0: none).
 int64_t gemm_f32_split_scratch(int M, int N, int K) {

@@ -54,7 +54,7 @@ def _lib():
         lib.st_gemm_can_fuse_norm.argtypes = [_c_int, _c_int, _c_int, _c_int]
         lib.st_gemm_wide_offered.argtypes = [_c_int, _c_int, _c_int, _c_int]
         lib.st_gemm_can_fuse_merge.argtypes = [_c_int] * 7
-        lib.st_gemm_scratch.argtypes, lib.st_gemm_scratch.restype = [_c_int] * 4, _c_i64
+        lib.st_gemm_scratch.argtypes, lib.st_gemm_scratch.restype = [_c_int] * 5, _c_i64
         lib.st_gemm_library_tuning.argtypes = [_c_int]
         lib.st_attn_rows_gated.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_p,
                                            _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_f, _c_int, _c_f,
@@ -424,11 +424,11 @@ def wide_offered(M: int, N: int, K: int, dtype: torch.dtype) -> bool:
 
 
 @functools.lru_cache(maxsize=4096)
-def _gemm_scratch(M: int, N: int, K: int, code: int, most: bool) -> int:
+def _gemm_scratch(M: int, N: int, K: int, code: int, most: bool, algo: int = 0) -> int:
     """Floats of scratch that a product of M rows asks for; ``most``: that one of any number of rows up to M may ask for (it
     depends on the tiles of 128 rows)."""
     of = list(range(128, M, 128)) + [M] if most else [M]
-    return max(_lib().st_gemm_scratch(m, N, K, code) for m in of)
+    return max(_lib().st_gemm_scratch(m, N, K, code, algo) for m in of)
 
 
 # functions of the products' epilogues and of ``activation_multiply``, by the C interface's number
@@ -543,7 +543,7 @@ def gemm(x, w: torch.Tensor, *, bias: Optional[torch.Tensor] = None,
         idx = empty((n_scratch,), torch.int32, device)
         keep += [val, idx]
         ex.best_ids, ex.best_val, ex.best_idx = _ptr(best), _ptr(val), _ptr(idx)
-    scratch = _gemm_scratch(M, N, K, code, arena.measuring()) if code == F32 and M and algo in (0, 3) else 0
+    scratch = _gemm_scratch(M, N, K, code, arena.measuring(), int(algo)) if code == F32 and M and algo in (0, 3) else 0
     if scratch:
         if ex is None:
             ex = _GemmExtras()

@@ -20,6 +20,11 @@ def operands(M, N, D, seed=0):
     return x, w, g
 
 
+def parted(M, N, D):
+    """Whether the product has tiles that are parted over the depth and summed (it asks for room for their sums)."""
+    return K._gemm_scratch(M, N, D, 0, False, 3) > 0
+
+
 def check(y, x, w, bias=None, residual=None, scale=1.0, extra=0.0):
     ref = x.double() @ w.double().T
     size = x.double().abs() @ w.double().abs().T
@@ -36,9 +41,11 @@ def check(y, x, w, bias=None, residual=None, scale=1.0, extra=0.0):
 
 
 # edges of the 128 x 128 tiles, depths that are no whole steps of 32, tiles in whole rounds, split ones and both (256 compute units)
-@pytest.mark.parametrize("M,N,D", [(1, 4, 4), (3, 12, 28), (127, 132, 32), (128, 128, 36), (129, 124, 64), (200, 260, 100), (96, 512, 96),
-                                   (257, 1028, 516), (701, 6144, 512), (1000, 4100, 1000), (130, 2048, 4096)])
-def test_shapes(M, N, D):
+@pytest.mark.parametrize("M,N,D,parts", [
+    (1, 4, 4, False), (3, 12, 28, False), (127, 132, 32, False), (128, 128, 36, False), (129, 124, 64, False), (200, 260, 100, False), (96, 512, 96, False),
+    (257, 1028, 516, True), (701, 5376, 512, False), (701, 6144, 512, True), (1000, 4100, 1000, True), (130, 2048, 4096, True), (1, 4, 2052, True)])
+def test_shapes(M, N, D, parts):
+    assert parted(M, N, D) == parts
     x, w, g = operands(M, N, D)
     bias = torch.empty(N, device="cuda").normal_(0, 1, generator=g)
     check(K.gemm(x, w, algo=3), x, w)
@@ -73,9 +80,11 @@ def test_most_scratch_of_smaller_steps():
     assert not arena.measuring()
 
 
-@pytest.mark.parametrize("M,N", [(300, 256), (701, 2048)])
-def test_epilogues(M, N):
-    x, w, g = operands(M, N, 512)
+# (every epilogue of the kernel and of the sum of parted tiles)
+@pytest.mark.parametrize("M,N,D,parts", [(300, 256, 516, True), (701, 2048, 512, False), (701, 2048, 2048, True)])
+def test_epilogues(M, N, D, parts):
+    assert parted(M, N, D) == parts
+    x, w, g = operands(M, N, D)
     bias = torch.empty(N, device="cuda").normal_(0, 1, generator=g)
     residual = torch.empty(M, N, device="cuda").normal_(0, 1, generator=g)
     plain = K.gemm(x, w, algo=3)
@@ -90,11 +99,12 @@ def test_epilogues(M, N):
     check(unscaled, x, w * 0.5, bias=bias)
 
 
-@pytest.mark.parametrize("M", [130, 701])
-def test_pages(M):
+@pytest.mark.parametrize("M,D,parts", [(130, 256, False), (701, 256, False), (701, 1024, True)])
+def test_pages(M, D, parts):
     """A fused query, key and value product writes its pages as the library's product and the page write do."""
-    heads, hd, page, D = 4, 32, 8, 256
+    heads, hd, page = 4, 32, 8
     N = 3 * heads * hd
+    assert parted(M, N, D) == parts
     x, w, _ = operands(M, N, D)
     pages = -(-M // page) + 2
     table = torch.randperm(pages, device="cuda").int()[None].contiguous()
@@ -115,9 +125,11 @@ def test_pages(M):
     assert torch.equal(made[0][1] != 0, made[1][1] != 0)
 
 
-def test_numbers_that_parts_do_not_hold():
+@pytest.mark.parametrize("D,parts", [(200, False), (1032, True)])
+def test_numbers_that_parts_do_not_hold(D, parts):
     """Infinities, NaN, numbers past bfloat16's largest and tiny ones give what float products give, and other rows are as without."""
-    M, N, D = 300, 256, 200
+    M, N = 300, 256
+    assert parted(M, N, D) == parts
     x, w, _ = operands(M, N, D)
     clean = K.gemm(x, w, algo=3)
     inf, big = float("inf"), 3.4e38
@@ -148,6 +160,7 @@ def test_numbers_that_parts_do_not_hold():
 def test_tiny_numbers_with_large_ones(M, N, D, tiny, large):
     """Numbers that three bfloat16 numbers do not hold, in rows of x and of W, times numbers that make ordinary sums of them: no further off
     than D roundings of a float sum."""
+    assert parted(M, N, D) == (D > 1000)
     x, w, g = operands(M, N, D)
     normal = lambda *s: torch.empty(*s, device="cuda").normal_(0, 1, generator=g).double()
     x[5], x[M - 2] = (normal(D) * 2.0 ** tiny).float(), torch.where(torch.arange(D, device="cuda") == D - 40, 2.0 ** tiny * 1.2345678, 0.0)
@@ -167,6 +180,7 @@ def test_tiny_numbers_with_large_ones(M, N, D, tiny, large):
 @pytest.mark.parametrize("M,N,D", [(300, 256, 200), (701, 2048, 2048)])
 def test_rows_do_not_change_each_other(M, N, D):
     """Infinities, NaN, numbers past bfloat16's largest and tiny ones in some rows of x: the others' results stay the same to the last bit."""
+    assert parted(M, N, D) == (D > 1000)
     x, w, _ = operands(M, N, D)
     clean = K.gemm(x, w, algo=3)
     x[3, 7], x[70, 0], x[140, D - 1], x[200, 5], x[201, 3] = float("inf"), -float("inf"), float("nan"), 3.4e38, 1e-42
@@ -176,6 +190,24 @@ def test_rows_do_not_change_each_other(M, N, D):
     y = K.gemm(x, w, algo=3)
     assert torch.equal(y[rows], clean[rows])
     assert not torch.equal(y[201], clean[201])
+
+
+def test_without_room_for_the_sums():
+    """A caller of the C entry that brings no scratch: the library, as before there was a kernel that asks for it; too little: the same."""
+    import ctypes
+    M, N, D = 200, 2048, 8192
+    x, w, _ = operands(M, N, D)
+    assert K._gemm_scratch(M, N, D, 0, False) > 4
+    room, out = torch.empty(4, device="cuda"), torch.empty(M, N, device="cuda")
+    ex = K._GemmExtras()
+    ex.scratch, ex.scratch_floats = room.data_ptr(), 4
+    for extras in (None, ctypes.byref(ex)):
+        K.gemm_path_counts(reset=True)
+        assert K._lib().st_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), None, None, M, N, D, 0, 0, 1, 0, extras,
+                                torch.cuda.current_stream().cuda_stream) == 0
+        assert K.gemm_path_counts()["library"] == 1 and K.gemm_path_counts()["split_f32"] == 0
+        ref, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+        assert bool(((out.double() - ref).abs() <= D * 2.0 ** -24 * size).all())
 
 
 def test_rows_off_16_bytes_go_to_the_library():
