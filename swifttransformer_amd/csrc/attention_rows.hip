@@ -393,8 +393,7 @@ static int launch_rows(void* out, float* part_o, float* part_lse, const void* q,
     while (lpk < need) lpk <<= 1;
     ST_CHECK(lpk <= 64, "attention: head_dim %d is too large for this kernel (at most %d)",
              head_dim, 64 * VEC);
-    const int G = num_waves * (64 / lpk);
-    const size_t lds = (size_t)(2 * G + G * head_dim + 16 + max_pages) * sizeof(float);
+    const size_t lds = (size_t)(16 + num_waves * head_dim + max_pages) * sizeof(float);      // (the kernel's layout)
     dim3 grid(num_q_heads, num_tokens, num_splits);
 #define ST_ROWS(L)                                                                              \
     attn_rows_kernel<T, L><<<grid, num_waves * 64, lds, stream>>>((T*)out, part_o, part_lse, (const T*)q,  \
