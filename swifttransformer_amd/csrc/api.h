@@ -299,14 +299,15 @@ int st_moe_down(float* out, const float* residual, float* pair_out, const void* 
                 float out_scale, int dtype, hipStream_t stream);
 // out[t, n] = residual[t, n] + out_scale * sum_j weights[t * top + j] * pair_out[place_of_pair[t * top + j], n]
 // (weights null: ones; residual null: zeros)
-// Both for one or two tokens of up to four choices and tiles of 16 places, in one kernel (ids: the choices; the same numbers).
-int st_moe_down_sum_offered(int num_tokens, int top);
-int st_moe_down_sum(float* out, const float* residual, const void* y, const void* w_down, const int* place_of_pair, const float* weights,
-                    const int* ids, const void* x, int experts, int num_tokens, int top, int width, int inner, float out_scale, int dtype,
-                    hipStream_t stream);
 int st_moe_combine(float* out, const float* residual, const float* pair_out, const int* place_of_pair,
                    const float* weights, const int* ids, const void* x, int experts, int num_tokens, int top, int width,
                    float out_scale, int dtype, hipStream_t stream);
+// st_moe_down and st_moe_combine for one or two tokens of up to four choices and tiles of 16 places, in one kernel (the same numbers).
+// ids: the choices, always; x: the tokens' rows where there are identity experts, or null.  offered: whether it is no slower than the two.
+int st_moe_down_sum_offered(int num_tokens, int top, int width, int inner, int dtype);
+int st_moe_down_sum(float* out, const float* residual, const void* y, const void* w_down, const int* place_of_pair, const float* weights,
+                    const int* ids, const void* x, int experts, int num_tokens, int top, int width, int inner, float out_scale, int dtype,
+                    hipStream_t stream);
 
 // ---- float operations on the residual stream (csrc/stream_ops.hip)
 // y = tanh(alpha[0] * x[row]) * w + b (b may be null) of every row, or of the rows picked by `rows`

@@ -20,6 +20,7 @@
 #include "activation.h"
 #include "fragment.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace st {
@@ -395,7 +396,8 @@ __global__ __launch_bounds__(1024) void moe_router_align_kernel(
 // features and so: gate and up of 2,048 x 2,048, one token of two experts 17.6 and 8.0, eight tokens of ten 34.7 and 30.9, output product
 // 8.8 and 5.0, 17.1 and 16.4; 24 tokens, 4,096 x 4,096, thirteen experts 155 and 151, 77.8 and 74.2; one of 768 x 768 5.9 and 5.3, 4.0 and 3.5.
 // (The output product with the rows of all 16 places read, pair or not: 12.3, 23.5, 101 and 4.8.)
-template <typename T, int MATS>
+// FIRST: pieces of depth a batch.
+template <typename T, int MATS, int FIRST = MATS == 1 ? 16 : 8>
 __device__ inline void moe_depth_share(floatx4* acc, const T* xr, const T* const* wr, int K, int vec) {
     constexpr int D = Frag<T>::kDepth, L = Frag<T>::kLane;
     const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3, g = lane >> 4;
@@ -421,7 +423,7 @@ __device__ inline void moe_depth_share(floatx4* acc, const T* xr, const T* const
         }
     };
     if (vec) {
-        batches(Steps<MATS == 1 ? 16 : 8>());
+        batches(Steps<FIRST>());
         batches(Steps<4>());
     }
     for (; k0 < end; k0 += D) {
@@ -518,13 +520,16 @@ __global__ __launch_bounds__(256) void moe_down_few_kernel(
 
 // The output product of one or two tokens with the sum over their choices: four waves a choice, whose sums meet in LDS in the order of the
 // choices, so that neither the pairs' results nor a kernel that adds them stand between (the same numbers to the last bit).  Tokens do
-// not share an expert's weights, so no more than two.  grid (ceil(width / 16), tokens), 256 threads a choice.
-template <typename T>
-__global__ __launch_bounds__(1024) void moe_down_sum_kernel(
+// not share an expert's weights, so no more than two.  An instance a number of choices, so that the registers are those of its own threads
+// (one of 1,024 threads for all spilled 27 of them: 2,048 x 2,048, 2 choices 23.6 us a call, 20.0 so); four choices, 128 registers a thread, ask
+// for 8 pieces of depth at once instead of 16.  grid (ceil(width / 16), tokens), 256 threads a choice.
+template <typename T, int TOP>
+__global__ __launch_bounds__(256 * TOP) void moe_down_sum_kernel(
     float* out, const float* residual, const T* __restrict__ y, const T* __restrict__ w_down, const int* __restrict__ place_of_pair,
-    const float* __restrict__ weights, const int* __restrict__ ids, const T* __restrict__ x, int experts, int top, int width, int inner,
+    const float* __restrict__ weights, const int* __restrict__ ids, const T* __restrict__ x, int experts, int width, int inner,
     float out_scale, int vec) {
-    __shared__ float lds[16][16];
+    constexpr int top = TOP;
+    __shared__ float lds[4 * TOP][16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, n0 = blockIdx.x * 16;
     const int64_t pair0 = (int64_t)blockIdx.y * top, at = (int64_t)blockIdx.y * width + min(n0 + r16, width - 1);
     const int place = place_of_pair[pair0 + (wave >> 2)], id = ids[pair0 + (wave >> 2)];
@@ -535,7 +540,7 @@ __global__ __launch_bounds__(1024) void moe_down_sum_kernel(
     if (place >= 0) {
         const T* wr[1] = {w_down + ((int64_t)id * width + min(n0 + r16, width - 1)) * inner};
         floatx4 acc[1] = {floatx4{0.f, 0.f, 0.f, 0.f}};
-        moe_depth_share<T, 1>(acc, y + (int64_t)place * inner, wr, inner, vec);
+        moe_depth_share<T, 1, TOP == 4 ? 8 : 16>(acc, y + (int64_t)place * inner, wr, inner, vec);
         if (lane < 16) lds[wave][lane] = acc[0][0];        // (all rows of the block are the pair's)
     }
     __syncthreads();
@@ -1305,31 +1310,45 @@ extern "C" int st_moe_down(float* out, const float* residual, float* pair_out, c
     return 0;
 }
 
-// ids and x (both or neither): a choice of `experts` or above is an identity expert, whose result is the token's row of x
-// [tokens, width] in the storage type.
-// Whether st_moe_down_sum takes so many tokens and choices.
-extern "C" int st_moe_down_sum_offered(int num_tokens, int top) { return num_tokens <= 2 && top >= 1 && top <= 4; }
+// Whether st_moe_down_sum is no slower than st_moe_down and st_moe_combine.  It saves a kernel, 1.5 to 2.5 us, but a workgroup reads all of a
+// token's choices where the other has one for each: where `width` has few blocks of 16 features, few compute units then read long rows.
+// So the bytes a workgroup reads of each feature are bounded, the more workgroups there are the less.  us a call, two kernels and one:
+// one token, bfloat16, 768 x 768 of 2, 3, 4 choices (3, 4.6, 6.1 KB) 14.5 and 13.4, 15.4 and 14.7, 16.5 and 16.1; width 768, inner 2,048 of
+// 2, 3, 4 (8, 12, 16 KB) 16.2 and 16.3, 18.2 and 20.3, 20.0 and 23.7; 2,048 x 2,048 of 2, 3, 4 20.7 and 20.0, 28.3 and 27.1, 29.4 and 30.8;
+// 1,024, inner 4,096 of 1, 2, 4 (8, 16, 32 KB) 19.0 and 17.4, 22.5 and 24.6, 31.9 and 39.9, in float 28.0 and 25.1, 34.5 and 39.5, 51.4 and 73.6;
+// 4,096 x 4,096 of 2 45.7 and 44.3.  Two tokens that share an expert read it twice, which large matrices do not forgive: 2,048 x 2,048 of 2
+// 28.6 and 26.2, in float (16 MB) 46.4 and 42.2, 4,096 x 4,096 of 2 46.7 and 54.5.
+extern "C" int st_moe_down_sum_offered(int num_tokens, int top, int width, int inner, int dtype) {
+    if (num_tokens > 2 || top < 1 || top > 4) return 0;
+    const int64_t elem = dtype == kF32 ? 4 : 2, units = device_compute_units();
+    const int64_t groups = std::min<int64_t>((int64_t)(width + 15) / 16 * num_tokens, units);
+    return (top == 1 || top * inner * elem <= 6144 + 12288 * groups / units) && (num_tokens < 2 || elem * width * inner <= 16 << 20);
+}
 
 // st_moe_down (into the pairs' results) and st_moe_combine at once, for the tokens of tiles of 16 places.
 extern "C" int st_moe_down_sum(float* out, const float* residual, const void* y, const void* w_down, const int* place_of_pair,
                                const float* weights, const int* ids, const void* x, int experts, int num_tokens, int top, int width, int inner,
                                float out_scale, int dtype, hipStream_t stream) {
     ST_CHECK(num_tokens >= 0 && width > 0 && inner > 0, "moe_down_sum: bad sizes");
-    ST_CHECK(st_moe_down_sum_offered(num_tokens, top), "moe_down_sum: one or two tokens of up to four choices, not %d of %d", num_tokens, top);
+    ST_CHECK(num_tokens <= 2 && top >= 1 && top <= 4, "moe_down_sum: one or two tokens of up to four choices, not %d of %d", num_tokens, top);
     ST_CHECK(out && y && w_down && place_of_pair && ids, "moe_down_sum: null operand");
     ST_CHECK(dtype == kF32 || dtype == kBF16, "moe_down_sum: unknown dtype %d", dtype);
     if (num_tokens == 0) return 0;
     const int vec = rows_vectorised(y, w_down, nullptr, inner, dtype);
     const dim3 grid((width + 15) / 16, num_tokens);
-#define ST_MDS(T)                                                                                                        \
-    moe_down_sum_kernel<T><<<grid, 256 * top, 0, stream>>>(out, residual, (const T*)y, (const T*)w_down, place_of_pair, weights, ids, \
-                                                           (const T*)x, experts, top, width, inner, out_scale, vec)
-    if (dtype == kF32) ST_MDS(float); else ST_MDS(bf16_t);
+#define ST_MDS(T, TOP)                                                                                                    \
+    moe_down_sum_kernel<T, TOP><<<grid, 256 * TOP, 0, stream>>>(out, residual, (const T*)y, (const T*)w_down, place_of_pair, weights, ids, \
+                                                                (const T*)x, experts, width, inner, out_scale, vec)
+#define ST_MDS_T(T) do { if (top == 1) ST_MDS(T, 1); else if (top == 2) ST_MDS(T, 2); else if (top == 3) ST_MDS(T, 3); else ST_MDS(T, 4); } while (0)
+    if (dtype == kF32) ST_MDS_T(float); else ST_MDS_T(bf16_t);
+#undef ST_MDS_T
 #undef ST_MDS
     ST_LAUNCH_CHECK("moe_down_sum");
     return 0;
 }
 
+// ids and x (both or neither): a choice of `experts` or above is an identity expert, whose result is the token's row of x
+// [tokens, width] in the storage type.
 extern "C" int st_moe_combine(float* out, const float* residual, const float* pair_out, const int* place_of_pair,
                               const float* weights, const int* ids, const void* x, int experts, int num_tokens, int top,
                               int width, float out_scale, int dtype, hipStream_t stream) {

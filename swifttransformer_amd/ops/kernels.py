@@ -112,7 +112,7 @@ def _lib():
                                   _c_f, _c_int, _c_int, _c_p]
         lib.st_moe_down.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                     _c_f, _c_int, _c_p]
-        lib.st_moe_down_sum_offered.argtypes = [_c_int] * 2
+        lib.st_moe_down_sum_offered.argtypes = [_c_int] * 5
         lib.st_moe_down_sum.argtypes = [_c_p] * 8 + [_c_int] * 5 + [_c_f, _c_int, _c_p]
         lib.st_moe_combine.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_f, _c_int,
                                        _c_p]
@@ -1535,7 +1535,7 @@ def routed_experts(x: torch.Tensor, logits: torch.Tensor, w_gate: Optional[torch
         _check(lib.st_moe_align(_ptr(sorted_pairs), _ptr(place), _ptr(tile_expert), _ptr(ids), T * top, E, cap, tile, st))
     _check(lib.st_moe_up(_ptr(y), _ptr(x), _ptr(w_gate), _ptr(w_up), _ptr(sorted_pairs), _ptr(tile_expert),
                          _ptr(wts), cap, tile, int(top), W, F, float(limit), 2 if w_gate is None else 3 if clamped else int(on_output), code, st))
-    if tile == 16 and (on_output or top > 1) and lib.st_moe_down_sum_offered(T, int(top)):
+    if tile == 16 and (on_output or top > 1) and lib.st_moe_down_sum_offered(T, int(top), W, F, code):
         # the fewest tokens: the output product sums over a token's choices itself
         out = residual if residual is not None else empty((T, W), torch.float32, dev)
         _check(lib.st_moe_down_sum(_ptr(out), _ptr(residual), _ptr(y), _ptr(w_down), _ptr(place), _ptr(wts) if on_output else None, _ptr(ids),

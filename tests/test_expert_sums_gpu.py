@@ -15,6 +15,7 @@ pytestmark = pytest.mark.gpu
     (20, 28, 5, 3, "softmax_corrected", 2, True),        # depths of no whole pieces; identity experts
     (1000, 520, 8, 4, "softmax_all", 0, False),
     (96, 2056, 7, 2, "scaled_input", 0, False),          # weights on the inputs
+    (96, 520, 7, 2, "scaled_input", 0, False),           # (the rows before are too long for the kernel)
     (64, 64, 9, 5, "softmax_output", 0, False),          # more choices than the kernel takes
 ])
 def test_few_tokens(dtype, W, F, E, top, style, identity, clamped):
@@ -39,3 +40,16 @@ def test_few_tokens(dtype, W, F, E, top, style, identity, clamped):
             for n in (1, 2):
                 assert torch.equal(run(n, None), many[:n])
     assert bool(torch.isfinite(many).all()) and float(many.abs().max()) > 0
+
+
+@pytest.mark.parametrize("dtype,W,F,top,one,two", [
+    (torch.bfloat16, 768, 768, 4, True, True), (torch.float32, 768, 768, 3, False, True),
+    (torch.bfloat16, 1024, 4096, 1, True, True), (torch.bfloat16, 1024, 4096, 2, False, False),      # few workgroups, long rows
+    (torch.float32, 2048, 2048, 1, True, True), (torch.float32, 2048, 2056, 1, True, False),         # 16 MB and more a matrix
+    (torch.bfloat16, 2048, 2048, 3, True, True), (torch.bfloat16, 2048, 2048, 4, False, True),
+    (torch.bfloat16, 64, 64, 5, False, False),
+])
+def test_which_sizes_are_summed_so(dtype, W, F, top, one, two):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the line depends on the number of compute units")
+    assert [bool(K._lib().st_moe_down_sum_offered(n, top, W, F, K.dtype_code(dtype))) for n in (1, 2, 3)] == [one, two, False]
