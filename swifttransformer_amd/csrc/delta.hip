@@ -745,9 +745,12 @@ extern "C" int st_delta_step(void* out, const float* proj, int64_t stride, float
     const int cols = value_dim / (vec ? 4 : 1), pieces = cols * key_dim;
     int threads = 256;
     // Four pieces of 16 bytes a thread, or eight where there are more workgroups than compute units: a unit then holds four of 512 threads
-    // and their states are on their way together, instead of two of 1,024 (32 heads of 128 x 128: 24 requests 41.0 -> 28.6 us, 9 23.8 ->
-    // 17.7, 48 75.8 -> 52.6; 8 requests, a workgroup a unit, 14.1).
-    const bool many = vec && pieces <= 8 * 512 && (int64_t)heads * num_items > device_compute_units();
+    // and their states are on their way together, instead of two of 1,024 (32 heads of 128 x 128: 24 requests 41.5 -> 28.9 us, 9 24.0 ->
+    // 17.9, 48 76.5 -> 47.4; 96 x 128, 24 requests 35.9 -> 24.0; 72 x 128 32.5 -> 21.0; 16 heads of 68 x 240 25.5 -> 19.4).  States that four
+    // pieces a thread make workgroups of 512 threads of take eight, and 256, only where there are some rounds of them: 32 heads of 64 x
+    // 128 and 128 x 64 12.9 and 12.9 us with four, 13.2 and 13.8 with eight at 12 requests, 19.0 and 19.0, 18.3 and 19.5 at 24, 33.1 and 33.5,
+    // 28.9 and 29.9 at 48.
+    const bool many = vec && pieces <= 8 * 512 && (int64_t)heads * num_items > (pieces > 4 * 512 ? 1 : 4) * (int64_t)device_compute_units();
     while (threads < (many ? 512 : 1024) && threads * (many ? 8 : vec ? 4 : 16) < pieces) threads <<= 1;
     const int lanes = threads / cols < key_dim ? threads / cols : key_dim;
     const int np = (key_dim + lanes - 1) / lanes;

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("items,heads,qk,dk,dv,taps", [(9, 32, 8, 128, 128, 4), (65, 4, 4, 128, 128, 1), (24, 12, 3, 100, 96, 3), (9, 32, 8, 64, 256, 4),
-                                                       (40, 8, 8, 68, 240, 2), (9, 32, 16, 256, 256, 4)])
+                                                       (40, 8, 8, 68, 240, 2), (9, 32, 16, 256, 256, 4),
+                                                       (32, 32, 8, 64, 128, 4), (33, 32, 8, 64, 128, 4)])   # (either side of four workgroups a unit)
 def test_many_requests(items, heads, qk, dk, dv, taps):
     g = torch.Generator(device="cuda").manual_seed(items + dk + dv)
     rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
