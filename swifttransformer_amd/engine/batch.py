@@ -58,6 +58,8 @@ class StepContext:
     # of this step (lengths, slots); kernels size their work for `max_kv_len` = the longest
     # context that the recording serves (`tuning.short_span`, or all that the model allows)
     static_shapes: bool = False
+    # of such a step for short contexts: the longest context that the model allows (0: `max_kv_len` is that)
+    longest_kv_len: int = 0
     # the model's position encoding, for mixers to call its ``rotate`` (set by the model)
     position: Optional[object] = None
     # work lists that parts asked for through their ``step_planner`` (key -> StepPlan); a key is
@@ -229,7 +231,7 @@ class DecodeBuffers:
     padding (token_item = -1): kernels skip them."""
 
     def __init__(self, capacity: int, groups: Sequence[int], max_pages: int, page_size: int, device,
-                 max_positions: int):
+                 max_positions: int, longest: int = 0):
         self.capacity = capacity
         self.lay = BatchLayout(capacity, capacity, capacity, groups, max_pages)
         self.host = torch.zeros(self.lay.total, dtype=torch.int32).pin_memory()
@@ -238,7 +240,7 @@ class DecodeBuffers:
         self.groups = list(groups)
         self.max_pages = max_pages
         self.ctx = self.lay.context(self.dev, page_size, max_kv_len=max_positions, all_single=True,
-                                    static_shapes=True)
+                                    static_shapes=True, longest_kv_len=longest)
         hv = lambda n: self.lay.view(self.host_np, n)
         self._tok, self._pos, self._item = hv("token_ids"), hv("positions"), hv("token_item")
         self._start, self._len, self._off, self._slot = (hv("item_start"), hv("item_len"),

@@ -301,7 +301,7 @@ class ModelRunner:
 
     def _record(self, capacity: int, span: int) -> _RecordedStep:
         buffers = DecodeBuffers(capacity, self.paged_group_ids, self.max_pages_per_seq,
-                                self.cache_param.page_size, self.device, span)
+                                self.cache_param.page_size, self.device, span, self.model.max_positions)
         # one unrecorded run on padding rows first: loads code objects, sizes the allocator, and
         # has the library's products of this row count timed and chosen
         # The rows' best tokens are left where the next step's token ids are read: a step that

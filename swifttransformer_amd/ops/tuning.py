@@ -29,10 +29,12 @@ class Tuning:
     # every compute unit, at least this many keys a split (two workgroups a unit were 0-2 %
     # slower at batch 2 to 12, OPT-1.3B sizes).
     min_keys_per_split: int = 256
-    # Decode steps of requests with contexts of up to this many tokens have recordings of their own: where few rows' keys are
-    # split until there is a workgroup for every compute unit, one row of 12 heads of 64 takes (attention and output projection, us)
-    # 8.8 whole and 12.5 in 16 splits that a kernel merges at 57 keys, 11.0 and 12.8 at 300, 12.4 and 12.9 at 500; merged by the
-    # projection itself, in 8 splits, 10.2 at 97 keys (whole 8.9), 10.5 at 300 (whole 11.0): the two meet at about 210.
+    # Decode steps of requests with contexts of up to this many tokens have recordings of their own, in which few rows' keys are split
+    # less than in those for all contexts.  What a mixer does with them is its own rule (``PagedAttention._short_splits`` and the
+    # ``_splits`` of the others).  Whole steps of four layers, us, for all contexts and for short ones, at 30 and at 185 tokens: one request,
+    # opt-125m 132 -> 125, 132 -> 130; gisedra-125m (shared entries of 160, window) 359 -> 356, 367 -> 363; zimorax-1.3b (sinks) 469 ->
+    # 453, 476 -> 461; pupalix-125m 278 -> 254, 278 -> 265; four, gisedra-1.3b 720 -> 691, 735 -> 711; eight, fefozen-125m (gated
+    # latent) 206 -> 201, 205 -> 202.  Whole keys and splits that the output projection merges meet at about 200 (heads of 64).
     short_span: int = 192
     # A step that is not plain decoding is recorded when its shape comes up for this many-th time.
     record_after: int = 2

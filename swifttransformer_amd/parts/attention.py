@@ -25,7 +25,7 @@ import numpy as np
 from ..ops import kernels as K
 from ..ops.tuning import tuning
 from ..weights.loader import TensorSpec
-from .base import CacheNeed, Mixer, StepPlan, count_bucket
+from .base import CacheNeed, KeySpan, Mixer, StepPlan, count_bucket
 
 _compute_units: Dict[int, int] = {}
 
@@ -159,13 +159,7 @@ class PagedAttention(Mixer):
         """The most keys a row of this step reads."""
         return ctx.max_kv_len if self.window <= 0 else min(ctx.max_kv_len, self.window)
 
-    def _shape_row_kernel(self, ctx, rows: int):
-        """(key splits, waves per workgroup) of the row kernel.  A workgroup serves one
-        (row, head, split); when rows * heads alone does not fill the chip, a row's keys are
-        split over workgroups (merged by a second kernel), at least tuning.min_keys_per_split keys
-        each.  ctx.max_kv_len is the longest sequence of this step, or, for a recorded step,
-        the longest context that the recording serves: then the shape depends on the recording and the batch size alone."""
-        span = self.key_span(ctx)
+    def _key_splits(self, rows: int, span: int) -> int:
         groups = max(1, rows * self.num_heads)
         units = _target_workgroups()
         splits = min(-(-units // groups), max(1, span // tuning.min_keys_per_split), 32)
@@ -175,7 +169,40 @@ class PagedAttention(Mixer):
             # others waiting.  Workgroups of half the keys even that out (batch 10, 11, 17, 18: +2 to
             # 3 % a step; nothing where the last round is fuller).
             splits = 2
-        return max(1, splits), 4
+        return max(1, splits)
+
+    merges_in_projection = True     # the output projection may merge a row's splits itself (``attend``)
+
+    def _short_splits(self, rows: int, splits: int, longer: int, span: int) -> int:
+        """Splits of a recorded step for short contexts, where one for all contexts has ``longer`` of them.  A workgroup reads its
+        keys in passes of a key a lane group.  Up to so many passes whole keys win, more of them where the alternative needs a
+        kernel that merges; beyond, four passes a split.  Attention and output projection, us, whole, split as below and as for all
+        contexts, bfloat16: one row of 12 heads of 64 (6 passes for 192 keys, merged by the projection) 7.1 / - / 8.9 at 16 keys,
+        8.2 / - / 8.8 at 185; 6 heads of 128 (12 passes) 7.2 / 8.4 / 9.0, 9.4 / 8.9 / 8.9; 12 heads over shared entries of 160 (24)
+        8.3 / 8.8 / 9.2, 13.5 / 9.7 / 9.5; 32 heads over entries of 160 (merged by a kernel) 11.7 / - / 16.8, 17.0 / - / 17.8; float32, 12
+        heads of 64 (12) 10.5 / - / 13.3, 13.4 / - / 13.9, of 128 (24) 11.7 / 15.2 / 15.8, 17.3 / 16.2 / 16.1."""
+        lanes = 1
+        while lanes * 16 < self.head_dim * self.dtype.itemsize:
+            lanes <<= 1
+        passes = -(-span * lanes // 256)            # (four waves)
+        fused = self.merges_in_projection and K.can_fuse_merge(rows, self.hidden_size, self.q_size, longer, self.num_heads, self.head_dim, self.dtype)
+        if passes <= (6 if fused else 24 if self.dtype == torch.bfloat16 else 12):
+            return splits
+        return max(splits, min(longer, -(-passes // 4)))
+
+    def _shape_row_kernel(self, ctx, rows: int):
+        """(key splits, waves per workgroup) of the row kernel.  A workgroup serves one
+        (row, head, split); when rows * heads alone does not fill the chip, a row's keys are
+        split over workgroups (merged by a second kernel), at least tuning.min_keys_per_split keys
+        each.  ctx.max_kv_len is the longest sequence of this step, or, for a recorded step,
+        the longest context that the recording serves: then the shape depends on the recording and the batch size alone."""
+        span = self.key_span(ctx)
+        splits, longest = self._key_splits(rows, span), getattr(ctx, "longest_kv_len", 0)
+        if longest > ctx.max_kv_len:
+            longer = self._key_splits(rows, self.key_span(KeySpan(longest)))
+            if longer > splits:
+                splits = self._short_splits(rows, splits, longer, span)
+        return splits, 4
 
     def attend(self, qkv: torch.Tensor, ctx, cache, unmerged_ok: bool = False):
         """Attention of every row of ``qkv`` [T, q+2kv] over ``cache`` (already holding the rows' keys).

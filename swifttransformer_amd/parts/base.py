@@ -177,6 +177,14 @@ def fold_output_scale(weight: torch.Tensor, bias: Optional[torch.Tensor], scale:
     return w, b
 
 
+@dataclass(frozen=True)
+class KeySpan:
+    """What a mixer shapes a recorded step of single tokens by: the longest context that it serves, and, if that is not all, the
+    longest that the model allows (the fields of ``engine.batch.StepContext``)."""
+    max_kv_len: int
+    longest_kv_len: int = 0
+
+
 class Mixer(Part):
     graph_safe = True   # its forward launches only capturable work
 

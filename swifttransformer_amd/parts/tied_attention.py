@@ -34,6 +34,7 @@ class TiedKeyValueAttention(PagedAttention):
 
     raw_output_ok = True
     accepts_norm = False
+    merges_in_projection = False
 
     def __init__(self, spec, hidden_size, dtype):
         p = spec.params

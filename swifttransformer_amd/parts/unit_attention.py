@@ -35,6 +35,7 @@ class UnitQueryKeyAttention(PagedAttention):
 
     raw_output_ok = True
     accepts_norm = False
+    merges_in_projection = False
 
     def __init__(self, spec, hidden_size, dtype):
         p = spec.params
