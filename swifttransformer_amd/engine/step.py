@@ -12,7 +12,8 @@ Steps are launch-bound below some hundreds of tokens: some two hundred kernels w
 launches cost the host more than they cost the device.  A step is therefore recorded
 once per shape as a HIP graph over fixed index buffers and replayed; the kernels and
 the cache are the same as in the unrecorded path.  Steps of single tokens (decoding)
-are recorded per batch-size bucket, for short contexts and for all, at their first use; steps of any other composition
+are recorded per batch-size bucket, for short contexts (where a mixer has
+another shape for those) and for all, at their first use; steps of any other composition
 (prompt portions, alone or beside decode tokens) per (padded token count, lengths of the
 parts' work lists) once that shape has come up ``record_after`` times; their final norm
 and head run after the replay on the rows that are wanted, so the number of wanted rows
@@ -35,7 +36,7 @@ from ..models.decoder import DecoderModel
 from ..ops import kernels as K
 from ..ops.arena import StepArena, using as using_arena
 from ..ops.tuning import tuning
-from ..parts.base import BatchInfo
+from ..parts.base import BatchInfo, KeySpan, decode_shape
 from .batch import (DecodeBuffers, StepBuffers, StepContext, StepItem, check_items, pack_batch, run_planners,
                     token_bucket)
 
@@ -103,6 +104,7 @@ class ModelRunner:
         self.steps_run = 0
         self._recorded_spans: Dict[Tuple[int, int], _RecordedStep] = {}      # by rows and longest context
         self._recorded: Dict[int, _RecordedStep] = {}                        # of these the last one used, by rows
+        self._short_differs: Dict[Tuple[int, int], bool] = {}                # whether short contexts' steps of so many rows have a shape of their own
         self._recorded_general: Dict[tuple, _RecordedStep] = {}
         self._seen: Dict[tuple, int] = {}
         self.record_after = int(tuning.record_after if record_after is None else record_after)
@@ -284,15 +286,23 @@ class ModelRunner:
             b <<= 1
         return min(b, self.cache_param.max_seqs)
 
-    def _decode_span(self, longest: int) -> int:
-        """The longest context that the recorded step of requests with contexts of up to ``longest`` tokens is made for:
-        ``tuning.short_span`` or all that the model allows.  The parts shape their attention by it (``ctx.max_kv_len``)."""
-        short = tuning.short_span
-        return short if self.paged_group_ids and longest <= short < self.model.max_positions else self.model.max_positions
+    def _decode_span(self, capacity: int, longest: int) -> int:
+        """The longest context that the recorded step of up to ``capacity`` requests with contexts of up to ``longest`` tokens is made
+        for: ``tuning.short_span``, if any mixer has another shape for those, or all that the model allows."""
+        short, most = tuning.short_span, self.model.max_positions
+        if not self.paged_group_ids or longest > short or short >= most:
+            return most
+        differ = self._short_differs.get((capacity, short))
+        if differ is None:
+            differ = any(decode_shape(layer.mixer, KeySpan(short, most), capacity) != decode_shape(layer.mixer, KeySpan(most, most), capacity)
+                         for layer in self.model.layers)
+            self._short_differs[capacity, short] = differ
+        return short if differ else most
 
     def _decode_step(self, n: int, longest: int) -> _RecordedStep:
         """The recorded step of ``n`` single tokens whose contexts, the tokens included, are up to ``longest`` long."""
-        cap, span = self._bucket(n), self._decode_span(longest)
+        cap = self._bucket(n)
+        span = self._decode_span(cap, longest)
         rec = self._recorded_spans.get((cap, span))
         if rec is None:
             rec = self._recorded_spans[cap, span] = self._record(cap, span)

@@ -204,6 +204,9 @@ class PagedAttention(Mixer):
                 splits = self._short_splits(rows, splits, longer, span)
         return splits, 4
 
+    def decode_shape(self, span: KeySpan, rows: int):
+        return self._shape_row_kernel(span, rows)
+
     def attend(self, qkv: torch.Tensor, ctx, cache, unmerged_ok: bool = False):
         """Attention of every row of ``qkv`` [T, q+2kv] over ``cache`` (already holding the rows' keys).
         With ``unmerged_ok`` the result may be a ``SplitAttention`` that the output projection merges."""

@@ -195,6 +195,17 @@ class Mixer(Part):
         """The model's position part (one for all layers), told once after construction."""
         self.position = position
 
+    def decode_shape(self, span: KeySpan, rows: int):
+        """What a recorded step of ``rows`` single tokens takes from ``span``: recordings for which all mixers answer alike are the
+        same step.  Here: all of it with a cache of pages, else nothing."""
+        needs = self.cache_parts().values() if hasattr(self, "cache_parts") else [self.cache_need()]
+        return span if any(n is not None and n.kind == "paged_kv" for n in needs) else None
+
+
+def decode_shape(mixer, span: KeySpan, rows: int):
+    """``mixer.decode_shape``; of a mixer without one, ``span`` itself."""
+    return mixer.decode_shape(span, rows) if hasattr(mixer, "decode_shape") else span
+
 
 class PositionEncoding(Part):
     rotates = False          # True: mixers must call ``rotate`` on their queries and keys

@@ -137,6 +137,9 @@ class GatedLatentAttention(Mixer):
         groups = max(1, rows * -(-self.num_heads // 32))
         return max(1, min(-(-_target_workgroups() // groups), -(-span // 128), 32))
 
+    def decode_shape(self, span, rows: int):
+        return self._splits(span, rows)
+
     def forward(self, x_t: torch.Tensor, residual32: Optional[torch.Tensor], ctx, cache, write: bool = True) -> torch.Tensor:
         """residual32 + mix(x_t) (``residual32`` None: the second alone)."""
         if write != self.own_latent:

@@ -13,7 +13,7 @@ from typing import Dict, List, Optional
 import torch
 
 from ..weights.loader import TensorSpec
-from .base import CacheNeed, Mixer, build_part
+from .base import CacheNeed, Mixer, build_part, decode_shape
 
 
 class ParallelMixers(Mixer):
@@ -55,6 +55,9 @@ class ParallelMixers(Mixer):
                 if need is not None:
                     parts[side] = need
         return parts
+
+    def decode_shape(self, span, rows: int):
+        return tuple(decode_shape(m, span, rows) for m in self.branches.values())
 
     def _cache_of(self, side: str, cache):
         m = self.branches[side]

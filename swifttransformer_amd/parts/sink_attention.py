@@ -100,6 +100,9 @@ class SinkAttention(Mixer):
         blocks = max(1, -(-span // 64))
         return max(1, min(256 // max(rows, 1), blocks, 16))
 
+    def decode_shape(self, span, rows: int):
+        return self._splits(span, rows)
+
     accepts_norm = True     # forward(..., norm=part) normalises residual32 itself
 
     def forward(self, x_t: Optional[torch.Tensor], residual32: torch.Tensor, ctx, cache, write: bool = True,

@@ -102,6 +102,9 @@ class GatedWindowAttention(Mixer):
         blocks = max(1, -(-span // 64))
         return max(1, min(256 // max(rows, 1), blocks, 16))
 
+    def decode_shape(self, span, rows: int):
+        return self._splits(span, rows)
+
     def forward(self, x_t: torch.Tensor, residual32: Optional[torch.Tensor], ctx, cache, write: bool = True) -> torch.Tensor:
         if not write:
             raise ValueError("this attention keeps a filter state that moves with every token: no read-only run")

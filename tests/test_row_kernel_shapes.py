@@ -40,3 +40,25 @@ def test_splits_of_short_contexts(monkeypatch, heads, head_dim, dtype, rows, win
     assert part._shape_row_kernel(KeySpan(192, 2048), rows) == (with_merge if fused else without, 4)
     if rows * heads < 256 and not window:
         assert part._shape_row_kernel(KeySpan(192), rows)[0] == 1 and part._shape_row_kernel(KeySpan(2048, 2048), rows)[0] > 1
+
+
+@pytest.mark.parametrize("rows,heads,window,same", [(8, 32, 0, True), (7, 32, 0, False), (1, 12, 0, False), (1, 12, 300, True), (16, 32, 0, True)])
+def test_steps_of_one_shape(monkeypatch, rows, heads, window, same):
+    """What decides whether short contexts have a recording of their own: the mixers' answers for both spans, whichever mixer it is."""
+    from swifttransformer_amd.parts import PartSpec, attention, build_part
+    from swifttransformer_amd.parts.base import CacheNeed, KeySpan, Mixer, decode_shape
+    monkeypatch.setattr(attention, "_target_workgroups", lambda: 256)
+    monkeypatch.setattr(attention.K, "can_fuse_merge", lambda *a: True)
+    part = build_part("mixer", PartSpec("paged_attention", {"num_heads": heads, "head_dim": 64, "scale": 0.125, "bias": False, "window": window},
+                                        {f"{n}.weight": n for n in ("q", "k", "v", "out")}), heads * 64, torch.bfloat16)
+    differ = lambda m: decode_shape(m, KeySpan(192, 2048), rows) != decode_shape(m, KeySpan(2048, 2048), rows)
+    assert differ(part) != same
+
+    class Other(Mixer):
+        def __init__(self, need):
+            self.need = need
+
+        def cache_need(self):
+            return self.need
+    assert not differ(Other(None)) and not differ(Other(CacheNeed("state", state_shape=(4,), state_dtype=torch.float32)))
+    assert differ(Other(CacheNeed("paged_kv", num_kv_heads=1, head_dim=64))) and differ(object())

@@ -76,3 +76,24 @@ def test_models_no_longer_than_short_contexts_have_one(tmp_path):
     runner.admit(0)
     runner.step([StepEntry(0, [5], [0])])
     assert set(runner._recorded_spans) == {(1, tuning.short_span)}
+
+
+def test_one_recording_where_the_step_is_the_same(tmp_path):
+    """Fewer positions than two splits of keys: a request that grows out of short contexts keeps its recording."""
+    from swifttransformer_amd.engine.step import StepEntry
+    from swifttransformer_amd.config import OptHyperParam
+    from swifttransformer_amd.ops.tuning import tuning
+    from swifttransformer_amd.weights import write_random_model
+    most = 2 * tuning.min_keys_per_split - 1
+    d = write_random_model(OptHyperParam(**dict(CFG, max_position_embeddings=most)).validate(), str(tmp_path / "m"), seed=3)
+    cfg, w = plain_opt.load_folder(d)
+    runner = make_runner(d, torch.float32, 16, num_pages=40, max_seqs=2)
+    seq, first = tiny.prompt(tuning.short_span + 3, CFG["vocab_size"], 5), tuning.short_span - 3
+    ref = plain_opt.forward(cfg, w, seq).numpy()
+    runner.admit(0)
+    runner.step([StepEntry(0, seq[:first], [])])
+    for p in range(first, len(seq)):
+        check(runner.step([StepEntry(0, [seq[p]], [0])]), ref[p:p + 1], torch.float32, f"position {p}")
+    assert set(runner._recorded_spans) == {(1, most)}
+    runner.finish(0)
+    assert runner.warm_up([], [1, 2]) == 1 and set(runner._recorded_spans) == {(1, most), (2, most)}
