@@ -17,7 +17,7 @@
 
 namespace st {
 
-static std::atomic<uint64_t> g_path_counts[kNumGemmPaths];
+static std::atomic<uint64_t> g_path_counts[kNumGemmPaths], g_split_count;
 void count_gemm_path(int path) {
     if (path >= 0 && path < kNumGemmPaths) g_path_counts[path].fetch_add(1, std::memory_order_relaxed);
 }
@@ -212,7 +212,7 @@ extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bia
           reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(ex.scratch) |
           reinterpret_cast<uintptr_t>(ex.k_cache) | reinterpret_cast<uintptr_t>(ex.v_cache)) & 15) == 0) {
         const int rc = gemm_f32_split((float*)out, (const float*)x, (const float*)w, bias, residual, M, N, K, act, ex, stream);
-        if (rc == 0) count_gemm_path(kPathSplitF32);
+        if (rc == 0) g_split_count.fetch_add(1, std::memory_order_relaxed);
         return rc;
     }
     const bool to_library = algo == 2 || (algo == 0 && !ex.ln_x && !ex.mg_o && library_can &&
@@ -281,7 +281,7 @@ extern "C" int st_gemm_library_rule(int min_rows, int64_t min_weights, int min_d
 }
 
 // Calls of st_gemm per kernel family since the last reset (order of st::GemmPath); returns the
-// number of families.  `out` may be null.
+// number of families.  `out` may be null.  (Float products of split operands: st_gemm_split_count.)
 extern "C" int st_gemm_path_counts(uint64_t* out, int reset) {
     for (int i = 0; i < kNumGemmPaths; ++i) {
         const uint64_t v = reset ? g_path_counts[i].exchange(0) : g_path_counts[i].load();
@@ -289,6 +289,9 @@ extern "C" int st_gemm_path_counts(uint64_t* out, int reset) {
     }
     return kNumGemmPaths;
 }
+
+// Calls of st_gemm that gemm_f32_split took since the last reset.
+extern "C" uint64_t st_gemm_split_count(int reset) { return reset ? g_split_count.exchange(0) : g_split_count.load(); }
 
 // Whether st_gemm (algo 0) can take a split attention output (partials and log-sum-exps) as its input.
 extern "C" int st_gemm_can_fuse_merge(int M, int N, int K, int splits, int heads, int head_dim, int dtype) {

@@ -83,7 +83,6 @@ enum GemmPath {
     kPathSkinny64,
     kPathTiledMfma,          // 128x128 matrix-core tiles
     kPathWide,               // persistent walk over a very wide matrix (few rows)
-    kPathSplitF32,           // float operands as bfloat16 parts
     kNumGemmPaths
 };
 void count_gemm_path(int path);

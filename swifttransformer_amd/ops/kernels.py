@@ -50,6 +50,7 @@ def _lib():
         lib.st_gemm.argtypes = [_c_p, _c_p, _c_p, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_int,
                                 _c_int, _c_int, _c_p, _c_p]
         lib.st_gemm_path_counts.argtypes = [_c_p, _c_int]
+        lib.st_gemm_split_count.argtypes, lib.st_gemm_split_count.restype = [_c_int], ctypes.c_uint64
         lib.st_gemm_library_rule.argtypes = [_c_int, _c_i64, _c_int]
         lib.st_gemm_can_fuse_norm.argtypes = [_c_int, _c_int, _c_int, _c_int]
         lib.st_gemm_wide_offered.argtypes = [_c_int, _c_int, _c_int, _c_int]
@@ -383,17 +384,23 @@ class tuned_products:
 
 
 GEMM_PATHS = ("library", "generic_f32", "generic_bf16", "resident", "resident_norm", "resident_merge",
-              "resident_staged", "skinny16", "skinny32", "skinny64", "tiled_mfma", "wide", "split_f32")
+              "resident_staged", "skinny16", "skinny32", "skinny64", "tiled_mfma", "wide")
 
 
 def gemm_path_counts(reset: bool = False) -> dict:
-    """Calls of ``gemm`` per kernel family since the last reset: which dispatch branches ran."""
+    """Calls of ``gemm`` per kernel family since the last reset: which dispatch branches ran.  (Float products of split operands are
+    counted by ``gemm_split_count``.)"""
     n = len(GEMM_PATHS)
     buf = (ctypes.c_uint64 * n)()
     got = _lib().st_gemm_path_counts(buf, int(reset))
     if got != n:
         raise KernelError(f"the library counts {got} product paths, this module names {n}")
     return {name: int(buf[i]) for i, name in enumerate(GEMM_PATHS)}
+
+
+def gemm_split_count(reset: bool = False) -> int:
+    """Float products that ran as products of bfloat16 parts since the last reset."""
+    return int(_lib().st_gemm_split_count(int(reset)))
 
 
 def gemm_library_rule(min_rows: int = -1, min_weights: int = -1, min_depth: int = -1) -> None:

@@ -57,9 +57,9 @@ def test_chosen_and_closer_than_the_library():
     x, w, _ = operands(701, 2048, 2048)
     assert K._gemm_scratch(701, 2048, 2048, 0, False) > 0 and K._gemm_scratch(64, 2048, 2048, 0, False) == 0
     ref = x.double() @ w.double().T
-    K.gemm_path_counts(reset=True)
+    K.gemm_path_counts(reset=True), K.gemm_split_count(reset=True)
     own, lib = K.gemm(x, w), K.gemm(x, w, algo=2)
-    assert {n: c for n, c in K.gemm_path_counts().items() if c} == {"split_f32": 1, "library": 1}
+    assert K.gemm_split_count() == 1 and {n: c for n, c in K.gemm_path_counts().items() if c} == {"library": 1}
     assert torch.equal(own, K.gemm(x, w, algo=3)) and torch.equal(own, K.gemm(x, w))
     assert float((own - ref).norm()) < float((lib - ref).norm())
 
@@ -202,10 +202,10 @@ def test_without_room_for_the_sums():
     ex = K._GemmExtras()
     ex.scratch, ex.scratch_floats = room.data_ptr(), 4
     for extras in (None, ctypes.byref(ex)):
-        K.gemm_path_counts(reset=True)
+        K.gemm_path_counts(reset=True), K.gemm_split_count(reset=True)
         assert K._lib().st_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), None, None, M, N, D, 0, 0, 1, 0, extras,
                                 torch.cuda.current_stream().cuda_stream) == 0
-        assert K.gemm_path_counts()["library"] == 1 and K.gemm_path_counts()["split_f32"] == 0
+        assert K.gemm_path_counts()["library"] == 1 and K.gemm_split_count() == 0
         ref, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
         assert bool(((out.double() - ref).abs() <= D * 2.0 ** -24 * size).all())
 
