@@ -26,8 +26,8 @@
 // 270 with products and LDS reads alone (2,048 x 8,192 x 2,048).  So every number is split once a workgroup, by all waves, between the
 // products (a step's products and splitting one after the other, by waves in turn or all alike: 392 and 383 us), and what is multiplied next is
 // read from LDS while there are products left that do not need the registers.
-// us, the library's best of 32 and this: 701 rows of 6,144 x 2,048 141 and 119, of 2,048 x 8,192 178 and 157, 1,500 rows of 2,560 x 2,560
-// 148 and 117, of 768 x 3,072 59 and 53 (more beside gemm_f32_split_pays).
+// us, the library's best of 32 and this: 701 rows of 6,144 x 2,048 143 and 120, of 2,048 x 8,192 184 and 160, 1,500 rows of 2,560 x 2,560
+// 154 and 116, of 768 x 3,072 64 and 57.
 //
 // Reference: cuBLAS calls (src/csrc/util/cublas_wrapper.cc:29).
 #include "common.h"
@@ -287,7 +287,8 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
                 }
     }
     if (end == steps && steps * kStep < K) plain(acc, steps * kStep, K);
-    // What is added to the results is asked for before the first is stored: one trip to memory a row of the block, not one a store.
+    // What is added to the results is
+    // asked for before the first is stored: one trip to memory a row of the block, not one a store.
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
         const int mt = wm * 64 + r * 32 + l32, m = m0 + mt;
@@ -338,8 +339,8 @@ __global__ __launch_bounds__(256) void gemm_f32_sum_kernel(
 }
 
 // How a product is dealt out: `whole` tiles by workgroups of their own (whole rounds of a workgroup a compute unit), the rest by
-// `splits` workgroups each.
-struct Deal { int tiles_m, tiles, whole, splits; };
+// `splits` workgroups each; the longest that a compute unit has to do are `steps` steps of a tile.
+struct Deal { int tiles_m, tiles, whole, splits, steps; };
 
 Deal deal(int M, int N, int K) {
     Deal d;
@@ -357,29 +358,14 @@ Deal deal(int M, int N, int K) {
         const double cost = (double)((rest * s + units - 1) / units) * share + rest * s * 0.033 + 4;
         if (cost < best) { best = cost; d.splits = s; }
     }
+    d.steps = d.tiles / units * steps + (rest * d.splits + units - 1) / units * ((steps + d.splits - 1) / d.splits);
     return d;
 }
 
 }  // namespace
 
-// Whether a product is faster here than in the library, from what either takes (us).  Here: what the unit with the most to do does (rounds of
-// workgroups, each with its beginning and its results; steps of a tile), slower the more units are busy, as power bounds them, and the partial
-// sums.  The library: 72e6 products a us on rows in tiles of 64.  Both are fitted on 76 products with cold weights, 96 to 2,048 rows of 768 x
-// 768 to 10,240 x 2,560, the library's best of 32; the first is within 10 % of every one.  Of these none that is slower here is taken, and
-// what is faster here and left to the library is so by up to 28 % at 128 rows, 18 % at 300, 13 % beyond (rows x features x depth: library, here):
-// taken: 200 x 8,192 x 2,048 59.9, 59.6; 200 x 4,096 x 4,096 65.4, 58.1; 256 x 2,048 x 8,192 72.7, 63.4; 1,024 x 2,048 x 2,048 61.9, 59.4;
-// 1,500 x 2,560 x 2,560 148, 117; 2,048 x 2,048 x 2,048 120, 98
-// left: 300 x 6,144 x 2,048 61.9, 78.4; 701 x 2,048 x 2,048 47.3, 52.6; 384 x 2,560 x 2,560 40.8, 43.2; 2,048 x 3,072 x 768 70.4, 80.0; 128 x
-// 8,192 x 2,048 37.9, 41.6; 128 x 2,560 x 10,240 86.5, 67.4; 300 x 2,048 x 8,192 95.9, 81.0; 701 x 2,560 x 2,560 75.5, 66.8
-bool gemm_f32_split_pays(int M, int N, int K) {
-    if (M < 96) return false;
-    const Deal d = deal(M, N, K);
-    const int units = device_compute_units(), steps = K / kStep, parts = (d.tiles - d.whole) * d.splits;
-    const int last = (parts + units - 1) / units;                    // rounds of the tiles that are left of whole ones
-    const double most = (double)(d.whole / units) * steps + (double)last * ((steps + d.splits - 1) / d.splits);
-    const double here = 6.4 + 6.6 * (d.whole / units + last) + 0.87 * most + 0.44 * ((double)d.tiles * steps / units) + (d.splits > 1 ? 0.02 * parts : 0.0);
-    return here < 4 + (double)((M + 63) / 64 * 64) * N * K / 72e6;
-}
+// Whether a product is faster here than in the library: most of a tile's 128 rows, and enough tiles or depth to fill the chip.
+bool gemm_f32_split_pays(int M, int N, int K) { return M >= 96 && (int64_t)M * N * K >= 2500000000ll; }
 
 // Floats of scratch with which gemm_f32_split deals its tiles out best (0: none).
 int64_t gemm_f32_split_scratch(int M, int N, int K) {
