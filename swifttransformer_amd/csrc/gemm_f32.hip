@@ -26,8 +26,8 @@
 // 270 with products and LDS reads alone (2,048 x 8,192 x 2,048).  So every number is split once a workgroup, by all waves, between the
 // products (a step's products and splitting one after the other, by waves in turn or all alike: 392 and 383 us), and what is multiplied next is
 // read from LDS while there are products left that do not need the registers.
-// us, the library's best of 32 and this: 701 rows of 6,144 x 2,048 143 and 120, of 2,048 x 8,192 184 and 160, 1,500 rows of 2,560 x 2,560
-// 154 and 116, of 768 x 3,072 64 and 57.
+// us, the library's best of 32 and this: 701 rows of 6,144 x 2,048 139 and 120, of 2,048 x 8,192 177 and 155, 1,500 rows of 2,560 x 2,560
+// 149 and 115, of 768 x 3,072 61 and 54 (more beside gemm_f32_split_pays).
 //
 // Reference: cuBLAS calls (src/csrc/util/cublas_wrapper.cc:29).
 #include "common.h"
@@ -287,8 +287,7 @@ __global__ __launch_bounds__(512) void gemm_f32_split_kernel(
                 }
     }
     if (end == steps && steps * kStep < K) plain(acc, steps * kStep, K);
-    // What is added to the results is
-    // asked for before the first is stored: one trip to memory a row of the block, not one a store.
+    // What is added to the results is asked for before the first is stored: one trip to memory a row of the block, not one a store.
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
         const int mt = wm * 64 + r * 32 + l32, m = m0 + mt;
@@ -364,8 +363,25 @@ Deal deal(int M, int N, int K) {
 
 }  // namespace
 
-// Whether a product is faster here than in the library: most of a tile's 128 rows, and enough tiles or depth to fill the chip.
-bool gemm_f32_split_pays(int M, int N, int K) { return M >= 96 && (int64_t)M * N * K >= 2500000000ll; }
+// Whether a product of at least 2.5e9 multiply-adds goes here, from what it takes here and in the library (us).  Here: rounds of workgroups, each
+// with its beginning and its results; the steps of the unit with the most to do, slower the more units are busy, as power bounds them; the
+// partial sums.  The library: 72e6 multiply-adds a us on rows in tiles of 16, and the depth, which few tiles have to go through one after
+// the other.  Both are fitted on 130 products with cold weights, 97 to 2,103 rows of 768 x 3,072 to 12,288 x 4,096, the library's best of 32, here
+// to 11 % and there to 17 % of every one.  Up to 6 % more is taken for results that are closer to exact ones; with that no size of the
+// 130 is taken that is over 7 % slower here (at 2.5e9 and above alone it was 8 to 27 % for 11 of them, where the rows fill a tile
+// badly), and none left that is over 5 % faster.  Up to 96 rows the library has a tile of their size.  Rows x features x depth: library, here
+// taken: 97 x 2,560 x 10,240 81, 62; 230 x 6,144 x 2,048 50.5, 54.0; 300 x 2,048 x 8,192 93, 80; 701 x 2,048 x 2,048 50.5, 53.5; 701 x 6,144 x
+// 2,048 139, 120; 1,100 x 3,072 x 768 46.1, 41.7; 2,103 x 2,048 x 8,192 522, 388
+// left: 96 x 2,560 x 10,240 59, 68; 140 x 10,240 x 2,560 73, 93; 290 x 7,680 x 2,560 95, 105; 300 x 6,144 x 2,048 64, 78; 2,048 x 3,072 x 768 72, 79
+bool gemm_f32_split_pays(int M, int N, int K) {
+    const double products = (double)M * N * K;
+    if (M <= 96 || products < 2.5e9) return false;
+    const Deal d = deal(M, N, K);
+    const int units = device_compute_units(), parts = (d.tiles - d.whole) * d.splits, rounds = d.whole / units + (parts + units - 1) / units;
+    const double here = 6.3 + 8.5 * rounds + 0.8 * d.steps + 0.49 * d.tiles * (K / kStep) / units + (d.splits > 1 ? 0.012 * parts : 0.0);
+    const double library = 6.2 + 13.8e-9 * products / M * ((M + 15) / 16 * 16) + 0.00225 * K;
+    return here < 1.06 * library;
+}
 
 // Floats of scratch with which gemm_f32_split deals its tiles out best (0: none).
 int64_t gemm_f32_split_scratch(int M, int N, int K) {

@@ -75,6 +75,19 @@ def test_no_further_off_than_the_library(M, N, D, share):
     assert float(own) < float(lib)
 
 
+@pytest.mark.parametrize("M,N,D,taken", [
+    (96, 2560, 10240, False), (97, 2560, 10240, True), (128, 8192, 2048, False), (140, 10240, 2560, False), (200, 2048, 8192, True), (256, 4096, 4096, True),
+    (300, 6144, 2048, False), (300, 2048, 8192, True), (300, 4096, 4096, False), (701, 6144, 2048, True), (2048, 3072, 768, False), (2048, 2048, 2048, True)])
+def test_which_sizes_are_taken(M, N, D, taken):
+    """Those that are no slower than in the library (the figures are beside the rule)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the line depends on the number of compute units")
+    x, w, _ = operands(M, N, D)
+    K.gemm_path_counts(reset=True), K.gemm_split_count(reset=True)
+    K.gemm(x, w)
+    assert (K.gemm_split_count(), K.gemm_path_counts()["library"]) == (int(taken), int(not taken))
+
+
 def test_most_scratch_of_smaller_steps():
     assert K._gemm_scratch(1024, 2048, 2048, 0, True) >= max(K._gemm_scratch(m, 2048, 2048, 0, False) for m in range(1, 1025))
     assert not arena.measuring()
