@@ -21,7 +21,7 @@
 //   (infinity times a part that is zero).
 // - Its sum is below 2^-90 and not zero: products of small parts may be below float's least number where the whole product is not.
 //
-// What bounds it: the chip's power, more than its matrix cores (six products a float product, 1.0 to 1.2 PFLOP/s of them where a large
+// What bounds it: the chip's power, more than its matrix cores (six products a float product, 0.9 to 1.1 PFLOP/s of them where a large
 // bfloat16 product reaches 1.6): with one sum for all six the same launch took 381 us on normal numbers and 320 on zeros, 290 without loads,
 // 270 with products and LDS reads alone (2,048 x 8,192 x 2,048).  So every number is split once a workgroup, by all waves, between the
 // products (a step's products and splitting one after the other, by waves in turn or all alike: 392 and 383 us), and what is multiplied next is

@@ -1358,7 +1358,8 @@ extern "C" int st_moe_combine(float* out, const float* residual, const float* pa
     if (num_tokens == 0) return 0;
     const bool vec = width % 4 == 0 && (((uintptr_t)out | (uintptr_t)residual | (uintptr_t)pair_out) & 15) == 0;
     // a turn is two trips to memory (a choice's place, then its result): few rows have a thread for every piece, up to 1,024 (us, 256 threads
-    // and so: 8 rows of 2,048 2.7 and 2.15, 24 of 4,096 4.0 and 2.5, 256 of 2,048 3.0 and 2.5)
+    // and so, alone: 8 rows of 2,048 2.7 and 2.15, 24 of 4,096 4.0 and 2.5, 256 of 2,048 3.0 and 2.5; a call in a step, behind the product that
+    // writes the results: 24 of 4,096 10.8 and 7.4, 8 of 2,048 5.0 either way)
     int threads = 256;
     while (num_tokens <= device_compute_units() && threads < 1024 && threads * (vec ? 4 : 1) < width) threads <<= 1;
 #define ST_MC(T, V)                                                                                                    \
