@@ -99,21 +99,6 @@ __device__ inline float group_sum(float s) {
     return s;
 }
 
-// The sum (or, MAX, the largest) of a value over the lanes that differ by O, where the lanes O apart from each other's are already
-// alike or distinct by it alone: turns of 32, 16 (row swaps), 8, 4, 2, 1 (rotations within 16 lanes), from the largest down to any of them.
-template <int O, bool MAX>
-__device__ inline float across(float x) {
-    float a, b;
-    if (O >= 16) {
-        const uint32_t u = __float_as_uint(x);
-        const auto v = O == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
-        a = __uint_as_float(v[0]); b = __uint_as_float(v[1]);
-    } else {
-        a = x;
-        b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + (O >= 16 ? 1 : O), 0xF, 0xF, false));
-    }
-    return MAX ? fmaxf(a, b) : a + b;
-}
 // over the 64 / LPK lanes that are `lane % LPK` alike
 template <int LPK, bool MAX>
 __device__ inline float across_groups(float x) {

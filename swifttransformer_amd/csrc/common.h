@@ -149,17 +149,35 @@ __device__ inline float exp_le0(float x) {
     return fmaf(p, lost * 0.693147181f, p);
 }
 
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
+// The sum (or, MAX, the largest) of a value over the lanes that differ by O, where the lanes O apart from each other's are already
+// alike or distinct by it alone: turns of 32, 16 (row swaps), 8, 4, 2, 1 (rotations within 16 lanes), from the largest down to any of them.
+template <int O, bool MAX>
+__device__ inline float across(float x) {
+    float a, b;
+    if (O >= 16) {
+        const uint32_t u = __float_as_uint(x);
+        const auto v = O == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        a = __uint_as_float(v[0]); b = __uint_as_float(v[1]);
+    } else {
+        a = x;
+        b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + (O >= 16 ? 1 : O), 0xF, 0xF, false));
+    }
+    return MAX ? fmaxf(a, b) : a + b;
 }
 
-__device__ inline float wave_max(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-    return v;
+// Over the 64 lanes, which are all there; every lane gets the result.  Moves between the lanes, not trips through LDS, six of which
+// one after the other are most of the time of a small norm; the same pairs, so the same bits.
+template <bool MAX>
+__device__ inline float across_wave(float v) {
+    v = across<32, MAX>(v);
+    v = across<16, MAX>(v);
+    v = across<8, MAX>(v);
+    v = across<4, MAX>(v);
+    v = across<2, MAX>(v);
+    return across<1, MAX>(v);
 }
+__device__ inline float wave_sum(float v) { return across_wave<false>(v); }
+__device__ inline float wave_max(float v) { return across_wave<true>(v); }
 
 // Sum over a workgroup of up to 1024 threads; every thread gets the result.
 // `red` is LDS scratch of at least 16 floats; safe to call repeatedly.
