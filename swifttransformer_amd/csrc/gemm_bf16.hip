@@ -31,6 +31,7 @@ namespace st {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 
 __device__ inline bf16x8 load8(const bf16_t* p) {
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
@@ -95,6 +96,62 @@ __device__ inline void store4(void* out, const float* bias, const float* residua
         }
     }
 }
+
+// The same with what it adds asked for beforehand: `ask` and `ask_place` where the loads may be on their way beside others, `finish`
+// with the sums.  (Element by element behind the sums they are up to ten trips to memory one after the other.)
+struct Epilogue4 {
+    floatx4 b, r;
+    int64_t place;
+    int which;
+    bool ahead;          // N and the pointers allow 16-byte accesses
+    __device__ inline void ask(const float* bias, const float* residual, int m, int n0, int N, bool here) {
+        ahead = (N & 3) == 0 && ((reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual)) & 15) == 0;
+        b = r = floatx4{0.f, 0.f, 0.f, 0.f};
+        place = -1;
+        which = 0;
+        if (!here || !ahead) return;
+        const int n = min(n0, N - 4);
+        if (bias) b = *reinterpret_cast<const floatx4*>(bias + n);
+        if (residual) r = *reinterpret_cast<const floatx4*>(residual + (int64_t)m * N + n);
+    }
+    // the place in the caches of the row of `item` at `pos`
+    __device__ inline void ask_place(int n0, int item, int pos, const StGemmExtras& ex) {
+        if (n0 >= ex.q_size) place = kv_scatter_place(ex, item, pos, n0, &which);
+    }
+    template <bool OUT_F32>
+    __device__ inline void finish(void* out, const float* bias, const float* residual, int act, int m, int n0, int N, floatx4 v,
+                                  const StGemmExtras& ex) const {
+        if (!ahead) {
+            store4<OUT_F32>(out, bias, residual, act, m, n0, N, v, ex);
+            return;
+        }
+        float s[4] = {v[0], v[1], v[2], v[3]};
+        if (bias && !ex.bias_unscaled) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] += b[i];
+        }
+        apply_activation4(act, s);
+        if (ex.out_scale != 0.f) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] *= ex.out_scale;
+        }
+        if (bias && ex.bias_unscaled) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] += b[i];
+        }
+        if (residual) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] += r[i];
+        }
+        if constexpr (OUT_F32) {
+            *reinterpret_cast<float4*>((float*)out + (int64_t)m * N + n0) = make_float4(s[0], s[1], s[2], s[3]);
+        } else {
+            const uint2 p = make_uint2(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]));
+            if (place >= 0) *reinterpret_cast<uint2*>((bf16_t*)(which ? ex.v_cache : ex.k_cache) + place) = p;
+            *reinterpret_cast<uint2*>((bf16_t*)out + (int64_t)m * N + n0) = p;
+        }
+    }
+};
 
 // ------------------------------------------------------------------------ skinny
 // One workgroup owns 16*NT output features and all of K; its WAVES waves split K and
@@ -200,8 +257,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
 }
 
 // ------------------------------------------------------- skinny, W slab in registers
-// M <= 16.  A workgroup owns 16 output features; wave w owns k in [w*KSTEPS*64, +KSTEPS*64)
-// and loads its whole slab of W (16 rows x KSTEPS*64 k) into registers with its first
+// M <= 16.  A workgroup owns ROWS output features; wave w owns k in [w*KSTEPS*64, +KSTEPS*64)
+// and loads its whole slab of W into registers with its first
 // instructions, so every byte of W is in flight before anything waits.  With LN the
 // workgroup meanwhile normalises the M input rows (float, from ex.ln_x) into LDS as
 // bfloat16, and the x operand is read from there.
@@ -211,12 +268,34 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
 // the stored input rows are copied into LDS first (asked for before the W slab, so they arrive
 // first): the K steps then read their x fragments from LDS instead of paying a trip to the L2
 // each, one after the other.
-// K % 8 == 0, K <= WAVES*KSTEPS*64; LN: K % 256 == 0 handled by guards, K <= 4096.
+// K % 8 == 0, K <= WAVES*KSTEPS*64; LN: K <= 4096.
+//
+// What bounds it beside the weights' stream: trips to memory one after the other, and the vector instructions of sixteen waves (four a
+// SIMD, so that an instruction of each costs 16 clocks) before W is asked for.  So the loads are unconditional, from addresses that are
+// clamped (a load behind a branch of a lane's makes the compiler wait for all that are on their way before it uses the first), W's
+// addresses are a scalar a step and one offset a lane, the staged rows are copied as they lie (where a piece goes in LDS is found
+// afterwards), and what the epilogue adds (bias, residual, the place in the cache) is asked for behind W instead of element by element
+// behind the sums.  us a call in a recorded chain, before and so: 1 row 768 to 768 3.5 and 2.7, 3,072 to 768 5.4 and 4.2, with the norm 768
+// to 2,304 4.5 and 3.9; 8 rows 2,048 to 2,048 5.5 and 4.1, to 4,096 7.4 and 5.6, 8,192 to 2,048 11.8 and 9.5, 2,560 to 2,560 9.0 and 8.5,
+// with the norm 2,048 to 6,144 9.5 and 8.4, with the merge 7.6 and 6.4; 16 rows with the norm 11.3 and 10.3, 8,192 to 2,048 13.1 and 13.1.
 constexpr int kLnMaxVec = 16;            // float4 per lane of a row held in registers (K <= 4096)
 constexpr int kMgElems = 2;              // merge prologue: float4 elements of the input per thread
 constexpr int kMgSplits = 8;             // and splits per element, all held in registers;
 constexpr int kMgElemsTwo = 8;           // or this many elements of at most two splits (PRO == 4: more rows)
 constexpr int kMgMaxWeights = 2048;      // rows * heads * splits weights in LDS
+
+// position `at` of `step`, `2 step`, ... behind a start, as (quotient, remainder) by a divisor
+struct DividedWalk {
+    int q, r, dq, dr, by;
+    __device__ inline DividedWalk(int start, int step, int divisor) : by(divisor) {
+        q = (unsigned)start / (unsigned)divisor; r = start - q * divisor;
+        dq = (unsigned)step / (unsigned)divisor; dr = step - dq * divisor;
+    }
+    __device__ inline void next() {
+        q += dq; r += dr;
+        if (r >= by) { r -= by; ++q; }
+    }
+};
 
 template <int WAVES, int KSTEPS, bool OUT_F32, int PRO, int ROWS>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
@@ -224,13 +303,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
     const float* __restrict__ bias, const float* __restrict__ residual,
     int M, int N, int K, int act, const StGemmExtras ex) {
     constexpr bool LN = PRO == 1, MG = PRO == 2 || PRO == 4, ST = PRO == 3;
+    constexpr int THREADS = WAVES * 64;
     // merge prologue: elements of the input per thread x splits held in registers
     constexpr int MGE = PRO == 4 ? kMgElemsTwo : kMgElems, MGS = PRO == 4 ? 2 : kMgSplits;
     extern __shared__ uint4 dyn[];
     constexpr int NT = (ROWS + 15) / 16;                                   // 16-row MFMA tiles of W per workgroup
     floatx4* red = reinterpret_cast<floatx4*>(dyn);                       // [WAVES][NT][64]
-    bf16_t* xs = nullptr;                                                  // [M][K + 8] input rows made here (LN, MG)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    bf16_t* xs = nullptr;                                                  // [M][K + 8] input rows made here (LN, MG, ST)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r16 = lane & 15;
     // ROWS output features per workgroup.  8: half of each MFMA's rows stay empty, but a narrow
     // matrix (N = hidden) then spreads over twice as many compute units.  24 and 32 (two tiles):
@@ -239,13 +319,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
     // two tiles are as long as those of one tile with 8, so as many bytes are in flight.
     const int n_base = blockIdx.x * ROWS;
     const int k_begin = wave * (KSTEPS * 64);
-    bool wvalid[NT];
-    const bf16_t* wrow[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        wvalid[t] = 16 * t + r16 < ROWS;
-        wrow[t] = w + (int64_t)min(n_base + 16 * t + r16, N - 1) * K;
-    }
+    // the wave's steps that lie in the depth whole, and how much of the next one does
+    const int whole = min(KSTEPS, max(0, K - k_begin) >> 6), rest = min(64, max(0, K - k_begin - whole * 64));
     const int xstride = K + 8;
 
     // Loads return in order, so what is needed first is asked for first: the norm's gain and
@@ -258,90 +333,132 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
     float* sb = sg + K;                                               // [K] bias
     xs = reinterpret_cast<bf16_t*>(sb + K);
     float4 gv[GV], bv[GV];
-    if (LN) {
-#pragma unroll
-        for (int i = 0; i < GV; ++i) {
-            const int c = threadIdx.x + i * (WAVES * 64);
-            gv[i] = (ex.ln_gamma && c < nvec) ? reinterpret_cast<const float4*>(ex.ln_gamma)[c]
-                                              : make_float4(1.f, 1.f, 1.f, 1.f);
-            bv[i] = (ex.ln_beta && c < nvec) ? reinterpret_cast<const float4*>(ex.ln_beta)[c]
-                                             : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    }
-    // merge prologue: this thread's elements of every split, asked for before the W slab so that
-    // they arrive first; the weights of the splits meanwhile go to LDS
-    float4 mo[MG ? MGE : 1][MG ? MGS : 1];
-    float* sw = sg;                                                   // [M * heads * splits] weights (MG only)
-    if (MG) {
-        xs = reinterpret_cast<bf16_t*>(sw + ((M * ex.mg_heads * ex.mg_splits + 3) & ~3));   // 16-byte aligned
-        const int S = ex.mg_splits, hd4 = ex.mg_head_dim >> 2, total = M * nvec;
-#pragma unroll
-        for (int e = 0; e < MGE; ++e) {
-            const int idx = threadIdx.x + e * (WAVES * 64);          // (row, float4 of K)
-            const int m = idx / nvec, c = idx - m * nvec;
-            const int head = c / hd4, d4 = c - head * hd4;
-            const float4* po = reinterpret_cast<const float4*>(ex.mg_o) +
-                               ((int64_t)(m * ex.mg_heads + head) * S) * hd4 + d4;
-#pragma unroll
-            for (int sp = 0; sp < MGS; ++sp)
-                mo[e][sp] = (idx < total && sp < S) ? po[(int64_t)sp * hd4] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    }
-    // staged input: this thread's 16-byte pieces of the M rows
-    constexpr int STV = 8;                                            // pieces per thread: M*K <= 8*8*threads
-    uint4 sx[ST ? STV : 1];
-    if (ST) {
-        xs = reinterpret_cast<bf16_t*>(sg);
-        const int pieces = K >> 3, total = M * pieces;
-#pragma unroll
-        for (int i = 0; i < STV; ++i) {
-            const int idx = threadIdx.x + i * (WAVES * 64);
-            const int m = idx / pieces, c = idx - m * pieces;
-            sx[i] = idx < total ? *reinterpret_cast<const uint4*>(x + (int64_t)m * K + c * 8) : make_uint4(0, 0, 0, 0);
-        }
-    }
     float4 v[LNV];
     auto load_row = [&](int m) {
-        const float* xr = ex.ln_x + (int64_t)m * K;
+        const float4* xr = reinterpret_cast<const float4*>(ex.ln_x + (int64_t)m * K);
 #pragma unroll
-        for (int i = 0; i < LNV; ++i) {
-            const int c = lane + i * 64;
-            v[i] = c < nvec ? reinterpret_cast<const float4*>(xr)[c] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+        for (int i = 0; i < LNV; ++i) v[i] = xr[min(lane + i * 64, nvec - 1)];
     };
-    if (LN && wave < M) load_row(wave);
-    bf16x8 a[NT][KSTEPS][2];
+    if constexpr (LN) {
+        // (a norm without one of them reads the first row in its place)
+        const float4 *gain = reinterpret_cast<const float4*>(ex.ln_gamma ? ex.ln_gamma : ex.ln_x),
+                     *shift = reinterpret_cast<const float4*>(ex.ln_beta ? ex.ln_beta : ex.ln_x);
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+        for (int i = 0; i < GV; ++i) {
+            const int c = min(tid + i * THREADS, nvec - 1);
+            gv[i] = gain[c];
+            bv[i] = shift[c];
+        }
+        if (wave < M) load_row(wave);
+    }
+    // merge prologue: this thread's elements of every split and its group's log-sum-exps, asked for before the W slab so that
+    // they arrive first.  Elements of the input in the order in which they lie: (row and head, piece of the head).
+    float4 mo[MG ? MGE : 1][MG ? MGS : 1];
+    float ls[MG ? MGS : 1];
+    float* sw = sg;                                                   // [M * heads * splits] weights (MG only)
+    const int S = ex.mg_splits, groups = M * ex.mg_heads, total4 = M * nvec;
+    if constexpr (MG) {
+        xs = reinterpret_cast<bf16_t*>(sw + ((groups * S + 3) & ~3));         // 16-byte aligned
+        // (a thread a group: rows * heads * splits <= 2,048, two splits and more)
+        const float* lse = ex.mg_lse + (int64_t)min(tid, groups - 1) * S;
+#pragma unroll
+        for (int sp = 0; sp < MGS; ++sp)
+            if (sp < S) ls[sp] = lse[sp];
+        const int hd4 = ex.mg_head_dim >> 2;
+        DividedWalk at(tid, THREADS, hd4);
+#pragma unroll
+        for (int e = 0; e < MGE; ++e, at.next()) {
+            if (e * THREADS >= total4) continue;
+            const bool there = tid + e * THREADS < total4;
+            const float4* po = reinterpret_cast<const float4*>(ex.mg_o) + (int64_t)(there ? at.q : 0) * S * hd4 + at.r;
+#pragma unroll
+            for (int sp = 0; sp < MGS; ++sp)
+                if (sp < S) mo[e][sp] = po[(int64_t)sp * hd4];
+        }
+    }
+    // staged input: this thread's 16-byte pieces of the M rows, which lie one behind the other
+    constexpr int STV = 8;                                            // pieces per thread: M*K <= 8*8*threads
+    uintx4 sx[ST ? STV : 1];
+    const int pieces = K >> 3, total = M * pieces;
+    if constexpr (ST) {
+        xs = reinterpret_cast<bf16_t*>(sg);
+#pragma unroll
+        for (int i = 0; i < STV; ++i)
+            sx[i] = i * THREADS < total ? reinterpret_cast<const uintx4*>(x)[(uint32_t)min(tid + i * THREADS, total - 1)] : uintx4{0, 0, 0, 0};
+    }
+    // where the lane's results go: wave t sums tile t, row r16, features n0 on
+    const int n0 = n_base + 16 * wave + 4 * g, m_own = min(r16, M - 1);
+    const bool own = wave < NT && r16 < M && 16 * wave + 4 * g < ROWS && n0 < N;
+    const bool scatter = !OUT_F32 && ex.k_cache && wave < NT && n_base + ROWS > ex.q_size;
+    int item = -1, pos = -1;
+    if (scatter) { item = ex.token_item[m_own]; pos = ex.positions[m_own]; }
+
+    // A tile of 8 features (the last one of 8 or 24): lanes 0 to 7 of a row hold the features' first half of a step's pieces, lanes 8 to
+    // 15 the same features' other half, so that a product with either half of x fills its own half of the tile's sums (the other half is
+    // not looked at): half the loads and registers, and as many products, as with eight rows left empty.
+    constexpr bool HALF = ROWS % 16 == 8;
+    const auto half_tile = [](int t) { return HALF && t == NT - 1; };
+    const int upper = r16 >> 3;
+    bf16x8 a[NT][KSTEPS][2];
+    const bf16_t* wb = w + (int64_t)n_base * K;
+    uint32_t wrow[NT];                                                // first element of the lane's row of W, from wb on
+#pragma unroll
+    for (int t = 0; t < NT; ++t)                                      // (rows past the matrix stand for its last: their results are not stored)
+        wrow[t] = (uint32_t)min(16 * t + (half_tile(t) ? r16 & 7 : r16), N - 1 - n_base) * (uint32_t)K;
+    if ((K & 63) == 0) {                                              // a wave's steps lie in the depth, or past it: the first 64 then
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            const bf16_t* ws = wb + (s < whole ? k_begin + s * 64 : 0);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                a[t][s][0] = load8(ws + (wrow[t] + g * 16 + (half_tile(t) ? upper * 8 : 0)));
+                if (!half_tile(t)) a[t][s][1] = load8(ws + (wrow[t] + g * 16 + 8));
+            }
+        }
+    } else {
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
             const int ko = k_begin + s * 64 + g * 16;
-            a[t][s][0] = (wvalid[t] && ko + 8 <= K) ? load8(wrow[t] + ko) : zero8();
-            a[t][s][1] = (wvalid[t] && ko + 16 <= K) ? load8(wrow[t] + ko + 8) : zero8();
-        }
-    const bool xvalid = r16 < M;
-    const bf16_t* xrow = x + (int64_t)(xvalid ? r16 : 0) * K;       // unused with LN, MG and ST
-    if (ST) {
-        const int pieces = K >> 3, total = M * pieces;
 #pragma unroll
-        for (int i = 0; i < STV; ++i) {
-            const int idx = threadIdx.x + i * (WAVES * 64);
-            if (idx < total) {
-                const int m = idx / pieces, c = idx - m * pieces;
-                *reinterpret_cast<uint4*>(xs + (int64_t)m * xstride + c * 8) = sx[i];
+            for (int t = 0; t < NT; ++t) {
+                const int k0 = ko + (half_tile(t) ? upper * 8 : 0);
+                a[t][s][0] = load8(wb + (wrow[t] + (k0 + 8 <= K ? k0 : 0)));
+                if (!half_tile(t)) a[t][s][1] = load8(wb + (wrow[t] + (ko + 16 <= K ? ko + 8 : 0)));
             }
         }
-        __syncthreads();
-        xrow = xs + (int64_t)(xvalid ? r16 : 0) * xstride;
     }
-    if (MG) {
-        const int S = ex.mg_splits, groups = M * ex.mg_heads;
-        for (int gidx = threadIdx.x; gidx < groups; gidx += WAVES * 64) {
-            const float* lse = ex.mg_lse + (int64_t)gidx * S;
-            float ls[MGS], mx = -INFINITY;
+    // (the rows of x as they lie, where a lane's registers hold them beside W)
+    const bf16_t* xrow = x + (int64_t)m_own * K;                      // unused with LN, MG and ST
+    constexpr bool BESIDE = PRO == 0 && KSTEPS <= 2;
+    bf16x8 bx[BESIDE ? KSTEPS : 1][2];
+    if constexpr (BESIDE) {
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            const int ko = k_begin + s * 64 + g * 16;
+            bx[s][0] = load8(xrow + (ko + 8 <= K ? ko : 0));
+            bx[s][1] = load8(xrow + (ko + 16 <= K ? ko + 8 : 0));
+        }
+    }
+    Epilogue4 ep;
+    const auto ask = [&] {
+        ep.ask(bias, residual, m_own, n0, N, wave < NT);
+        if (scatter) ep.ask_place(n0, item, pos, ex);
+    };
+    if constexpr (!MG) ask();                                         // (with the partial results there are no registers left for it)
+
+    if constexpr (ST) {
+        DividedWalk at(tid, THREADS, pieces);
+#pragma unroll
+        for (int i = 0; i < STV; ++i, at.next())
+            if (i * THREADS < total && tid + i * THREADS < total) *reinterpret_cast<uintx4*>(xs + at.q * xstride + at.r * 8) = sx[i];
+        __syncthreads();
+    }
+    if constexpr (MG) {
+        if (tid < groups) {
+            float mx = -INFINITY;
 #pragma unroll
             for (int sp = 0; sp < MGS; ++sp) {
-                ls[sp] = sp < S ? lse[sp] : -INFINITY;
+                if (sp >= S) ls[sp] = -INFINITY;
                 mx = fmaxf(mx, ls[sp]);
             }
             float wsum = 0.f;
@@ -353,16 +470,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
             const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
 #pragma unroll
             for (int sp = 0; sp < MGS; ++sp)
-                if (sp < S) sw[gidx * S + sp] = ls[sp] * inv;
+                if (sp < S) sw[tid * S + sp] = ls[sp] * inv;
         }
         __syncthreads();
-        const int hd4 = ex.mg_head_dim >> 2, total = M * nvec;
+        DividedWalk head(tid, THREADS, ex.mg_head_dim >> 2), row(tid, THREADS, nvec);
 #pragma unroll
-        for (int e = 0; e < MGE; ++e) {
-            const int idx = threadIdx.x + e * (WAVES * 64);
-            if (idx >= total) continue;
-            const int m = idx / nvec, c = idx - m * nvec;
-            const float* wg = sw + (m * ex.mg_heads + c / hd4) * S;
+        for (int e = 0; e < MGE; ++e, head.next(), row.next()) {
+            if (e * THREADS >= total4 || tid + e * THREADS >= total4) continue;
+            const float* wg = sw + head.q * S;
             float y0 = 0.f, y1 = 0.f, y2 = 0.f, y3 = 0.f;
 #pragma unroll
             for (int sp = 0; sp < MGS; ++sp) {
@@ -375,28 +490,28 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
             uint2 p;
             p.x = pack_bf16x2(y0, y1);
             p.y = pack_bf16x2(y2, y3);
-            *reinterpret_cast<uint2*>(xs + (int64_t)m * xstride + c * 4) = p;
+            *reinterpret_cast<uint2*>(xs + row.q * xstride + row.r * 4) = p;
         }
+        ask();
         __syncthreads();
-        xrow = xs + (int64_t)(xvalid ? r16 : 0) * xstride;
     }
-    if (LN) {
+    if constexpr (LN) {
 #pragma unroll
         for (int i = 0; i < GV; ++i) {
-            const int c = threadIdx.x + i * (WAVES * 64);
+            const int c = tid + i * THREADS;
             if (c < nvec) {
-                reinterpret_cast<float4*>(sg)[c] = gv[i];
-                reinterpret_cast<float4*>(sb)[c] = bv[i];
+                reinterpret_cast<float4*>(sg)[c] = ex.ln_gamma ? gv[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+                reinterpret_cast<float4*>(sb)[c] = ex.ln_beta ? bv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
             }
         }
-        // rows beyond the first of a wave (M > WAVES) are loaded when their turn comes
         float mean = 0.f, rstd = 0.f;
-        bool first = true;
-        for (int m = wave; m < M; m += WAVES) {
-            if (!first) load_row(m);
+        auto statistics = [&] {
             float sum = 0.f;
 #pragma unroll
-            for (int i = 0; i < LNV; ++i) sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+            for (int i = 0; i < LNV; ++i) {
+                if ((i + 1) * 64 > nvec && lane + i * 64 >= nvec) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+            }
             mean = ex.ln_no_center ? 0.f : wave_sum(sum) / (float)K;
             float sq = 0.f;
 #pragma unroll
@@ -407,8 +522,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
                 }
             }
             rstd = 1.0f / sqrtf(wave_sum(sq) / (float)K + ex.ln_eps);
-            if (first) __syncthreads();              // gain and bias are in LDS (every wave passes here once)
-            first = false;
+        };
+        auto write_row = [&](int m) {
 #pragma unroll
             for (int i = 0; i < LNV; ++i) {
                 const int c = lane + i * 64;
@@ -420,44 +535,82 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
                 uint2 p;
                 p.x = pack_bf16x2(y0, y1);
                 p.y = pack_bf16x2(y2, y3);
-                *reinterpret_cast<uint2*>(xs + (int64_t)m * xstride + c * 4) = p;
+                *reinterpret_cast<uint2*>(xs + m * xstride + c * 4) = p;
             }
+        };
+        if (wave < M) statistics();
+        __syncthreads();                             // gain and bias are in LDS
+        if (wave < M) write_row(wave);
+        for (int m = wave + WAVES; m < M; m += WAVES) {                  // rows beyond the first of a wave
+            load_row(m);
+            statistics();
+            write_row(m);
         }
-        if (first) __syncthreads();                  // waves without a row still meet the others
         __syncthreads();
-        xrow = xs + (int64_t)(xvalid ? r16 : 0) * xstride;
     }
-    // x fragments are fetched step by step (from cache or LDS): loads return in order, so they
-    // queue behind the W slab already in flight and need no registers until then
-    floatx4 acc[NT];
+    // x fragments from LDS, or (without a prologue and a long slab) step by step from the cache: those queue behind the W slab and
+    // need no registers until then
+    if constexpr (PRO != 0) xrow = xs + m_own * xstride;
+    floatx4 acc[NT], other = floatx4{0.f, 0.f, 0.f, 0.f};             // (other: the half tile's products with the second half of x)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < KSTEPS; ++s) {
-        const int ko = k_begin + s * 64 + g * 16;
-        const bf16x8 b0 = (xvalid && ko + 8 <= K) ? load8(xrow + ko) : zero8();
-        const bf16x8 b1 = (xvalid && ko + 16 <= K) ? load8(xrow + ko + 8) : zero8();
+    auto multiply = [&](int s, const bf16x8& b0, const bf16x8& b1) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][0], b0, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][1], b1, acc[t], 0, 0, 0);
+            if (half_tile(t)) other = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][0], b1, other, 0, 0, 0);
+            else acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][1], b1, acc[t], 0, 0, 0);
+        }
+    };
+    if (whole == KSTEPS) {
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            if constexpr (BESIDE) multiply(s, bx[s][0], bx[s][1]);
+            else multiply(s, load8(xrow + k_begin + s * 64 + g * 16), load8(xrow + k_begin + s * 64 + g * 16 + 8));
+        }
+    } else {
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            if (s > whole || (s == whole && rest == 0)) continue;
+            const int ko = k_begin + s * 64 + g * 16;
+            const bool in0 = ko + 8 <= K, in1 = ko + 16 <= K;
+            bf16x8 b0, b1;
+            if constexpr (BESIDE) { b0 = bx[s][0]; b1 = bx[s][1]; }
+            else { b0 = load8(xrow + (in0 ? ko : 0)); b1 = load8(xrow + (in1 ? ko + 8 : 0)); }
+            if (s == whole) {                        // past the depth: zeros on both sides
+                if (!in0) b0 = zero8();
+                if (!in1) b1 = zero8();
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    if (half_tile(t) && upper ? !in1 : !in0) a[t][s][0] = zero8();
+                    if (!half_tile(t) && !in1) a[t][s][1] = zero8();
+                }
+            }
+            multiply(s, b0, b1);
         }
     }
     // the waves' partial tiles meet in LDS (a slot per wave and tile); one barrier, then wave t sums tile t
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-        if (wave != t) red[(wave * NT + t) * 64 + lane] = acc[t];
+    for (int t = 0; t < NT; ++t) red[(wave * NT + t) * 64 + lane] = half_tile(t) && g >= 2 ? other : acc[t];
     __syncthreads();
     if (wave >= NT) return;
-    floatx4 sum = acc[0];
+    // (in two batches where two workgroups' registers fit a unit: sixteen partial sums are 64 of them)
+    constexpr int BATCH = WAVES > 8 && KSTEPS <= (HALF ? 4 : 2) && (PRO == 0 || PRO == 3) ? 8 : WAVES;
+    floatx4 sum = red[wave * 64 + lane];
 #pragma unroll
-    for (int t = 1; t < NT; ++t)
-        if (wave == t) sum = acc[t];
+    for (int w0 = 0; w0 < WAVES; w0 += BATCH) {
+        floatx4 part[BATCH];
 #pragma unroll
-    for (int wv = 0; wv < WAVES; ++wv)
-        if (wv != wave) sum += red[(wv * NT + wave) * 64 + lane];
-    const int n0 = n_base + 16 * wave + 4 * g;
-    if (r16 < M && 16 * wave + 4 * g < ROWS && n0 < N) store4<OUT_F32>(out, bias, residual, act, r16, n0, N, sum, ex);
+        for (int i = 0; i < BATCH; ++i) part[i] = red[((w0 + i) * NT + wave) * 64 + lane];
+#pragma unroll
+        for (int i = w0 == 0; i < BATCH; ++i) sum += part[i];
+        if (w0 + BATCH < WAVES) asm volatile("" : "+v"(sum) : : "memory");
+    }
+    if (HALF && wave == NT - 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] = across<32, false>(sum[i]);
+    }
+    if (own) ep.finish<OUT_F32>(out, bias, residual, act, r16, n0, N, sum, ex);
 }
 
 // ------------------------------------------------------------------------- tiled

@@ -91,11 +91,9 @@ void count_gemm_path(int path);
 #ifdef __HIPCC__
 namespace st {
 
-// Destination of output feature n (>= q_size) of row m inside the caches, or -1.
+// Destination of output feature n (>= q_size) of a row of `item` at `pos` inside the caches, or -1.
 // which: 0 = key, 1 = value.
-__device__ inline int64_t kv_scatter_offset(const StGemmExtras& e, int m, int n, int* which) {
-    const int item = e.token_item[m];
-    const int pos = e.positions[m];
+__device__ inline int64_t kv_scatter_place(const StGemmExtras& e, int item, int pos, int n, int* which) {
     if (item < 0 || pos < 0) return -1;
     int c = n - e.q_size;
     *which = c >= e.kv_size ? 1 : 0;
@@ -105,6 +103,10 @@ __device__ inline int64_t kv_scatter_offset(const StGemmExtras& e, int m, int n,
     const int page = e.block_table[(int64_t)item * e.max_pages + pi];
     if (page < 0) return -1;
     return (int64_t)page * e.page_stride + ((int64_t)head * e.page_size + (pos - pi * e.page_size)) * e.head_dim + d;
+}
+// the same for row m
+__device__ inline int64_t kv_scatter_offset(const StGemmExtras& e, int m, int n, int* which) {
+    return kv_scatter_place(e, e.token_item[m], e.positions[m], n, which);
 }
 
 }  // namespace st
