@@ -27,6 +27,7 @@
 #include "api.h"
 
 #include <mutex>
+#include <type_traits>
 
 namespace st {
 
@@ -141,22 +142,27 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
     const int d0 = sub * VEC;
     const bool dvalid = d0 < head_dim;
 
+    // whole pages in a number of positions, by a shift where that will do (a division by a number that is known only here is some
+    // thirty instructions one after the other, before the first key is asked for)
+    const bool shifts = (page_size & (page_size - 1)) == 0;
+    const int page_bits = 31 - __builtin_clz(page_size);
+    const auto pages_in = [&](int n) { return shifts ? n >> page_bits : n / page_size; };
+
     int kb = 0, ke = 0;
     if (item >= 0 && pos >= 0) {
         const int hi = pos + 1;
         // window > 0: the last `window` positions; window < 0: the positions of the row's own chunk of
         // -window positions, chunks counted from the sequence's start
         const int lo = window > 0 ? (hi > window ? hi - window : 0) : window < 0 ? pos - pos % (-window) : 0;
-        const int chunk = (hi - lo + num_splits - 1) / num_splits;
+        const int chunk = num_splits == 1 ? hi - lo : (hi - lo + num_splits - 1) / num_splits;
         kb = lo + split * chunk;
         ke = min(hi, kb + chunk);
     }
     // the pages this workgroup will touch go to LDS first: key addresses then need no
     // dependent global load
-    int p_lo = 0;
     if (kb < ke) {
-        p_lo = kb / page_size;
-        const int p_n = (ke - 1) / page_size - p_lo + 1;
+        const int p_lo = pages_in(kb);
+        const int p_n = pages_in(ke - 1) - p_lo + 1;
         const int* bt = block_table + (int64_t)item * max_pages + p_lo;
         for (int i = threadIdx.x; i < p_n; i += blockDim.x) s_bt[i] = bt[i];
     }
@@ -178,8 +184,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
         }
     }
     const float post_scale = DOT2 ? scale : 1.f;
-    const int kvh = h / (num_q_heads / num_kv_heads);
-    const int64_t head_off = (int64_t)kvh * page_size * head_dim + d0;
+    const int kvh = num_q_heads == num_kv_heads ? h : h / (num_q_heads / num_kv_heads);
     // a position encoding may add slope * (key position - query position) to this head's scores
     const float slope = head_slopes ? head_slopes[h] : 0.f;
     const float inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;   // scores pass through softcap * tanh(s / softcap)
@@ -190,27 +195,42 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
 #pragma unroll
     for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
 
-    // U keys of this lane group per round, two rounds in registers: one being used, one in flight
+    // U keys of this lane group per round, two rounds in registers: one being used, one in flight.  Every load is unconditional: a place
+    // past the last key stands for that key (its values are cleared and its score is that of none), and all groups take the same number
+    // of rounds.  (Behind a branch of a lane's the compiler waits for every load that is on its way before it uses the first, so that no
+    // round was on its way beside another's arithmetic.)  The pages of the round after next come from LDS a round ahead.  32 heads of 64, us
+    // before and so: 8 rows of 60 keys 5.1 and 5.0, of 300 7.6 and 7.1, of 1,536 23.4 and 21.3 (4.7 TB/s), of 300 to 1,700 22.0 and 18.2;
+    // 16 rows of 1,000 27.7 and 26.5, 64 93.0 and 90.4; 8 rows of 700 keys, 20 heads of 80, 17.1 and 12.5; of 900, 8 heads of 128 over 2,
+    // 18.9 and 12.3.
     constexpr int U = 4;
     uint4 kA[U], vA[U], kB[U], vB[U];
     const int round_keys = G * U;
-    auto issue = [&](uint4* kr, uint4* vr, int j0) {
+    // (lanes that hold nothing of the head read its start, and their part of a score is zero)
+    const int64_t lane_off = (int64_t)kvh * page_size * head_dim + (dvalid ? d0 : 0);
+    int page_of[U], row_of[U];                           // (rows counted in elements)
+    int jn = kb + gi, jq = 0, jr = 0, last_q = 0, last_r = 0;
+    const int step_q = pages_in(G), page_rows = page_size * head_dim, step_r = G * head_dim - step_q * page_rows;
+    const auto look_up = [&] {                           // the next U keys' pages and rows of them
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int j = j0 + u * G;
-            if (j < ke && dvalid) {
-                const int pi = j / page_size;
-                const int64_t off = (int64_t)s_bt[pi - p_lo] * page_stride + head_off +
-                                    (int64_t)(j - pi * page_size) * head_dim;
-                kr[u] = *reinterpret_cast<const uint4*>(k_cache + off);
-                vr[u] = *reinterpret_cast<const uint4*>(v_cache + off);
-            } else {
-                kr[u] = make_uint4(0, 0, 0, 0);
-                vr[u] = make_uint4(0, 0, 0, 0);
-            }
+            const bool in = jn < ke;
+            page_of[u] = s_bt[in ? jq : last_q];
+            row_of[u] = in ? jr : last_r;
+            jn += G; jq += step_q; jr += step_r;
+            if (jr >= page_rows) { jr -= page_rows; ++jq; }
         }
     };
-    auto consume = [&](const uint4* kr, const uint4* vr, int j0) {
+    const auto issue = [&](uint4* kr, uint4* vr) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t off = (int64_t)((uint64_t)(uint32_t)page_of[u] * (uint64_t)page_stride) + lane_off + row_of[u];
+            kr[u] = *reinterpret_cast<const uint4*>(k_cache + off);
+            vr[u] = *reinterpret_cast<const uint4*>(v_cache + off);
+        }
+    };
+    // TAIL: the last round, in which there may be fewer keys
+    const auto consume = [&](uint4* kr, uint4* vr, int j0, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
         float s[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -226,14 +246,17 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) d = fmaf(qv[i], kf[i], d);
             }
-            s[u] = d;
+            s[u] = dvalid ? d : 0.f;
         }
         float mn = m;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             s[u] = fmaf(slope, (float)(j0 + u * G - pos), group_sum<LPK>(s[u]) * post_scale);   // slope 0: the score itself
             if (softcap > 0.f) s[u] = softcap * (ACC ? tanhf(s[u] * inv_cap) : tanh_fast(s[u] * inv_cap));
-            if (j0 + u * G >= ke) s[u] = -INFINITY;      // the same for all lanes of a group
+            if (TAIL && j0 + u * G >= ke) {              // the same for all lanes of a group
+                s[u] = -INFINITY;
+                vr[u] = make_uint4(0, 0, 0, 0);
+            }
             mn = fmaxf(mn, s[u]);
         }
         const float alpha = exp_<ACC>(m - mn);           // m = -inf in the first round: 0
@@ -252,17 +275,49 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(
         l = l * alpha + psum;
         m = mn;
     };
-    {
-        int j0 = kb + gi;                                // this group's first key; j0 < ke: it has work
-        if (j0 < ke) issue(kA, vA, j0);
-        while (j0 < ke) {
-            if (j0 + round_keys < ke) issue(kB, vB, j0 + round_keys);
-            consume(kA, vA, j0);
+    // everything up to here has been formed before anything behind is asked for
+    const auto settle = [&] {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) asm volatile("" : "+v"(acc[i]));
+        asm volatile("" : "+v"(l), "+v"(m) : : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (kb < ke) {
+        const int first = pages_in(kb);
+        last_q = pages_in(ke - 1);
+        last_r = (ke - 1 - last_q * page_size) * head_dim;
+        last_q -= first;
+        jq = pages_in(jn);
+        jr = (jn - jq * page_size) * head_dim;
+        jq -= first;
+        // (a loop with one way out: where two meet the compiler would wait for what either has on its way)
+        const int more = __builtin_amdgcn_readfirstlane((ke - kb - 1) >> (31 - __builtin_clz(round_keys)));   // rounds behind the first (of a power of two)
+        int j0 = kb + gi;
+        look_up();
+        issue(kA, vA);
+        look_up();
+        for (int r = 0; r + 2 <= more; r += 2) {
+            issue(kB, vB);
+            look_up();
+            __builtin_amdgcn_sched_barrier(0);
+            consume(kA, vA, j0, std::false_type());
+            settle();                                    // (the next round's registers are this one's)
             j0 += round_keys;
-            if (j0 >= ke) break;
-            if (j0 + round_keys < ke) issue(kA, vA, j0 + round_keys);
-            consume(kB, vB, j0);
+            issue(kA, vA);
+            look_up();
+            __builtin_amdgcn_sched_barrier(0);
+            consume(kB, vB, j0, std::false_type());
+            settle();
             j0 += round_keys;
+        }
+        if (more & 1) {
+            issue(kB, vB);
+            __builtin_amdgcn_sched_barrier(0);
+            consume(kA, vA, j0, std::false_type());
+            j0 += round_keys;
+            if (j0 < ke) consume(kB, vB, j0, std::true_type());
+        } else if (j0 < ke) {
+            consume(kA, vA, j0, std::true_type());
         }
     }
 
