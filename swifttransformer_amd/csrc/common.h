@@ -151,33 +151,50 @@ __device__ inline float exp_le0(float x) {
 
 // The sum (or, MAX, the largest) of a value over the lanes that differ by O, where the lanes O apart from each other's are already
 // alike or distinct by it alone: turns of 32, 16 (row swaps), 8, 4, 2, 1 (rotations within 16 lanes), from the largest down to any of them.
-template <int O, bool MAX>
-__device__ inline float across(float x) {
-    float a, b;
-    if (O >= 16) {
-        const uint32_t u = __float_as_uint(x);
-        const auto v = O == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
-        a = __uint_as_float(v[0]); b = __uint_as_float(v[1]);
+// (Both sides of such a pair, in one order or the other.)
+template <int O>
+__device__ inline void pair_across(uint32_t x, uint32_t& a, uint32_t& b) {
+    if constexpr (O >= 16) {
+        const auto v = O == 32 ? __builtin_amdgcn_permlane32_swap(x, x, false, false) : __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        a = v[0]; b = v[1];
     } else {
         a = x;
-        b = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + (O >= 16 ? 1 : O), 0xF, 0xF, false));
+        b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x120 + O, 0xF, 0xF, false);
     }
-    return MAX ? fmaxf(a, b) : a + b;
+}
+template <int O, bool MAX>
+__device__ inline float across(float x) {
+    uint32_t a, b;
+    pair_across<O>(__float_as_uint(x), a, b);
+    return MAX ? fmaxf(__uint_as_float(a), __uint_as_float(b)) : __uint_as_float(a) + __uint_as_float(b);
+}
+// over G neighbouring lanes, a power of two; every lane gets the result
+template <int G, bool MAX>
+__device__ inline float across_lanes(float v) {
+    if constexpr (G > 32) v = across<32, MAX>(v);
+    if constexpr (G > 16) v = across<16, MAX>(v);
+    if constexpr (G > 8) v = across<8, MAX>(v);
+    if constexpr (G > 4) v = across<4, MAX>(v);
+    if constexpr (G > 2) v = across<2, MAX>(v);
+    if constexpr (G > 1) v = across<1, MAX>(v);
+    return v;
 }
 
 // Over the 64 lanes, which are all there; every lane gets the result.  Moves between the lanes, not trips through LDS, six of which
-// one after the other are most of the time of a small norm; the same pairs, so the same bits.
-template <bool MAX>
-__device__ inline float across_wave(float v) {
-    v = across<32, MAX>(v);
-    v = across<16, MAX>(v);
-    v = across<8, MAX>(v);
-    v = across<4, MAX>(v);
-    v = across<2, MAX>(v);
-    return across<1, MAX>(v);
+// one after the other are most of the time of a small norm.
+__device__ inline float wave_sum(float v) { return across_lanes<64, false>(v); }
+__device__ inline float wave_max(float v) { return across_lanes<64, true>(v); }
+
+// what the lanes up to and with one's own hold together, over the 64 lanes: within 16 by shifts, then the rows' ends to the rows behind
+__device__ inline int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);        // lane 15 to the second row, lane 47 to the fourth
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);        // lane 31 to the upper half
+    return v;
 }
-__device__ inline float wave_sum(float v) { return across_wave<false>(v); }
-__device__ inline float wave_max(float v) { return across_wave<true>(v); }
 
 // Sum over a workgroup of up to 1024 threads; every thread gets the result.
 // `red` is LDS scratch of at least 16 floats; safe to call repeatedly.
