@@ -44,6 +44,7 @@ int st_gemm(void* out, const void* x, const void* w, const float* bias, const fl
             const StGemmExtras* extras, hipStream_t stream);
 int st_gemm_path_counts(uint64_t* out, int reset);
 uint64_t st_gemm_split_count(int reset);
+uint64_t st_gemm_parts_count(int reset);
 int st_gemm_library_rule(int min_rows, int64_t min_weights, int min_depth);
 // Which workgroup shapes a product with the norm prologue may take (for measurements and tests):
 // bit 1 the wide ones (24 features) at all, bit 2 sixteen waves for them, and 32 features, bit 4

@@ -17,7 +17,7 @@
 
 namespace st {
 
-static std::atomic<uint64_t> g_path_counts[kNumGemmPaths], g_split_count;
+static std::atomic<uint64_t> g_path_counts[kNumGemmPaths], g_split_count, g_parts_count;
 void count_gemm_path(int path) {
     if (path >= 0 && path < kNumGemmPaths) g_path_counts[path].fetch_add(1, std::memory_order_relaxed);
 }
@@ -106,6 +106,11 @@ int gemm_wide(float* out, const bf16_t* x, const bf16_t* w, const float* bias, i
               const StGemmExtras& ex, hipStream_t stream);
 int gemm_library(void* out, const void* x, const void* w, const float* bias, const float* residual,
                  int M, int N, int K, int act, int out_f32, int dtype, float alpha, hipStream_t stream, bool* handled);
+bool gemm_parts_can(int M, int N, int K);
+bool gemm_parts_pays(int M, int N, int K);
+int64_t gemm_parts_scratch(int M, int N, int K);
+int gemm_parts(void* out, const bf16_t* x, const bf16_t* w, const float* bias, const float* residual, int M, int N, int K, int act, int out_f32,
+               const StGemmExtras& ex, hipStream_t stream);
 bool gemm_f32_split_pays(int M, int N, int K);
 int64_t gemm_f32_split_scratch(int M, int N, int K);
 int gemm_f32_split(float* out, const float* x, const float* w, const float* bias, const float* residual, int M, int N, int K, int act,
@@ -146,7 +151,8 @@ using namespace st;
 // (residual stream, logits) whatever `dtype` is.  algo: 0 = best available,
 // 1 = the generic tiled kernel (the plain one that the others are checked against),
 // 2 = the vendor library (an error if it has no kernel for the shape),
-// 3 = the hand-written matrix-core kernels whatever the number of rows.
+// 3 = the hand-written matrix-core kernels whatever the number of rows,
+// 4 = the bfloat16 product of a depth in parts (an error where it does not take the shape or lacks its scratch).
 // extras: optional fused work (see gemm_extras.h), or null.
 extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bias,
                        const float* residual, int M, int N, int K, int activation, int dtype,
@@ -215,6 +221,17 @@ extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bia
         if (rc == 0) g_split_count.fetch_add(1, std::memory_order_relaxed);
         return rc;
     }
+    const bool parts = dtype == kBF16 && !ex.ln_x && !ex.mg_o && !ex.k_cache && !ex.best_ids &&
+        (algo == 4 || (algo == 0 && M >= g_library_min_rows && gemm_parts_pays(M, N, K))) && gemm_parts_can(M, N, K) &&
+        (ex.scratch ? ex.scratch_floats : 0) >= gemm_parts_scratch(M, N, K) &&
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(out) |
+          reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(ex.scratch)) & 15) == 0;
+    ST_CHECK(algo != 4 || parts, "gemm: no product of a depth in parts for M=%d N=%d K=%d dtype=%d", M, N, K, dtype);
+    if (parts) {
+        const int rc = gemm_parts(out, (const bf16_t*)x, (const bf16_t*)w, bias, residual, M, N, K, act, out_f32, ex, stream);
+        if (rc == 0) g_parts_count.fetch_add(1, std::memory_order_relaxed);
+        return rc;
+    }
     const bool to_library = algo == 2 || (algo == 0 && !ex.ln_x && !ex.mg_o && library_can &&
         (dtype == kF32 || M >= g_library_min_rows ||
          ((int64_t)N * K >= g_library_min_weights && K >= g_library_min_depth)));
@@ -258,9 +275,11 @@ extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bia
     return 0;
 }
 
-// Floats of scratch (StGemmExtras::scratch) that a product asks for, by algo (0 or 3): with less, one of algo 0 goes to the library, one of
+// Floats of scratch (StGemmExtras::scratch) that a product asks for, by algo (0, 3 or 4): with less, one of algo 0 goes to the library, one of
 // algo 3 runs with fewer workgroups at its end.
 extern "C" int64_t st_gemm_scratch(int M, int N, int K, int dtype, int algo) {
+    if (dtype == kBF16)
+        return (algo == 4 && gemm_parts_can(M, N, K)) || (algo == 0 && M >= g_library_min_rows && gemm_parts_pays(M, N, K)) ? gemm_parts_scratch(M, N, K) : 0;
     if (dtype != kF32 || !f32_split_can(M, N, K) || !(algo == 3 || (algo == 0 && gemm_f32_split_pays(M, N, K)))) return 0;
     return gemm_f32_split_scratch(M, N, K);
 }
@@ -281,7 +300,8 @@ extern "C" int st_gemm_library_rule(int min_rows, int64_t min_weights, int min_d
 }
 
 // Calls of st_gemm per kernel family since the last reset (order of st::GemmPath); returns the
-// number of families.  `out` may be null.  (Float products of split operands: st_gemm_split_count.)
+// number of families.  `out` may be null.  (Float products of split operands: st_gemm_split_count; bfloat16
+// products of depths in parts: st_gemm_parts_count.)
 extern "C" int st_gemm_path_counts(uint64_t* out, int reset) {
     for (int i = 0; i < kNumGemmPaths; ++i) {
         const uint64_t v = reset ? g_path_counts[i].exchange(0) : g_path_counts[i].load();
@@ -291,6 +311,7 @@ extern "C" int st_gemm_path_counts(uint64_t* out, int reset) {
 }
 
 // Calls of st_gemm that gemm_f32_split took since the last reset.
+extern "C" uint64_t st_gemm_parts_count(int reset) { return reset ? g_parts_count.exchange(0) : g_parts_count.load(); }
 extern "C" uint64_t st_gemm_split_count(int reset) { return reset ? g_split_count.exchange(0) : g_split_count.load(); }
 
 // Whether st_gemm (algo 0) can take a split attention output (partials and log-sum-exps) as its input.

@@ -51,6 +51,7 @@ def _lib():
                                 _c_int, _c_int, _c_p, _c_p]
         lib.st_gemm_path_counts.argtypes = [_c_p, _c_int]
         lib.st_gemm_split_count.argtypes, lib.st_gemm_split_count.restype = [_c_int], ctypes.c_uint64
+        lib.st_gemm_parts_count.argtypes, lib.st_gemm_parts_count.restype = [_c_int], ctypes.c_uint64
         lib.st_gemm_library_rule.argtypes = [_c_int, _c_i64, _c_int]
         lib.st_gemm_can_fuse_norm.argtypes = [_c_int, _c_int, _c_int, _c_int]
         lib.st_gemm_wide_offered.argtypes = [_c_int, _c_int, _c_int, _c_int]
@@ -403,6 +404,11 @@ def gemm_split_count(reset: bool = False) -> int:
     return int(_lib().st_gemm_split_count(int(reset)))
 
 
+def gemm_parts_count(reset: bool = False) -> int:
+    """bfloat16 products whose depth was dealt to several workgroups, with a kernel for their sums, since the last reset."""
+    return int(_lib().st_gemm_parts_count(int(reset)))
+
+
 def gemm_library_rule(min_rows: int = -1, min_weights: int = -1, min_depth: int = -1) -> None:
     """Change when bfloat16 products go to the vendor library (for measurements): from ``min_rows``
     rows on, and below that for matrices of ``min_weights`` elements and ``min_depth`` depth.  -1
@@ -433,8 +439,9 @@ def wide_offered(M: int, N: int, K: int, dtype: torch.dtype) -> bool:
 @functools.lru_cache(maxsize=4096)
 def _gemm_scratch(M: int, N: int, K: int, code: int, most: bool, algo: int = 0) -> int:
     """Floats of scratch that a product of M rows asks for; ``most``: that one of any number of rows up to M may ask for (it
-    depends on the tiles of 128 rows)."""
-    of = list(range(128, M, 128)) + [M] if most else [M]
+    depends on the tiles, of 128 rows, or of 64 and only up to some hundred rows)."""
+    each = 128 if code == F32 else 64
+    of = list(range(each, M if code == F32 else min(M, 1024), each)) + [M] if most else [M]
     return max(_lib().st_gemm_scratch(m, N, K, code, algo) for m in of)
 
 
@@ -550,7 +557,8 @@ def gemm(x, w: torch.Tensor, *, bias: Optional[torch.Tensor] = None,
         idx = empty((n_scratch,), torch.int32, device)
         keep += [val, idx]
         ex.best_ids, ex.best_val, ex.best_idx = _ptr(best), _ptr(val), _ptr(idx)
-    scratch = _gemm_scratch(M, N, K, code, arena.measuring(), int(algo)) if code == F32 and M and algo in (0, 3) else 0
+    asks = algo in (0, 3) if code == F32 else algo in (0, 4) and x_ptr is not None and kv_scatter is None and best is None
+    scratch = _gemm_scratch(M, N, K, code, arena.measuring(), int(algo)) if M and asks else 0
     if scratch:
         if ex is None:
             ex = _GemmExtras()
