@@ -778,6 +778,11 @@ __global__ __launch_bounds__(256) void moe_down_kernel(
 // 64 on 256 rows: 145 us at 753 tokens.  With the meeting before a step's last quarter instead of between two steps: 2,011 tokens
 // 219 -> 205 us, 1,024 tokens 129 -> 123; 4,096 x 4,096, 2,048 tokens 656 -> 619, 951 tokens 395 -> 386; tiles of 64 within 2 %.
 // (2,011 tokens before: 153 us with the loads taken out, 176 with the products taken out; 205 on matrices stored in the order of the tiles.)
+// A workgroup of 256 rows is a unit's only one, so a die's last round may be nearly empty: what its whole rounds of a unit each leave over goes in
+// halves (128 rows) where that is up to half of a round, in quarters (and 64 places) up to a quarter; 128 x 128 and 128 x 64 take two thirds and
+// half of a whole one's time, the bytes of their operands.  Up and output product, us: 16 experts of 2,048 x 2,048, 2,011 tokens (8 to 16 of 32
+// units in the last round) 127 + 80 -> 111 + 61, 1,024 tokens 88 + 44 -> 77 + 45; 8 of 2,048 x 3,072, 2,048 tokens 165 + 105 -> 151 + 81; 14 of
+// 4,096 x 4,096 426 + 220 -> 403 + 205.
 // Tried and no better: 256 places a tile (at 753 tokens 187 us; as the loop is now 195 to 199 at 2,011, 173 at 753, 413 at 951 of 4,096),
 // 128 weight rows on 256 places (220 at 2,011), four waves with 128 weight rows each (206), two buffers for 256 rows (156),
 // four and five for 128 rows, workgroups that stay and take the next item while the last one's results are stored (no gain), loads of
@@ -788,56 +793,73 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 // a row's chunk of 8 in depth lies at chunk ^ swizzle(row): 16 neighbouring rows' like chunks lie in different banks
 __device__ inline int swizzle(int row) { return (row >> 1) & 7; }
 
-// the tile and the block of weight rows of a workgroup; false where there is none left
-__device__ inline bool moe_work_item(int& tile, int& block, int& expert, const int* __restrict__ tile_expert, int max_tiles, int blocks) {
+// the tile and the block of weight rows of a workgroup, and which of how many pieces of it; false where there is none left
+struct MoeWork { int tile, block, expert, piece, pieces; };
+__device__ inline bool moe_work_item(MoeWork& w, const int* __restrict__ tile_expert, int max_tiles, int blocks, int per_die) {
     const int lane = threadIdx.x & 63;
     int tiles = 0;
     for (int b = 0; b < max_tiles; b += 64)
         tiles += __popcll(__ballot(b + lane < max_tiles && tile_expert[min(b + lane, max_tiles - 1)] >= 0));
     const int items = tiles * blocks, share = (items + 7) / 8;       // (the host checks that the numbers fit)
-    const int j = blockIdx.x >> 3, i = (blockIdx.x & 7) * share + j;
-    if (j >= share || i >= items) return false;
-    expert = tile_expert[i / blocks];                                // (an expert's tiles are neighbours)
+    const int die = blockIdx.x & 7, j = blockIdx.x >> 3, mine = min(share, items - die * share);
+    int at = j;
+    w.piece = 0;
+    w.pieces = 1;
+    if (per_die > 0) {                                               // what whole rounds leave over goes in pieces, where those fill no more than a round
+        const int whole = mine / per_die * per_die, rest = mine - whole;
+        w.pieces = j < whole ? 1 : 4 * rest <= per_die ? 4 : 2 * rest <= per_die ? 2 : 1;
+        at = j < whole ? j : whole + (j - whole) / w.pieces;
+        w.piece = j < whole ? 0 : (j - whole) % w.pieces;
+    }
+    if (at >= mine) return false;
+    const int i = die * share + at;
+    w.expert = tile_expert[i / blocks];                              // (an expert's tiles are neighbours)
     int before = 0, own = 0;
     for (int b = 0; b < max_tiles; b += 64) {
         const int v = tile_expert[min(b + lane, max_tiles - 1)];
         const bool in = b + lane < max_tiles && v >= 0;
-        before += __popcll(__ballot(in && v < expert));
-        own += __popcll(__ballot(in && v == expert));
+        before += __popcll(__ballot(in && v < w.expert));
+        own += __popcll(__ballot(in && v == w.expert));
     }
     const int r = i - before * blocks;
-    block = r / own;
-    tile = before + (r - block * own);
+    w.block = r / own;
+    w.tile = before + (r - w.block * own);
     return true;
 }
 
 enum TiledKind : int { kTiledDown = 0, kTiledUp = 1, kTiledGelu = 2 };
 
-// AHEAD: steps on their way beside the one that is multiplied
-template <int KIND, int WN, int NJ, int AHEAD>
-__global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 1) void moe_tiled_kernel(
-    bf16_t* __restrict__ y_out, float* out, const float* residual, float* __restrict__ pair_out, const bf16_t* __restrict__ a_rows,
-    const bf16_t* __restrict__ w0, const bf16_t* __restrict__ w1, const int* __restrict__ sorted, const int* __restrict__ tile_expert,
-    const float* __restrict__ weights, int max_tiles, int blocks, int top, int N, int K, float limit, float out_scale, int style) {
+struct MoeTiled {
+    bf16_t* y_out; float* out; const float* residual; float* pair_out;
+    const bf16_t *a_rows, *w0, *w1;
+    const int* sorted; const float* weights;
+    int top, N, K; float limit, out_scale; int style;
+};
+
+// PLACES places from `base` on by 64 RG weight rows from feature n0 on, of expert e, by RG x PG waves: each has 64 rows and NJ blocks of 32 places
+// (waves past the places load with the others and multiply nothing).  AHEAD: steps on their way beside the one that is multiplied; DOUBLE:
+// sums are carried in double every few steps.
+template <int KIND, int RG, int PG, int NJ, int PLACES, int AHEAD, bool DOUBLE>
+__device__ __forceinline__ void moe_tile_body(const MoeTiled& arg, uint4* lds, int buf_stride, int base, int n0, int turn, int e) {
+    bf16_t* y_out = arg.y_out;
+    float *out = arg.out, *pair_out = arg.pair_out;
+    const float *residual = arg.residual, *weights = arg.weights;
+    const bf16_t *a_rows = arg.a_rows, *w0 = arg.w0, *w1 = arg.w1;
+    const int* sorted = arg.sorted;
+    const int top = arg.top, N = arg.N, K = arg.K, style = arg.style;
+    const float limit = arg.limit, out_scale = arg.out_scale;
     constexpr bool UP = KIND == kTiledUp, GATHER = KIND != kTiledDown;
-    // Results that stay float, of tiles of 64 places: sums are carried in double every few steps.  With 7 to 31 pairs an expert the tiles of
-    // 16 were used before, whose waves share the depth: their chains are an eighth as long (2,048 deep: 2.7e-7 off float64 in one chain,
-    // 1.3e-7 in theirs).
-    constexpr bool DOUBLE = KIND == kTiledDown && NJ == 1;
-    constexpr int WAVES = 2 * WN, ROWS = 64 * WN, PLACES = 64 * NJ;
-    constexpr int BUF = (ROWS + PLACES) * 8;               // 16-byte pieces a buffer: weight rows, then places
+    constexpr int WAVES = RG * PG, ROWS = 64 * RG;
     constexpr int NW = ROWS / (8 * WAVES), NP = PLACES / (8 * WAVES), NL = NW + NP;      // direct loads a wave and step, eight rows each
-    __shared__ uint4 lds[(AHEAD + 1) * BUF];
-    int tile, block, e;
-    if (!moe_work_item(tile, block, e, tile_expert, max_tiles, blocks)) return;
+    static_assert(NW * 8 * WAVES == ROWS && NP * 8 * WAVES == PLACES, "whole loads");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave % WN, wm = wave / WN, l32 = lane & 31, lh = lane >> 5;
-    const int base = tile * PLACES, n0 = block * (UP ? ROWS / 2 : ROWS);
+    const int wn = wave % RG, wm = wave / RG, l32 = lane & 31, lh = lane >> 5;
+    const bool on = NJ * PG * 32 == PLACES || wm * 32 < PLACES;      // (where there are more waves than blocks, NJ is 1)
     int pair[NJ], full = 0;                        // the pairs of the lane's columns of results; how many of the wave's blocks hold one
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        pair[j] = sorted[base + (2 * j + wm) * 32 + l32];
-        full += __ballot(pair[j] >= 0) != 0;       // (an expert's pairs come first in its tiles)
+        pair[j] = sorted[base + (on ? (PG * j + wm) * 32 : 0) + l32];
+        full += on && __ballot(pair[j] >= 0) != 0;       // (an expert's pairs come first in its tiles)
     }
     // Load t of a wave brings rows 8 (wave + WAVES t) on, a lane 16 bytes of row + lane / 8: piece lane % 8 of the row's place in
     // LDS, which is the chunk that the row's swizzle puts there, the same for all t.  Rows past the matrix stand for row 0 and places
@@ -857,11 +879,11 @@ __global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 
         }
         src[t] += chunk * 8;
     }
-    const int whole = K >> 6, steps = (K + 63) >> 6, begin = block * 3 % steps;
+    const int whole = K >> 6, steps = (K + 63) >> 6, begin = turn * 3 % steps;
     auto stage = [&](int s, int buf) {
         int k = s + begin;
         if (k >= steps) k -= steps;
-        uint4* dst = lds + buf * BUF + wave * 64;
+        uint4* dst = lds + buf * buf_stride + wave * 64;
         if (k < whole) {
 #pragma unroll
             for (int t = 0; t < NL; ++t)
@@ -901,11 +923,11 @@ __global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 
         constexpr int B = decltype(blocks32)::value;
         auto fetch = [&](int cur, int kk) {                         // the operands of a product of depth 16
             if constexpr (B > 0) {
-                const uint4* at = own + cur * BUF + ((kk * 2 + lh) ^ swz);
+                const uint4* at = own + cur * buf_stride + ((kk * 2 + lh) ^ swz);
 #pragma unroll
                 for (int q = 0; q < 2; ++q) a[kk & 1][q] = __builtin_bit_cast(bf16x8, at[(wn * 64 + q * 32) * 8]);
 #pragma unroll
-                for (int j = 0; j < B; ++j) b[kk & 1][j] = __builtin_bit_cast(bf16x8, at[(ROWS + (j * 2 + wm) * 32) * 8]);
+                for (int j = 0; j < B; ++j) b[kk & 1][j] = __builtin_bit_cast(bf16x8, at[(ROWS + (j * PG + wm) * 32) * 8]);
             }
         };
         auto multiply = [&](int kk) {
@@ -961,7 +983,8 @@ __global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 
     if (full == NJ) walk(Steps<NJ>());
     else if (NJ > 1 && full > 0) walk(Steps<1>());
     else walk(Steps<0>());
-    // acc[q][j][u]: weight row wn * 64 + q * 32 + 8 * (u / 4) + 4 * lh + u % 4, place base + (2 * j + wm) * 32 + l32
+    if (!on) return;
+    // acc[q][j][u]: weight row wn * 64 + q * 32 + 8 * (u / 4) + 4 * lh + u % 4, place base + (PG * j + wm) * 32 + l32
     auto store_row = [&](int place, int f, const float* r) {
         bf16_t* dst = y_out + (int64_t)place * N + f;
         if (f + 3 < N && (N & 3) == 0) Elem<bf16_t>::store4(dst, r);
@@ -970,7 +993,7 @@ __global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 
     };
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
-        const int place = base + (j * 2 + wm) * 32 + l32;
+        const int place = base + (j * PG + wm) * 32 + l32;
         const int p = pair[j];
         if (UP) {
             const float scale = p >= 0 && style == 0 ? weights[p] : 1.f;
@@ -1031,6 +1054,33 @@ __global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 
     }
 }
 
+// per_die: compute units of a die, where what whole rounds of them leave over goes in pieces (workgroups of 256 rows by 128 places), else 0
+template <int KIND, int WN, int NJ, int AHEAD>
+__global__ __launch_bounds__(128 * WN, WN == 2 && (NJ == 1 || AHEAD == 1) ? 2 : 1) void moe_tiled_kernel(
+    const MoeTiled arg, const int* __restrict__ tile_expert, int max_tiles, int blocks, int per_die) {
+    constexpr int ROWS = 64 * WN, PLACES = 64 * NJ, BUF = (ROWS + PLACES) * 8;           // 16-byte pieces a buffer: weight rows, then places
+    __shared__ uint4 lds[(AHEAD + 1) * BUF];
+    // Results that stay float, of tiles of 64 places: sums are carried in double every few steps.  With 7 to 31 pairs an expert the tiles of
+    // 16 were used before, whose waves share the depth: their chains are an eighth as long (2,048 deep: 2.7e-7 off float64 in one chain,
+    // 1.3e-7 in theirs).
+    constexpr bool DOUBLE = KIND == kTiledDown && NJ == 1;
+    constexpr int FEATURES = KIND == kTiledUp ? ROWS / 2 : ROWS;                         // of a block
+    MoeWork w;
+    if (!moe_work_item(w, tile_expert, max_tiles, blocks, per_die)) return;
+    const int base = w.tile * PLACES, n0 = w.block * FEATURES;
+    if constexpr (WN == 4 && NJ == 2) {
+        if (w.pieces == 2) {
+            moe_tile_body<KIND, 2, 4, 1, 128, AHEAD, DOUBLE>(arg, lds, BUF, base, n0 + w.piece * (FEATURES / 2), w.block, w.expert);
+            return;
+        }
+        if (w.pieces == 4) {
+            moe_tile_body<KIND, 2, 4, 1, 64, AHEAD, DOUBLE>(arg, lds, BUF, base + (w.piece >> 1) * 64, n0 + (w.piece & 1) * (FEATURES / 2), w.block, w.expert);
+            return;
+        }
+    }
+    moe_tile_body<KIND, WN, 2, NJ, PLACES, AHEAD, DOUBLE>(arg, lds, BUF, base, n0, w.block, w.expert);
+}
+
 template <int KIND>
 static int launch_tiled(bf16_t* y, float* out, const float* residual, float* pair_out, const void* a_rows, const void* w0,
                         const void* w1, const int* sorted, const int* tile_expert, const float* weights, int capacity, int tile, int top,
@@ -1040,9 +1090,11 @@ static int launch_tiled(bf16_t* y, float* out, const float* residual, float* pai
         constexpr int WN = decltype(wn)::value, NJ = decltype(nj)::value, AHEAD = decltype(ahead)::value;
         const int features = KIND == kTiledUp ? 32 * WN : 64 * WN, blocks = (N + features - 1) / features;
         ST_CHECK((int64_t)tiles * blocks < (1ll << 30), "moe: too many tiles");
-        const unsigned grid = (unsigned)((tiles * blocks + 7) / 8 * 8);
-        moe_tiled_kernel<KIND, WN, NJ, AHEAD><<<grid, 128 * WN, 0, stream>>>(y, out, residual, pair_out, (const bf16_t*)a_rows,
-            (const bf16_t*)w0, (const bf16_t*)w1, sorted, tile_expert, weights, tiles, blocks, top, N, K, limit, out_scale, style);
+        const int per_die = WN == 4 && NJ == 2 ? device_compute_units() / 8 : 0;
+        const unsigned grid = (unsigned)((tiles * blocks + 7) / 8 + per_die) * 8;        // (pieces: up to a round more)
+        const MoeTiled arg{y, out, residual, pair_out, (const bf16_t*)a_rows, (const bf16_t*)w0, (const bf16_t*)w1, sorted, weights, top, N, K,
+                           limit, out_scale, style};
+        moe_tiled_kernel<KIND, WN, NJ, AHEAD><<<grid, 128 * WN, 0, stream>>>(arg, tile_expert, tiles, blocks, per_die);
         return 0;
     };
     int rc;
