@@ -47,7 +47,8 @@ def test_rows_and_features_stay_apart():
     assert got[69].isnan().all() and got[:69, 131].isinf().all() and got[:69, :131].isfinite().all()
 
 
-@pytest.mark.parametrize("rows,features,depth,taken", [(64, 2048, 8192, False), (65, 2048, 8192, True), (512, 2048, 8192, True), (513, 2048, 8192, False), (150, 4096, 16384, True), (12, 4096, 16384, False),
+@pytest.mark.parametrize("rows,features,depth,taken", [(64, 2048, 8192, False), (65, 2048, 8192, True), (512, 2048, 8192, True), (513, 2048, 8192, True), (577, 2048, 16384, True), (768, 768, 8192, True),
+                                                       (769, 768, 8192, False), (576, 1024, 4096, False), (577, 4096, 8192, False), (150, 4096, 16384, True), (12, 4096, 16384, False),
                                                        (64, 2048, 2048, False), (150, 8192, 2048, False), (100, 2560, 10240, True), (100, 2560, 10208, False)])
 def test_which_products_go_there(rows, features, depth, taken):
     x, w = draw(1, rows, depth).bfloat16(), draw(2, features, depth, scale=0.05).bfloat16()
