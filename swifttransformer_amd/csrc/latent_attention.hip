@@ -647,6 +647,76 @@ __global__ __launch_bounds__(256) void latent_up_rows_kernel(
     }
 }
 
+// The same numbers where a head's matrix fits the registers (up to 32 VR values and 8 VEC DR entries) and the splits a wave: weights, partial results,
+// their log-sum-exps and gates are asked for before anything waits, and every wave weighs the splits for itself.  What bounds it is trips to memory
+// one after the other, of which the kernel above has eight.  us a call, cold matrices, above and so: 24 tokens of 32 heads of 128 x 128 6.15, 5.22, one
+// of them 6.6, 5.35, 64 8.9, 8.3; eight of 16 heads of 64 x 96 4.5, 3.2; 48 of 32 heads of 64 x 64 5.2, 4.7.
+template <typename T, int VR, int DR>
+__global__ __launch_bounds__(256) void latent_up_few_kernel(
+    T* __restrict__ y, const float* __restrict__ part_o, const float* __restrict__ part_lse, const T* __restrict__ w,
+    const float* __restrict__ gate, int64_t gate_stride, const int* __restrict__ token_item, int heads, int value_dim,
+    int out_dim, int splits) {
+    constexpr int VEC = Elem<T>::kVec, B = 8;
+    __shared__ __attribute__((aligned(16))) float s_o[8 * VEC * DR];
+    const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, sub = tid & 7;
+    const int64_t at = ((int64_t)t * heads + h) * splits;
+    const int item = token_item[t];
+    const float lse = part_lse[at + min(lane, splits - 1)];
+    float part[B];
+    const float* po = part_o + at * out_dim + min(tid, out_dim - 1);
+    auto load = [&](int s0) {
+#pragma unroll
+        for (int u = 0; u < B; ++u) part[u] = po[(int64_t)min(s0 + u, splits - 1) * out_dim];
+    };
+    load(0);
+    uint4 raw[VR][DR];
+    float logit[VR];
+    const T* wh = w + (int64_t)h * value_dim * out_dim;
+    const float* gp = gate ? gate + (int64_t)t * gate_stride + (int64_t)h * value_dim : part_lse;
+#pragma unroll
+    for (int r = 0; r < VR; ++r) {
+        const int v = min(32 * r + (tid >> 3), value_dim - 1);
+#pragma unroll
+        for (int q = 0; q < DR; ++q)
+            raw[r][q] = *reinterpret_cast<const uint4*>(wh + (int64_t)v * out_dim + min((sub + 8 * q) * VEC, out_dim - VEC));
+        logit[r] = gp[gate ? v : 0];
+    }
+    if (item < 0) return;
+    const float M = wave_max(lane < splits ? lse : -INFINITY);
+    const float e = lane < splits && M > -INFINITY ? expf(lse - M) : 0.f;
+    const float W = wave_sum(e), weight = W > 0.f ? e / W : 0.f;
+    float o = 0.f;
+    for (int s0 = 0; s0 < splits; s0 += B) {
+        if (s0) load(s0);
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+            if (s0 + u < splits) o = fmaf(__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), s0 + u)), part[u], o);
+    }
+    if (tid < out_dim) s_o[tid] = o;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < VR; ++r) {
+        const int v = 32 * r + (tid >> 3);
+        if (32 * r >= value_dim) break;                                // uniform
+        float dot = 0.f;
+#pragma unroll
+        for (int q = 0; q < DR; ++q) {
+            const int d = (sub + 8 * q) * VEC;
+            if (d >= out_dim) continue;
+            float x[VEC];
+            Elem<T>::unpack(raw[r][q], x);
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) dot = fmaf(x[k], s_o[d + k], dot);
+        }
+#pragma unroll
+        for (int k = 4; k > 0; k >>= 1) dot += __shfl_xor(dot, k, 64);
+        if (sub == 0 && v < value_dim) {
+            if (gate) dot /= 1.f + expf(-logit[r]);
+            Elem<T>::store(y + ((int64_t)t * heads + h) * value_dim + v, dot);
+        }
+    }
+}
+
 // Prompts: a wave takes 16 tokens of a head on the matrix cores; DS steps over out_dim at most.
 template <typename T, int DS>
 __global__ __launch_bounds__(256) void latent_up_kernel(
@@ -925,6 +995,17 @@ extern "C" int st_latent_up(void* y, const void* o, const float* part_o, const f
         ST_CHECK(num_tokens <= 65535, "latent_up: %d decoded tokens", num_tokens);
         const size_t lds = sizeof(float) * ((size_t)out_dim + num_splits);
         const dim3 grid(heads, num_tokens);
+        if (value_dim <= 128 && out_dim <= 128 && num_splits <= 64) {
+#define ST_LF(T, VR, DR) latent_up_few_kernel<T, VR, DR><<<grid, 256, 0, stream>>>((T*)y, part_o, part_lse, (const T*)w, gate, gate_stride, token_item, heads, value_dim, out_dim, num_splits)
+#define ST_LF_D(T, VR) do { if (out_dim <= 64) ST_LF(T, VR, 8 / Elem<T>::kVec); else ST_LF(T, VR, 16 / Elem<T>::kVec); } while (0)
+#define ST_LF_V(T) do { if (value_dim <= 64) ST_LF_D(T, 2); else ST_LF_D(T, 4); } while (0)
+            if (dtype == kF32) ST_LF_V(float); else ST_LF_V(bf16_t);
+#undef ST_LF_V
+#undef ST_LF_D
+#undef ST_LF
+            ST_LAUNCH_CHECK("latent_up (few)");
+            return 0;
+        }
         if (dtype == kF32)
             latent_up_rows_kernel<float><<<grid, 256, lds, stream>>>((float*)y, part_o, part_lse, (const float*)w, gate, gate_stride, token_item, heads, value_dim, out_dim, num_splits);
         else
