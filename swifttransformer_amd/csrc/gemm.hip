@@ -276,10 +276,11 @@ extern "C" int st_gemm(void* out, const void* x, const void* w, const float* bia
 }
 
 // Floats of scratch (StGemmExtras::scratch) that a product asks for, by algo (0, 3 or 4): with less, one of algo 0 goes to the library, one of
-// algo 3 runs with fewer workgroups at its end.
+// algo 3 runs with fewer workgroups at its end.  The same whatever st_gemm_library_rule says (callers keep the number): a product that the rule
+// sends elsewhere leaves its scratch alone.
 extern "C" int64_t st_gemm_scratch(int M, int N, int K, int dtype, int algo) {
     if (dtype == kBF16)
-        return (algo == 4 && gemm_parts_can(M, N, K)) || (algo == 0 && M >= g_library_min_rows && gemm_parts_pays(M, N, K)) ? gemm_parts_scratch(M, N, K) : 0;
+        return (algo == 4 && gemm_parts_can(M, N, K)) || (algo == 0 && gemm_parts_pays(M, N, K)) ? gemm_parts_scratch(M, N, K) : 0;
     if (dtype != kF32 || !f32_split_can(M, N, K) || !(algo == 3 || (algo == 0 && gemm_f32_split_pays(M, N, K)))) return 0;
     return gemm_f32_split_scratch(M, N, K);
 }
