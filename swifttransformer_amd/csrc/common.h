@@ -168,16 +168,17 @@ __device__ inline float across(float x) {
     pair_across<O>(__float_as_uint(x), a, b);
     return MAX ? fmaxf(__uint_as_float(a), __uint_as_float(b)) : __uint_as_float(a) + __uint_as_float(b);
 }
-// over G neighbouring lanes, a power of two; every lane gets the result
+// over G neighbouring lanes, 16, 32 or 64 (fewer are not a group of their own: the turns of 8 and less go round all 16 of a row); every
+// lane gets the result
 template <int G, bool MAX>
 __device__ inline float across_lanes(float v) {
+    static_assert(G == 16 || G == 32 || G == 64, "whole rows of 16 lanes");
     if constexpr (G > 32) v = across<32, MAX>(v);
     if constexpr (G > 16) v = across<16, MAX>(v);
-    if constexpr (G > 8) v = across<8, MAX>(v);
-    if constexpr (G > 4) v = across<4, MAX>(v);
-    if constexpr (G > 2) v = across<2, MAX>(v);
-    if constexpr (G > 1) v = across<1, MAX>(v);
-    return v;
+    v = across<8, MAX>(v);
+    v = across<4, MAX>(v);
+    v = across<2, MAX>(v);
+    return across<1, MAX>(v);
 }
 
 // Over the 64 lanes, which are all there; every lane gets the result.  Moves between the lanes, not trips through LDS, six of which

@@ -36,7 +36,7 @@ struct RouteRule {
     int experts, top, mode, groups, keep;
 };
 
-// the largest v of G neighbouring lanes and the lowest index that has it; every lane gets both
+// the larger v of a lane and those O apart from it, and the lower index of equal ones
 template <int O>
 __device__ inline void better_across(float& v, int& i) {
     uint32_t va, vb, ia, ib;
@@ -47,17 +47,19 @@ __device__ inline void better_across(float& v, int& i) {
     v = second ? b : a;
     i = second ? (int)ib : (int)ia;
 }
+// The largest v of G neighbouring lanes (16, 32 or 64, as across_lanes) and the lowest index that has it; every lane gets both.
 // (By moves between the lanes: a choice is one after the other of these, and by way of LDS one of two words takes some 130 clocks.
 // With what the rule needs asked for at the start and a wave's two pieces of a router 768 deep at once: router, choice and sorting of one
 // token 6.0 -> 5.1 us, of eight 2,048 deep 9.7 -> 9.0, choice and sorting of 33 tokens 5.0 -> 4.2; a pass of fiterax-125m 7,706 -> 7,547.)
 template <int G>
 __device__ inline void group_best(float& v, int& i) {
+    static_assert(G == 16 || G == 32 || G == 64, "whole rows of 16 lanes");
     if constexpr (G > 32) better_across<32>(v, i);
     if constexpr (G > 16) better_across<16>(v, i);
-    if constexpr (G > 8) better_across<8>(v, i);
-    if constexpr (G > 4) better_across<4>(v, i);
-    if constexpr (G > 2) better_across<2>(v, i);
-    if constexpr (G > 1) better_across<1>(v, i);
+    better_across<8>(v, i);
+    better_across<4>(v, i);
+    better_across<2>(v, i);
+    better_across<1>(v, i);
 }
 
 // What a lane needs beside its token's logit, asked for at the kernel's start: behind the choice, or behind the products that make the
