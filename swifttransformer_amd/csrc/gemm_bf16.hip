@@ -25,6 +25,7 @@
 #include "activation.h"
 
 #include <atomic>
+#include <type_traits>
 
 namespace st {
 
@@ -278,6 +279,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
 // behind the sums.  us a call in a recorded chain, before and so: 1 row 768 to 768 3.5 and 2.7, 3,072 to 768 5.4 and 4.2, with the norm 768
 // to 2,304 4.5 and 3.9; 8 rows 2,048 to 2,048 5.5 and 4.1, to 4,096 7.4 and 5.6, 8,192 to 2,048 11.8 and 9.5, 2,560 to 2,560 9.0 and 8.5,
 // with the norm 2,048 to 6,144 9.5 and 8.4, with the merge 7.6 and 6.4; 16 rows with the norm 11.3 and 10.3, 8,192 to 2,048 13.1 and 13.1.
+// Waves whose steps all lie past the depth ask for no weights: these go a way of their own through the prologue, so that on the others' way the
+// number of loads that are on their way is known.  us a call, cold weights, with all waves asking (for the first step again) and so: 16 rows
+// 256 to 5,120 5.4 and 3.2, 8 rows 512 to 5,120 5.1 and 4.0, 640 to 5,120 5.7 and 4.5, 2,560 to 2,560 8.4 and 6.8; one row 2,560 to 5,120
+// 11.7 and 9.8, 5,120 to 8,192 23.1 and 20.0.
 constexpr int kLnMaxVec = 16;            // float4 per lane of a row held in registers (K <= 4096)
 constexpr int kMgElems = 2;              // merge prologue: float4 elements of the input per thread
 constexpr int kMgSplits = 8;             // and splits per element, all held in registers;
@@ -297,8 +302,14 @@ struct DividedWalk {
     }
 };
 
+// Waves a SIMD whose registers an instance is kept to: two workgroups a unit (64 registers a lane) where that spills nothing.  One row 2,048 to
+// 2,560, 320 workgroups: 67 registers 6.3 us a call, 64 5.2.
+constexpr int resident_waves(int waves, int ksteps, int pro, int rows) {
+    return waves == 16 && ((pro == 0 && ksteps == 1) || (pro == 3 && ksteps == 2 && rows == 8)) ? 8 : waves / 4;
+}
+
 template <int WAVES, int KSTEPS, bool OUT_F32, int PRO, int ROWS>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
+__global__ __launch_bounds__(WAVES * 64, resident_waves(WAVES, KSTEPS, PRO, ROWS)) void gemm_skinny_resident_kernel(
     void* __restrict__ out, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
     const float* __restrict__ bias, const float* __restrict__ residual,
     int M, int N, int K, int act, const StGemmExtras ex) {
@@ -399,194 +410,202 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_resident_kernel(
     constexpr bool HALF = ROWS % 16 == 8;
     const auto half_tile = [](int t) { return HALF && t == NT - 1; };
     const int upper = r16 >> 3;
-    bf16x8 a[NT][KSTEPS][2];
-    const bf16_t* wb = w + (int64_t)n_base * K;
-    uint32_t wrow[NT];                                                // first element of the lane's row of W, from wb on
-#pragma unroll
-    for (int t = 0; t < NT; ++t)                                      // (rows past the matrix stand for its last: their results are not stored)
-        wrow[t] = (uint32_t)min(16 * t + (half_tile(t) ? r16 & 7 : r16), N - 1 - n_base) * (uint32_t)K;
-    if ((K & 63) == 0) {                                              // a wave's steps lie in the depth, or past it: the first 64 then
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            const bf16_t* ws = wb + (s < whole ? k_begin + s * 64 : 0);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                a[t][s][0] = load8(ws + (wrow[t] + g * 16 + (half_tile(t) ? upper * 8 : 0)));
-                if (!half_tile(t)) a[t][s][1] = load8(ws + (wrow[t] + g * 16 + 8));
-            }
-        }
-    } else {
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            const int ko = k_begin + s * 64 + g * 16;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const int k0 = ko + (half_tile(t) ? upper * 8 : 0);
-                a[t][s][0] = load8(wb + (wrow[t] + (k0 + 8 <= K ? k0 : 0)));
-                if (!half_tile(t)) a[t][s][1] = load8(wb + (wrow[t] + (ko + 16 <= K ? ko + 8 : 0)));
-            }
-        }
-    }
-    // (the rows of x as they lie, where a lane's registers hold them beside W)
-    const bf16_t* xrow = x + (int64_t)m_own * K;                      // unused with LN, MG and ST
-    constexpr bool BESIDE = PRO == 0 && KSTEPS <= 2;
-    bf16x8 bx[BESIDE ? KSTEPS : 1][2];
-    if constexpr (BESIDE) {
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            const int ko = k_begin + s * 64 + g * 16;
-            bx[s][0] = load8(xrow + (ko + 8 <= K ? ko : 0));
-            bx[s][1] = load8(xrow + (ko + 16 <= K ? ko + 8 : 0));
-        }
-    }
     Epilogue4 ep;
     const auto ask = [&] {
         ep.ask(bias, residual, m_own, n0, N, wave < NT);
         if (scatter) ep.ask_place(n0, item, pos, ex);
     };
-    if constexpr (!MG) ask();                                         // (with the partial results there are no registers left for it)
-
-    if constexpr (ST) {
-        DividedWalk at(tid, THREADS, pieces);
+    // The rows of the input in LDS, by all waves.  What the epilogue adds is asked for before them, or, with the merge, whose partial results
+    // leave no registers for it, behind them.
+    const auto make_rows = [&](auto asks) {
+        if constexpr (!MG && decltype(asks)::value) ask();
+        if constexpr (ST) {
+            DividedWalk at(tid, THREADS, pieces);
 #pragma unroll
-        for (int i = 0; i < STV; ++i, at.next())
-            if (i * THREADS < total && tid + i * THREADS < total) *reinterpret_cast<uintx4*>(xs + at.q * xstride + at.r * 8) = sx[i];
-        __syncthreads();
-    }
-    if constexpr (MG) {
-        if (tid < groups) {
-            float mx = -INFINITY;
-#pragma unroll
-            for (int sp = 0; sp < MGS; ++sp) {
-                if (sp >= S) ls[sp] = -INFINITY;
-                mx = fmaxf(mx, ls[sp]);
-            }
-            float wsum = 0.f;
-#pragma unroll
-            for (int sp = 0; sp < MGS; ++sp) {
-                ls[sp] = ls[sp] > -INFINITY ? __expf(ls[sp] - mx) : 0.f;
-                wsum += ls[sp];
-            }
-            const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
-#pragma unroll
-            for (int sp = 0; sp < MGS; ++sp)
-                if (sp < S) sw[tid * S + sp] = ls[sp] * inv;
+            for (int i = 0; i < STV; ++i, at.next())
+                if (i * THREADS < total && tid + i * THREADS < total) *reinterpret_cast<uintx4*>(xs + at.q * xstride + at.r * 8) = sx[i];
+            __syncthreads();
         }
-        __syncthreads();
-        DividedWalk head(tid, THREADS, ex.mg_head_dim >> 2), row(tid, THREADS, nvec);
+        if constexpr (MG) {
+            if (tid < groups) {
+                float mx = -INFINITY;
 #pragma unroll
-        for (int e = 0; e < MGE; ++e, head.next(), row.next()) {
-            if (e * THREADS >= total4 || tid + e * THREADS >= total4) continue;
-            const float* wg = sw + head.q * S;
-            float y0 = 0.f, y1 = 0.f, y2 = 0.f, y3 = 0.f;
-#pragma unroll
-            for (int sp = 0; sp < MGS; ++sp) {
-                if (sp < S) {
-                    const float ww = wg[sp];
-                    y0 = fmaf(ww, mo[e][sp].x, y0); y1 = fmaf(ww, mo[e][sp].y, y1);
-                    y2 = fmaf(ww, mo[e][sp].z, y2); y3 = fmaf(ww, mo[e][sp].w, y3);
+                for (int sp = 0; sp < MGS; ++sp) {
+                    if (sp >= S) ls[sp] = -INFINITY;
+                    mx = fmaxf(mx, ls[sp]);
                 }
-            }
-            uint2 p;
-            p.x = pack_bf16x2(y0, y1);
-            p.y = pack_bf16x2(y2, y3);
-            *reinterpret_cast<uint2*>(xs + row.q * xstride + row.r * 4) = p;
-        }
-        ask();
-        __syncthreads();
-    }
-    if constexpr (LN) {
+                float wsum = 0.f;
 #pragma unroll
-        for (int i = 0; i < GV; ++i) {
-            const int c = tid + i * THREADS;
-            if (c < nvec) {
-                reinterpret_cast<float4*>(sg)[c] = ex.ln_gamma ? gv[i] : make_float4(1.f, 1.f, 1.f, 1.f);
-                reinterpret_cast<float4*>(sb)[c] = ex.ln_beta ? bv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-        }
-        float mean = 0.f, rstd = 0.f;
-        auto statistics = [&] {
-            float sum = 0.f;
-#pragma unroll
-            for (int i = 0; i < LNV; ++i) {
-                if ((i + 1) * 64 > nvec && lane + i * 64 >= nvec) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-            }
-            mean = ex.ln_no_center ? 0.f : wave_sum(sum) / (float)K;
-            float sq = 0.f;
-#pragma unroll
-            for (int i = 0; i < LNV; ++i) {
-                if (lane + i * 64 < nvec) {
-                    const float p = v[i].x - mean, q = v[i].y - mean, r = v[i].z - mean, t = v[i].w - mean;
-                    sq += (p * p + q * q) + (r * r + t * t);
+                for (int sp = 0; sp < MGS; ++sp) {
+                    ls[sp] = ls[sp] > -INFINITY ? __expf(ls[sp] - mx) : 0.f;
+                    wsum += ls[sp];
                 }
-            }
-            rstd = 1.0f / sqrtf(wave_sum(sq) / (float)K + ex.ln_eps);
-        };
-        auto write_row = [&](int m) {
+                const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
 #pragma unroll
-            for (int i = 0; i < LNV; ++i) {
-                const int c = lane + i * 64;
-                if (c >= nvec) continue;
-                const float4 gm = reinterpret_cast<const float4*>(sg)[c];
-                const float4 bt = reinterpret_cast<const float4*>(sb)[c];
-                const float y0 = (v[i].x - mean) * rstd * gm.x + bt.x, y1 = (v[i].y - mean) * rstd * gm.y + bt.y;
-                const float y2 = (v[i].z - mean) * rstd * gm.z + bt.z, y3 = (v[i].w - mean) * rstd * gm.w + bt.w;
+                for (int sp = 0; sp < MGS; ++sp)
+                    if (sp < S) sw[tid * S + sp] = ls[sp] * inv;
+            }
+            __syncthreads();
+            DividedWalk head(tid, THREADS, ex.mg_head_dim >> 2), row(tid, THREADS, nvec);
+#pragma unroll
+            for (int e = 0; e < MGE; ++e, head.next(), row.next()) {
+                if (e * THREADS >= total4 || tid + e * THREADS >= total4) continue;
+                const float* wg = sw + head.q * S;
+                float y0 = 0.f, y1 = 0.f, y2 = 0.f, y3 = 0.f;
+#pragma unroll
+                for (int sp = 0; sp < MGS; ++sp) {
+                    if (sp < S) {
+                        const float ww = wg[sp];
+                        y0 = fmaf(ww, mo[e][sp].x, y0); y1 = fmaf(ww, mo[e][sp].y, y1);
+                        y2 = fmaf(ww, mo[e][sp].z, y2); y3 = fmaf(ww, mo[e][sp].w, y3);
+                    }
+                }
                 uint2 p;
                 p.x = pack_bf16x2(y0, y1);
                 p.y = pack_bf16x2(y2, y3);
-                *reinterpret_cast<uint2*>(xs + m * xstride + c * 4) = p;
+                *reinterpret_cast<uint2*>(xs + row.q * xstride + row.r * 4) = p;
             }
-        };
-        if (wave < M) statistics();
-        __syncthreads();                             // gain and bias are in LDS
-        if (wave < M) write_row(wave);
-        for (int m = wave + WAVES; m < M; m += WAVES) {                  // rows beyond the first of a wave
-            load_row(m);
-            statistics();
-            write_row(m);
+            if constexpr (decltype(asks)::value) ask();
+            __syncthreads();
         }
-        __syncthreads();
-    }
-    // x fragments from LDS, or (without a prologue and a long slab) step by step from the cache: those queue behind the W slab and
-    // need no registers until then
-    if constexpr (PRO != 0) xrow = xs + m_own * xstride;
+        if constexpr (LN) {
+#pragma unroll
+            for (int i = 0; i < GV; ++i) {
+                const int c = tid + i * THREADS;
+                if (c < nvec) {
+                    reinterpret_cast<float4*>(sg)[c] = ex.ln_gamma ? gv[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+                    reinterpret_cast<float4*>(sb)[c] = ex.ln_beta ? bv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+                }
+            }
+            float mean = 0.f, rstd = 0.f;
+            auto statistics = [&] {
+                float sum = 0.f;
+#pragma unroll
+                for (int i = 0; i < LNV; ++i) {
+                    if ((i + 1) * 64 > nvec && lane + i * 64 >= nvec) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    sum += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+                }
+                mean = ex.ln_no_center ? 0.f : wave_sum(sum) / (float)K;
+                float sq = 0.f;
+#pragma unroll
+                for (int i = 0; i < LNV; ++i) {
+                    if (lane + i * 64 < nvec) {
+                        const float p = v[i].x - mean, q = v[i].y - mean, r = v[i].z - mean, t = v[i].w - mean;
+                        sq += (p * p + q * q) + (r * r + t * t);
+                    }
+                }
+                rstd = 1.0f / sqrtf(wave_sum(sq) / (float)K + ex.ln_eps);
+            };
+            auto write_row = [&](int m) {
+#pragma unroll
+                for (int i = 0; i < LNV; ++i) {
+                    const int c = lane + i * 64;
+                    if (c >= nvec) continue;
+                    const float4 gm = reinterpret_cast<const float4*>(sg)[c];
+                    const float4 bt = reinterpret_cast<const float4*>(sb)[c];
+                    const float y0 = (v[i].x - mean) * rstd * gm.x + bt.x, y1 = (v[i].y - mean) * rstd * gm.y + bt.y;
+                    const float y2 = (v[i].z - mean) * rstd * gm.z + bt.z, y3 = (v[i].w - mean) * rstd * gm.w + bt.w;
+                    uint2 p;
+                    p.x = pack_bf16x2(y0, y1);
+                    p.y = pack_bf16x2(y2, y3);
+                    *reinterpret_cast<uint2*>(xs + m * xstride + c * 4) = p;
+                }
+            };
+            if (wave < M) statistics();
+            __syncthreads();                             // gain and bias are in LDS
+            if (wave < M) write_row(wave);
+            for (int m = wave + WAVES; m < M; m += WAVES) {                  // rows beyond the first of a wave
+                load_row(m);
+                statistics();
+                write_row(m);
+            }
+            __syncthreads();
+        }
+    };
     floatx4 acc[NT], other = floatx4{0.f, 0.f, 0.f, 0.f};             // (other: the half tile's products with the second half of x)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](int s, const bf16x8& b0, const bf16x8& b1) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][0], b0, acc[t], 0, 0, 0);
-            if (half_tile(t)) other = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][0], b1, other, 0, 0, 0);
-            else acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][1], b1, acc[t], 0, 0, 0);
-        }
-    };
-    if (whole == KSTEPS) {
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            if constexpr (BESIDE) multiply(s, bx[s][0], bx[s][1]);
-            else multiply(s, load8(xrow + k_begin + s * 64 + g * 16), load8(xrow + k_begin + s * 64 + g * 16 + 8));
-        }
+    if (k_begin >= K) {
+        make_rows(std::bool_constant<(NT > 1)>());                      // (the first wave is never one of these)
     } else {
+        bf16x8 a[NT][KSTEPS][2];
+        const bf16_t* wb = w + (int64_t)n_base * K;
+        uint32_t wrow[NT];                                                // first element of the lane's row of W, from wb on
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
-            if (s > whole || (s == whole && rest == 0)) continue;
-            const int ko = k_begin + s * 64 + g * 16;
-            const bool in0 = ko + 8 <= K, in1 = ko + 16 <= K;
-            bf16x8 b0, b1;
-            if constexpr (BESIDE) { b0 = bx[s][0]; b1 = bx[s][1]; }
-            else { b0 = load8(xrow + (in0 ? ko : 0)); b1 = load8(xrow + (in1 ? ko + 8 : 0)); }
-            if (s == whole) {                        // past the depth: zeros on both sides
-                if (!in0) b0 = zero8();
-                if (!in1) b1 = zero8();
+        for (int t = 0; t < NT; ++t)                                      // (rows past the matrix stand for its last: their results are not stored)
+            wrow[t] = (uint32_t)min(16 * t + (half_tile(t) ? r16 & 7 : r16), N - 1 - n_base) * (uint32_t)K;
+        if ((K & 63) == 0) {                                              // a wave's steps lie in the depth, or past it: the first 64 then
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                const bf16_t* ws = wb + (s < whole ? k_begin + s * 64 : 0);
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    if (half_tile(t) && upper ? !in1 : !in0) a[t][s][0] = zero8();
-                    if (!half_tile(t) && !in1) a[t][s][1] = zero8();
+                    a[t][s][0] = load8(ws + (wrow[t] + g * 16 + (half_tile(t) ? upper * 8 : 0)));
+                    if (!half_tile(t)) a[t][s][1] = load8(ws + (wrow[t] + g * 16 + 8));
                 }
             }
-            multiply(s, b0, b1);
+        } else {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                const int ko = k_begin + s * 64 + g * 16;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const int k0 = ko + (half_tile(t) ? upper * 8 : 0);
+                    a[t][s][0] = load8(wb + (wrow[t] + (k0 + 8 <= K ? k0 : 0)));
+                    if (!half_tile(t)) a[t][s][1] = load8(wb + (wrow[t] + (ko + 16 <= K ? ko + 8 : 0)));
+                }
+            }
+        }
+        // (the rows of x as they lie, where a lane's registers hold them beside W)
+        const bf16_t* xrow = x + (int64_t)m_own * K;                      // unused with LN, MG and ST
+        constexpr bool BESIDE = PRO == 0 && KSTEPS == 1;
+        bf16x8 bx[BESIDE ? KSTEPS : 1][2];
+        if constexpr (BESIDE) {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                const int ko = k_begin + s * 64 + g * 16;
+                bx[s][0] = load8(xrow + (ko + 8 <= K ? ko : 0));
+                bx[s][1] = load8(xrow + (ko + 16 <= K ? ko + 8 : 0));
+            }
+        }
+        make_rows(std::true_type());
+        // x fragments from LDS, or (without a prologue and a long slab) step by step from the cache: those queue behind the W slab and
+        // need no registers until then
+        if constexpr (PRO != 0) xrow = xs + m_own * xstride;
+        auto multiply = [&](int s, const bf16x8& b0, const bf16x8& b1) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][0], b0, acc[t], 0, 0, 0);
+                if (half_tile(t)) other = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][0], b1, other, 0, 0, 0);
+                else acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t][s][1], b1, acc[t], 0, 0, 0);
+            }
+        };
+        if (whole == KSTEPS) {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                if constexpr (BESIDE) multiply(s, bx[s][0], bx[s][1]);
+                else multiply(s, load8(xrow + k_begin + s * 64 + g * 16), load8(xrow + k_begin + s * 64 + g * 16 + 8));
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                if (s > whole || (s == whole && rest == 0)) continue;
+                const int ko = k_begin + s * 64 + g * 16;
+                const bool in0 = ko + 8 <= K, in1 = ko + 16 <= K;
+                bf16x8 b0, b1;
+                if constexpr (BESIDE) { b0 = bx[s][0]; b1 = bx[s][1]; }
+                else { b0 = load8(xrow + (in0 ? ko : 0)); b1 = load8(xrow + (in1 ? ko + 8 : 0)); }
+                if (s == whole) {                        // past the depth: zeros on both sides
+                    if (!in0) b0 = zero8();
+                    if (!in1) b1 = zero8();
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        if (half_tile(t) && upper ? !in1 : !in0) a[t][s][0] = zero8();
+                        if (!half_tile(t) && !in1) a[t][s][1] = zero8();
+                    }
+                }
+                multiply(s, b0, b1);
+            }
         }
     }
     // the waves' partial tiles meet in LDS (a slot per wave and tile); one barrier, then wave t sums tile t
@@ -848,10 +867,15 @@ static int launch_resident_k(void* out, const bf16_t* x, const bf16_t* w, const 
 #define ST_RES(KS)                                                                                                 \
     (out_f32 ? launch_resident_rows<WAVES, KS, true, PRO>(out, x, w, bias, residual, M, N, K, act, ex, stream, wide_rows, narrow) \
              : launch_resident_rows<WAVES, KS, false, PRO>(out, x, w, bias, residual, M, N, K, act, ex, stream, wide_rows, narrow))
-    if (ksteps <= 1) return ST_RES(1);
-    if (ksteps <= 2) return ST_RES(2);
-    if constexpr (kMax >= 4) {
-        if (ksteps <= 4) return ST_RES(4);
+    // (rows as they lie are 1,024 deep at most, or so many and deep that LDS does not hold them; staged ones are deeper than 1,024)
+    if constexpr (PRO != 3) {
+        if (ksteps <= 1) return ST_RES(1);
+    }
+    if constexpr (PRO != 0) {
+        if (ksteps <= 2) return ST_RES(2);
+        if constexpr (kMax >= 4) {
+            if (ksteps <= 4) return ST_RES(4);
+        }
     }
     if constexpr (kMax >= 8) return ST_RES(8);
     return -1;
