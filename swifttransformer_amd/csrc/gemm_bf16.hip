@@ -283,7 +283,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
 // Waves whose steps all lie past the depth ask for no weights: these go a way of their own through the prologue, so that on the others' way the
 // number of loads that are on their way is known.  us a call, cold weights, with all waves asking (for the first step again) and so: 16 rows
 // 256 to 5,120 5.4 and 3.2, 8 rows 512 to 5,120 5.1 and 4.0, 640 to 5,120 5.7 and 4.5, 2,560 to 2,560 8.4 and 6.8; one row 2,560 to 5,120
-// 11.7 and 9.8, 5,120 to 8,192 23.1 and 20.0.
+// 11.7 and 9.8, 5,120 to 8,192 23.1 and 20.0; with the norm, 8 rows 2,560 to 8,192 19.3 and 16.8 (its rows of up to 3,072 in 48 registers).
 constexpr int kLnMaxVec = 16;            // float4 per lane of a row held in registers (K <= 4096)
 constexpr int kMgElems = 2;              // merge prologue: float4 elements of the input per thread
 constexpr int kMgSplits = 8;             // and splits per element, all held in registers;
@@ -357,6 +357,7 @@ __global__ __launch_bounds__(WAVES * 64, resident_waves(WAVES, KSTEPS, PRO, ROWS
                      *shift = reinterpret_cast<const float4*>(ex.ln_beta ? ex.ln_beta : ex.ln_x);
 #pragma unroll
         for (int i = 0; i < GV; ++i) {
+            if (i > 0 && i * THREADS >= nvec) continue;
             const int c = min(tid + i * THREADS, nvec - 1);
             gv[i] = gain[c];
             bv[i] = shift[c];
@@ -879,6 +880,9 @@ static int launch_resident_k(void* out, const bf16_t* x, const bf16_t* w, const 
         if constexpr (kMax >= 4) {
             if (ksteps <= 4) return ST_RES(4);
         }
+    }
+    if constexpr (PRO == 1 && kMax >= 8) {
+        if (ksteps <= 6) return ST_RES(6);          // (rows of up to 3,072: 48 registers for the one being normalised, not 64)
     }
     if constexpr (kMax >= 8) return ST_RES(8);
     return -1;
