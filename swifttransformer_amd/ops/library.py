@@ -40,12 +40,17 @@ FILE_FLAGS = {"attention_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "attention_prefill_dma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "attention_prefill_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "latent_attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
-# Loads stay where the sources ask for them.  The sources clamp a load's address and clear afterwards what should not be there, so that a
-# batch of loads is on its way together; the optimiser, left to itself, moves a load to the one place that uses it, behind the lane's
-# condition, and each then waits for its own trip to memory (single tokens of the gated linear attention, 80 x 80 states: 29.8 us a call,
-# 9.8 so; outputs of the delta rule's chunks 113 -> 95 us).  The kernels of LOADS_MOVE have no such loads and fewer registers without it.
+# Files whose loads stay where the sources ask for them.  Many kernels clamp a load's address and clear afterwards what should not be there, so
+# that a batch of loads is on its way together; the optimiser may move such a load to the one place that uses it, behind the lane's condition,
+# where each waits for its own trip to memory.  Left in place they hold registers longer, so a file is here only where both ways were timed
+# and this one is faster: steps of all families at the layer sizes of 125m to 6.7b, both builds in turn, time with the flag over time without.
+# delta: outputs of chunks 0.90, carry 0.98.  gla_chunks: the walk 0.41, outputs 0.99.  group_norm: with the filter 0.95.  latent: cache
+# entries 0.98.  moe: float tiles 0.60 to 0.92 (its bfloat16 tiles 1.007, one and two float tokens 1.013).  sink_attention: 0.97 at
+# 32 heads of 128, 1.00 elsewhere.  Not here: state_chunks, whose outputs take 1.01 with it at 64 channels and whole calls 1.06 to 1.15 at 80 to
+# 128 (2,011 tokens, 32 heads of 128: 203 us, 179 without; a workgroup a unit less), attention_prefill_dma 1.005, hyper_streams 1.03 (the start
+# of the streams), and the others, where both are within 0.5 %.
 LOADS_STAY = ["-mllvm", "-instcombine-code-sinking=0"]
-LOADS_MOVE = {"gemm_bf16.hip", "attention_prefill.hip"}
+LOADS_STAY_IN = {"delta.hip", "gla_chunks.hip", "group_norm.hip", "latent.hip", "moe.hip", "sink_attention.hip"}
 # the vendor's matrix-product library backs the large bfloat16 products (csrc/gemm_library.hip)
 LINK_LIBS = ["-lhipblaslt"]
 
@@ -59,7 +64,7 @@ class KernelLibraryError(RuntimeError):
 
 def flags_of(source: str) -> List[str]:
     """What a file is compiled with beside ``HIPCC_FLAGS``."""
-    return FILE_FLAGS.get(source, []) + ([] if source in LOADS_MOVE else LOADS_STAY)
+    return FILE_FLAGS.get(source, []) + (LOADS_STAY if source in LOADS_STAY_IN else [])
 
 
 def sources() -> List[str]:
