@@ -10,8 +10,9 @@ namespace st {
 
 // A workgroup a row; NP pieces of V neighbouring columns a thread stay in registers between the sums.  Both norms' gains are asked for at the
 // start: a few rows are bound by trips to memory one after the other, and a load behind the stores of x' waits for those too (24 rows of 4,096 with both norms 3.75 -> 3.15 us, 968 9.9 -> 9.5,
-// 2,048 18.5 -> 18.1).
-template <typename T, int V, int NP>
+// 2,048 18.5 -> 18.1).  THEN: there is a second norm; without one its gains' place in the registers and in the queue is not taken either (2,048
+// rows of 5,120, cold: 31.8 us with the first gains asked for twice, 29.0 so).
+template <typename T, int V, int NP, bool THEN>
 __global__ __launch_bounds__(256) void rms_onto_kernel(
     float* __restrict__ out32, T* __restrict__ out_t, const float* __restrict__ y, const float* __restrict__ x,
     const float* __restrict__ gain, const float* __restrict__ gain2, int width, float eps, float eps2) {
@@ -46,7 +47,7 @@ __global__ __launch_bounds__(256) void rms_onto_kernel(
     load(y + row, a);
     load(x + row, b);
     load(gain, w);
-    load(gain2 ? gain2 : gain, w2);
+    if constexpr (THEN) load(gain2, w2);
     const float r = 1.f / sqrtf(mean_square(a) + eps);
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(256) void rms_onto_kernel(
             else out32[row + c] = b[i][0];
         }
     }
-    if (!gain2) return;
+    if constexpr (!THEN) return;
     const float r2 = 1.f / sqrtf(mean_square(b) + eps2);
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
@@ -107,7 +108,9 @@ extern "C" int st_rms_onto(float* out32, void* out_t, const float* y, const floa
     ST_CHECK(out32 && y && x && gain && (!gain2 || out_t), "rms_onto: null operand");
     const bool vec = width % 4 == 0 && (((uintptr_t)out32 | (uintptr_t)out_t | (uintptr_t)y | (uintptr_t)x | (uintptr_t)gain |
                                          (uintptr_t)gain2) & 15) == 0;
-#define ST_RO(T, V, NP) rms_onto_kernel<T, V, NP><<<num_rows, 256, 0, stream>>>(out32, (T*)out_t, y, x, gain, gain2, width, eps, eps2)
+#define ST_RO(T, V, NP)                                                                                                 \
+    (gain2 ? rms_onto_kernel<T, V, NP, true><<<num_rows, 256, 0, stream>>>(out32, (T*)out_t, y, x, gain, gain2, width, eps, eps2) \
+           : rms_onto_kernel<float, V, NP, false><<<num_rows, 256, 0, stream>>>(out32, nullptr, y, x, gain, nullptr, width, eps, eps2))
 #define ST_RO_T(T)                                                                                                     \
     do {                                                                                                               \
         if (vec && width <= 1024) ST_RO(T, 4, 1);                                                                      \

@@ -52,7 +52,9 @@ def test_no_private_memory(tmp_path):
     ("state_out_kernelILi32ELi4E", 2, 256), ("state_out_kernelILi32ELi8ELb1E", 1, 256),
     # eight: two workgroups of sixteen waves a unit
     ("gemm_skinny_resident_kernelILi16ELi1ELb0ELi0E", 2, 64), ("gemm_skinny_resident_kernelILi16ELi1ELb1ELi0E", 2, 64),
-    ("gemm_skinny_resident_kernelILi16ELi2ELb0ELi3ELi8E", 1, 64), ("gemm_skinny_resident_kernelILi16ELi2ELb1ELi3ELi8E", 1, 64)])
+    ("gemm_skinny_resident_kernelILi16ELi2ELb0ELi3ELi8E", 1, 64), ("gemm_skinny_resident_kernelILi16ELi2ELb1ELi3ELi8E", 1, 64),
+    # four: no second norm's gains
+    ("rms_onto_kernelIfLi4ELi8ELb0E", 1, 128)])
 def test_registers_leave_room_for_another_workgroup(tmp_path, kernel, instances, most):
     counts = noted(library.find_built() or library.build(), tmp_path, "vgpr_count")
     of = {n: v for n, v in counts.items() if kernel in n}
