@@ -99,7 +99,8 @@ __device__ inline void dot_rows(const float* __restrict__ qs, int q_stride, cons
 // where the value size is a multiple of that)
 template <typename T, int NG, int W>
 __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnArgs a) {
-    constexpr int VB = NG == 1 && sizeof(T) == 2 ? 8 : 4;      // keys whose values a thread asks for at once
+    constexpr bool EARLY = NG == 1 && sizeof(T) == 2;
+    constexpr int VB = EARLY ? 8 : 4;      // keys whose values a thread asks for at once
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int H = a.heads, G = a.kv_heads, dk = a.key_dim, dv = a.value_dim, per = a.heads / a.kv_heads;
     float* qs = lds;                               // [H * dk]
@@ -185,8 +186,9 @@ __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnArgs a) {
             if (b + 1 < b1) page = bt[own_key(b + 1) / a.page_size];
         }
         __syncthreads();
-        // The values' first keys are asked for before the scores are formed and the others VB at a time, where a thread has one group of
-        // columns (with more the registers that this takes would cost workgroups).
+        // EARLY: the values' first keys are asked for before the scores are formed and the others VB at a time, where a thread has one group of
+        // columns of bfloat16.  (With more groups the registers that this takes would cost workgroups.  In float, four keys at a time, it is
+        // 30 registers for nothing: 12 heads of 64, 2,300 rows 455 us with it, 426 without, eight rows 183 and 170.)
         uint4 vraw[VB][NG];
         const auto ask = [&](int j) {
 #pragma unroll
@@ -194,7 +196,7 @@ __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnArgs a) {
 #pragma unroll
                 for (int i = 0; i < NG; ++i) vraw[u][i] = *reinterpret_cast<const uint4*>(vc + ov[i] + voff[j + u]);
         };
-        if constexpr (W > 1 && NG == 1) ask(0);
+        if constexpr (W > 1 && EARLY) ask(0);
         // a thread a (key head, key): the key row is loaded once for the heads that share it
         for (int p = tid; p < G * kKeyBlock; p += 256) {
             const int c = p >> 6, jj = p & 63;
@@ -202,10 +204,10 @@ __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnArgs a) {
             for (int g0 = c * per; g0 < (c + 1) * per; g0 += 4) {
                 const int n = min(4, (c + 1) * per - g0);
                 float acc[4] = {0.f, 0.f, 0.f, 0.f};
-                if (n == 4) dot_rows<T, 4, NG == 1 && sizeof(T) == 2>(qs + g0 * dk, dk, kp, dk, acc);
-                else if (n == 3) dot_rows<T, 3, NG == 1 && sizeof(T) == 2>(qs + g0 * dk, dk, kp, dk, acc);
-                else if (n == 2) dot_rows<T, 2, NG == 1 && sizeof(T) == 2>(qs + g0 * dk, dk, kp, dk, acc);
-                else dot_rows<T, 1, NG == 1 && sizeof(T) == 2>(qs + g0 * dk, dk, kp, dk, acc);
+                if (n == 4) dot_rows<T, 4, EARLY>(qs + g0 * dk, dk, kp, dk, acc);
+                else if (n == 3) dot_rows<T, 3, EARLY>(qs + g0 * dk, dk, kp, dk, acc);
+                else if (n == 2) dot_rows<T, 2, EARLY>(qs + g0 * dk, dk, kp, dk, acc);
+                else dot_rows<T, 1, EARLY>(qs + g0 * dk, dk, kp, dk, acc);
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
                     if (u < n) sraw[(g0 + u) * kKeyBlock + jj] = acc[u];
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnArgs a) {
         if constexpr (W > 1) {
 #pragma unroll 1
             for (int jj = 0; jj < kKeyBlock; jj += VB) {
-                if constexpr (NG > 1) ask(jj);
+                if constexpr (!EARLY) ask(jj);
 #pragma unroll
                 for (int u = 0; u < VB; u += 4)
 #pragma unroll
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(256) void sink_attention_kernel(SinkAttnArgs a) {
                         for (int w = 0; w < W; ++w)
                             o[i][w] = fmaf(p3, x3[w], fmaf(p2, x2[w], fmaf(p1, x1[w], fmaf(p0, x0[w], o[i][w]))));
                     }
-                if (NG == 1 && jj + VB < kKeyBlock) ask(jj + VB);
+                if (EARLY && jj + VB < kKeyBlock) ask(jj + VB);
             }
         } else {
 #pragma unroll 1

@@ -54,7 +54,9 @@ def test_no_private_memory(tmp_path):
     ("gemm_skinny_resident_kernelILi16ELi1ELb0ELi0E", 2, 64), ("gemm_skinny_resident_kernelILi16ELi1ELb1ELi0E", 2, 64),
     ("gemm_skinny_resident_kernelILi16ELi2ELb0ELi3ELi8E", 1, 64), ("gemm_skinny_resident_kernelILi16ELi2ELb1ELi3ELi8E", 1, 64),
     # four: no second norm's gains
-    ("rms_onto_kernelIfLi4ELi8ELb0E", 1, 128)])
+    ("rms_onto_kernelIfLi4ELi8ELb0E", 1, 128),
+    # three, with some to spare: no values held beside the scores in float
+    ("sink_attention_kernelIfLi1ELi4E", 1, 144)])
 def test_registers_leave_room_for_another_workgroup(tmp_path, kernel, instances, most):
     counts = noted(library.find_built() or library.build(), tmp_path, "vgpr_count")
     of = {n: v for n, v in counts.items() if kernel in n}
