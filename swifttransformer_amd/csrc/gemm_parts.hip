@@ -207,25 +207,34 @@ bool gemm_parts_can(int M, int N, int K) {
     return M >= 1 && M <= 64 * kMaxRowBlocks * 4 && K % kStep == 0 && K >= 2 * kStep && N % 4 == 0 && deal(M, N, K).splits > 1;
 }
 
-// Whether a product of 65 to 768 rows goes here: up to 512 where it takes 5 % less than the library's best of 32, whose time (to a standard deviation of
-// 10 % of 180 measured, 16 to 512 rows of 768 x 3,072 to 16,384 x 4,096) is that of the weights' stream, of the products on rows in tiles of 16, of the
-// depth that few tiles walk one after the other, and of rows times depth and features.  Cold weights, library and here, us:
-// taken: 100 x 2,048 x 8,192 19.2, 15.8; 150 25.4, 18.5; 256 26.7, 23.6; 512 37.5, 32.4; 150 x 4,096 x 4,096 21.2, 19.0; 100 x 4,096 x 16,384
-// 49.2, 33.3; 150 68.2, 39.5; 512 97.5, 88.3; 100 x 2,560 x 10,240 34.3, 20.2; 512 52.9, 47.3; 100 x 16,384 x 4,096 40.2, 33.6
-// left: 64 rows and fewer, for which the library has tiles of their size (64 x 2,048 x 8,192 16.2, 13.0 alone, but 15.7, 16.4 in a step of 64
-// requests); 150 x 2,048 x 2,048 11.9, 13.0; 150 x 6,144 x 2,048 15.0, 17.7; 150 x 8,192 x 2,048 15.6, 18.8; 256 x 4,096 x 4,096 22.4, 24.2;
-// 100 x 768 x 3,072 6.9, 9.7; 100 x 2,560 x 2,560 11.8, 13.8
-// With more rows the library fills the chip where the depth is 5,120 or less (576 x 1,024 x 4,096 18.3, 21.9; 5,120 x 5,120 46.6, 48.1).  Deeper ones:
-// up to 576 rows, three tiles of 192, its time is as estimated or more (520 x 2,048 x 8,192 44.6, 33.8; 576 x 3,072 x 12,288 77.8, 66.3;
-// 575 x 4,096 x 16,384 131.8, 120.8; 576 x 5,120 x 13,824 108.3, 105.9); up to 768, in tiles of 256, the line is lower (taken: 640 x 2,048 x 16,384
-// 84.0, 62.8; 700 x 768 x 8,192 34.8, 24.4; 768 x 2,560 x 10,240 67.6, 63.3; left: 640 x 4,096 x 8,192 64.2, 71.9; 768 x 5,120 x 13,824 124.6, 138.2;
-// 768 x 2,048 x 5,504 32.9, 35.8).  Past that it is the library's (900 x 2,048 x 8,192 47.2, 49.0).
+// Whether a product of 65 to 768 rows goes here: where what it takes is less than a part of the estimate for the library's best of 32, that of the
+// weights' stream, of the products on rows in tiles of 16, of the depth that few tiles walk one after the other, and of rows times depth
+// and features.  Both estimates are some tenths low, and by what depends on the sizes, so the part does too; it was set by 812 products timed
+// beside the library's, 66 to 768 rows of 256 x 16,384 to 8,192 x 8,192 (cold weights; library and here, us).  394 go here, in 0.73 of the library's time; five of them
+// in more, 256 x 256 x 16,384 in 1.14, the others in up to 1.05.
+// Tiles of up to 192 rows: 0.95 up to 512 rows (100 x 2,048 x 8,192 19.2, 15.8; 150 25.4, 18.5; 150 x 4,096 x 4,096 21.2, 19.0; 100 x 4,096 x 16,384
+// 49.2, 33.3; 150 x 2,560 x 10,240 32.8, 23.3; 100 x 16,384 x 4,096 40.2, 33.6; left: 150 x 2,048 x 2,048 11.9, 13.0; 150 x 6,144 x 2,048 15.0, 17.7;
+// 100 x 768 x 3,072 6.9, 9.7) and all of it up to 576, where the library's time is a tenth above the estimate (of 105 products 0.78 of its time, at
+// worst 1.04: 520 x 2,048 x 8,192 44.6, 33.8; 575 x 4,096 x 16,384 130.6, 117.0; 576 x 5,120 x 13,824 119.8, 119.4; 530 x 3,072 x 5,632 36.5, 37.9).
+// Tiles of 256 rows take longer than estimated where there are two or three to a column: 0.84 (taken: 512 x 2,048 x 8,192 38.0, 33.7; 512 x 4,096 x 16,384
+// 110.3, 90.2; left: 512 x 7,168 x 7,168 75.3, 86.7; 512 x 8,192 x 8,192 87.8, 103.4; 512 x 5,120 x 5,120 50.7, 53.6) and 0.82 (taken: 640 x 2,048 x
+// 16,384 84.0, 62.8; left: 704 x 4,096 x 8,192 69.1, 84.6; 768 x 5,120 x 13,824 124.6, 138.2).
+// Of narrow results the library deals out the depth too, which its estimate does not know: 0.82 below 1,024 features (taken: 192 x 768 x 12,288 28.5,
+// 18.3; 704 x 768 x 8,192 34.9, 24.8; left: 150 x 768 x 8,192 14.6, 17.3; 192 x 640 x 8,192 14.7, 17.3), 0.7 up to 512 (taken: 320 x 512 x 12,288 28.1,
+// 20.2; left: 256 x 512 x 8,192 13.1, 18.1; 480 17.4, 19.3).
+// Left by their sizes: 64 rows and fewer, for which the library has tiles of their size (64 x 2,048 x 8,192 16.2, 13.0 alone, but 15.7, 16.4 in a step
+// of 64 requests); more than 768 (900 x 2,048 x 8,192 47.2, 49.0); and more than 512 of a depth below 5,504, the least that was timed when that line was
+// drawn (575 x 5,120 x 5,120 51.9, 55.4; 576 x 1,024 x 4,096 18.3, 21.9; but 560 x 2,048 x 5,120 31.7, 26.6; 575 x 2,560 x 5,312 40.0, 30.6).
 bool gemm_parts_pays(int M, int N, int K) {
     if (M <= 64 || M > 768 || (M > 512 && K < 5504) || !gemm_parts_can(M, N, K)) return false;
+    const Deal d = deal(M, N, K);
     const double rows = (M + 15) / 16 * 16;
     const double library = 3.3 + 0.78 * N * K * 2e-6 / 5 + 0.69 * 2e-9 * rows * N * K / 1.2 + 0.00058 * K + 0.305e-5 * rows * K +
                            0.31e-5 * (rows * N < 1e6 ? rows * N : 1e6);
-    return deal(M, N, K).us < (M <= 512 ? 0.95 : M <= 576 ? 1.0 : 0.82) * library;
+    double part = d.nj < kMaxRowBlocks ? (M <= 512 ? 0.95 : 1.0) : M <= 256 ? 0.95 : M <= 512 ? 0.84 : 0.82;
+    if (N < 1024 && part > 0.82) part = 0.82;
+    if (N <= 512 && part > 0.7) part = 0.7;
+    return d.us < part * library;
 }
 
 // Floats of scratch that it takes.
