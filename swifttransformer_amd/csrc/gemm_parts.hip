@@ -3,7 +3,7 @@
 //
 // What bounds such a product is the way of its operands into a compute unit's LDS, some 40 bytes a nanosecond: a narrow result (the
 // hidden size) has fewer tiles than the chip has units, and a unit that walks the whole depth of its tile alone takes four times as long as the
-// weights' stream does.  So: tiles of 128 features by all rows (up to 256; a tile of 64, 128, 192 or 256 rows) and as many parts of
+// weights' stream does.  So: tiles of 128 features by all rows (up to 256; a tile of 128, 192 or 256 rows) and as many parts of
 // the depth as make a workgroup a unit.  A tile's operands go from memory into LDS directly (16 bytes a lane, rows' chunks rotated
 // for the matrix instruction's reads), two steps of 64 in depth ahead of the one that is multiplied; four waves, each with 64 features and
 // every other block of 32 rows (v_mfma_f32_32x32x16_bf16).  The parts of a depth are dealt to the dies in their order, so that an eighth of x
@@ -40,7 +40,7 @@ template <int N> using Number = std::integral_constant<int, N>;
 
 // NJ: blocks of 64 rows of a tile.  part [splits][tiles][2 NJ 4 of 4 waves][64 lanes][4]; grid: items rounded up to eights.
 template <int NJ>
-__global__ __launch_bounds__(256, NJ == 1 ? 2 : 1) void gemm_parts_kernel(
+__global__ __launch_bounds__(256, 1) void gemm_parts_kernel(
     float* __restrict__ part, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, int M, int N, int K, int tiles_n, int tiles, int splits) {
     constexpr int ROWS = 64 * NJ, BUF = (kFeatures + ROWS) * 8;                         // 16-byte pieces of a buffer: features, then rows
     constexpr int NW = kFeatures / 32, NL = NW + ROWS / 32;                             // direct loads a wave and step, eight rows each
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256, NJ == 1 ? 2 : 1) void gemm_parts_kernel(
     };
     // (a tile has more than 64 (NJ - 1) rows, but where several make up the rows the last may have fewer: it multiplies what it need not)
     if (m0 + (2 * (NJ - 1) + wm) * 32 < M) walk(Number<NJ>());
-    else walk(Number<(NJ > 1 ? NJ - 1 : 1)>());
+    else walk(Number<NJ - 1>());
     float* dst = part + ((int64_t)split * tiles + tile) * (kFeatures * ROWS) + wave * (32 * NJ * 64) + lane * 4;
 #pragma unroll
     for (int q = 0; q < 2; ++q)
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256) void gemm_parts_sum_kernel(
     }
 }
 
-// How a product is dealt out: tiles of 64 nj rows, the depth in `splits` parts, no more workgroups than compute units (a second one on some
+// How a product is dealt out: tiles of 64 nj rows (nj of 2 to 4), the depth in `splits` parts, no more workgroups than compute units (a second one on some
 // takes as long as on all), and what that takes (us, to some 10 % of 700 measured): launches, beginnings and ends, the steps of a
 // workgroup or the weights' stream, the partial sums there and back.
 struct Deal { int nj, tiles_n, tiles, splits; double us; };
@@ -188,7 +188,7 @@ struct Deal { int nj, tiles_n, tiles, splits; double us; };
 Deal deal(int M, int N, int K) {
     Deal d{};
     const int units = device_compute_units(), blocks = (M + 63) / 64, tiles_m = (blocks + kMaxRowBlocks - 1) / kMaxRowBlocks, all = K / kStep;
-    d.nj = (blocks + tiles_m - 1) / tiles_m;
+    d.nj = blocks == 1 ? 2 : (blocks + tiles_m - 1) / tiles_m;       // (64 rows and fewer come by demand alone: half of a tile of 128)
     d.tiles_n = (N + kFeatures - 1) / kFeatures;
     d.tiles = d.tiles_n * ((M + 64 * d.nj - 1) / (64 * d.nj));
     const double step = (kFeatures + 64 * d.nj) * 128 / 56e3, stream = (double)N * K * 2 / 5.2e6, sums = (double)d.tiles * 64 * d.nj * kFeatures * 8 / 7e6;
@@ -251,7 +251,6 @@ int gemm_parts(void* out, const bf16_t* x, const bf16_t* w, const float* bias, c
     const unsigned grid = (unsigned)((d.tiles * d.splits + 7) / 8 * 8);
 #define ST_PARTS(NJ) gemm_parts_kernel<NJ><<<grid, 256, 0, stream>>>(ex.scratch, x, w, M, N, K, d.tiles_n, d.tiles, d.splits)
     switch (d.nj) {
-        case 1: ST_PARTS(1); break;
         case 2: ST_PARTS(2); break;
         case 3: ST_PARTS(3); break;
         default: ST_PARTS(4); break;
