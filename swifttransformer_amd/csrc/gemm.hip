@@ -311,8 +311,10 @@ extern "C" int st_gemm_path_counts(uint64_t* out, int reset) {
     return kNumGemmPaths;
 }
 
-// Calls of st_gemm that gemm_f32_split took since the last reset.
+// Calls of st_gemm that gemm_parts took since the last reset.
 extern "C" uint64_t st_gemm_parts_count(int reset) { return reset ? g_parts_count.exchange(0) : g_parts_count.load(); }
+
+// Calls of st_gemm that gemm_f32_split took since the last reset.
 extern "C" uint64_t st_gemm_split_count(int reset) { return reset ? g_split_count.exchange(0) : g_split_count.load(); }
 
 // Whether st_gemm (algo 0) can take a split attention output (partials and log-sum-exps) as its input.

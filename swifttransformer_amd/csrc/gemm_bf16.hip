@@ -324,7 +324,7 @@ __global__ __launch_bounds__(WAVES * 64, resident_waves(WAVES, KSTEPS, PRO, ROWS
     bf16_t* xs = nullptr;                                                  // [M][K + 8] input rows made here (LN, MG, ST)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r16 = lane & 15;
-    // ROWS output features per workgroup.  8: half of each MFMA's rows stay empty, but a narrow
+    // ROWS output features per workgroup.  8: the two halves of each MFMA's rows hold the two halves of a step of the same features (below); a narrow
     // matrix (N = hidden) then spreads over twice as many compute units.  24 and 32 (two tiles):
     // a wide matrix then makes one workgroup a compute unit instead of one and a half or two,
     // and its prologue (the norm of all rows) is done half as often; with 16 waves the slabs of

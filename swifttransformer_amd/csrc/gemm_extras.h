@@ -16,7 +16,9 @@
 //  * K/V scatter epilogue: output features [q_size, q_size + 2*kv_size) of a fused QKV
 //    product are the new tokens' keys and values; besides the normal store they go
 //    straight into their cache pages (the reference does this with a separate kernel,
-//    src/csrc/kernel/kvcache_mgmt.cu:34-80).  Every product kernel offers it.
+//    src/csrc/kernel/kvcache_mgmt.cu:34-80).  The kernels of gemm.hip, gemm_bf16.hip and gemm_f32.hip offer it; behind a product
+//    of the library a copy does the same, and the products by parts of their depth (gemm_parts.hip) leave such ones to it.
+//  * Scratch: room for the partial sums of products whose depth is dealt out (gemm_f32.hip, gemm_parts.hip).
 #pragma once
 #include <stdint.h>
 
@@ -57,12 +59,13 @@ extern "C" struct StGemmExtras {
     float* best_val;
     int* best_idx;
     // scaled result: what the product, bias and activation gave is multiplied by out_scale before
-    // the residual is added (0 means 1).  The kernels of gemm.hip and gemm_bf16.hip and the library
+    // the residual is added (0 means 1).  The kernels of gemm.hip, gemm_bf16.hip, gemm_f32.hip and gemm_parts.hip and the library
     // (as its alpha, for products without activation, and without bias or with bias_unscaled) offer it.
     float out_scale;
     // != 0: the bias is added after the factor, out = residual + out_scale * x W^T + bias (no activation)
     int bias_unscaled;
-    // float products: room for partial sums (st_gemm_scratch floats make the best split of them), or null
+    // room for partial sums, or null: st_gemm_scratch floats make the best split of a float product, and without them no bfloat16 product goes by
+    // parts of its depth
     float* scratch;
     int64_t scratch_floats;
 };
