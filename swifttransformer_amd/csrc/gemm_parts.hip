@@ -215,7 +215,7 @@ bool gemm_parts_can(int M, int N, int K) {
 // Tiles of up to 192 rows: 0.95 up to 512 rows (100 x 2,048 x 8,192 19.2, 15.8; 150 25.4, 18.5; 150 x 4,096 x 4,096 21.2, 19.0; 100 x 4,096 x 16,384
 // 49.2, 33.3; 150 x 2,560 x 10,240 32.8, 23.3; 100 x 16,384 x 4,096 40.2, 33.6; left: 150 x 2,048 x 2,048 11.9, 13.0; 150 x 6,144 x 2,048 15.0, 17.7;
 // 100 x 768 x 3,072 6.9, 9.7) and all of it up to 576, where the library's time is a tenth above the estimate (of 105 products 0.78 of its time, at
-// worst 1.04: 520 x 2,048 x 8,192 44.6, 33.8; 575 x 4,096 x 16,384 130.6, 117.0; 576 x 5,120 x 13,824 119.8, 119.4; 530 x 3,072 x 5,632 36.5, 37.9).
+// worst 1.04: 520 x 2,048 x 8,192 44.6, 33.8; 575 x 4,096 x 16,384 130.6, 117.0, of which a step of 575 rows keeps 4; 576 x 5,120 x 13,824 119.8, 119.4; 530 x 3,072 x 5,632 36.5, 37.9).
 // Tiles of 256 rows take longer than estimated where there are two or three to a column: 0.84 (taken: 512 x 2,048 x 8,192 38.0, 33.7; 512 x 4,096 x 16,384
 // 110.3, 90.2; left: 512 x 7,168 x 7,168 75.3, 86.7; 512 x 8,192 x 8,192 87.8, 103.4; 512 x 5,120 x 5,120 50.7, 53.6) and 0.82 (taken: 640 x 2,048 x
 // 16,384 84.0, 62.8; left: 704 x 4,096 x 8,192 69.1, 84.6; 768 x 5,120 x 13,824 124.6, 138.2).

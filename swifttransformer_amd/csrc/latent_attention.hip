@@ -650,7 +650,8 @@ __global__ __launch_bounds__(256) void latent_up_rows_kernel(
 // The same numbers where a head's matrix fits the registers (up to 32 VR values and 8 VEC DR entries) and the splits a wave: weights, partial results,
 // their log-sum-exps and gates are asked for before anything waits, and every wave weighs the splits for itself.  What bounds it is trips to memory
 // one after the other, of which the kernel above has eight.  us a call, cold matrices, above and so: 24 tokens of 32 heads of 128 x 128 6.15, 5.22, one
-// of them 6.6, 5.35, 64 8.9, 8.3; eight of 16 heads of 64 x 96 4.5, 3.2; 48 of 32 heads of 64 x 64 5.2, 4.7.
+// of them 6.6, 5.35, 64 8.9, 8.3; eight of 16 heads of 64 x 96 4.5, 3.2; 48 of 32 heads of 64 x 64 5.2, 4.7.  (Waves past the entries ask for no more
+// splits than the first eight: 64 tokens of 32 heads of 64 x 64, 40 splits 8.3 above, 9.6 with them, 7.8 so.)
 template <typename T, int VR, int DR>
 __global__ __launch_bounds__(256) void latent_up_few_kernel(
     T* __restrict__ y, const float* __restrict__ part_o, const float* __restrict__ part_lse, const T* __restrict__ w,
@@ -686,7 +687,8 @@ __global__ __launch_bounds__(256) void latent_up_few_kernel(
     const float e = lane < splits && M > -INFINITY ? expf(lse - M) : 0.f;
     const float W = wave_sum(e), weight = W > 0.f ? e / W : 0.f;
     float o = 0.f;
-    for (int s0 = 0; s0 < splits; s0 += B) {
+    const int mine = __builtin_amdgcn_readfirstlane(tid) < out_dim ? splits : 0;          // (waves past the entries have none to sum)
+    for (int s0 = 0; s0 < mine; s0 += B) {
         if (s0) load(s0);
 #pragma unroll
         for (int u = 0; u < B; ++u)

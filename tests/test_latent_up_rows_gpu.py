@@ -10,7 +10,7 @@ DEV = "cuda:0"
 
 
 # values, entries, splits: up to 128, 128 and 64 are one kernel's, the rest the other's
-@pytest.mark.parametrize("vd,od,splits", [(1, 16, 1), (33, 112, 8), (96, 80, 9), (128, 128, 16), (128, 128, 64), (128, 128, 65), (129, 128, 3), (64, 144, 5)])
+@pytest.mark.parametrize("vd,od,splits", [(1, 16, 1), (33, 112, 8), (96, 80, 9), (128, 128, 16), (128, 128, 64), (128, 128, 65), (129, 128, 3), (64, 144, 5), (64, 48, 40), (80, 64, 17)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_splits_product_and_gate(vd, od, splits, dtype):
     g = torch.Generator().manual_seed(vd * 100 + od + splits)
