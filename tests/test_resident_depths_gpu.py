@@ -51,8 +51,8 @@ def seconds(x, ws):
 
 
 def test_a_shallow_product_takes_less_than_a_deep_one():
-    """A quarter of the depth leaves twelve of the sixteen waves without a step: half of the time where they ask for no weights (3.2 us of 6.5),
-    four fifths where they do."""
+    """A quarter of the depth leaves twelve of the sixteen waves without a step.  Where they ask for no weights it takes 0.54 to 0.56 of the time
+    (3.4 us of 6.1, 16 runs on two cards), where they ask for the first step again 0.88 to 0.89 (5.6 of 6.4, 8 runs): the line is in the middle."""
     rows, features = 16, 5120
     took = {depth: seconds(draw(1, rows, depth).bfloat16(), [draw(i, features, depth, scale=0.05).bfloat16() for i in range(24)]) for depth in (256, 1024)}
-    assert took[256] < 0.65 * took[1024], took
+    assert took[256] < 0.72 * took[1024], took
